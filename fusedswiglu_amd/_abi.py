@@ -20,6 +20,8 @@ DTYPE_BF16 = 0
 DTYPE_FP16 = 1
 #: OR-ed into a dtype code (or a workspace step): weights are stored "out x in" like nn.Linear.weight
 WEIGHTS_OUT_IN = 0x100
+#: OR-ed into a dtype code: rows are padded to a multiple of 8 elements (FSW_ROWS_PADDED)
+ROWS_PADDED = 0x400
 STEP_DOWN_FORWARD, STEP_DOWN_INPUT_GRAD, STEP_DOWN_WEIGHT_GRAD = 4, 5, 6
 
 STEP_FORWARD, STEP_INPUT_GRAD, STEP_WEIGHT_GRAD = 0, 1, 2
@@ -37,6 +39,8 @@ EXPORTED_SYMBOLS = (
     "fsw_workspace_bytes",
     "fsw_swiglu_forward",
     "fsw_elementwise_backward",
+    "fsw_elementwise_backward_rows",
+    "fsw_repack_rows",
     "fsw_gating_grad_recompute",
     "fsw_input_grad",
     "fsw_input_grad_noalloc",
@@ -108,6 +112,10 @@ def lib() -> ctypes.CDLL:
         L.fsw_swiglu_forward.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, ci, vp]
         L.fsw_elementwise_backward.restype = ci
         L.fsw_elementwise_backward.argtypes = [vp, vp, vp, vp, vp, i64, ci, vp]
+        L.fsw_elementwise_backward_rows.restype = ci
+        L.fsw_elementwise_backward_rows.argtypes = [vp] * 5 + [i64] * 5 + [ci, vp]
+        L.fsw_repack_rows.restype = ci
+        L.fsw_repack_rows.argtypes = [vp] * 4 + [i64] * 4 + [ci, vp]
         L.fsw_gating_grad_recompute.restype = ci
         L.fsw_gating_grad_recompute.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, ci, vp]
         L.fsw_input_grad.restype = ci

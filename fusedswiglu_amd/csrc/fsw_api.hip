@@ -21,10 +21,11 @@ int fail(int code, const char* fmt, ...) {
 // `dtype` arguments carry the element type in the low byte and optional FSW_* layout flags above it
 bool dtype_ok(int d) {
   const int e = d & 0xff;
-  return (e == FSW_DTYPE_BF16 || e == FSW_DTYPE_FP16) && (d & ~(0xff | FSW_WEIGHTS_OUT_IN)) == 0;
+  return (e == FSW_DTYPE_BF16 || e == FSW_DTYPE_FP16) && (d & ~(0xff | FSW_WEIGHTS_OUT_IN | FSW_ROWS_PADDED)) == 0;
 }
 int elem_of(int d) { return d & 0xff; }
 bool out_in_of(int d) { return (d & FSW_WEIGHTS_OUT_IN) != 0; }
+bool padded_of(int d) { return (d & FSW_ROWS_PADDED) != 0; }
 bool al2(const void* p) { return ((uintptr_t)p & 1) == 0; }
 
 int check_dims(const char* fn, int64_t T, int64_t D, int64_t I) {
@@ -37,11 +38,19 @@ int check_dims(const char* fn, int64_t T, int64_t D, int64_t I) {
   return FSW_OK;
 }
 
-int check_ld(const char* fn, const char* name, int64_t ld, int64_t cols) {
+// `padded`: rows reach up to the next multiple of 8 elements
+int check_ld(const char* fn, const char* name, int64_t ld, int64_t cols, bool padded = false) {
+  if (padded) cols = (cols + 7) & ~(int64_t)7;
   if (ld < cols)
     return fail(FSW_ERR_BAD_STRIDE, "%s: leading dimension %s=%lld is smaller than the row length %lld",
                 fn, name, (long long)ld, (long long)cols);
   return FSW_OK;
+}
+
+// What FSW_ROWS_PADDED promises (aligned pointers and row pitches) is not there: the edge-shape kernel does not keep the
+// padding of results, so the call is refused.
+int not_padded(const char* fn) {
+  return fail(FSW_ERR_ALIGNMENT, "%s: FSW_ROWS_PADDED needs 16-byte aligned pointers and leading dimensions that are multiples of 8 (below 2^21)", fn);
 }
 
 int launched(const char* fn, hipError_t e) {
@@ -89,7 +98,7 @@ int fsw_uses_tiled_kernel(int step, int64_t T, int64_t D, int64_t I, int64_t ldx
   }
   // the down projection: y, grad_y [T,D] (ldx)   w_down (ldw)   act, grad_act [T,I] (ldo)   grad_w_down (ld_grad)
   const bool oi = p.w_out_in;
-  fsw::GemmProblem q{ptr, ptr, (void*)ptr, 0, 0, 0, 0, 0, 0, 0};
+  fsw::GemmProblem q{ptr, ptr, (void*)ptr, 0, 0, 0, 0, 0, 0, 0, false};
   switch (step & 0xff) {
     case 4: q.M = T; q.N = D; q.K = I; q.lda = ldo; q.ldb = ldw; q.ldc = ldx; q.layout = oi ? 1 : 0; break;
     case 5: q.M = T; q.N = I; q.K = D; q.lda = ldx; q.ldb = ldw; q.ldc = ldo; q.layout = oi ? 0 : 1; break;
@@ -127,19 +136,20 @@ int fsw_swiglu_forward(const void* x, const void* w_gate, const void* w_up, void
     return fail(FSW_ERR_NULL_POINTER, "%s: xw_gate and xw_up must both be given or both be null", fn);
   if (!dtype_ok(dtype)) return fail(FSW_ERR_BAD_DTYPE, "%s: dtype %d is neither bf16 (0) nor fp16 (1)", fn, dtype);
   if (int e = check_dims(fn, T, D, I)) return e;
-  const bool oi = out_in_of(dtype);
+  const bool oi = out_in_of(dtype), padded = padded_of(dtype);
   dtype = elem_of(dtype);
-  if (int e = check_ld(fn, "ldx", ldx, D)) return e;
-  if (int e = check_ld(fn, "ldw", ldw, oi ? D : I)) return e;
-  if (int e = check_ld(fn, "ldo", ldo, I)) return e;
+  if (int e = check_ld(fn, "ldx", ldx, D, padded)) return e;
+  if (int e = check_ld(fn, "ldw", ldw, oi ? D : I, padded)) return e;
+  if (int e = check_ld(fn, "ldo", ldo, I, padded)) return e;
   if (!al2(x) || !al2(w_gate) || !al2(w_up) || !al2(out) || !al2(xw_gate) || !al2(xw_up))
     return fail(FSW_ERR_ALIGNMENT, "%s: pointers must be 2-byte aligned", fn);
   fsw::Problem p{};
   p.x = x; p.wg = w_gate; p.wu = w_up; p.out = out; p.g = xw_gate; p.u = xw_up;
-  p.T = T; p.D = D; p.I = I; p.ldx = ldx; p.ldw = ldw; p.ldo = ldo; p.w_out_in = oi;
+  p.T = T; p.D = D; p.I = I; p.ldx = ldx; p.ldw = ldw; p.ldo = ldo; p.w_out_in = oi; p.padded = padded;
   hipStream_t s = (hipStream_t)stream;
   if (fsw::skinny_forward_ok(p)) return launched(fn, fsw::launch_forward_skinny(dtype, p, s));
   if (fsw::fast_path_ok_forward(p)) return launched(fn, fsw::launch_forward_fast(dtype, p, s));
+  if (padded) return not_padded(fn);
   return launched(fn, fsw::launch_forward_generic(dtype, p, s));
 }
 
@@ -152,19 +162,51 @@ int fsw_gating_grad_recompute(const void* x, const void* w_gate, const void* w_u
     return fail(FSW_ERR_NULL_POINTER, "%s: all six arrays must be non-null", fn);
   if (!dtype_ok(dtype)) return fail(FSW_ERR_BAD_DTYPE, "%s: dtype %d is neither bf16 (0) nor fp16 (1)", fn, dtype);
   if (int e = check_dims(fn, T, D, I)) return e;
-  const bool oi = out_in_of(dtype);
+  const bool oi = out_in_of(dtype), padded = padded_of(dtype);
   dtype = elem_of(dtype);
-  if (int e = check_ld(fn, "ldx", ldx, D)) return e;
-  if (int e = check_ld(fn, "ldw", ldw, oi ? D : I)) return e;
-  if (int e = check_ld(fn, "ldo", ldo, I)) return e;
+  if (int e = check_ld(fn, "ldx", ldx, D, padded)) return e;
+  if (int e = check_ld(fn, "ldw", ldw, oi ? D : I, padded)) return e;
+  if (int e = check_ld(fn, "ldo", ldo, I, padded)) return e;
   if (!al2(x) || !al2(w_gate) || !al2(w_up) || !al2(grad_out) || !al2(grad_xw_up) || !al2(grad_xw_gate))
     return fail(FSW_ERR_ALIGNMENT, "%s: pointers must be 2-byte aligned", fn);
   fsw::Problem p{};
   p.x = x; p.wg = w_gate; p.wu = w_up; p.dout = grad_out; p.g = grad_xw_gate; p.u = grad_xw_up;
-  p.T = T; p.D = D; p.I = I; p.ldx = ldx; p.ldw = ldw; p.ldo = ldo; p.w_out_in = oi;
+  p.T = T; p.D = D; p.I = I; p.ldx = ldx; p.ldw = ldw; p.ldo = ldo; p.w_out_in = oi; p.padded = padded;
   hipStream_t s = (hipStream_t)stream;
   if (fsw::fast_path_ok_forward(p)) return launched(fn, fsw::launch_forward_fast(dtype, p, s));
+  if (padded) return not_padded(fn);
   return launched(fn, fsw::launch_forward_generic(dtype, p, s));
+}
+
+int fsw_repack_rows(const void* src0, void* dst0, const void* src1, void* dst1, int64_t rows, int64_t cols, int64_t ld_src,
+                    int64_t ld_dst, int pad, void* stream) {
+  const char* fn = "fsw_repack_rows";
+  if (!src0 || !dst0 || (src1 == nullptr) != (dst1 == nullptr))
+    return fail(FSW_ERR_NULL_POINTER, "%s: src0 and dst0 must be non-null, src1 and dst1 both given or both null", fn);
+  if (rows <= 0 || cols <= 0 || rows > 0x7fffffffLL || cols > 0x7fffffffLL - 8)
+    return fail(FSW_ERR_BAD_SHAPE, "%s: rows and columns must be positive and below 2^31 (rows=%lld cols=%lld)", fn, (long long)rows, (long long)cols);
+  if (int e = check_ld(fn, "ld_src", ld_src, cols)) return e;
+  if (int e = check_ld(fn, "ld_dst", ld_dst, cols, pad != 0)) return e;
+  if (!al2(src0) || !al2(dst0) || !al2(src1) || !al2(dst1)) return fail(FSW_ERR_ALIGNMENT, "%s: pointers must be 2-byte aligned", fn);
+  return launched(fn, fsw::launch_repack(src0, dst0, src1, dst1, rows, cols, ld_src, ld_dst, pad != 0, (hipStream_t)stream));
+}
+
+int fsw_elementwise_backward_rows(const void* grad_out, const void* xw_gate, const void* xw_up, void* grad_xw_up,
+                                  void* grad_xw_gate, int64_t T, int64_t I, int64_t ld_grad_out, int64_t ld_xw, int64_t ld_grad,
+                                  int dtype, void* stream) {
+  const char* fn = "fsw_elementwise_backward_rows";
+  if (!grad_out || !xw_gate || !xw_up || !grad_xw_up || !grad_xw_gate)
+    return fail(FSW_ERR_NULL_POINTER, "%s: all five arrays must be non-null", fn);
+  if (!dtype_ok(dtype)) return fail(FSW_ERR_BAD_DTYPE, "%s: dtype %d is neither bf16 (0) nor fp16 (1)", fn, dtype);
+  if (int e = check_dims(fn, T, I, I)) return e;
+  if (int e = check_ld(fn, "ld_grad_out", ld_grad_out, I)) return e;
+  if (int e = check_ld(fn, "ld_xw", ld_xw, I)) return e;
+  if (int e = check_ld(fn, "ld_grad", ld_grad, I, true)) return e;
+  if (!al2(grad_out) || !al2(xw_gate) || !al2(xw_up)) return fail(FSW_ERR_ALIGNMENT, "%s: pointers must be 2-byte aligned", fn);
+  if ((((uintptr_t)grad_xw_up | (uintptr_t)grad_xw_gate) & 15) || (ld_grad & 7))
+    return fail(FSW_ERR_ALIGNMENT, "%s: the rows of the results must be 16-byte aligned", fn);
+  return launched(fn, fsw::launch_elementwise_rows(elem_of(dtype), grad_out, ld_grad_out, xw_gate, xw_up, ld_xw, grad_xw_up,
+                                                   grad_xw_gate, ld_grad, T, I, (hipStream_t)stream));
 }
 
 int fsw_elementwise_backward(const void* grad_out, const void* xw_gate, const void* xw_up,
@@ -189,9 +231,10 @@ static int check_input_grad_args(const char* fn, const void* grad_xw_gate, const
     return fail(FSW_ERR_NULL_POINTER, "%s: all five arrays must be non-null", fn);
   if (!dtype_ok(dtype)) return fail(FSW_ERR_BAD_DTYPE, "%s: dtype %d is neither bf16 (0) nor fp16 (1)", fn, dtype);
   if (int e = check_dims(fn, T, D, I)) return e;
-  if (int e = check_ld(fn, "ldo", ldo, I)) return e;
-  if (int e = check_ld(fn, "ldw", ldw, out_in_of(dtype) ? D : I)) return e;
-  if (int e = check_ld(fn, "ld_dx", ld_dx, D)) return e;
+  const bool padded = padded_of(dtype);
+  if (int e = check_ld(fn, "ldo", ldo, I, padded)) return e;
+  if (int e = check_ld(fn, "ldw", ldw, out_in_of(dtype) ? D : I, padded)) return e;
+  if (int e = check_ld(fn, "ld_dx", ld_dx, D, padded)) return e;
   if (!al2(grad_xw_gate) || !al2(grad_xw_up) || !al2(w_gate) || !al2(w_up) || !al2(grad_x))
     return fail(FSW_ERR_ALIGNMENT, "%s: pointers must be 2-byte aligned", fn);
   return FSW_OK;
@@ -204,12 +247,14 @@ static int input_grad_checked(const char* fn, const void* grad_xw_gate, const vo
   fsw::Problem p{};
   p.dG = grad_xw_gate; p.dU = grad_xw_up; p.wg = w_gate; p.wu = w_up; p.dx = grad_x;
   p.T = T; p.D = D; p.I = I; p.ldo = ldo; p.ldw = ldw; p.lddx = ld_dx; p.w_out_in = out_in_of(dtype);
+  p.padded = padded_of(dtype);
   dtype = elem_of(dtype);
   hipStream_t s = (hipStream_t)stream;
   if (fsw::fast_path_ok_input_grad(p)) {
     const bool ws_ok = workspace && workspace_bytes > 0 && ((uintptr_t)workspace & 15) == 0;
     return launched(fn, fsw::launch_input_grad_fast(dtype, p, s, ws_ok ? workspace : nullptr, ws_ok ? workspace_bytes : 0));
   }
+  if (p.padded) return not_padded(fn);
   return launched(fn, fsw::launch_input_grad_generic(dtype, p, s));
 }
 
@@ -231,9 +276,10 @@ static int check_weight_grad_args(const char* fn, const void* x, const void* gra
     return fail(FSW_ERR_NULL_POINTER, "%s: all five arrays must be non-null", fn);
   if (!dtype_ok(dtype)) return fail(FSW_ERR_BAD_DTYPE, "%s: dtype %d is neither bf16 (0) nor fp16 (1)", fn, dtype);
   if (int e = check_dims(fn, T, D, I)) return e;
-  if (int e = check_ld(fn, "ldx", ldx, D)) return e;
-  if (int e = check_ld(fn, "ldo", ldo, I)) return e;
-  if (int e = check_ld(fn, "ld_dw", ld_dw, out_in_of(dtype) ? D : I)) return e;
+  const bool padded = padded_of(dtype);
+  if (int e = check_ld(fn, "ldx", ldx, D, padded)) return e;
+  if (int e = check_ld(fn, "ldo", ldo, I, padded)) return e;
+  if (int e = check_ld(fn, "ld_dw", ld_dw, out_in_of(dtype) ? D : I, padded)) return e;
   if (!al2(x) || !al2(grad_xw_up) || !al2(grad_xw_gate) || !al2(grad_w_up) || !al2(grad_w_gate))
     return fail(FSW_ERR_ALIGNMENT, "%s: pointers must be 2-byte aligned", fn);
   return FSW_OK;
@@ -246,16 +292,17 @@ int fsw_weight_grad(const void* x, const void* grad_xw_up, const void* grad_xw_g
   const char* fn = "fsw_weight_grad";
   if (int e = check_weight_grad_args(fn, x, grad_xw_up, grad_xw_gate, grad_w_up, grad_w_gate, T, D, I, ldx, ldo, ld_dw, dtype))
     return e;
-  const bool oi = out_in_of(dtype);
+  const bool oi = out_in_of(dtype), padded = padded_of(dtype);
   dtype = elem_of(dtype);
   fsw::Problem p{};
   p.x = x; p.dG = grad_xw_gate; p.dU = grad_xw_up; p.dWg = grad_w_gate; p.dWu = grad_w_up;
-  p.T = T; p.D = D; p.I = I; p.ldx = ldx; p.ldo = ldo; p.lddw = ld_dw; p.w_out_in = oi;
+  p.T = T; p.D = D; p.I = I; p.ldx = ldx; p.ldo = ldo; p.lddw = ld_dw; p.w_out_in = oi; p.padded = padded;
   hipStream_t s = (hipStream_t)stream;
   if (fsw::fast_path_ok_weight_grad(p)) {
     const bool ws_ok = workspace && workspace_bytes > 0 && ((uintptr_t)workspace & 15) == 0;
     return launched(fn, fsw::launch_weight_grad_fast(dtype, p, s, ws_ok ? workspace : nullptr, ws_ok ? workspace_bytes : 0));
   }
+  if (padded) return not_padded(fn);
   return launched(fn, fsw::launch_weight_grad_generic(dtype, p, s));
 }
 
@@ -276,22 +323,29 @@ int fsw_swiglu_backward(const void* grad_out, const void* xw_gate, const void* x
   if (int e = check_dims(fn, T, D, I)) return e;
   if (!al2(grad_out) || !al2(xw_gate) || !al2(xw_up))
     return fail(FSW_ERR_ALIGNMENT, "%s: pointers must be 2-byte aligned", fn);
+  const bool padded = padded_of(dtype);
+  const int64_t ldi = padded ? (I + 7) & ~(int64_t)7 : I;
   if (grad_x)
-    if (int e = check_input_grad_args(fn, grad_xw_gate, grad_xw_up, w_gate, w_up, grad_x, T, D, I, I, ldw, ld_dx, dtype))
+    if (int e = check_input_grad_args(fn, grad_xw_gate, grad_xw_up, w_gate, w_up, grad_x, T, D, I, ldi, ldw, ld_dx, dtype))
       return e;
   if (grad_w_gate)
-    if (int e = check_weight_grad_args(fn, x, grad_xw_up, grad_xw_gate, grad_w_up, grad_w_gate, T, D, I, ldx, I, ld_dw, dtype))
+    if (int e = check_weight_grad_args(fn, x, grad_xw_up, grad_xw_gate, grad_w_up, grad_w_gate, T, D, I, ldx, ldi, ld_dw, dtype))
       return e;
-  if (int e = fsw_elementwise_backward(grad_out, xw_gate, xw_up, grad_xw_up, grad_xw_gate, T * I, elem_of(dtype), stream))
+  if (padded) {
+    if (int e = fsw_elementwise_backward_rows(grad_out, xw_gate, xw_up, grad_xw_up, grad_xw_gate, T, I, I, ldi, ldi,
+                                              elem_of(dtype), stream))
+      return e;
+  } else if (int e = fsw_elementwise_backward(grad_out, xw_gate, xw_up, grad_xw_up, grad_xw_gate, T * I, elem_of(dtype), stream)) {
     return e;
+  }
   // the weight gradient first: measured at 8192 x 4096 x 12288, the input gradient runs 4 % faster behind it than
   // behind the gating-gradient kernel (its dG / dU operand is still in the memory-side cache), the step 0.3 % faster
   if (grad_w_gate)
-    if (int e = fsw_weight_grad(x, grad_xw_up, grad_xw_gate, grad_w_up, grad_w_gate, T, D, I, ldx, I, ld_dw, workspace,
+    if (int e = fsw_weight_grad(x, grad_xw_up, grad_xw_gate, grad_w_up, grad_w_gate, T, D, I, ldx, ldi, ld_dw, workspace,
                                 workspace_bytes, dtype, stream))
       return e;
   if (grad_x)
-    if (int e = fsw_input_grad(grad_xw_gate, grad_xw_up, w_gate, w_up, grad_x, T, D, I, I, ldw, ld_dx, workspace,
+    if (int e = fsw_input_grad(grad_xw_gate, grad_xw_up, w_gate, w_up, grad_x, T, D, I, ldi, ldw, ld_dx, workspace,
                                workspace_bytes, dtype, stream))
       return e;
   return FSW_OK;
@@ -301,7 +355,8 @@ int fsw_swiglu_backward(const void* grad_out, const void* xw_gate, const void* x
 static int run_gemm(const char* fn, int layout, const void* a, const void* b, void* c, int64_t M, int64_t N,
                     int64_t K, int64_t lda, int64_t ldb, int64_t ldc, void* workspace, int64_t workspace_bytes,
                     int dtype, void* stream) {
-  fsw::GemmProblem p{a, b, c, M, N, K, lda, ldb, ldc, layout};
+  fsw::GemmProblem p{a, b, c, M, N, K, lda, ldb, ldc, layout, padded_of(dtype)};
+  dtype = elem_of(dtype);
   hipStream_t s = (hipStream_t)stream;
   if (fsw::fast_path_ok_gemm(p)) {
     const bool ws_ok = workspace && workspace_bytes > 0 && ((uintptr_t)workspace & 15) == 0;
@@ -309,6 +364,7 @@ static int run_gemm(const char* fn, int layout, const void* a, const void* b, vo
       return launched(fn, fsw::launch_gemm_skinny(dtype, p, s, ws_ok ? workspace : nullptr, ws_ok ? workspace_bytes : 0));
     return launched(fn, fsw::launch_gemm_fast(dtype, p, s, ws_ok ? workspace : nullptr, ws_ok ? workspace_bytes : 0));
   }
+  if (p.padded) return not_padded(fn);
   return launched(fn, fsw::launch_gemm_generic(dtype, p, s));
 }
 
@@ -317,9 +373,10 @@ static int check_down_proj(const char* fn, const void* p0, const void* p1, const
   if (!p0 || !p1 || !p2) return fail(FSW_ERR_NULL_POINTER, "%s: all three arrays must be non-null", fn);
   if (!dtype_ok(dtype)) return fail(FSW_ERR_BAD_DTYPE, "%s: dtype %d is neither bf16 (0) nor fp16 (1)", fn, dtype);
   if (int e = check_dims(fn, T, D, I)) return e;
-  if (int e = check_ld(fn, "ld_act", ld_act, I)) return e;
-  if (int e = check_ld(fn, "ldw", ldw, out_in_of(dtype) ? I : D)) return e;
-  if (int e = check_ld(fn, "ldy", ldy, D)) return e;
+  const bool padded = padded_of(dtype);
+  if (int e = check_ld(fn, "ld_act", ld_act, I, padded)) return e;
+  if (int e = check_ld(fn, "ldw", ldw, out_in_of(dtype) ? I : D, padded)) return e;
+  if (int e = check_ld(fn, "ldy", ldy, D, padded)) return e;
   if (!al2(p0) || !al2(p1) || !al2(p2)) return fail(FSW_ERR_ALIGNMENT, "%s: pointers must be 2-byte aligned", fn);
   return FSW_OK;
 }
@@ -331,7 +388,7 @@ int fsw_down_proj_forward(const void* act, const void* w_down, void* y, int64_t 
   if (int e = check_down_proj(fn, act, w_down, y, T, I, D, ld_act, ldw, ldy, dtype)) return e;
   // y [T,D] = act [T,I] W_down [I,D]   (or act W_down^T for W_down [D,I])
   return run_gemm(fn, out_in_of(dtype) ? 1 : 0, act, w_down, y, T, D, I, ld_act, ldw, ldy, workspace, workspace_bytes,
-                  elem_of(dtype), stream);
+                  dtype, stream);
 }
 
 int fsw_down_proj_input_grad(const void* grad_y, const void* w_down, void* grad_act, int64_t T, int64_t I,
@@ -341,7 +398,7 @@ int fsw_down_proj_input_grad(const void* grad_y, const void* w_down, void* grad_
   if (int e = check_down_proj(fn, grad_y, w_down, grad_act, T, I, D, ld_act, ldw, ldy, dtype)) return e;
   // grad_act [T,I] = grad_y [T,D] W_down^T   (or grad_y W_down for W_down [D,I])
   return run_gemm(fn, out_in_of(dtype) ? 0 : 1, grad_y, w_down, grad_act, T, I, D, ldy, ldw, ld_act, workspace,
-                  workspace_bytes, elem_of(dtype), stream);
+                  workspace_bytes, dtype, stream);
 }
 
 int fsw_down_proj_weight_grad(const void* act, const void* grad_y, void* grad_w_down, int64_t T, int64_t I,
@@ -352,9 +409,9 @@ int fsw_down_proj_weight_grad(const void* act, const void* grad_y, void* grad_w_
   // grad_W_down [I,D] = act^T grad_y   (or [D,I] = grad_y^T act)
   if (out_in_of(dtype))
     return run_gemm(fn, 2, grad_y, act, grad_w_down, D, I, T, ldy, ld_act, ld_dw, workspace, workspace_bytes,
-                    elem_of(dtype), stream);
+                    dtype, stream);
   return run_gemm(fn, 2, act, grad_y, grad_w_down, I, D, T, ld_act, ldy, ld_dw, workspace, workspace_bytes,
-                  elem_of(dtype), stream);
+                  dtype, stream);
 }
 
 }  // extern "C"

@@ -68,4 +68,107 @@ hipError_t launch_elementwise(int dtype, const void* dout, const void* g, const 
                     : launch_elementwise_t<FP16>(dout, g, u, dU, dG, n, stream);
 }
 
+// ---- rows that are not 16-byte aligned -----------------------------------------------------------------------------
+// Eight elements at a 2-byte aligned address: one unaligned 16-byte access (the compiler knows the alignment).
+struct __attribute__((packed, aligned(2))) Chunk { u32x4 v; };
+FSW_DEV u32x4 load_chunk(const unsigned short* p, int left) {
+  if (left >= 8) return ((const Chunk*)p)->v;
+  u32x4 r{0, 0, 0, 0};
+  for (int e = 0; e < left; e++) r[e >> 1] |= (unsigned)p[e] << (16 * (e & 1));
+  return r;
+}
+FSW_DEV void store_chunk(unsigned short* p, u32x4 v, int left) {
+  if (left >= 8) {
+    ((Chunk*)p)->v = v;
+    return;
+  }
+  for (int e = 0; e < left; e++) p[e] = (unsigned short)(v[e >> 1] >> (16 * (e & 1)));
+}
+
+// One thread per 8 columns of a row; a workgroup takes 256 consecutive chunks of the (row, chunk) order, so short rows
+// fill it too.
+constexpr int kRowThreads = 256;
+FSW_DEV bool row_chunk(unsigned rows, unsigned chunks, long long& row, int& col) {
+  const unsigned i = blockIdx.x * (unsigned)kRowThreads + threadIdx.x;  // the host keeps rows * chunks below 2^31
+  const unsigned r = i / chunks;
+  row = r;
+  col = (int)(i - r * chunks) * 8;
+  return r < rows;
+}
+// Calls launch(first row, rows, blocks) for as many rows at a time as a launch can index.
+template <typename F>
+static hipError_t for_row_ranges(long long rows, long long chunks, F&& launch) {
+  const long long most = 0x7fffff00LL / chunks;
+  for (long long r = 0; r < rows; r += most) {
+    const long long n = rows - r < most ? rows - r : most;
+    launch(r, (unsigned)n, (unsigned)((n * chunks + kRowThreads - 1) / kRowThreads));
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+// Bound: HBM, 4 bytes per element (one read, one write); the unaligned side's accesses straddle a line now and then.
+__global__ __launch_bounds__(kRowThreads) void fsw_repack_kernel(const unsigned short* __restrict__ src0, unsigned short* __restrict__ dst0,
+                                                                 const unsigned short* __restrict__ src1, unsigned short* __restrict__ dst1,
+                                                                 unsigned rows, unsigned chunks, int cols, long long ld_src,
+                                                                 long long ld_dst, int pad) {
+  long long row;
+  int col;
+  if (!row_chunk(rows, chunks, row, col)) return;
+  const unsigned short* src = blockIdx.y ? src1 : src0;
+  unsigned short* dst = blockIdx.y ? dst1 : dst0;
+  const u32x4 v = load_chunk(src + row * ld_src + col, cols - col);
+  store_chunk(dst + row * ld_dst + col, v, pad ? 8 : cols - col);
+}
+
+hipError_t launch_repack(const void* src0, void* dst0, const void* src1, void* dst1, long long rows, long long cols,
+                         long long ld_src, long long ld_dst, bool pad, hipStream_t s) {
+  typedef const unsigned short* cus;
+  typedef unsigned short* us;
+  const long long chunks = (cols + 7) / 8;
+  return for_row_ranges(rows, chunks, [&](long long r, unsigned n, unsigned blocks) {
+    fsw_repack_kernel<<<dim3(blocks, src1 ? 2 : 1), kRowThreads, 0, s>>>(
+        (cus)src0 + r * ld_src, (us)dst0 + r * ld_dst, src1 ? (cus)src1 + r * ld_src : nullptr,
+        src1 ? (us)dst1 + r * ld_dst : nullptr, n, (unsigned)chunks, (int)cols, ld_src, ld_dst, pad);
+  });
+}
+
+// The gating gradient on rows: the upstream gradient dense as autograd delivers it, everything else padded.
+template <typename E>
+__global__ __launch_bounds__(kRowThreads) void elementwise_backward_rows_kernel(
+    const unsigned short* __restrict__ dout, long long ld_dout, const unsigned short* __restrict__ g,
+    const unsigned short* __restrict__ u, long long ld_gu, unsigned short* __restrict__ dU, unsigned short* __restrict__ dG,
+    long long ld_out, unsigned rows, unsigned chunks, int cols) {
+  long long row;
+  int col;
+  if (!row_chunk(rows, chunks, row, col)) return;
+  const int left = cols - col;
+  const u32x4 a = load_chunk(dout + row * ld_dout + col, left);
+  const u32x4 b = load_chunk(g + row * ld_gu + col, left);
+  const u32x4 c = load_chunk(u + row * ld_gu + col, left);
+  u32x4 ru, rg;  // zeros beyond the row: the loads are zero there
+#pragma unroll
+  for (int w = 0; w < 4; w++) {
+    float u0, g0, u1, g1;
+    gating_grad(E::to_float(a[w] & 0xffff), E::to_float(b[w] & 0xffff), E::to_float(c[w] & 0xffff), u0, g0);
+    gating_grad(E::to_float(a[w] >> 16), E::to_float(b[w] >> 16), E::to_float(c[w] >> 16), u1, g1);
+    ru[w] = E::pack2(u0, u1);
+    rg[w] = E::pack2(g0, g1);
+  }
+  *(u32x4*)(dU + row * ld_out + col) = ru;
+  *(u32x4*)(dG + row * ld_out + col) = rg;
+}
+
+hipError_t launch_elementwise_rows(int dtype, const void* dout, long long ld_dout, const void* g, const void* u, long long ld_gu,
+                                   void* dU, void* dG, long long ld_out, long long rows, long long cols, hipStream_t stream) {
+  typedef const unsigned short* cus;
+  typedef unsigned short* us;
+  const long long chunks = (cols + 7) / 8;
+  auto kernel = dtype == kDtypeBF16 ? elementwise_backward_rows_kernel<BF16> : elementwise_backward_rows_kernel<FP16>;
+  return for_row_ranges(rows, chunks, [&](long long r, unsigned n, unsigned blocks) {
+    kernel<<<blocks, kRowThreads, 0, stream>>>((cus)dout + r * ld_dout, ld_dout, (cus)g + r * ld_gu, (cus)u + r * ld_gu, ld_gu,
+                                               (us)dU + r * ld_out, (us)dG + r * ld_out, ld_out, n, (unsigned)chunks, (int)cols);
+  });
+}
+
 }  // namespace fsw

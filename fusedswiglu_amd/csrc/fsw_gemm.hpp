@@ -47,6 +47,9 @@ struct GemmParams {
   // dU = d0 * silu(g), dG = d0 * u * silu'(g) computed from the fp32 accumulators (d0 has ldc too)
   const void* d0;
   int M, N, K;     // result rows x columns (per result) and reduction length (per pass)
+  // rows of a k-contiguous B that exist.  Equal to N, except that N is rounded up to a multiple of 8 when the
+  // caller's rows are padded: the padding columns of a result are written (zeros), the rows of B are not there.
+  int n_rows_b;
   int lda, ldb, ldc;  // leading dimensions in elements
   int tiles_m, tiles_n, group_m;
   // split-K (every mode but the forwards, on small problems): `splits` workgroups per tile each reduce
@@ -415,8 +418,8 @@ __global__ __launch_bounds__(kThreads) void fsw_gemm_kernel(GemmParams p) {
   if constexpr (A_KC) kc_setup(ka, p.a0, C::kPasses == 2 ? p.a1 : p.a0, m0, p.M, p.K, p.lda, wave, lane);
   else if constexpr (C::kDualM) mc_setup(ma, p.a0, p.a1, p.a0, p.a1, m0, m0, p.M, p.K, p.lda, wave, lane);
   else mc_setup(ma, p.a0, p.a0, p.a0, p.a0, m0, m0 + 128, p.M, p.K, p.lda, wave, lane);
-  if constexpr (MODE == kFwdT) kc_setup_interleaved(kb, p.b0, p.b1, n0, p.N, p.K, p.ldb, wave, lane);
-  else if constexpr (B_KC) kc_setup(kb, p.b0, C::kPasses == 2 ? p.b1 : p.b0, n0, p.N, p.K, p.ldb, wave, lane);
+  if constexpr (MODE == kFwdT) kc_setup_interleaved(kb, p.b0, p.b1, n0, p.n_rows_b, p.K, p.ldb, wave, lane);
+  else if constexpr (B_KC) kc_setup(kb, p.b0, C::kPasses == 2 ? p.b1 : p.b0, n0, p.n_rows_b, p.K, p.ldb, wave, lane);
   else if constexpr (C::kDualN) mc_setup(mb, p.b0, p.b1, p.b0, p.b1, n0, n0, p.N, p.K, p.ldb, wave, lane);
   else mc_setup(mb, p.b0, p.b0, C::kPasses == 2 ? p.b1 : p.b0, C::kPasses == 2 ? p.b1 : p.b0, n0, n0 + 128, p.N, p.K,
                 p.ldb, wave, lane);

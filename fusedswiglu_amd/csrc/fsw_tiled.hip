@@ -11,9 +11,10 @@ static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 static bool ld_ok(long long ld) { return mult8(ld) && ld < (1LL << 21); }
 // leading dimension of a result: a wave addresses its up to 128 rows through 32-bit byte offsets from the first
 static bool ld_out_ok(long long ld) { return mult8(ld) && ld < (1LL << 23); }
+// With padded rows the dimensions are free: the last chunk of a row is loaded and stored whole.
 static bool dims_ok(const Problem& p) {
-  return mult8(p.D) && mult8(p.I) && p.T > 0 && p.T < (1LL << 31) && p.D < (1LL << 31) &&
-         p.I < (1LL << 31);
+  return ((mult8(p.D) && mult8(p.I)) || (p.padded && p.D > 0 && p.I > 0)) && p.T > 0 && p.T < (1LL << 31) &&
+         p.D < (1LL << 31) - 8 && p.I < (1LL << 31) - 8;
 }
 
 // With [I,D] weights the roles of D and I as contiguous index swap for the weight operands, but both must be
@@ -101,6 +102,7 @@ static int steps_of(int mode, long long K) {
 template <int MODE>
 static long long workspace_of(long long M, long long N, long long K, bool with_tail = true) {
   using C = Cfg<MODE>;
+  N = result_cols(N);
   const long long tiles = ((M + C::kTileM - 1) / C::kTileM) * ((N + C::kTileN - 1) / C::kTileN);
   const SplitPlan pl = plan_split_unbounded(tiles, steps_of(MODE, K), M, N, C::kResults);
   if (pl.splits > 1) return (long long)pl.splits * M * N * 4 * C::kResults;
@@ -202,7 +204,7 @@ static hipError_t launch(int dtype, GemmParams g, hipStream_t s, void* ws = null
 hipError_t launch_forward_fast(int dtype, const Problem& p, hipStream_t s) {
   GemmParams g{};
   g.a0 = p.x; g.b0 = p.wg; g.b1 = p.wu; g.c0 = p.out; g.c1 = p.g; g.c2 = p.u; g.d0 = p.dout;
-  g.M = (int)p.T; g.N = (int)p.I; g.K = (int)p.D;
+  g.M = (int)p.T; g.N = (int)result_cols(p.I); g.n_rows_b = (int)p.I; g.K = (int)p.D;
   g.lda = (int)p.ldx; g.ldb = (int)p.ldw; g.ldc = (int)p.ldo;
   return p.w_out_in ? launch<kFwdT>(dtype, g, s) : launch<kFwd>(dtype, g, s);
 }
@@ -210,7 +212,7 @@ hipError_t launch_forward_fast(int dtype, const Problem& p, hipStream_t s) {
 hipError_t launch_input_grad_fast(int dtype, const Problem& p, hipStream_t s, void* ws, long long ws_bytes) {
   GemmParams g{};
   g.a0 = p.dG; g.a1 = p.dU; g.b0 = p.wg; g.b1 = p.wu; g.c0 = p.dx;
-  g.M = (int)p.T; g.N = (int)p.D; g.K = (int)p.I;
+  g.M = (int)p.T; g.N = (int)result_cols(p.D); g.n_rows_b = (int)p.D; g.K = (int)p.I;
   g.lda = (int)p.ldo; g.ldb = (int)p.ldw; g.ldc = (int)p.lddx;
   return p.w_out_in ? launch<kDxT>(dtype, g, s, ws, ws_bytes) : launch<kDx>(dtype, g, s, ws, ws_bytes);
 }
@@ -219,27 +221,27 @@ hipError_t launch_weight_grad_fast(int dtype, const Problem& p, hipStream_t s, v
   GemmParams g{};
   if (p.w_out_in) {  // dWg [I,D] = dG^T x: the two results share the B tile (x)
     g.a0 = p.dG; g.a1 = p.dU; g.b0 = p.x; g.c0 = p.dWg; g.c1 = p.dWu;
-    g.M = (int)p.I; g.N = (int)p.D; g.K = (int)p.T;
+    g.M = (int)p.I; g.N = (int)result_cols(p.D); g.n_rows_b = (int)p.D; g.K = (int)p.T;
     g.lda = (int)p.ldo; g.ldb = (int)p.ldx; g.ldc = (int)p.lddw;
     return launch<kDwT>(dtype, g, s, ws, ws_bytes);
   }
   g.a0 = p.x; g.b0 = p.dG; g.b1 = p.dU; g.c0 = p.dWg; g.c1 = p.dWu;
-  g.M = (int)p.D; g.N = (int)p.I; g.K = (int)p.T;
+  g.M = (int)p.D; g.N = (int)result_cols(p.I); g.n_rows_b = (int)p.I; g.K = (int)p.T;
   g.lda = (int)p.ldx; g.ldb = (int)p.ldo; g.ldc = (int)p.lddw;
   return launch<kDw>(dtype, g, s, ws, ws_bytes);
 }
 
 bool fast_path_ok_gemm(const GemmProblem& p) {
-  return p.M > 0 && p.N > 0 && p.K > 0 && p.M < (1LL << 31) && p.N < (1LL << 31) && p.K < (1LL << 31) &&
-         // the contiguous index of each operand must be a multiple of 8 elements
-         mult8(p.layout == 2 ? p.M : p.K) && mult8(p.layout == 1 ? p.K : p.N) && mult8(p.N) &&
+  return p.M > 0 && p.N > 0 && p.K > 0 && p.M < (1LL << 31) - 8 && p.N < (1LL << 31) - 8 && p.K < (1LL << 31) - 8 &&
+         // the contiguous index of each operand must be a multiple of 8 elements, unless its rows are padded
+         (p.padded || (mult8(p.layout == 2 ? p.M : p.K) && mult8(p.layout == 1 ? p.K : p.N) && mult8(p.N))) &&
          ld_ok(p.lda) && ld_ok(p.ldb) && ld_out_ok(p.ldc) && al16(p.a) && al16(p.b) && al16(p.c);
 }
 
 hipError_t launch_gemm_fast(int dtype, const GemmProblem& p, hipStream_t s, void* ws, long long ws_bytes) {
   GemmParams g{};
   g.a0 = p.a; g.b0 = p.b; g.c0 = p.c;
-  g.M = (int)p.M; g.N = (int)p.N; g.K = (int)p.K;
+  g.M = (int)p.M; g.N = (int)result_cols(p.N); g.n_rows_b = (int)p.N; g.K = (int)p.K;
   g.lda = (int)p.lda; g.ldb = (int)p.ldb; g.ldc = (int)p.ldc;
   switch (p.layout) {
     case 0: return launch<kNN>(dtype, g, s, ws, ws_bytes);

@@ -96,8 +96,71 @@ def _ld(t2: torch.Tensor) -> int:
     return t2.stride(0) if t2.shape[0] > 1 else t2.shape[1]
 
 
-def _code(dtype: torch.dtype, weights_out_in: bool) -> int:
-    return _DTYPE_CODE[dtype] | (_abi.WEIGHTS_OUT_IN if weights_out_in else 0)
+def _code(dtype: torch.dtype, weights_out_in: bool, padded: bool = False) -> int:
+    return (_DTYPE_CODE[dtype] | (_abi.WEIGHTS_OUT_IN if weights_out_in else 0)
+            | (_abi.ROWS_PADDED if padded else 0))
+
+
+# ---- operands the tiled kernels cannot read as they are ---------------------------------------
+# Rows that are not whole 16-byte chunks (a dimension that is not a multiple of 8) or do not start on 16-byte
+# boundaries are copied once into padded rows; the padded results are copied back.  Each copy moves an array once in
+# each direction; the kernels behind it run at 10 to 30 times the rate of the edge-shape kernel (a training step of 2048
+# tokens, 1024 x 2730, bf16: 1716 us on the edge-shape kernel, 237 us on padded copies).  Below this many multiply-adds per
+# matrix product the edge-shape kernel's fewer launches win: forward / backward at 2^21.5 33 / 56 against 46 / 75 us, at
+# 2^23.5 38 / 79 against 46 / 76, at 2^24.5 39 / 100 against 46 / 77, at 2^25.2 69 / 224 against 46 / 77.
+_PAD_MIN_WORK = 1 << 24
+
+
+def _pad8(n: int) -> int:
+    return (n + 7) & ~7
+
+
+def _whole_chunks(t2: torch.Tensor) -> bool:
+    return not (t2.shape[1] & 7 or _ld(t2) & 7 or t2.data_ptr() & 15)
+
+
+def _repack(src: torch.Tensor, dst: torch.Tensor, cols: int, pad: bool, src1: Optional[torch.Tensor] = None,
+            dst1: Optional[torch.Tensor] = None) -> None:
+    """Copies `cols` columns of every row between row pitches (one or two arrays of the same shape and pitch)."""
+    _abi.check(_abi.lib().fsw_repack_rows(
+        src.data_ptr(), dst.data_ptr(), src1.data_ptr() if src1 is not None else None,
+        dst1.data_ptr() if dst1 is not None else None, src.shape[0], cols, _ld(src), _ld(dst), int(pad),
+        _stream_ptr(src.device)))
+
+
+def _padded_copies(*ts: torch.Tensor) -> Tuple[torch.Tensor, ...]:
+    """[rows, cols] tensors (one, or two with the same shape and row pitch) as padded, aligned copies
+    [rows, cols rounded up to 8]; as they are when the tiled kernels can read them directly."""
+    if all(_whole_chunks(t) for t in ts):
+        return ts
+    rows, cols = ts[0].shape
+    out = tuple(torch.empty((rows, _pad8(cols)), device=t.device, dtype=t.dtype) for t in ts)
+    _repack(ts[0], out[0], cols, True, *((ts[1], out[1]) if len(ts) > 1 else ()))
+    return out
+
+
+def _padded_result(rows: int, cols: int, like: torch.Tensor) -> torch.Tensor:
+    return torch.empty((rows, _pad8(cols)), device=like.device, dtype=like.dtype)
+
+
+def _unpadded(t: torch.Tensor, cols: int) -> torch.Tensor:
+    """The dense [rows, cols] copy of a padded result (the result itself when it has no padding)."""
+    if t.shape[1] == cols:
+        return t
+    out = torch.empty((t.shape[0], cols), device=t.device, dtype=t.dtype)
+    _repack(t, out, cols, False)
+    return out
+
+
+def pads_rows(x: torch.Tensor, I: int) -> bool:
+    """Whether a problem with this x and dimensions that are not multiples of 8 runs on padded copies."""
+    return x.numel() * I >= _PAD_MIN_WORK
+
+
+def _wants_padding(T: int, D: int, I: int, *ts: torch.Tensor) -> bool:
+    if T * D * I < _PAD_MIN_WORK:
+        return False
+    return bool((D | I) & 7) or not all(_whole_chunks(t) for t in ts)
 
 
 def _weight_dims(w: torch.Tensor, weights_out_in: bool) -> Tuple[int, int]:
@@ -130,26 +193,58 @@ def fused_swiglu_fwd(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, 
         wg, wu = wg.contiguous(), wu.contiguous()
     T = x2.shape[0]
     out_shape = tuple(x.shape[:-1]) + (I,)
+    px, pg, pu, ldx, ldw = x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), _ld(x2), _ld(wg)
+    if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and T * D * I >= _PAD_MIN_WORK:
+        return _padded_fwd(x2, wg, wu, dtype, out_shape, D, I, save_preactivations, weights_out_in)
     out = torch.empty(out_shape, device=dev, dtype=dtype)
     g = torch.empty_like(out) if save_preactivations else None
     u = torch.empty_like(out) if save_preactivations else None
     with _on_device(dev):
         _abi.check(_abi.lib().fsw_swiglu_forward(
+            px, pg, pu, out.data_ptr(), g.data_ptr() if g is not None else None, u.data_ptr() if u is not None else None,
+            T, D, I, ldx, ldw, I, _code(dtype, weights_out_in), _stream_ptr(dev)))
+    return out, g, u
+
+
+def _padded_fwd(x2, wg, wu, dtype, out_shape, D, I, save_preactivations, weights_out_in):
+    """fused_swiglu_fwd on padded copies.  The pre-activations stay padded: views of [T, I rounded up to 8]."""
+    T, dev = x2.shape[0], x2.device
+    with _on_device(dev):
+        (x2,), (wg, wu) = _padded_copies(x2), _padded_copies(wg, wu)
+        out = _padded_result(T, I, x2)
+        g, u = (torch.empty_like(out), torch.empty_like(out)) if save_preactivations else (None, None)
+        _abi.check(_abi.lib().fsw_swiglu_forward(
             x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), out.data_ptr(),
             g.data_ptr() if g is not None else None, u.data_ptr() if u is not None else None,
-            T, D, I, _ld(x2), _ld(wg), I, _code(dtype, weights_out_in), _stream_ptr(dev)))
+            T, D, I, _ld(x2), _ld(wg), _pad8(I), _code(dtype, weights_out_in, True), _stream_ptr(dev)))
+        out = _unpadded(out, I).view(out_shape)
+    if g is not None:
+        wide = out_shape[:-1] + (_pad8(I),)
+        g, u = g.view(wide)[..., :I], u.view(wide)[..., :I]
     return out, g, u
 
 
 def elementwise_backward(grad_output: torch.Tensor, xw_gate: torch.Tensor, xw_up: torch.Tensor,
-                         dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Returns (grad_xw_up, grad_xw_gate) -- the reference's order (kernels_bf16.py:255)."""
+                         dtype: torch.dtype, padded: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Returns (grad_xw_up, grad_xw_gate) -- the reference's order (kernels_bf16.py:255).  With `padded`, as
+    [tokens, I rounded up to 8] arrays whose last columns are zeros: what the gradient GEMMs take as they are."""
     _require(grad_output.shape == xw_gate.shape == xw_up.shape,
              "grad_output, xw_gate and xw_up must have the same shape")
     _require(grad_output.dtype == dtype and xw_gate.dtype == dtype and xw_up.dtype == dtype,
              f"Expected {dtype} tensors")
     dev = _check_device(grad_output, xw_gate, xw_up)
     _require(grad_output.numel() > 0, "empty input")
+    if padded:
+        dout, g, u = _rows(grad_output), _rows(xw_gate), _rows(xw_up)
+        if _ld(g) != _ld(u):
+            g, u = g.contiguous(), u.contiguous()
+        T, I = dout.shape
+        grad_xw_up, grad_xw_gate = _padded_result(T, I, dout), _padded_result(T, I, dout)
+        with _on_device(dev):
+            _abi.check(_abi.lib().fsw_elementwise_backward_rows(
+                dout.data_ptr(), g.data_ptr(), u.data_ptr(), grad_xw_up.data_ptr(), grad_xw_gate.data_ptr(), T, I,
+                _ld(dout), _ld(g), _pad8(I), _DTYPE_CODE[dtype], _stream_ptr(dev)))
+        return grad_xw_up, grad_xw_gate
     # the kernel indexes flat, dense arrays (the reference silently assumes this, :224-226)
     dout, g, u = grad_output.contiguous(), xw_gate.contiguous(), xw_up.contiguous()
     grad_xw_up = torch.empty_like(dout)
@@ -163,7 +258,7 @@ def elementwise_backward(grad_output: torch.Tensor, xw_gate: torch.Tensor, xw_up
 
 def gating_grad_recompute(grad_output: torch.Tensor, x: torch.Tensor, w_gate: torch.Tensor,
                           w_up: torch.Tensor, dtype: torch.dtype,
-                          weights_out_in: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
+                          weights_out_in: bool = False, padded: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
     """(grad_xw_up, grad_xw_gate) like elementwise_backward, but from x and the weights: the
     pre-activations x@w_gate and x@w_up are recomputed in fp32 inside the kernel and never stored.
     For backward passes that did not save them (fused_swiglu/swiglu.py:28 saves them always)."""
@@ -182,6 +277,21 @@ def gating_grad_recompute(grad_output: torch.Tensor, x: torch.Tensor, w_gate: to
     x2, wg, wu = _rows(x), _rows(w_gate), _rows(w_up)
     if _ld(wg) != _ld(wu):
         wg, wu = wg.contiguous(), wu.contiguous()
+    T = x2.shape[0]
+    dout = _rows(grad_output)
+    if padded or _wants_padding(T, D, I, x2, wg, wu, dout):
+        with _on_device(dev):
+            (x2,), (wg, wu), (dout,) = _padded_copies(x2), _padded_copies(wg, wu), _padded_copies(dout)
+            if _ld(dout) != _pad8(I):
+                dout = dout.contiguous()
+            grad_xw_up, grad_xw_gate = _padded_result(T, I, dout), _padded_result(T, I, dout)
+            _abi.check(_abi.lib().fsw_gating_grad_recompute(
+                x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), dout.data_ptr(), grad_xw_up.data_ptr(),
+                grad_xw_gate.data_ptr(), T, D, I, _ld(x2), _ld(wg), _pad8(I), _code(dtype, weights_out_in, True),
+                _stream_ptr(dev)))
+            if not padded:
+                grad_xw_up, grad_xw_gate = (_unpadded(t, I).view(grad_output.shape) for t in (grad_xw_up, grad_xw_gate))
+        return grad_xw_up, grad_xw_gate
     dout = grad_output.contiguous()
     grad_xw_up = torch.empty_like(dout)
     grad_xw_gate = torch.empty_like(dout)
@@ -193,14 +303,46 @@ def gating_grad_recompute(grad_output: torch.Tensor, x: torch.Tensor, w_gate: to
     return grad_xw_up, grad_xw_gate
 
 
+def _padded_input_grad(dg, du, wg, wu, dtype, D, I, weights_out_in) -> torch.Tensor:
+    """Dense [T, D] input gradient from operands with padded rows (current device: theirs)."""
+    T, dev = dg.shape[0], dg.device
+    grad_x = _padded_result(T, D, dg)
+    ws, ws_bytes = _workspace(_abi.STEP_INPUT_GRAD | (_abi.WEIGHTS_OUT_IN if weights_out_in else 0), T, D, I, dev)
+    _abi.check(_abi.lib().fsw_input_grad(
+        dg.data_ptr(), du.data_ptr(), wg.data_ptr(), wu.data_ptr(), grad_x.data_ptr(),
+        T, D, I, _ld(dg), _ld(wg), _pad8(D), ws.data_ptr() if ws is not None else None, ws_bytes,
+        _code(dtype, weights_out_in, True), _stream_ptr(dev)))
+    return _unpadded(grad_x, D)
+
+
+def _padded_weight_grad(x2, du, dg, dtype, D, I, weights_out_in, out=None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(grad_w_up, grad_w_gate) from operands with padded rows, dense or in the two arrays of `out`."""
+    T, dev = x2.shape[0], x2.device
+    rows, cols = (I, D) if weights_out_in else (D, I)
+    grad_w_up, grad_w_gate = _padded_result(rows, cols, x2), _padded_result(rows, cols, x2)
+    ws, ws_bytes = _workspace(_abi.STEP_WEIGHT_GRAD | (_abi.WEIGHTS_OUT_IN if weights_out_in else 0), T, D, I, dev)
+    _abi.check(_abi.lib().fsw_weight_grad(
+        x2.data_ptr(), du.data_ptr(), dg.data_ptr(), grad_w_up.data_ptr(), grad_w_gate.data_ptr(),
+        T, D, I, _ld(x2), _ld(du), _pad8(cols), ws.data_ptr() if ws is not None else None, ws_bytes,
+        _code(dtype, weights_out_in, True), _stream_ptr(dev)))
+    if out is None:
+        if cols % 8 == 0:
+            return grad_w_up, grad_w_gate
+        out = tuple(torch.empty((rows, cols), device=dev, dtype=dtype) for _ in range(2))
+    _repack(grad_w_up, out[0], cols, False, grad_w_gate, out[1])
+    return out
+
+
 def fused_input_grad(grad_xw_gate: torch.Tensor, grad_xw_up: torch.Tensor, w_gate: torch.Tensor,
-                     w_up: torch.Tensor, dtype: torch.dtype, weights_out_in: bool = False) -> torch.Tensor:
-    """grad_x = grad_xw_gate @ w_gate.T + grad_xw_up @ w_up.T in one kernel (swiglu.py:45)."""
+                     w_up: torch.Tensor, dtype: torch.dtype, weights_out_in: bool = False,
+                     padded: bool = False) -> torch.Tensor:
+    """grad_x = grad_xw_gate @ w_gate.T + grad_xw_up @ w_up.T in one kernel (swiglu.py:45).  `padded`: the two
+    gradients are [tokens, I rounded up to 8] as elementwise_backward(padded=True) returns them."""
     _require(grad_xw_gate.shape == grad_xw_up.shape, "gate/up gradient shapes differ")
     _require(w_gate.ndim == 2 and w_gate.shape == w_up.shape,
              "Expected both weight matrices to have same shape")
     D, I = _weight_dims(w_gate, weights_out_in)
-    _require(grad_xw_gate.shape[-1] == I, "Dimension mismatch between gradients and weights")
+    _require(grad_xw_gate.shape[-1] == (_pad8(I) if padded else I), "Dimension mismatch between gradients and weights")
     _require(all(t.dtype == dtype for t in (grad_xw_gate, grad_xw_up, w_gate, w_up)),
              f"Expected {dtype} tensors")
     dev = _check_device(grad_xw_gate, grad_xw_up, w_gate, w_up)
@@ -210,6 +352,11 @@ def fused_input_grad(grad_xw_gate: torch.Tensor, grad_xw_up: torch.Tensor, w_gat
     if _ld(wg) != _ld(wu):
         wg, wu = wg.contiguous(), wu.contiguous()
     T = dg.shape[0]
+    if padded or _wants_padding(T, D, I, dg, du, wg, wu):
+        with _on_device(dev):
+            dg, du = (dg, du) if padded else _padded_copies(dg, du)
+            grad_x = _padded_input_grad(dg, du, *_padded_copies(wg, wu), dtype, D, I, weights_out_in)
+        return grad_x.view(tuple(grad_xw_gate.shape[:-1]) + (D,))
     grad_x = torch.empty(tuple(grad_xw_gate.shape[:-1]) + (D,), device=dev, dtype=dtype)
     with _on_device(dev):
         flag = _abi.WEIGHTS_OUT_IN if weights_out_in else 0
@@ -245,9 +392,21 @@ def swiglu_backward(grad_output: torch.Tensor, x: torch.Tensor, w_gate: torch.Te
     x2, wg, wu = _rows(x), _rows(w_gate), _rows(w_up)
     if _ld(wg) != _ld(wu):
         wg, wu = wg.contiguous(), wu.contiguous()
+    T = x2.shape[0]
+    px, pg, pu, ldx, ldw = x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), _ld(x2), _ld(wg)
+    if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and T * D * I >= _PAD_MIN_WORK:
+        grad_xw_up, grad_xw_gate = elementwise_backward(grad_output, xw_gate, xw_up, dtype, padded=True)
+        grad_w_up = grad_w_gate = grad_x = None
+        if need_weight_grad or need_input_grad:
+            with _on_device(dev):
+                (x2,), (wg, wu) = _padded_copies(x2), _padded_copies(wg, wu)
+        if need_weight_grad:
+            grad_w_up, grad_w_gate = _padded_weight_grad(x2, grad_xw_up, grad_xw_gate, dtype, D, I, weights_out_in)
+        if need_input_grad:
+            grad_x = _padded_input_grad(grad_xw_gate, grad_xw_up, wg, wu, dtype, D, I, weights_out_in).view(x.shape)
+        return grad_x, grad_w_gate, grad_w_up
     # the gating gradient indexes flat, dense arrays
     dout, g, u = grad_output.contiguous(), xw_gate.contiguous(), xw_up.contiguous()
-    T = x2.shape[0]
     grad_xw_gate, grad_xw_up = torch.empty_like(dout), torch.empty_like(dout)
     grad_x = torch.empty(x.shape, device=dev, dtype=dtype) if need_input_grad else None
     grad_w_gate = torch.empty(w_gate.shape, device=dev, dtype=dtype) if need_weight_grad else None
@@ -260,25 +419,26 @@ def swiglu_backward(grad_output: torch.Tensor, x: torch.Tensor, w_gate: torch.Te
         ws = torch.empty(nbytes, device=dev, dtype=torch.uint8) if nbytes > 0 else None
         ld_dw = w_gate.shape[1]
         _abi.check(L.fsw_swiglu_backward(
-            dout.data_ptr(), g.data_ptr(), u.data_ptr(), x2.data_ptr(), wg.data_ptr(), wu.data_ptr(),
+            dout.data_ptr(), g.data_ptr(), u.data_ptr(), px, pg, pu,
             grad_xw_gate.data_ptr(), grad_xw_up.data_ptr(), grad_x.data_ptr() if need_input_grad else None,
             grad_w_gate.data_ptr() if need_weight_grad else None, grad_w_up.data_ptr() if need_weight_grad else None,
-            T, D, I, _ld(x2), _ld(wg), D, ld_dw, ws.data_ptr() if ws is not None else None, nbytes,
+            T, D, I, ldx, ldw, D, ld_dw, ws.data_ptr() if ws is not None else None, nbytes,
             _code(dtype, weights_out_in), _stream_ptr(dev)))
     return grad_x, grad_w_gate, grad_w_up
 
 
 def fused_weight_grad(x: torch.Tensor, grad_xw_up: torch.Tensor, grad_xw_gate: torch.Tensor,
                       dtype: torch.dtype,
-                      out: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
-                      weights_out_in: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
+                      out: Optional[Tuple[torch.Tensor, torch.Tensor]] = None, weights_out_in: bool = False,
+                      padded_from: Optional[int] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     """(grad_w_up, grad_w_gate) = (x^T grad_xw_up, x^T grad_xw_gate), each [D, I], reduced over
     every token in fp32.  Same argument and return order as fused_bmm (kernels_bf16.py:385-412),
     with the batch sum of swiglu.py:56-57 folded in.  `out` = (grad_w_up, grad_w_gate) lets the
     caller supply the two result arrays, e.g. the halves of one packed [D, 2I] gradient; they must
-    have unit inner stride and the same row stride."""
+    have unit inner stride and the same row stride.  `padded_from` = I: the two gradients are [tokens, I rounded
+    up to 8] as elementwise_backward(padded=True) returns them."""
     _require(grad_xw_up.shape == grad_xw_gate.shape, "gate/up gradient shapes differ")
-    _require(x.shape[:-1] == grad_xw_up.shape[:-1],
+    _require(x.numel() // x.shape[-1] == grad_xw_up.shape[0] if padded_from else x.shape[:-1] == grad_xw_up.shape[:-1],
              f"Dimension mismatch. x {tuple(x.shape)} vs gradients {tuple(grad_xw_up.shape)}")
     _require(all(t.dtype == dtype for t in (x, grad_xw_up, grad_xw_gate)), f"Expected {dtype} tensors")
     dev = _check_device(x, grad_xw_up, grad_xw_gate)
@@ -286,8 +446,14 @@ def fused_weight_grad(x: torch.Tensor, grad_xw_up: torch.Tensor, grad_xw_gate: t
     if _ld(dg) != _ld(du):
         dg, du = dg.contiguous(), du.contiguous()
     T, D = x2.shape
-    I = du.shape[1]
+    I = padded_from or du.shape[1]
     wshape = (I, D) if weights_out_in else (D, I)
+    pad = bool(padded_from) or _wants_padding(T, D, I, x2, du, dg) or (
+        out is not None and T * D * I >= _PAD_MIN_WORK and not all(_whole_chunks(t) for t in out))
+    if pad and out is None:
+        with _on_device(dev):
+            (x2,), (du, dg) = _padded_copies(x2), (du, dg) if padded_from else _padded_copies(du, dg)
+            return _padded_weight_grad(x2, du, dg, dtype, D, I, weights_out_in)
     if out is None:
         grad_w_up = torch.empty(wshape, device=dev, dtype=dtype)
         grad_w_gate = torch.empty(wshape, device=dev, dtype=dtype)
@@ -300,6 +466,10 @@ def fused_weight_grad(x: torch.Tensor, grad_xw_up: torch.Tensor, grad_xw_gate: t
         _require(grad_w_up.stride(-1) == 1 and grad_w_gate.stride(-1) == 1 and _ld(grad_w_up) == _ld(grad_w_gate)
                  and _ld(grad_w_up) >= wshape[1],
                  "weight-gradient outputs need unit inner stride and equal row strides")
+        if pad:
+            with _on_device(dev):
+                (x2,), (du, dg) = _padded_copies(x2), (du, dg) if padded_from else _padded_copies(du, dg)
+                return _padded_weight_grad(x2, du, dg, dtype, D, I, weights_out_in, out=(grad_w_up, grad_w_gate))
     with _on_device(dev):
         flag = _abi.WEIGHTS_OUT_IN if weights_out_in else 0
         ws, ws_bytes = _workspace(_abi.STEP_WEIGHT_GRAD | flag, T, D, I, dev)
@@ -326,14 +496,18 @@ def down_proj_forward(act: torch.Tensor, w_down: torch.Tensor, dtype: torch.dtyp
     _require(act.numel() > 0 and D > 0, "empty input")
     a2, w2 = _rows(act), _rows(w_down)
     T = a2.shape[0]
-    y = torch.empty(tuple(act.shape[:-1]) + (D,), device=dev, dtype=dtype)
+    shape = tuple(act.shape[:-1]) + (D,)
     flag = _abi.WEIGHTS_OUT_IN if weights_out_in else 0
+    pad = _wants_padding(T, D, I, a2, w2)
     with _on_device(dev):
+        if pad:
+            (a2,), (w2,) = _padded_copies(a2), _padded_copies(w2)
+        y = _padded_result(T, D, a2) if pad else torch.empty(shape, device=dev, dtype=dtype)
         ws, ws_bytes = _workspace(_abi.STEP_DOWN_FORWARD | flag, T, D, I, dev)
         _abi.check(_abi.lib().fsw_down_proj_forward(
-            a2.data_ptr(), w2.data_ptr(), y.data_ptr(), T, I, D, _ld(a2), _ld(w2), D,
-            ws.data_ptr() if ws is not None else None, ws_bytes, _code(dtype, weights_out_in), _stream_ptr(dev)))
-    return y
+            a2.data_ptr(), w2.data_ptr(), y.data_ptr(), T, I, D, _ld(a2), _ld(w2), _pad8(D) if pad else D,
+            ws.data_ptr() if ws is not None else None, ws_bytes, _code(dtype, weights_out_in, pad), _stream_ptr(dev)))
+        return _unpadded(y, D).view(shape) if pad else y
 
 
 def down_proj_input_grad(grad_y: torch.Tensor, w_down: torch.Tensor, dtype: torch.dtype,
@@ -345,14 +519,18 @@ def down_proj_input_grad(grad_y: torch.Tensor, w_down: torch.Tensor, dtype: torc
     dev = _check_device(grad_y, w_down)
     g2, w2 = _rows(grad_y), _rows(w_down)
     T = g2.shape[0]
-    grad_act = torch.empty(tuple(grad_y.shape[:-1]) + (I,), device=dev, dtype=dtype)
+    shape = tuple(grad_y.shape[:-1]) + (I,)
     flag = _abi.WEIGHTS_OUT_IN if weights_out_in else 0
+    pad = _wants_padding(T, D, I, g2, w2)
     with _on_device(dev):
+        if pad:
+            (g2,), (w2,) = _padded_copies(g2), _padded_copies(w2)
+        grad_act = _padded_result(T, I, g2) if pad else torch.empty(shape, device=dev, dtype=dtype)
         ws, ws_bytes = _workspace(_abi.STEP_DOWN_INPUT_GRAD | flag, T, D, I, dev)
         _abi.check(_abi.lib().fsw_down_proj_input_grad(
-            g2.data_ptr(), w2.data_ptr(), grad_act.data_ptr(), T, I, D, _ld(g2), _ld(w2), I,
-            ws.data_ptr() if ws is not None else None, ws_bytes, _code(dtype, weights_out_in), _stream_ptr(dev)))
-    return grad_act
+            g2.data_ptr(), w2.data_ptr(), grad_act.data_ptr(), T, I, D, _ld(g2), _ld(w2), _pad8(I) if pad else I,
+            ws.data_ptr() if ws is not None else None, ws_bytes, _code(dtype, weights_out_in, pad), _stream_ptr(dev)))
+        return _unpadded(grad_act, I).view(shape) if pad else grad_act
 
 
 def down_proj_weight_grad(act: torch.Tensor, grad_y: torch.Tensor, dtype: torch.dtype,
@@ -364,14 +542,18 @@ def down_proj_weight_grad(act: torch.Tensor, grad_y: torch.Tensor, dtype: torch.
     a2, g2 = _rows(act), _rows(grad_y)
     T, I = a2.shape
     D = g2.shape[1]
-    grad_w = torch.empty((D, I) if weights_out_in else (I, D), device=dev, dtype=dtype)
+    rows, cols = (D, I) if weights_out_in else (I, D)
     flag = _abi.WEIGHTS_OUT_IN if weights_out_in else 0
+    pad = _wants_padding(T, D, I, a2, g2)
     with _on_device(dev):
+        if pad:
+            (a2,), (g2,) = _padded_copies(a2), _padded_copies(g2)
+        grad_w = torch.empty((rows, _pad8(cols) if pad else cols), device=dev, dtype=dtype)
         ws, ws_bytes = _workspace(_abi.STEP_DOWN_WEIGHT_GRAD | flag, T, D, I, dev)
         _abi.check(_abi.lib().fsw_down_proj_weight_grad(
             a2.data_ptr(), g2.data_ptr(), grad_w.data_ptr(), T, I, D, _ld(a2), _ld(g2), grad_w.shape[1],
-            ws.data_ptr() if ws is not None else None, ws_bytes, _code(dtype, weights_out_in), _stream_ptr(dev)))
-    return grad_w
+            ws.data_ptr() if ws is not None else None, ws_bytes, _code(dtype, weights_out_in, pad), _stream_ptr(dev)))
+        return _unpadded(grad_w, cols) if pad else grad_w
 
 
 def fused_bmm(x_t: torch.Tensor, grad_xw_up: torch.Tensor, grad_xw_gate: torch.Tensor,

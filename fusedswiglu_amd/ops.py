@@ -90,29 +90,35 @@ def swiglu_backward(grad_out: Tensor, x: Tensor, w_gate: Tensor, w_up: Tensor, x
         dx, dw_gate, dw_up = _launch.swiglu_backward(grad_out, x, w_gate, w_up, xw_gate, xw_up, dtype, need_input_grad=need_x,
                                                      need_weight_grad=need_w_gate or need_w_up, weights_out_in=oi)
         return (dx if dx is not None else e, dw_gate if need_w_gate else e.clone(), dw_up if need_w_up else e.clone())
+    # rows of I elements that are not whole 16-byte chunks stay padded between the steps of the backward
+    I = w_gate.shape[0 if oi else 1]
+    padded = bool(I & 7) and _launch.pads_rows(x, I)
     if xw_gate.numel() == 0:
-        d_up, d_gate = _launch.gating_grad_recompute(grad_out, x, w_gate, w_up, dtype, weights_out_in=oi)
+        d_up, d_gate = _launch.gating_grad_recompute(grad_out, x, w_gate, w_up, dtype, weights_out_in=oi, padded=padded)
     else:
-        d_up, d_gate = _launch.elementwise_backward(grad_out, xw_gate, xw_up, dtype)
+        d_up, d_gate = _launch.elementwise_backward(grad_out, xw_gate, xw_up, dtype, padded=padded)
+    padded_from = I if padded else None
     dx = dw_gate = dw_up = None
     # the weight gradient first: the input gradient then finds d_gate and d_up in the memory-side cache
     if need_w_gate or need_w_up:
         if packed and oi:
             I, D = w_gate.shape
             dw_gate = torch.empty((2 * I, D), device=x.device, dtype=dtype)
-            _launch.fused_weight_grad(x, d_up, d_gate, dtype, out=(dw_gate[I:], dw_gate[:I]), weights_out_in=True)
+            _launch.fused_weight_grad(x, d_up, d_gate, dtype, out=(dw_gate[I:], dw_gate[:I]), weights_out_in=True,
+                                      padded_from=padded_from)
         elif packed:
             D, I = w_gate.shape
             dw_gate = torch.empty((D, 2 * I), device=x.device, dtype=dtype)
-            _launch.fused_weight_grad(x, d_up, d_gate, dtype, out=(dw_gate[:, I:], dw_gate[:, :I]))
+            _launch.fused_weight_grad(x, d_up, d_gate, dtype, out=(dw_gate[:, I:], dw_gate[:, :I]),
+                                      padded_from=padded_from)
         else:
-            dw_up, dw_gate = _launch.fused_weight_grad(x, d_up, d_gate, dtype, weights_out_in=oi)
+            dw_up, dw_gate = _launch.fused_weight_grad(x, d_up, d_gate, dtype, weights_out_in=oi, padded_from=padded_from)
             if not need_w_gate:
                 dw_gate = None
             if not need_w_up:
                 dw_up = None
     if need_x:
-        dx = _launch.fused_input_grad(d_gate, d_up, w_gate, w_up, dtype, weights_out_in=oi)
+        dx = _launch.fused_input_grad(d_gate, d_up, w_gate, w_up, dtype, weights_out_in=oi, padded=padded).view(x.shape)
     return (dx if dx is not None else e, dw_gate if dw_gate is not None else e.clone(),
             dw_up if dw_up is not None else e.clone())
 

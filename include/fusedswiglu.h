@@ -24,8 +24,9 @@
  *   - Return value: FSW_OK or an FSW_ERR_* code; arguments are validated before anything is
  *     enqueued.  fsw_last_error() gives a thread-local message for the last failure.
  *   - Operands whose dimensions and leading dimensions are multiples of 8 elements and whose
- *     pointers are 16-byte aligned run on the tiled direct-to-LDS MFMA kernels; anything else
- *     runs on a slower edge-shape kernel with identical arithmetic.
+ *     pointers are 16-byte aligned run on the tiled direct-to-LDS MFMA kernels, and so does any
+ *     dimension whose rows are padded (FSW_ROWS_PADDED); anything else runs on a much slower
+ *     edge-shape kernel with identical arithmetic.  fsw_repack_rows pads and unpads rows.
  */
 #ifndef FUSEDSWIGLU_H_
 #define FUSEDSWIGLU_H_
@@ -57,6 +58,13 @@ enum { FSW_DTYPE_BF16 = 0, FSW_DTYPE_FP16 = 1 };
  * transposed in memory: other variants of the tiled kernels and of the weight-streaming kernel (T <= 128) read
  * and write the layout in place. */
 #define FSW_WEIGHTS_OUT_IN 0x100
+
+/* May be OR-ed into the `dtype` of every entry point that takes leading dimensions and of fsw_swiglu_backward: D and I
+ * need not be multiples of 8, but every row of every 16-bit array of the call has room for the next multiple of 8
+ * elements - zeros in inputs; in results the kernels write zeros there - every leading dimension is a multiple of 8
+ * (below 2^21) and every pointer is 16-byte aligned (else FSW_ERR_ALIGNMENT).  The exception is grad_out of
+ * fsw_swiglu_backward, which stays dense, [T,I] with leading dimension I. */
+#define FSW_ROWS_PADDED 0x400
 
 enum {
   FSW_OK = 0,
@@ -106,6 +114,22 @@ FSW_API int fsw_swiglu_forward(const void* x, const void* w_gate, const void* w_
 FSW_API int fsw_elementwise_backward(const void* grad_out, const void* xw_gate, const void* xw_up,
                              void* grad_xw_up, void* grad_xw_gate, int64_t numel, int dtype,
                              void* stream);
+
+/*
+ * The same on rows of any alignment: grad_out (ld_grad_out), xw_gate, xw_up (ld_xw) -> grad_xw_up, grad_xw_gate (ld_grad,
+ * a multiple of 8, 16-byte aligned rows whose columns up to the next multiple of 8 are set to zero, as FSW_ROWS_PADDED
+ * wants its inputs).
+ */
+FSW_API int fsw_elementwise_backward_rows(const void* grad_out, const void* xw_gate, const void* xw_up, void* grad_xw_up,
+                                          void* grad_xw_gate, int64_t T, int64_t I, int64_t ld_grad_out, int64_t ld_xw,
+                                          int64_t ld_grad, int dtype, void* stream);
+
+/*
+ * Copies the rows of one or two (src1, dst1 may be NULL) 16-bit arrays [rows, cols] from row pitch ld_src to row pitch
+ * ld_dst; any alignment.  pad != 0: the columns up to the next multiple of 8 are set to zero in the destination.
+ */
+FSW_API int fsw_repack_rows(const void* src0, void* dst0, const void* src1, void* dst1, int64_t rows, int64_t cols,
+                            int64_t ld_src, int64_t ld_dst, int pad, void* stream);
 
 /*
  * Gating gradient without saved pre-activations: recomputes g = x Wg and u = x Wu (fp32, never
