@@ -12,7 +12,13 @@
 //   kDxT   dx  = dG Wg + dU Wu             B = Wg | Wu [I,D] (n-contiguous), two passes
 //   kDwT   dWg = dG^T x, dWu = dU^T x      A = dG | dU [T,I] (m-contiguous), B = x [T,D] (n-contiguous)
 //
-// One workgroup = 8 wavefronts (4 along M x 2 along N) = one 256 x 256 fp32 accumulator tile (in the dual
+// What both forms of the tiled kernel share - modes, parameters, LDS formats, fragment reads, epilogue - and the
+// eight-wave form.  The four-wave form (fsw_gemm4.hpp) runs everything it can address: with the same tile it is as fast
+// or faster at every reduction length (8192 tokens, forward / dx / dW: 102 / 93 / 103 -> 97 / 79 / 97 us at 1024 x 3072,
+// 38 / 43 / 45 -> 36 / 35 / 40 at 512 x 1536, in part from its lower tiles).  The eight-wave form is left for operands
+// that span 2^31 bytes or more along the reduction.
+//
+// Eight-wave form: one workgroup = 8 wavefronts (4 along M x 2 along N) = one 256 x 256 fp32 accumulator tile (in the dual
 // modes 256 rows x 128 columns of EACH of the two results sharing the A tile; kDwT: 128 rows of each result
 // sharing the B tile).
 // The reduction advances 32 elements per step and is organised in PAIRS of steps.  Operand tiles are
@@ -216,7 +222,7 @@ FSW_DEV void static_for(F&& f) {
 // ---- the epilogue of both forms of the tiled kernel: rounding, silu(g) * u or the gating gradients, and whole
 // 128-byte lines to memory.
 //
-// A wave holds 32*NQ rows x 128 columns of accumulators: acc[nb][mb][r] of lane l is the wave's row
+// A wave holds 16*MB rows x 128 columns of accumulators: acc[nb][mb][r] of lane l is the wave's row
 // mb*16 + (l & 15) and, within the wave's half h = nb >> 2, column (nb & 3)*16 + 4*(l >> 4) + r of 64 consecutive
 // result columns (128 bytes).  Half h goes to result res_half[h] (0: c0, 1: c1) at columns col_half[h]..; in the
 // forwards the two halves are gate and up of the same 64 columns col_half[0].
@@ -232,10 +238,12 @@ FSW_DEV void static_for(F&& f) {
 // ACC_ASM: the accumulators live in the accumulation registers behind inline-asm MFMAs (four-wave form); they are
 // then moved out by explicit instructions at their turn and not earlier (left to the compiler, they are moved out
 // wholesale after the main loop and spill).
-template <typename E, int MODE, int NQ, bool ACC_ASM>
-FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][2 * NQ], FSW_LDS char* patch, int lane, int row_base,
+template <typename E, int MODE, int MB, bool ACC_ASM>
+FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][MB], FSW_LDS char* patch, int lane, int row_base,
                         int col_half0, int col_half1, int res_half0, int res_half1) {
   using C = Cfg<MODE>;
+  constexpr int NQ = (MB + 1) / 2;                                        // groups of 32 rows,
+  auto blocks_of = [](int q) constexpr { return 2 * q + 1 < MB ? 2 : 1; };  // the last one of 16 when MB is odd
   constexpr int kPatchPitch = 128, kPatchBytes = 32 * kPatchPitch;
   const int wr_row = (lane & 15) * kPatchPitch, wr_swz = (lane >> 1) & 7, wr_grp = lane >> 4;
   // 8 bytes of column group wr_grp of 16-column block c:  chunk 2c + (wr_grp >> 1), half wr_grp & 1
@@ -247,7 +255,7 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][2 * NQ], FSW_LDS ch
     const int row = 8 * i + (lane >> 3);
     return row * kPatchPitch + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
   };
-  const int rows_left = p.M - row_base;             // rows of this wave that exist (may be <= 0 or >= 32*NQ)
+  const int rows_left = p.M - row_base;             // rows of this wave that exist (may be <= 0 or >= 16*MB)
   const unsigned ldc_bytes = (unsigned)p.ldc * 2u;  // the host keeps 128 rows of a result below 2^31 bytes
   // a result seen from the wave's first row and column `col_base`
   auto result_rsrc = [&](const void* base, int col_base) {
@@ -257,14 +265,14 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][2 * NQ], FSW_LDS ch
   // line store i of a part: lane l holds chunk l & 7 of row 8*i + (l >> 3) of the part's 32 rows
   const unsigned st_lane = (unsigned)(lane >> 3) * ldc_bytes + (unsigned)(lane & 7) * 16u;
   u32x4 in_flight[4];
-  auto read_part = [&](int k) {
+  auto read_part = [&](int k, int q) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) in_flight[i] = *(const FSW_LDS u32x4*)(patch + (k & 1) * kPatchBytes + rd_off(i));
+    for (int i = 0; i < 2 * blocks_of(q); i++) in_flight[i] = *(const FSW_LDS u32x4*)(patch + (k & 1) * kPatchBytes + rd_off(i));
   };
   // st_cols: st_lane, or the out-of-range offset in lanes whose columns do not exist
   auto store_part = [&](__amdgpu_buffer_rsrc_t rs, unsigned st_cols, int q) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < 2 * blocks_of(q); i++) {
       const int r0 = q * 32 + 8 * i;
       // The row offset goes through the vector offset, not the scalar one: behind a 16-byte store with a scalar
       // offset REGISTER the compiler leaves out the wait state before the next instruction that overwrites the
@@ -311,7 +319,7 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][2 * NQ], FSW_LDS ch
         constexpr int k = decltype(kc)::value, q = k / count, which = first + k % count;
         if constexpr (k % count == 0) {
 #pragma unroll
-          for (int mbl = 0; mbl < 2; mbl++)
+          for (int mbl = 0; mbl < blocks_of(q); mbl++)
 #pragma unroll
             for (int c = 0; c < 4; c++) {
               gq[mbl][c] = acc_read4(acc[c][2 * q + mbl]);
@@ -319,7 +327,7 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][2 * NQ], FSW_LDS ch
             }
           if constexpr (gating) {
 #pragma unroll
-            for (int mbl = 0; mbl < 2; mbl++)
+            for (int mbl = 0; mbl < blocks_of(q); mbl++)
 #pragma unroll
               for (int c = 0; c < 4; c++) {
                 const int r0 = (2 * q + mbl) * 16;
@@ -328,9 +336,9 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][2 * NQ], FSW_LDS ch
               }
           }
         }
-        if constexpr (k > 0) read_part(k - 1);
+        if constexpr (k > 0) read_part(k - 1, (k - 1) / count);
 #pragma unroll
-        for (int mbl = 0; mbl < 2; mbl++)
+        for (int mbl = 0; mbl < blocks_of(q); mbl++)
 #pragma unroll
           for (int c = 0; c < 4; c++) {
             const f32x4 g = gq[mbl][c], u = uq[mbl][c];
@@ -350,7 +358,7 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][2 * NQ], FSW_LDS ch
           }
         if constexpr (k > 0) store_part(rs[first + (k - 1) % count], st_cols, (k - 1) / count);
       });
-      read_part(NQ * count - 1);
+      read_part(NQ * count - 1, NQ - 1);
       store_part(rs[first + count - 1], st_cols, NQ - 1);
     };
     if (p.d0 != nullptr) forward_tile(std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{});
@@ -366,11 +374,14 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][2 * NQ], FSW_LDS ch
       if constexpr (ACC_ASM) {
         // (one result per half: pinning the registers costs a copy, which two or three tiles per launch do not feel)
 #pragma unroll
-        for (int c = 0; c < 4; c++) asm volatile("" : "+a"(acc[4 * h + c][2 * q]), "+a"(acc[4 * h + c][2 * q + 1]));
+        for (int c = 0; c < 4; c++) {
+          asm volatile("" : "+a"(acc[4 * h + c][2 * q]));
+          if constexpr (blocks_of(q) > 1) asm volatile("" : "+a"(acc[4 * h + c][2 * q + 1]));
+        }
       }
-      if constexpr (k > 0) read_part(k - 1);
+      if constexpr (k > 0) read_part(k - 1, (k - 1) >> 1);
 #pragma unroll
-      for (int mbl = 0; mbl < 2; mbl++)
+      for (int mbl = 0; mbl < blocks_of(q); mbl++)
 #pragma unroll
         for (int c = 0; c < 4; c++) {
           const f32x4 t = acc[4 * h + c][2 * q + mbl];
@@ -378,7 +389,7 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][2 * NQ], FSW_LDS ch
         }
       if constexpr (k > 0) store_part(rs[(k - 1) & 1], st_cols[(k - 1) & 1], (k - 1) >> 1);
     });
-    read_part(2 * NQ - 1);
+    read_part(2 * NQ - 1, NQ - 1);
     store_part(rs[1], st_cols[1], NQ - 1);
   }
 }
@@ -592,7 +603,7 @@ __global__ __launch_bounds__(kThreads) void fsw_gemm_kernel(GemmParams p) {
     }
     return;
   }
-  store_tile<E, MODE, 2, false>(p, acc, (FSW_LDS char*)smem + wave * (2 * 32 * 128), lane, row_base, col_of_half(0),
+  store_tile<E, MODE, 4, false>(p, acc, (FSW_LDS char*)smem + wave * (2 * 32 * 128), lane, row_base, col_of_half(0),
                                 col_of_half(1), result_of_half(0), result_of_half(1));
 }
 

@@ -1,26 +1,32 @@
-// Four-wave form of the tiled MFMA kernel (same modes, operands, LDS formats and rings as fsw_gemm.hpp).
+// Four-wave form of the tiled MFMA kernel (same modes, operands and LDS formats as fsw_gemm.hpp).
 //
-// One workgroup = 4 wavefronts, ONE per SIMD (2 along M x 2 along N), each owning a 128 x 128 block of the
-// 256 x 256 fp32 accumulator tile: 256 accumulator registers per lane, 8 + 8 operand fragments per 32-element
-// step for 64 MFMAs.  Against the eight-wave form (64 x 128 per wave, 4 + 8 fragments for 32 MFMAs) a step
+// One workgroup = 4 wavefronts, ONE per SIMD (2 along M x 2 along N), each owning a 16 MB x 128 block of the
+// 32 MB x 256 fp32 accumulator tile, MB = 8 down to 4: a tile has 256, 224, 192, 160 or 128 rows (plan() in
+// fsw_tiled.hpp chooses).  At MB = 8 that is 256 accumulator registers per lane, 8 + 8 operand fragments per
+// 32-element step for 64 MFMAs.  Against the eight-wave form (64 x 128 per wave, 4 + 8 fragments for 32 MFMAs) a step
 // reads 64 instead of 96 KiB of LDS per workgroup - the matrix cores are power limited with real data, and
 // LDS traffic is the largest part of what a GEMM adds to the MFMAs themselves.
+// A lower tile costs more per row: all CUs at work, a step takes 0.72 us at MB = 8, 0.65, 0.59, 0.50 and 0.435 at
+// MB = 7 .. 4 (forward); below that the loads of B (16 KiB a step whatever MB is) would bound it - tiles of 128 rows made
+// of 32 x 128 or of K-split 64 x 128 wave tiles in the eight-wave form take 0.63 .. 0.73 of a whole tile's time, their
+// loads alone 0.5 us a step.
 //
 // With a single wave per SIMD nothing hides a bubble in that wave's instruction stream, so the main loop is
-// written out MFMA by MFMA: after each of the 128 MFMAs of a pair of steps there is one "gap" that holds at
+// written out MFMA by MFMA: after each of the 16 MB MFMAs of a pair of steps there is one "gap" that holds at
 // most a few other instructions, and nothing is allowed to move between gaps.  What a gap can hold for free was
 // measured with one wave per SIMD issuing 16x16x32 MFMAs back to back (16 cycles each): one scalar instruction
 // (every further one costs 8 cycles), two vector ALU instructions, one LDS read (two behind the same MFMA cost
 // 17 cycles), or one direct-to-LDS load (about 12 cycles in any case).  Per pair p (steps 2p and 2p+1, fragment
-// register sets 0 and 1):
-//   gaps   0.. 14   the A stream moves on to pair p+2, one or two scalar instructions per gap
-//   gaps  15.. 58   the 8 loads of A(p+2) (ring slot of pair p-1, released at the last barrier), one per 6 gaps
+// register sets 0 and 1), at MB = 8 (the others keep the order and close up):
+//   gaps   0.. 14   the A stream moves on to its next pair, one or two scalar instructions per gap
+//   gaps  15.. 58   the 8 loads of that pair of A (ring slot of pair p-1, released at the last barrier), one per 6 gaps
 //   gaps  16.. 47   fragment reads of step 2p+1 into set 1, one LDS instruction per gap
-//   gaps  46.. 60   the B stream moves on to pair p+2
-//   gap   64        s_waitcnt vmcnt(8) lgkmcnt(0); s_barrier: pair p+1 has landed for every wave, and every
+//   gaps  46.. 60   the B stream moves on to its next pair
+//   gap   64        s_waitcnt vmcnt(n) lgkmcnt(0); s_barrier: pair p+1 has landed for every wave, and every
 //                   wave has finished reading pair p out of LDS
-//   gaps  66..109   the 8 loads of B(p+2) into pair p's B space
+//   gaps  66..109   the 8 loads of that pair of B into pair p's B space
 //   gaps  80..111   fragment reads of step 2p+2 into set 0
+// The rings are 3 pairs of A and 2 of B deep at MB >= 6, 4 and 3 at MB = 4 (Rings4).
 #pragma once
 #include <utility>
 
@@ -92,16 +98,17 @@ FSW_DEV void kc4_setup(Loader4& L, const void* p0, const void* p1, int row0, int
   L.records[0] = L.records[1] = records_of(((long long)rows_total - row0 - 1) * ld * 2 + (((long long)K + 7) & ~7LL) * 2);
 }
 
+// panel_cols: columns of each panel that the tile has (the others of its 128 are not fetched)
 FSW_DEV void mc4_setup(Loader4& L, const void* p_panel0, const void* p_panel1, const void* q_panel0,
                        const void* q_panel1, int col0_panel0, int col0_panel1, int cols_total, int K, int ld,
-                       int wave, int lane) {
+                       int wave, int lane, int panel_cols = 128) {
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int row = 4 * wave + 16 * (j & 1) + (lane >> 4);
     // physical 16-byte chunk (lane & 15) of k-row `row` holds logical columns `col`.. (see read_frag_mc16)
     const int col = (((lane >> 2) & 3) ^ (row & 3)) * 32 + ((((lane >> 1) ^ (row >> 3)) & 1) * 16) + (lane & 1) * 8;
     const int col0 = (j >> 1) ? col0_panel1 : col0_panel0;
-    L.voff[j] = (col0 + col < cols_total) ? (unsigned)row * (unsigned)ld * 2u + col * 2u : kOobOffset;
+    L.voff[j] = (col0 + col < cols_total && col < panel_cols) ? (unsigned)row * (unsigned)ld * 2u + col * 2u : kOobOffset;
     L.voff[4 + j] = L.voff[j];
     if (j < 2) L.klim[j] = K - row;
   }
@@ -118,13 +125,32 @@ FSW_DEV void mc4_setup(Loader4& L, const void* p_panel0, const void* p_panel1, c
   if (col0_panel1 >= cols_total) L.records[1] = 0;
 }
 
-template <typename E, int MODE, bool STREAM_B = false>
+// LDS rings, in pairs of steps.  A pair of B takes 32 KiB; a tile of fewer rows leaves room for a third one, and needs it:
+// its pairs are shorter, and a load of B issued into the space of the pair just read has one pair's time less to arrive
+// than the ring is deep.  With 3 + 2 pairs at every MB a weight gradient of 8192 x 1024 x 3072 whose operands are not
+// cached took 147 us (MB = 4), with 4 + 3 it takes 123; a training step of that size 342 -> 322 us, 8192 x 512 x 1536
+// 142 -> 134, 2048 x 1024 x 2736 122 -> 117.
+template <int LOADS_A>
+struct Rings4 {
+  static constexpr int kAreaA = LOADS_A * 4096, kAreaB = kKcAreaBytes;
+  static constexpr int kLds = 160 * 1024;
+  static constexpr int kPairsB = 3 * (kAreaA + kAreaB) <= kLds ? 3 : 2;
+  static constexpr int kPairsA = kPairsB == 3 && 4 * kAreaA + 3 * kAreaB <= kLds ? 4 : 3;
+  static constexpr int kBytesA = kPairsA * kAreaA, kBytesB = kPairsB * kAreaB;
+  static_assert(kBytesA + kBytesB <= kLds, "LDS");
+};
+
+template <typename E, int MODE, int MB = 8, bool STREAM_B = false>
 __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
   using C = Cfg<MODE>;
-  __shared__ __attribute__((aligned(1024))) char smem[C::kBytesA + C::kBytesB];
   constexpr bool A_KC = C::kAKc, B_KC = C::kBKc;
   constexpr bool B_INTER = (MODE == kFwdT);
-  constexpr int TM = C::kTileM, TN = C::kTileN;
+  constexpr int TM = C::kTileM * MB / 8, TN = C::kTileN;
+  // An m-contiguous A of 128 columns fits one panel; otherwise each wave row has a panel (kDwT: a result) of its own.
+  constexpr bool kOnePanelA = !A_KC && !C::kDualM && MB == 4;
+  constexpr int kLdA = A_KC || kOnePanelA ? MB : 8, kLdB = 8;  // load instructions (4 KiB of the workgroup) per wave and pair
+  using R = Rings4<kLdA>;
+  __shared__ __attribute__((aligned(1024))) char smem[R::kBytesA + R::kBytesB];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -149,12 +175,13 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
   const int kt_total = C::kForward ? kt_all : min(in_tail ? p.tail_steps : p.steps_per_split, kt_all - kbase);
 
   const unsigned smem_a = (unsigned)(uintptr_t)(FSW_LDS char*)smem;
-  const unsigned smem_b = smem_a + C::kBytesA;
+  const unsigned smem_b = smem_a + R::kBytesA;
 
   Loader4 la, lb;
   if constexpr (A_KC) kc4_setup(la, p.a0, C::kPasses == 2 ? p.a1 : p.a0, m0, p.M, p.K, p.lda, wave, lane, false);
-  else if constexpr (C::kDualM) mc4_setup(la, p.a0, p.a1, p.a0, p.a1, m0, m0, p.M, p.K, p.lda, wave, lane);
-  else mc4_setup(la, p.a0, p.a0, p.a0, p.a0, m0, m0 + 128, p.M, p.K, p.lda, wave, lane);
+  else if constexpr (C::kDualM) mc4_setup(la, p.a0, p.a1, p.a0, p.a1, m0, m0, p.M, p.K, p.lda, wave, lane, 16 * MB);
+  else if constexpr (kOnePanelA) mc4_setup(la, p.a0, p.a0, p.a0, p.a0, m0, m0, p.M, p.K, p.lda, wave, lane);
+  else mc4_setup(la, p.a0, p.a0, p.a0, p.a0, m0, m0 + 16 * MB, p.M, p.K, p.lda, wave, lane, 16 * MB);
   if constexpr (B_INTER) kc4_setup(lb, p.b0, p.b1, n0, p.n_rows_b, p.K, p.ldb, wave, lane, true);
   else if constexpr (B_KC) kc4_setup(lb, p.b0, C::kPasses == 2 ? p.b1 : p.b0, n0, p.n_rows_b, p.K, p.ldb, wave, lane, false);
   else if constexpr (C::kDualN) mc4_setup(lb, p.b0, p.b1, p.b0, p.b1, n0, n0, p.N, p.K, p.ldb, wave, lane);
@@ -224,7 +251,7 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
   // gathered at the top of the loop).
 #define FSW_PIN_S(x) asm volatile("" : "+s"(x))
   unsigned wrap_mask = 0, wrap_lo = 0, wrap_hi = 0;
-  auto stream_micro = [&](Stream4& S, const Loader4& L, bool kc, unsigned lds_base, int pairs, uint64_t wrap0,
+  auto stream_micro = [&](Stream4& S, const Loader4& L, bool kc, unsigned lds_base, int pairs, int area, uint64_t wrap0,
                           uint64_t wrap1, int n) {
     const bool two = C::kPasses == 2;
     if (n == 0) { FSW_PIN_S(S.koff); S.koff += kc ? 2 * kBK * 2 : 2 * kBK; FSW_PIN_S(S.koff); }
@@ -242,28 +269,30 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
     if (n == 7 && two) { FSW_PIN_S(S.rs[0]); rsrc_advance64(S.rs[0], wrap_lo, wrap_hi); FSW_PIN_S(S.rs[0]); }
     if (n == 10 && two && !kc) { FSW_PIN_S(wrap_mask); wrap_lo = (unsigned)wrap1 & wrap_mask; wrap_hi = (unsigned)(wrap1 >> 32) & wrap_mask; FSW_PIN_S(wrap_lo); FSW_PIN_S(wrap_hi); }
     if (n == 11 && two && !kc) { FSW_PIN_S(S.rs[1]); rsrc_advance64(S.rs[1], wrap_lo, wrap_hi); FSW_PIN_S(S.rs[1]); }
-    if (n == 12) { FSW_PIN_S(S.dst); S.dst += kKcAreaBytes; FSW_PIN_S(S.dst); }
+    if (n == 12) { FSW_PIN_S(S.dst); S.dst += area; FSW_PIN_S(S.dst); }
     if (n == 13) {
       FSW_PIN_S(S.dst);
-      S.dst = (S.dst == lds_base + wave * 1024 + pairs * kKcAreaBytes) ? lds_base + wave * 1024 : S.dst;
+      S.dst = (S.dst == lds_base + wave * 1024 + pairs * area) ? lds_base + wave * 1024 : S.dst;
       FSW_PIN_S(S.dst);
     }
     if (n == 14) { FSW_PIN_S(S.koff); stream_edge(S, L, kc); }
   };
-  auto stream_next = [&](Stream4& S, const Loader4& L, bool kc, unsigned lds_base, int pairs, uint64_t wrap0,
+  auto stream_next = [&](Stream4& S, const Loader4& L, bool kc, unsigned lds_base, int pairs, int area, uint64_t wrap0,
                          uint64_t wrap1) {
 #pragma unroll
-    for (int n = 0; n < 15; n++) stream_micro(S, L, kc, lds_base, pairs, wrap0, wrap1, n);
+    for (int n = 0; n < 15; n++) stream_micro(S, L, kc, lds_base, pairs, area, wrap0, wrap1, n);
   };
-  // Load i (0..7) of the pair: it goes to LDS at dst + i * 4 KiB (KC: LDS rows 8*(wave + 4i); MC: step i >> 2,
-  // KiB wave + 4*(i & 3) of its 16 KiB slot).  load_prep sets the destination (M0) and selects the lane's
+  // Load n of the pair goes to LDS at dst + n * 4 KiB (KC: LDS rows 8*(wave + 4n); MC: step i >> 2, KiB wave + 4*(i & 3)
+  // of its slot, i = load_index(n)).  load_prep sets the destination (M0) and selects the lane's
   // offset; the load itself comes at least one instruction later (M0 write -> LDS-DMA use).
-  auto load_prep = [&](const Stream4& S, const Loader4& L, bool kc, int i) -> unsigned {
-    asm volatile("s_add_u32 m0, %0, %1" : : "s"(S.dst), "n"(i * 4096) : "scc", "memory");
+  auto load_prep = [&](const Stream4& S, const Loader4& L, bool kc, int n, int i) -> unsigned {
+    asm volatile("s_add_u32 m0, %0, %1" : : "s"(S.dst), "n"(n * 4096) : "scc", "memory");
     // the whole offset goes through the vector operand, which the descriptor's range check covers for certain
     if (kc) return S.ok[0] ? L.voff[i] + S.koff : kOobOffset;
     return S.ok[(i >> 2) * 2 + (i & 1)] ? L.voff[i & 3] + S.soff[i >> 2] : kOobOffset;
   };
+  // the loads of a pair in issue order; an operand of one panel has no instructions for the second (i & 2)
+  auto load_index = [](bool one_panel, int n) constexpr { return one_panel ? (n >> 1) * 4 + (n & 1) : n; };
   auto load_go = [&](const Stream4& S, const Loader4& L, bool kc, bool inter, int i, unsigned off, auto nt) {
     constexpr bool kNt = decltype(nt)::value;
     if (kc) dma_load16<kNt>(inter ? S.rs[(i >> 1) & 1] : S.rs[0], off);
@@ -271,11 +300,12 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
   };
   constexpr std::false_type keep{};
   constexpr std::bool_constant<STREAM_B> hint_b{};
-  // all 8 loads of a pair back to back (prologue only)
-  auto pair_all = [&](const Stream4& S, const Loader4& L, bool kc, bool inter, auto nt) {
+  // all loads of a pair back to back (prologue only)
+  auto pair_all = [&](const Stream4& S, const Loader4& L, bool kc, bool inter, auto nt, int count, bool one_panel) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const unsigned off = load_prep(S, L, kc, i);
+    for (int n = 0; n < count; n++) {
+      const int i = load_index(one_panel, n);
+      const unsigned off = load_prep(S, L, kc, n, i);
       asm volatile("s_nop 3" ::: "memory");
       load_go(S, L, kc, inter, i, off, nt);
     }
@@ -289,26 +319,27 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
 #pragma unroll
   for (int h = 0; h < 2; h++) {
     const unsigned kc_lane = (unsigned)(lane & 15) * 128u + (unsigned)(((h * 4 + (lane >> 4)) ^ ((lane >> 1) & 7)) * 16);
-    const unsigned mc_lane = mc_lane_offset(lane) + h * kMcSlotBytes;
-    rd_a[h] = A_KC ? kc_lane + wm * 128 * 128 : mc_lane + wm * kMcPanelBytes;
-    rd_b[h] = B_KC ? kc_lane + wn * 128 * 128 : mc_lane;
+    const unsigned mc_lane = mc_lane_offset(lane);
+    rd_a[h] = A_KC ? kc_lane + wm * (16 * MB * 128) : mc_lane + (kOnePanelA ? h : h * 2 + wm) * kMcPanelBytes;
+    rd_b[h] = B_KC ? kc_lane + wn * 128 * 128 : mc_lane + h * kMcSlotBytes;
   }
   const FSW_LDS char* lds0 = (const FSW_LDS char*)smem;
-  // Read slot r (0..31) of a step: fragment r >> 1 (0..7 of A, then 0..7 of B).  A KC fragment is one
+  // Read slot r of a step: fragment r >> 1 (0..MB-1 of A, then 0..7 of B).  A KC fragment is one
   // ds_read_b128 in the even slot; an MC fragment is two transposing reads, one per slot (two LDS reads behind
   // the same MFMA cost four times what they cost one MFMA apart).
-  i16x8 fq[2][8], fp[2][8];
+  constexpr int kSlots = 2 * (MB + 8);
+  i16x8 fq[2][MB], fp[2][8];
   i16x4 half_lo;
   auto read_slot = [&](int set, int r, const FSW_LDS char* ra, const FSW_LDS char* rb) {
     const int f = r >> 1, second = r & 1;
-    const bool is_a = f < 8;
-    const int fi = is_a ? f : f - 8;
+    const bool is_a = f < MB;
+    const int fi = is_a ? f : f - MB;
     i16x8& dst = is_a ? fq[set][fi] : fp[set][fi];
     if (is_a ? A_KC : B_KC) {
       if (!second) dst = *(const FSW_LDS i16x8*)((is_a ? ra : rb) + fi * 2048);
     } else {
       const FSW_LDS char* base = is_a ? ra : rb + (fi >> 2) * kMcPanelBytes;
-      const int f16 = is_a ? fi : wn * 4 + (fi & 3);
+      const int f16 = is_a ? (kOnePanelA ? wm * 4 : 0) + fi : wn * 4 + (fi & 3);
       const FSW_LDS char* q = (const FSW_LDS char*)(uintptr_t)((unsigned)(uintptr_t)base ^ (unsigned)(f16 << 5));
       if (!second) {
         half_lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((FSW_LDS i16x4*)q);
@@ -322,30 +353,44 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
   // acc[nb][mb]: 16x16 block of rows wm*128 + mb*16.. and 16-column block nb of this wave:
   //   dual-N modes  nb = 4*a + c: matrix a (gate | up), columns wn*64 + c*16..
   //   else          B rows / columns wn*128 + nb*16.. (KC) or panel nb >> 2, columns wn*64 + (nb & 3)*16.. (MC)
-  f32x4 acc[8][8];
+  f32x4 acc[8][MB];
 #pragma unroll
   for (int nb = 0; nb < 8; nb++)
 #pragma unroll
-    for (int mb = 0; mb < 8; mb++) acc[nb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int mb = 0; mb < MB; mb++) acc[nb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // ---- prologue: pairs 0 and 1 of both operands, then the fragments of step 0
   Stream4 sa, sb;
   stream_init(sa, la, A_KC, smem_a);
   stream_init(sb, lb, B_KC, smem_b);
-  pair_all(sa, la, A_KC, false, keep);
-  pair_all(sb, lb, B_KC, B_INTER, hint_b);
-  stream_next(sa, la, A_KC, smem_a, C::kPairsA, wrap_a0, wrap_a1);
-  stream_next(sb, lb, B_KC, smem_b, C::kPairsB, wrap_b0, wrap_b1);
-  pair_all(sa, la, A_KC, false, keep);
-  pair_all(sb, lb, B_KC, B_INTER, hint_b);
-  wait_vmcnt_and_barrier<16>();
+  auto issue_a = [&]() { pair_all(sa, la, A_KC, false, keep, kLdA, kOnePanelA); };
+  auto issue_b = [&]() { pair_all(sb, lb, B_KC, B_INTER, hint_b, kLdB, false); };
+  auto next_a = [&]() { stream_next(sa, la, A_KC, smem_a, R::kPairsA, R::kAreaA, wrap_a0, wrap_a1); };
+  auto next_b = [&]() { stream_next(sb, lb, B_KC, smem_b, R::kPairsB, R::kAreaB, wrap_b0, wrap_b1); };
+  issue_a();
+  issue_b();
+  next_b();
+  if constexpr (R::kPairsB == 3 && R::kPairsA == 3) {  // (B(1) before A(1): what the loop waits for comes first)
+    issue_b();
+    next_a(), issue_a();
+    next_b(), issue_b();
+    wait_vmcnt_and_barrier<kLdA + 2 * kLdB>();
+  } else {
+    next_a(), issue_a();
+    issue_b();
+    if constexpr (R::kPairsB == 3) {
+      next_a(), issue_a();
+      next_b(), issue_b();
+    }
+    wait_vmcnt_and_barrier<(R::kPairsB - 1) * (kLdA + kLdB)>();
+  }
   // LDS byte offsets of the pair being multiplied inside the A and B rings
   unsigned rd_pair_a = 0, rd_pair_b = 0;
   {
     const FSW_LDS char* ra = lds0 + rd_a[0];
-    const FSW_LDS char* rb = lds0 + C::kBytesA + rd_b[0];
+    const FSW_LDS char* rb = lds0 + R::kBytesA + rd_b[0];
 #pragma unroll
-    for (int r = 0; r < 32; r++) read_slot(0, r, ra, rb);
+    for (int r = 0; r < kSlots; r++) read_slot(0, r, ra, rb);
   }
 
   // The schedule of one pair: which gap (after MFMA g of 128) holds what.
@@ -356,49 +401,59 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
   //   kBLd0 + kLdStrideB*i, +1     loads of B(p+2), after the barrier
   //   kRdNext .. +3                the ring offsets of pair p+1
   //   kRd0_0 + r                   read slot r of step 2p+2 (set 0), after the barrier
-  constexpr int kLdStrideA = 6, kLdStrideB = 6;
-  constexpr int kAMicro0 = 0, kALd0 = 15, kRd1_0 = 16;
-  constexpr int kBMicro0 = 46, kBarrier = 64, kBLd0 = 66, kRdNext = 74, kRd0_0 = 80;
-  static_assert(kALd0 + 1 + 7 * kLdStrideA < kBarrier && kBLd0 > kBarrier && kBLd0 + 1 + 7 * kLdStrideB < 128, "load gaps");
-  static_assert(kRd1_0 + 31 < kBarrier && kRd0_0 > kBarrier && kRd0_0 + 31 < 128, "read gaps");
+  constexpr int kHalf = 8 * MB;  // MFMAs of a step
+  // loads issued after those of pair p+1, which the barrier of pair p waits for
+  constexpr int kInFlight = R::kPairsB == 2 ? kLdA : R::kPairsA == 3 ? kLdA + kLdB : 2 * kLdA + kLdB;
+  constexpr int kLdStrideA = (kHalf - 18) / (kLdA - 1) < 6 ? (kHalf - 18) / (kLdA - 1) : 6;
+  constexpr int kLdStrideB = (kHalf - 4) / kLdB < 6 ? (kHalf - 4) / kLdB : 6;
+  constexpr int kAMicro0 = 0, kALd0 = 15, kRd1_0 = kHalf - 1 - kSlots < 16 ? kHalf - 1 - kSlots : 16;
+  constexpr int kBMicro0 = kHalf - 18, kBarrier = kHalf, kBLd0 = kHalf + 2;
+  constexpr int kRd0_0 = kHalf - 2 - kSlots < 16 ? 2 * kHalf - 2 - kSlots : kHalf + 16, kRdNext = kRd0_0 - (kRd0_0 - 6 > kHalf ? 6 : 4);
+  static_assert(kALd0 + 1 + (kLdA - 1) * kLdStrideA < kBarrier && kBLd0 > kBarrier && kBLd0 + 1 + (kLdB - 1) * kLdStrideB < 2 * kHalf, "load gaps");
+  static_assert(kRd1_0 + kSlots - 1 < kBarrier && kRd1_0 > 0 && kRdNext > kBarrier && kRd0_0 + kSlots - 1 < 2 * kHalf, "read gaps");
 
   for (int kt = 0; kt < kt_total; kt += 2) {
     unsigned off_a = 0, off_b = 0;
     const FSW_LDS char* ra;
     const FSW_LDS char* rb;
-    static_for<128>([&](auto gc) {
+    static_for<2 * kHalf>([&](auto gc) {
       constexpr int g = decltype(gc)::value;
-      constexpr int h = g >> 6, idx = g & 63, nb = idx >> 3, ii = idx & 7, mb = (nb & 1) ? 7 - ii : ii;
+      constexpr int h = g / kHalf, idx = g % kHalf, nb = idx / MB, ii = idx % MB, mb = (nb & 1) ? MB - 1 - ii : ii;
       mfma16_acc<E>(acc[nb][mb], fp[h][nb], fq[h][mb]);
       __builtin_amdgcn_sched_barrier(0);
       // --- the A stream moves on to pair p+2 (ring slot of pair p-1, released at the last barrier); its loads
       if constexpr (g >= kAMicro0 && g < kAMicro0 + 15)
-        stream_micro(sa, la, A_KC, smem_a, C::kPairsA, wrap_a0, wrap_a1, g - kAMicro0);
-      constexpr int ia_prep = gap_index(g, kALd0, kLdStrideA, 8), ia_go = gap_index(g, kALd0 + 1, kLdStrideA, 8);
-      if constexpr (ia_prep >= 0) off_a = load_prep(sa, la, A_KC, ia_prep);
-      if constexpr (ia_go >= 0) load_go(sa, la, A_KC, false, ia_go, off_a, keep);
+        stream_micro(sa, la, A_KC, smem_a, R::kPairsA, R::kAreaA, wrap_a0, wrap_a1, g - kAMicro0);
+      constexpr int ia_prep = gap_index(g, kALd0, kLdStrideA, kLdA), ia_go = gap_index(g, kALd0 + 1, kLdStrideA, kLdA);
+      if constexpr (ia_prep >= 0) off_a = load_prep(sa, la, A_KC, ia_prep, load_index(kOnePanelA, ia_prep));
+      if constexpr (ia_go >= 0) load_go(sa, la, A_KC, false, load_index(kOnePanelA, ia_go), off_a, keep);
       // --- fragments of step kt+1 (second half of the same pair) into set 1
       if constexpr (g == kRd1_0 - 1) {
         ra = lds0 + rd_pair_a + rd_a[1];
-        rb = lds0 + C::kBytesA + rd_pair_b + rd_b[1];
+        rb = lds0 + R::kBytesA + rd_pair_b + rd_b[1];
       }
-      if constexpr (g >= kRd1_0 && g < kRd1_0 + 32) read_slot(1, g - kRd1_0, ra, rb);
+      if constexpr (g >= kRd1_0 && g < kRd1_0 + kSlots) read_slot(1, g - kRd1_0, ra, rb);
       // --- the B stream moves on to pair p+2; the barrier of pair p; the loads of B(p+2) into pair p's space
       if constexpr (g >= kBMicro0 && g < kBMicro0 + 15)
-        stream_micro(sb, lb, B_KC, smem_b, C::kPairsB, wrap_b0, wrap_b1, g - kBMicro0);
-      if constexpr (g == kBarrier) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      constexpr int ib_prep = gap_index(g, kBLd0, kLdStrideB, 8), ib_go = gap_index(g, kBLd0 + 1, kLdStrideB, 8);
-      if constexpr (ib_prep >= 0) off_b = load_prep(sb, lb, B_KC, ib_prep);
+        stream_micro(sb, lb, B_KC, smem_b, R::kPairsB, R::kAreaB, wrap_b0, wrap_b1, g - kBMicro0);
+      if constexpr (g == kBarrier) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(kInFlight) : "memory");
+      constexpr int ib_prep = gap_index(g, kBLd0, kLdStrideB, kLdB), ib_go = gap_index(g, kBLd0 + 1, kLdStrideB, kLdB);
+      if constexpr (ib_prep >= 0) off_b = load_prep(sb, lb, B_KC, ib_prep, ib_prep);
       if constexpr (ib_go >= 0) load_go(sb, lb, B_KC, B_INTER, ib_go, off_b, hint_b);
       // --- fragments of step kt+2 (pair p+1) into set 0
-      if constexpr (g == kRdNext) { FSW_PIN_S(rd_pair_a); rd_pair_a += kKcAreaBytes; FSW_PIN_S(rd_pair_a); }
-      if constexpr (g == kRdNext + 1) { FSW_PIN_S(rd_pair_a); rd_pair_a = rd_pair_a == C::kPairsA * kKcAreaBytes ? 0u : rd_pair_a; FSW_PIN_S(rd_pair_a); }
-      if constexpr (g == kRdNext + 2) { FSW_PIN_S(rd_pair_b); rd_pair_b ^= kKcAreaBytes; FSW_PIN_S(rd_pair_b); }
+      if constexpr (g == kRdNext) { FSW_PIN_S(rd_pair_a); rd_pair_a += R::kAreaA; FSW_PIN_S(rd_pair_a); }
+      if constexpr (g == kRdNext + 1) { FSW_PIN_S(rd_pair_a); rd_pair_a = rd_pair_a == R::kBytesA ? 0u : rd_pair_a; FSW_PIN_S(rd_pair_a); }
+      if constexpr (g == kRdNext + 2) {
+        FSW_PIN_S(rd_pair_b);
+        if constexpr (R::kPairsB == 2) rd_pair_b ^= R::kAreaB;
+        else rd_pair_b = rd_pair_b == 2 * R::kAreaB ? 0u : rd_pair_b + R::kAreaB;
+        FSW_PIN_S(rd_pair_b);
+      }
       if constexpr (g == kRdNext + 3) {
         ra = lds0 + rd_pair_a + rd_a[0];
-        rb = lds0 + C::kBytesA + rd_pair_b + rd_b[0];
+        rb = lds0 + R::kBytesA + rd_pair_b + rd_b[0];
       }
-      if constexpr (g >= kRd0_0 && g < kRd0_0 + 32) read_slot(0, g - kRd0_0, ra, rb);
+      if constexpr (g >= kRd0_0 && g < kRd0_0 + kSlots) read_slot(0, g - kRd0_0, ra, rb);
       __builtin_amdgcn_sched_barrier(0);
     });
   }
@@ -419,7 +474,7 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
     else if constexpr (C::kDualN) return n0 + wn * 64;
     else return n0 + h * 128 + wn * 64;
   };
-  const int row_base = C::kDualM ? m0 : m0 + wm * 128;
+  const int row_base = C::kDualM ? m0 : m0 + wm * 16 * MB;
   auto result_of_half = [&](int h) -> int {
     if constexpr (MODE == kDw) return h;
     else if constexpr (C::kDualM) return wm;
@@ -429,7 +484,7 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
     // fp32 partial tile in tile-local coordinates [result][row][column], 16 bytes per lane and store
     float* part = p.ws + ((size_t)tail_tile * p.tail_parts + tail_part) * kTileFloats;
 #pragma unroll
-    for (int mb = 0; mb < 8; mb++) {
+    for (int mb = 0; mb < MB; mb++) {
       const int r = row_base - m0 + mb * 16 + (lane & 15);
 #pragma unroll
       for (int nb = 0; nb < 8; nb++) {
@@ -442,7 +497,7 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
   if (!C::kForward && p.splits > 1) {
     const size_t plane = (size_t)p.M * p.N;
 #pragma unroll
-    for (int mb = 0; mb < 8; mb++) {
+    for (int mb = 0; mb < MB; mb++) {
       const int m = row_base + mb * 16 + (lane & 15);
       if (m >= p.M) continue;
 #pragma unroll
@@ -456,7 +511,7 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
     }
     return;
   }
-  store_tile<E, MODE, 4, true>(p, acc, (FSW_LDS char*)smem + wave * (2 * 32 * 128), lane, row_base, col_of_half(0),
+  store_tile<E, MODE, MB, true>(p, acc, (FSW_LDS char*)smem + wave * (2 * 32 * 128), lane, row_base, col_of_half(0),
                                col_of_half(1), result_of_half(0), result_of_half(1));
 }
 
