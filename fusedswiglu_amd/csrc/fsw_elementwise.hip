@@ -38,8 +38,11 @@ __global__ __launch_bounds__(256) void elementwise_backward_kernel(
       ru[w] = E::pack2(u0, u1);
       rg[w] = E::pack2(g0, g1);
     }
-    __builtin_nontemporal_store(ru, (u32x4*)dU + v);
-    __builtin_nontemporal_store(rg, (u32x4*)dG + v);
+    // Inputs are read for the last time (non-temporal); the gradients are the next two kernels' operands and stay
+    // cacheable: a step of 8192 tokens takes 134 -> 125 us at d_model 512 (i = 3 d), 321 -> 307 at 1024, 964 -> 957 at
+    // 2048 and the same at 4096, where they exceed the memory-side cache.
+    ((u32x4*)dU)[v] = ru;
+    ((u32x4*)dG)[v] = rg;
   }
   // scalar tail (everything, when the pointers are not 16-byte aligned)
   for (size_t i = nvec * 8 + tid; i < n; i += stride) gate_grad<E>(dout[i], g[i], u[i], dU[i], dG[i]);
