@@ -617,10 +617,17 @@ __global__ __launch_bounds__(256) void fsw_splitk_reduce_kernel(const float* __r
   if (i4 >= n) return;
   ws += (size_t)blockIdx.y * splits * n;
   unsigned short* out = blockIdx.y ? out1 : out0;
-  f32x4 a = *(const f32x4*)(ws + i4);
-  for (int s = 1; s < splits; s++) {
-    const f32x4 b = *(const f32x4*)(ws + (size_t)s * n + i4);
-    a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+  // Loads of eight partials at a time: one after the other, each add waits for its own trip to memory (16 planes of
+  // 1 x 4096: 5.4 us).  The order of the sum is the same.
+  f32x4 a{-0.f, -0.f, -0.f, -0.f};
+  for (int s = 0; s < splits; s += 8) {
+    f32x4 b[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      if (s + j < splits) b[j] = *(const f32x4*)(ws + (size_t)(s + j) * n + i4);
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      if (s + j < splits) { a.x += b[j].x; a.y += b[j].y; a.z += b[j].z; a.w += b[j].w; }
   }
   const size_t m = i4 / (size_t)N, c = i4 - m * (size_t)N;
   u32x2 v;
