@@ -8,13 +8,15 @@
 // applies silu(g)*u in registers.  The weight loads carry the non-temporal hint: bytes that are read once
 // then leave L2 and the memory-side cache to x.  Fragment reads of the next half stage overlap the MFMAs
 // of the current one, and a slot goes back to the loader as soon as its fragments are in registers.
-#include "fsw_gemm.hpp"
+//
+// Where blocks of 128 columns leave CUs without work or their LDS slots half empty, the same idea runs on blocks of 16,
+// 32 or 64 columns (fsw_narrow.hpp); choose() below decides.
+#include "fsw_narrow.hpp"
 #include "fsw_internal.hpp"
+#include <algorithm>
 #include <atomic>
 
 namespace fsw {
-
-constexpr int kSkThreads = 256;
 
 // A stage holds 64 k-elements: BM rows of x, one full 128-byte line each, in the k-contiguous LDS format of the
 // tiled kernels (16-byte chunk c of row r at position c ^ ((r >> 1) & 7), read with ds_read_b128), and 32 KiB of
@@ -39,16 +41,6 @@ FSW_DEV i16x8 read_frag_kc32(const FSW_LDS char* area, int row_base, int ks, int
   const int chunk = (ks * 2 + (lane >> 5)) ^ ((row >> 1) & 7);
   return *(const FSW_LDS i16x8*)(area + row * 128 + chunk * 16);
 }
-
-// How a launch is cut up.  plain == 0: the SwiGLU forward (b0 = Wg, b1 = Wu, N = I).  plain == 1: one plain GEMM
-// C = A B whose B is given as its two column halves (b0 = columns 0.., b1 = columns N.. of a matrix 2N wide;
-// c1 = C, ws = fp32 partial planes [splits][M][2N] or null): the down projection for few tokens.  blockIdx.y
-// = k-split: this workgroup reduces stages split*stages_per_split .. of the reduction.
-struct SkArgs {
-  int bn;                 // output columns per workgroup (of each half), <= 128
-  int plain;
-  int splits, stages_per_split;
-};
 
 template <typename E, int BM, bool W_KC>
 __global__ __launch_bounds__(kSkThreads) void fsw_skinny_forward_kernel(GemmParams p, SkArgs a) {
@@ -180,41 +172,9 @@ __global__ __launch_bounds__(kSkThreads) void fsw_skinny_forward_kernel(GemmPara
     for (int r4 = 0; r4 < 4; r4++) {
       const int nc = wave * 32 + 8 * r4 + 4 * (lane >> 5), n = n0 + nc;
       if (nc >= bn || n >= p.N) continue;
-      if (a.plain) {
-        // the two halves are columns n and N + n of one result, 2N wide
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-          const float v[4] = {acc[h][q][r4 * 4], acc[h][q][r4 * 4 + 1], acc[h][q][r4 * 4 + 2], acc[h][q][r4 * 4 + 3]};
-          if (p.ws) {
-            float* dst = p.ws + ((size_t)split * p.M + m) * (2 * (size_t)p.N) + (size_t)h * p.N + n;
-            *(f32x4*)dst = f32x4{v[0], v[1], v[2], v[3]};
-          } else {
-            u32x2 w;
-            w.x = E::pack2(v[0], v[1]);
-            w.y = E::pack2(v[2], v[3]);
-            *(u32x2*)((unsigned short*)p.c1 + (size_t)m * p.ldc + (size_t)h * p.N + n) = w;
-          }
-        }
-        continue;
-      }
-      const size_t o = (size_t)m * p.ldc + n;
-      unsigned short ho[4], hg[4], hu[4];
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const float g = acc[0][q][r4 * 4 + e], u = acc[1][q][r4 * 4 + e];
-        ho[e] = E::from_float(silu_mul(g, u));
-        hg[e] = E::from_float(g);
-        hu[e] = E::from_float(u);
-      }
-      u32x2 v;
-      v.x = ho[0] | ((unsigned)ho[1] << 16); v.y = ho[2] | ((unsigned)ho[3] << 16);
-      *(u32x2*)((unsigned short*)p.c0 + o) = v;
-      if (p.c1) {
-        v.x = hg[0] | ((unsigned)hg[1] << 16); v.y = hg[2] | ((unsigned)hg[3] << 16);
-        *(u32x2*)((unsigned short*)p.c1 + o) = v;
-        v.x = hu[0] | ((unsigned)hu[1] << 16); v.y = hu[2] | ((unsigned)hu[3] << 16);
-        *(u32x2*)((unsigned short*)p.c2 + o) = v;
-      }
+      const float g[4] = {acc[0][q][r4 * 4], acc[0][q][r4 * 4 + 1], acc[0][q][r4 * 4 + 2], acc[0][q][r4 * 4 + 3]};
+      const float u[4] = {acc[1][q][r4 * 4], acc[1][q][r4 * 4 + 1], acc[1][q][r4 * 4 + 2], acc[1][q][r4 * 4 + 3]};
+      store_few<E>(p, a.plain, split, m, n, g, u);
     }
   }
 }
@@ -259,13 +219,109 @@ static int cu_count() {
   return cus;
 }
 
+// A launch: column blocks of `slot` = 128 (fsw_skinny_forward_kernel) or 16, 32, 64 columns (fsw_narrow_kernel; mq
+// 16-row blocks of x), of which bn are used, times k-splits.
+struct SkPlan { int slot, mq, bn, splits, stages_per_split; };
+
 template <typename E, bool W_KC>
-static hipError_t launch_skinny_t(const GemmParams& g, const SkArgs& a, hipStream_t s) {
+static hipError_t launch_skinny_t(const GemmParams& g, const SkPlan& pl, int plain, hipStream_t s) {
+  const SkArgs a{pl.bn, plain, pl.splits, pl.stages_per_split};
   const dim3 grid((unsigned)((g.N + a.bn - 1) / a.bn), (unsigned)a.splits);
-  if (g.M <= 32) fsw_skinny_forward_kernel<E, 32, W_KC><<<grid, kSkThreads, 0, s>>>(g, a);
-  else if (g.M <= 64) fsw_skinny_forward_kernel<E, 64, W_KC><<<grid, kSkThreads, 0, s>>>(g, a);
-  else fsw_skinny_forward_kernel<E, 128, W_KC><<<grid, kSkThreads, 0, s>>>(g, a);
+  switch (pl.slot * 16 + pl.mq) {
+#define FSW_NARROW(SLOT, MQ) case SLOT * 16 + MQ: fsw_narrow_kernel<E, MQ, SLOT, W_KC><<<grid, kSkThreads, 0, s>>>(g, a); break
+    FSW_NARROW(16, 1);
+    FSW_NARROW(16, 2);
+    FSW_NARROW(16, 4);
+    FSW_NARROW(32, 1);
+    FSW_NARROW(32, 2);
+    FSW_NARROW(32, 4);
+    FSW_NARROW(32, 8);
+#undef FSW_NARROW
+    default:
+      if constexpr (W_KC) {
+        if (pl.slot == 64) {
+          if (pl.mq == 2) fsw_narrow_kernel<E, 2, 64, true><<<grid, kSkThreads, 0, s>>>(g, a);
+          else if (pl.mq == 4) fsw_narrow_kernel<E, 4, 64, true><<<grid, kSkThreads, 0, s>>>(g, a);
+          else fsw_narrow_kernel<E, 8, 64, true><<<grid, kSkThreads, 0, s>>>(g, a);
+          break;
+        }
+      }
+      if (g.M <= 32) fsw_skinny_forward_kernel<E, 32, W_KC><<<grid, kSkThreads, 0, s>>>(g, a);
+      else if (g.M <= 64) fsw_skinny_forward_kernel<E, 64, W_KC><<<grid, kSkThreads, 0, s>>>(g, a);
+      else fsw_skinny_forward_kernel<E, 128, W_KC><<<grid, kSkThreads, 0, s>>>(g, a);
+  }
   return hipGetLastError();
+}
+
+// Blocks of 128 columns for the down projection: full blocks and as many k-splits as fit into one round of workgroups
+// (measured at N = 8192, K = 28672: 32 blocks x 8 splits beat every narrower block with fewer splits in this kernel,
+// although the partial planes then cost 2 x 8 x M x N x 4 bytes of traffic: narrow blocks leave the 32 KiB weight slots
+// half empty).  Enough column blocks for a round on their own, or the forward: no split, and the width rule above.
+static SkPlan plan_wide(long long M, long long Nh, long long K, int cus, bool w_kc, long long max_splits) {
+  const int stages = (int)((K + 63) / 64);
+  const long long tiles = (Nh + 127) / 128;
+  // a split shorter than 8 stages does not fill the ring
+  const long long splits = std::min({cus / tiles, 16LL, max_splits, (long long)stages / 8});
+  if (max_splits < 1 || splits <= 1) return SkPlan{128, 0, block_width((int)Nh, cus, w_kc, (int)M), 1, stages};
+  const int sps = (int)((stages + splits - 1) / splits);
+  return SkPlan{128, 0, 128, (stages + sps - 1) / sps, sps};
+}
+
+// Microseconds of a launch by what it moves, fitted to 9700 measured launches with weights that are not in the caches (1 to
+// 128 rows, d_model 1024 .. 8192, d_intermediate 2 .. 4 times that, both layouts, forward and down projection; rms error
+// 10 %): all weights once at 6 TB/s; per CU its weights at 49 (128-column blocks: 26) bytes/ns and its LDS fill, x
+// included, at 50 (62) bytes/ns; start and end of a launch and of every further round of workgroups; the second launch of a
+// split and its fp32 partials.  Rows of [D, I] weights shorter than a 128-byte line are fetched as whole lines by every
+// block.
+static double estimate_us(const SkPlan& p, long long M, long long Nh, long long K, int cus, bool w_kc) {
+  const bool wide = p.slot == 128;
+  const long long wgs = (Nh + p.bn - 1) / p.bn * p.splits, rounds = (wgs + cus - 1) / cus;
+  const int x_rows = !wide ? 16 * p.mq : (M <= 32 ? 32 : (M <= 64 ? 64 : 128));
+  const double stage = p.slot == 16 || (p.slot == 32 && p.mq == 1) ? 128 : 64;
+  const double k64 = (double)rounds * p.stages_per_split * stage / 64;  // 64-element blocks a CU goes through
+  const double lines = w_kc || p.slot >= 64 ? 1 : 64 / p.slot;
+  const double useful = k64 * p.bn * 256 * lines, fill = k64 * (256 * p.slot * lines + 128 * x_rows);
+  const double cu_rate = w_kc ? (wide ? 26e3 : 49e3) : (wide ? 30e3 : 36e3), fill_rate = w_kc ? (wide ? 62e3 : 50e3) : (wide ? 55e3 : 47e3);
+  const double start = w_kc ? (wide ? 0.6 : 4.2) : (wide ? 1.2 : 4.3), round = wide ? 2.0 : (w_kc ? 1.3 : 0.0);
+  double us = std::max({4.0 * K * Nh / 6.0e6, useful / cu_rate, fill / fill_rate}) + start + round * (rounds - 1);
+  if (p.splits > 1) us += (w_kc ? 1.7 : 2.3) + p.splits * M * Nh * 8.0 / 1.3e6;
+  return us;
+}
+
+// Nh: columns of each half.  Narrow blocks are taken where the estimate sees them ahead by more than it errs among the
+// launches above, whose times they then beat on average by 31 / 23 / 28 / 21 % (forward, [I, D], up to 16 / 32 / 64 / 128
+// rows), 15 / 16 / 19 / 15 % (down projection, nn.Linear's layout), 5 / 2 / 4 / 12 % and 10 / 9 / 2 / 0 % (the other
+// layout), at most 3 % slower anywhere: 1 x 1024 x 3072 [I, D] 10.5 -> 5.6 us, 16 x 2048 x 4096 19 -> 10, 1 x 4096 x 11008
+// 37 -> 33, its down projection 24 -> 21.  [D, I] weights of more than 150 MB stay on blocks of 128: their rows, one
+// segment per k and block, are then read 15 to 20 % slower in shorter segments.
+static SkPlan choose(long long M, long long Nh, long long K, int cus, bool w_kc, bool plain, long long max_splits) {
+  SkPlan best = plan_wide(M, Nh, K, cus, w_kc, plain ? max_splits : 0);
+  if (!w_kc && 4.0 * K * Nh > 150e6) return best;
+  double best_us = estimate_us(best, M, Nh, K, cus, w_kc);
+  best_us /= plain ? (M <= 16 ? 1.05 : 1.15) : (w_kc ? 1.10 : 1.0);
+  for (int slot = 16; slot <= (w_kc ? 64 : 32); slot *= 2) {
+    int mq = slot == 64 ? 2 : 1;
+    while (16 * mq < M) mq *= 2;
+    if (slot == 16 && mq > 4) continue;
+    const int stage = slot == 16 || (slot == 32 && mq == 1) ? 128 : 64;
+    const int stages = (int)((K + stage - 1) / stage);
+    // widths: the whole slot; rows of [I, D] weights are lines of their own, so also what fills 1 .. 5 rounds, and 8
+    // columns for short results
+    for (int i = 0; i <= (w_kc ? 6 : 0); i++) {
+      const int bn = i == 0 ? slot : (i == 6 ? 8 : (int)(((Nh + cus * i - 1) / (cus * i) + 3) & ~3LL));
+      if (bn > slot || bn < slot / 2 || (i == 6 && !plain)) continue;
+      const long long blocks = (Nh + bn - 1) / bn;
+      for (int splits : {1, 2, 3, 4, 6, 8}) {
+        if (splits > 1 && (!plain || splits > max_splits || blocks * splits > 560 || K < 128 * splits)) break;
+        if (blocks * splits < (splits > 1 ? 48 : 40)) continue;
+        const int sps = (stages + splits - 1) / splits;
+        const SkPlan pl{slot, mq, bn, (stages + sps - 1) / sps, sps};
+        const double us = estimate_us(pl, M, Nh, K, cus, w_kc);
+        if (us < best_us) { best_us = us; best = pl; }
+      }
+    }
+  }
+  return best;
 }
 
 bool skinny_forward_ok(const Problem& p) { return p.T <= kSkMaxRows && fast_path_ok_forward(p); }
@@ -275,34 +331,15 @@ hipError_t launch_forward_skinny(int dtype, const Problem& p, hipStream_t s) {
   g.a0 = p.x; g.b0 = p.wg; g.b1 = p.wu; g.c0 = p.out; g.c1 = p.g; g.c2 = p.u;
   g.M = (int)p.T; g.N = (int)result_cols(p.I); g.n_rows_b = (int)p.I; g.K = (int)p.D;
   g.lda = (int)p.ldx; g.ldb = (int)p.ldw; g.ldc = (int)p.ldo;
-  const int stages = (int)((p.D + 63) / 64);
-  const SkArgs a{block_width(g.N, cu_count(), p.w_out_in, g.M), 0, 1, stages};
-  if (p.w_out_in) return dtype == kDtypeBF16 ? launch_skinny_t<BF16, true>(g, a, s) : launch_skinny_t<FP16, true>(g, a, s);
-  return dtype == kDtypeBF16 ? launch_skinny_t<BF16, false>(g, a, s) : launch_skinny_t<FP16, false>(g, a, s);
+  const SkPlan pl = choose(g.M, g.N, g.K, cu_count(), p.w_out_in, false, 1);
+  if (p.w_out_in) return dtype == kDtypeBF16 ? launch_skinny_t<BF16, true>(g, pl, 0, s) : launch_skinny_t<FP16, true>(g, pl, 0, s);
+  return dtype == kDtypeBF16 ? launch_skinny_t<BF16, false>(g, pl, 0, s) : launch_skinny_t<FP16, false>(g, pl, 0, s);
 }
 
 // ---- the down projection for few tokens: y [M, N] = a [M, K] W, W stored [K, N] (layout 0) or [N, K] (layout 1)
 // The same kernel with W's two column halves in the places of Wg and Wu.  N is short and K long here (D and I
 // of the SwiGLU), so column blocks alone do not fill the chip: the reduction is split as well, the fp32 partial
 // planes go to the caller's scratch and fsw_splitk_reduce_kernel adds them in a fixed order.
-struct SkPlan { int bn, splits, stages_per_split; };
-
-// Full 128-column blocks and as many k-splits as fit into one round of workgroups (measured at N = 8192,
-// K = 28672: 32 blocks x 8 splits beat every narrower block with fewer splits, although the partial planes
-// then cost 2 x 8 x M x N x 4 bytes of traffic: narrow blocks leave the 32 KiB weight slots half empty).
-// Enough column blocks for a round on their own: no split, and the width rule of the forward.
-static SkPlan plan_plain(long long M, long long Nh, long long K, int cus, bool w_kc, long long max_splits) {
-  const int stages = (int)((K + 63) / 64);
-  const long long tiles = (Nh + 127) / 128;
-  long long splits = cus / tiles;
-  if (splits > 16) splits = 16;
-  if (splits > max_splits) splits = max_splits;
-  if (splits > stages / 8) splits = stages / 8;   // a split shorter than 8 stages does not fill the ring
-  if (splits <= 1) return SkPlan{block_width((int)Nh, cus, w_kc, (int)M), 1, stages};
-  const int sps = (int)((stages + splits - 1) / splits);
-  return SkPlan{128, (stages + sps - 1) / sps, sps};
-}
-
 bool skinny_gemm_ok(const GemmProblem& p) {
   if (p.layout > 1 || p.M > kSkMaxRows || (p.N & 7) || !fast_path_ok_gemm(p)) return false;
   const long long nh = p.N / 2;
@@ -311,7 +348,7 @@ bool skinny_gemm_ok(const GemmProblem& p) {
 
 long long skinny_gemm_workspace_bytes(int layout, long long M, long long N, long long K) {
   if (layout > 1 || M > kSkMaxRows || M <= 0 || (N & 7) || (N / 2) % (layout == 1 ? 8 : 64)) return 0;
-  const SkPlan pl = plan_plain(M, N / 2, K, cu_count(), layout == 1, 16);
+  const SkPlan pl = choose(M, N / 2, K, cu_count(), layout == 1, true, 16);
   return pl.splits > 1 ? (long long)pl.splits * M * N * 4 : 0;
 }
 
@@ -319,7 +356,7 @@ hipError_t launch_gemm_skinny(int dtype, const GemmProblem& p, hipStream_t s, vo
   const bool w_kc = p.layout == 1;
   const long long nh = p.N / 2;
   const long long fit = ws ? ws_bytes / (p.M * p.N * 4) : 1;
-  const SkPlan pl = plan_plain(p.M, nh, p.K, cu_count(), w_kc, fit < 1 ? 1 : fit);
+  const SkPlan pl = choose(p.M, nh, p.K, cu_count(), w_kc, true, fit < 1 ? 1 : fit);
   GemmParams g{};
   g.a0 = p.a; g.b0 = p.b;
   g.b1 = (const char*)p.b + (w_kc ? (size_t)nh * p.ldb * 2 : (size_t)nh * 2);
@@ -327,10 +364,9 @@ hipError_t launch_gemm_skinny(int dtype, const GemmProblem& p, hipStream_t s, vo
   g.M = (int)p.M; g.N = g.n_rows_b = (int)nh; g.K = (int)p.K;
   g.lda = (int)p.lda; g.ldb = (int)p.ldb; g.ldc = (int)p.ldc;
   g.ws = pl.splits > 1 ? (float*)ws : nullptr;
-  const SkArgs a{pl.bn, 1, pl.splits, pl.stages_per_split};
   hipError_t e;
-  if (w_kc) e = dtype == kDtypeBF16 ? launch_skinny_t<BF16, true>(g, a, s) : launch_skinny_t<FP16, true>(g, a, s);
-  else e = dtype == kDtypeBF16 ? launch_skinny_t<BF16, false>(g, a, s) : launch_skinny_t<FP16, false>(g, a, s);
+  if (w_kc) e = dtype == kDtypeBF16 ? launch_skinny_t<BF16, true>(g, pl, 1, s) : launch_skinny_t<FP16, true>(g, pl, 1, s);
+  else e = dtype == kDtypeBF16 ? launch_skinny_t<BF16, false>(g, pl, 1, s) : launch_skinny_t<FP16, false>(g, pl, 1, s);
   if (e != hipSuccess || pl.splits == 1) return e;
   const size_t n = (size_t)p.M * p.N;
   const dim3 blocks((unsigned)((n / 4 + 255) / 256), 1);
