@@ -17,7 +17,7 @@ FSW_DEV void gate_grad(unsigned short dout, unsigned short g, unsigned short u, 
   dG = E::from_float(fg);
 }
 
-template <typename E>
+template <typename E, bool KEEP>
 __global__ __launch_bounds__(256) void elementwise_backward_kernel(
     const unsigned short* __restrict__ dout, const unsigned short* __restrict__ g,
     const unsigned short* __restrict__ u, unsigned short* __restrict__ dU,
@@ -38,11 +38,14 @@ __global__ __launch_bounds__(256) void elementwise_backward_kernel(
       ru[w] = E::pack2(u0, u1);
       rg[w] = E::pack2(g0, g1);
     }
-    // Inputs are read for the last time (non-temporal); the gradients are the next two kernels' operands and stay
-    // cacheable: a step of 8192 tokens takes 134 -> 125 us at d_model 512 (i = 3 d), 321 -> 307 at 1024, 964 -> 957 at
-    // 2048 and the same at 4096, where they exceed the memory-side cache.
-    ((u32x4*)dU)[v] = ru;
-    ((u32x4*)dG)[v] = rg;
+    // Inputs are read for the last time (non-temporal); the gradients are the next two kernels' operands
+    if constexpr (KEEP) {
+      ((u32x4*)dU)[v] = ru;
+      ((u32x4*)dG)[v] = rg;
+    } else {
+      __builtin_nontemporal_store(ru, (u32x4*)dU + v);
+      __builtin_nontemporal_store(rg, (u32x4*)dG + v);
+    }
   }
   // scalar tail (everything, when the pointers are not 16-byte aligned)
   for (size_t i = nvec * 8 + tid; i < n; i += stride) gate_grad<E>(dout[i], g[i], u[i], dU[i], dG[i]);
@@ -59,7 +62,11 @@ static hipError_t launch_elementwise_t(const void* dout, const void* g, const vo
   if (blocks > 65536) blocks = (blocks + 1) / 2;
   if (blocks > 0x7fffffffu) blocks = 0x7fffffffu;
   if (blocks == 0) return hipSuccess;
-  elementwise_backward_kernel<E><<<(unsigned)blocks, 256, 0, stream>>>(
+  // Gradients that fit into the 256 MB memory-side cache stay cacheable for the two GEMMs that read them: a step of 8192
+  // tokens takes 134 -> 125 us at d_model 512 (i = 3 d), 321 -> 307 at 1024, 964 -> 957 at 2048.  Larger ones (4096: 403
+  // MB) are gone before they are read, and plain stores cost this kernel 177 instead of 159 us.
+  auto kernel = n * 4 <= (256u << 20) ? elementwise_backward_kernel<E, true> : elementwise_backward_kernel<E, false>;
+  kernel<<<(unsigned)blocks, 256, 0, stream>>>(
       (const unsigned short*)dout, (const unsigned short*)g, (const unsigned short*)u,
       (unsigned short*)dU, (unsigned short*)dG, n, vec_ok);
   return hipGetLastError();

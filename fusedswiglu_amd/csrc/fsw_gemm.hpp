@@ -233,7 +233,10 @@ FSW_DEV void static_for(F&& f) {
 // conflict), the lines of part k-1 are on their way from the other patch to memory.  Everything is branch free -
 // edges are masked through the offsets of buffer stores and loads, which the descriptors' range check drops - so
 // the whole epilogue is one basic block that the compiler schedules across parts.  The results are written once
-// and read by a later kernel at the earliest: non-temporal stores keep them out of the way of the operands.
+// and read by a later kernel at the earliest: non-temporal stores keep them out of the way of the operands.  The gating
+// gradients are the exception: the next two kernels read them, so they stay cacheable (a step of 8192 tokens that
+// recomputes its pre-activations, i = 3 d: d_model 512 149 -> 138 us, 1024 373 -> 360, 2048 1236 -> 1217, the same at
+// 4096; out, g and u cacheable as well: no further gain).
 //
 // ACC_ASM: the accumulators live in the accumulation registers behind inline-asm MFMAs (four-wave form); they are
 // then moved out by explicit instructions at their turn and not earlier (left to the compiler, they are moved out
@@ -269,8 +272,8 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][MB], FSW_LDS char* 
 #pragma unroll
     for (int i = 0; i < 2 * blocks_of(q); i++) in_flight[i] = *(const FSW_LDS u32x4*)(patch + (k & 1) * kPatchBytes + rd_off(i));
   };
-  // st_cols: st_lane, or the out-of-range offset in lanes whose columns do not exist
-  auto store_part = [&](__amdgpu_buffer_rsrc_t rs, unsigned st_cols, int q) {
+  // st_cols: st_lane, or the out-of-range offset in lanes whose columns do not exist; keep: cacheable
+  auto store_part = [&](__amdgpu_buffer_rsrc_t rs, unsigned st_cols, int q, auto keep) {
 #pragma unroll
     for (int i = 0; i < 2 * blocks_of(q); i++) {
       const int r0 = q * 32 + 8 * i;
@@ -278,7 +281,7 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][MB], FSW_LDS char* 
       // offset REGISTER the compiler leaves out the wait state before the next instruction that overwrites the
       // store's data registers, and on this hardware the store then picks up the new value in some lanes.
       const unsigned off = ((lane >> 3) < rows_left - r0 ? st_cols : kOobOffset) + (unsigned)r0 * ldc_bytes;
-      __builtin_amdgcn_raw_buffer_store_b128(in_flight[i], rs, off, 0, 2 /* nt */);
+      __builtin_amdgcn_raw_buffer_store_b128(in_flight[i], rs, off, 0, decltype(keep)::value ? 0 : 2 /* nt */);
     }
   };
   auto write_part = [&](int k, int mbl, int c, float a, float b, float cc, float d) {
@@ -305,6 +308,7 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][MB], FSW_LDS char* 
     auto forward_tile = [&](auto first_tag, auto count_tag) {
       constexpr int first = decltype(first_tag)::value, count = decltype(count_tag)::value;
       constexpr bool gating = first == 1;
+      constexpr std::integral_constant<bool, gating> keep{};
       __amdgpu_buffer_rsrc_t rs[3] = {result_rsrc(p.c0, colw), result_rsrc(count > 1 ? p.c1 : p.c0, colw),
                                       result_rsrc(count > 1 ? p.c2 : p.c0, colw)};
       __amdgpu_buffer_rsrc_t rs_d = result_rsrc(gating ? p.d0 : p.c0, colw);
@@ -356,10 +360,10 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][MB], FSW_LDS char* 
             }
             write_part(k, mbl, c, v[0], v[1], v[2], v[3]);
           }
-        if constexpr (k > 0) store_part(rs[first + (k - 1) % count], st_cols, (k - 1) / count);
+        if constexpr (k > 0) store_part(rs[first + (k - 1) % count], st_cols, (k - 1) / count, keep);
       });
       read_part(NQ * count - 1, NQ - 1);
-      store_part(rs[first + count - 1], st_cols, NQ - 1);
+      store_part(rs[first + count - 1], st_cols, NQ - 1, keep);
     };
     if (p.d0 != nullptr) forward_tile(std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{});
     else if (p.c1 != nullptr) forward_tile(std::integral_constant<int, 0>{}, std::integral_constant<int, 3>{});
@@ -387,10 +391,10 @@ FSW_DEV void store_tile(const GemmParams& p, f32x4 (&acc)[8][MB], FSW_LDS char* 
           const f32x4 t = acc[4 * h + c][2 * q + mbl];
           write_part(k, mbl, c, t[0], t[1], t[2], t[3]);
         }
-      if constexpr (k > 0) store_part(rs[(k - 1) & 1], st_cols[(k - 1) & 1], (k - 1) >> 1);
+      if constexpr (k > 0) store_part(rs[(k - 1) & 1], st_cols[(k - 1) & 1], (k - 1) >> 1, std::false_type{});
     });
     read_part(2 * NQ - 1, NQ - 1);
-    store_part(rs[1], st_cols[1], NQ - 1);
+    store_part(rs[1], st_cols[1], NQ - 1, std::false_type{});
   }
 }
 
