@@ -77,6 +77,8 @@ def _rows(t: torch.Tensor) -> torch.Tensor:
     """2-D [rows, cols] view with unit inner stride (copies only if it must)."""
     if t.ndim == 2 and t.stride(1) == 1 and (t.shape[0] <= 1 or t.stride(0) >= t.shape[1]):
         return t
+    if t.is_contiguous():
+        return t.view(-1, t.shape[-1])
     t2 = t.reshape(-1, t.shape[-1])
     if t2.stride(-1) != 1 or (t2.shape[0] > 1 and t2.stride(0) < t2.shape[1]):
         t2 = t2.contiguous()
@@ -160,7 +162,10 @@ def pads_rows(x: torch.Tensor, I: int) -> bool:
 def _wants_padding(T: int, D: int, I: int, *ts: torch.Tensor) -> bool:
     if T * D * I < _PAD_MIN_WORK:
         return False
-    return bool((D | I) & 7) or not all(_whole_chunks(t) for t in ts)
+    bits = D | I
+    for t in ts:
+        bits |= t.shape[1] | _ld(t) | (t.data_ptr() >> 1)  # 16-byte aligned: bits 1 to 3 of the address
+    return bool(bits & 7)
 
 
 def _weight_dims(w: torch.Tensor, weights_out_in: bool) -> Tuple[int, int]:

@@ -51,15 +51,34 @@ def _require_gpu(*tensors: Tensor) -> None:
             raise _launch.ShapeError(f"fused SwiGLU needs tensors on a HIP GPU, got device '{t.device}'")
 
 
+def _unobserved(*tensors: Tensor) -> bool:
+    """Whether a call that records no gradient may go straight to the launcher: a custom operator is there for what
+    watches the dispatcher (a compiler or tracer, a mode, a transform, forward-mode AD, the profiler, a tensor subclass),
+    and its way through Python costs 10 us of host time: one token through a 4096 x 11008 MLP block 61 -> 41 us of host
+    time, 49 us of GPU time."""
+    return (not torch.compiler.is_compiling() and all(type(t) in (Tensor, torch.nn.Parameter) for t in tensors)
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None
+            and torch.autograd.forward_ad._current_level < 0 and not torch.autograd._profiler_enabled())
+
+
+def _pick(op, launcher, *tensors: Tensor):
+    """The operator, or the function behind it inside an autograd function, where nothing watches and no graph is recorded
+    (a backward pass that records one, create_graph=True, keeps the operator and its refusal to be differentiated)."""
+    return launcher if not torch.is_grad_enabled() and _unobserved(*tensors) else op
+
+
 # ---- forward -----------------------------------------------------------------------------------
-@torch.library.custom_op("fusedswiglu_amd::swiglu_forward", mutates_args=(), device_types="cuda")
-def swiglu_forward(x: Tensor, w_gate: Tensor, w_up: Tensor, save_preactivations: bool,
+def _swiglu_forward(x: Tensor, w_gate: Tensor, w_up: Tensor, save_preactivations: bool,
                    weights_out_in: bool = False) -> Tuple[Tensor, Tensor, Tensor]:
     out, g, u = _launch.fused_swiglu_fwd(x, w_gate, w_up, _dtype_of(x),
                                          save_preactivations=save_preactivations, weights_out_in=weights_out_in)
     if not save_preactivations:
         g, u = _empty(out), _empty(out)
     return out, g, u
+
+
+swiglu_forward = torch.library.custom_op("fusedswiglu_amd::swiglu_forward", mutates_args=(), device_types="cuda")(_swiglu_forward)
 
 
 @swiglu_forward.register_fake
@@ -71,8 +90,7 @@ def _(x, w_gate, w_up, save_preactivations, weights_out_in=False):
 
 
 # ---- backward ----------------------------------------------------------------------------------
-@torch.library.custom_op("fusedswiglu_amd::swiglu_backward", mutates_args=(), device_types="cuda")
-def swiglu_backward(grad_out: Tensor, x: Tensor, w_gate: Tensor, w_up: Tensor, xw_gate: Tensor,
+def _swiglu_backward(grad_out: Tensor, x: Tensor, w_gate: Tensor, w_up: Tensor, xw_gate: Tensor,
                     xw_up: Tensor, need_x: bool, need_w_gate: bool, need_w_up: bool,
                     packed: bool, weights_out_in: bool = False) -> Tuple[Tensor, Tensor, Tensor]:
     """(dx, dw_gate, dw_up); a gradient that is not needed comes back with zero elements.  With
@@ -123,6 +141,9 @@ def swiglu_backward(grad_out: Tensor, x: Tensor, w_gate: Tensor, w_up: Tensor, x
             dw_up if dw_up is not None else e.clone())
 
 
+swiglu_backward = torch.library.custom_op("fusedswiglu_amd::swiglu_backward", mutates_args=(), device_types="cuda")(_swiglu_backward)
+
+
 @swiglu_backward.register_fake
 def _(grad_out, x, w_gate, w_up, xw_gate, xw_up, need_x, need_w_gate, need_w_up, packed, weights_out_in=False):
     r, c = w_gate.shape
@@ -144,8 +165,9 @@ def _setup_context(ctx, inputs, output):
 def _autograd_backward(ctx, grad_out, _grad_g, _grad_u):
     x, w_gate, w_up, g, u = ctx.saved_tensors
     need = ctx.needs_input_grad
-    dx, dwg, dwu = swiglu_backward(grad_out.contiguous(), x, w_gate, w_up, g, u,
-                                   need[0], need[1], need[2], False, ctx.weights_out_in)
+    backward = _pick(swiglu_backward, _swiglu_backward, grad_out, x, w_gate, w_up, g, u)
+    dx, dwg, dwu = backward(grad_out.contiguous(), x, w_gate, w_up, g, u,
+                            need[0], need[1], need[2], False, ctx.weights_out_in)
     return (dx if need[0] else None, dwg if need[1] else None, dwu if need[2] else None, None, None)
 
 
@@ -153,9 +175,11 @@ swiglu_forward.register_autograd(_autograd_backward, setup_context=_setup_contex
 
 
 # ---- the down projection that follows --------------------------------------------------------------
-@torch.library.custom_op("fusedswiglu_amd::down_proj_forward", mutates_args=(), device_types="cuda")
-def down_proj_forward(act: Tensor, w_down: Tensor, weights_out_in: bool = False) -> Tensor:
+def _down_proj_forward(act: Tensor, w_down: Tensor, weights_out_in: bool = False) -> Tensor:
     return _launch.down_proj_forward(act, w_down, _dtype_of(act), weights_out_in=weights_out_in)
+
+
+down_proj_forward = torch.library.custom_op("fusedswiglu_amd::down_proj_forward", mutates_args=(), device_types="cuda")(_down_proj_forward)
 
 
 @down_proj_forward.register_fake
@@ -163,8 +187,7 @@ def _(act, w_down, weights_out_in=False):
     return act.new_empty(tuple(act.shape[:-1]) + (w_down.shape[0 if weights_out_in else 1],))
 
 
-@torch.library.custom_op("fusedswiglu_amd::down_proj_backward", mutates_args=(), device_types="cuda")
-def down_proj_backward(grad_y: Tensor, act: Tensor, w_down: Tensor, need_act: bool, need_w: bool,
+def _down_proj_backward(grad_y: Tensor, act: Tensor, w_down: Tensor, need_act: bool, need_w: bool,
                        weights_out_in: bool = False) -> Tuple[Tensor, Tensor]:
     """(grad_act, grad_w_down); a gradient that is not needed comes back with zero elements."""
     dtype = _dtype_of(act)
@@ -174,6 +197,9 @@ def down_proj_backward(grad_y: Tensor, act: Tensor, w_down: Tensor, need_act: bo
     d_act = _launch.down_proj_input_grad(grad_y, w_down, dtype, weights_out_in=weights_out_in) if need_act else e
     d_w = _launch.down_proj_weight_grad(act, grad_y, dtype, weights_out_in=weights_out_in) if need_w else e.clone()
     return d_act, d_w
+
+
+down_proj_backward = torch.library.custom_op("fusedswiglu_amd::down_proj_backward", mutates_args=(), device_types="cuda")(_down_proj_backward)
 
 
 @down_proj_backward.register_fake
@@ -191,7 +217,8 @@ def _down_setup(ctx, inputs, output):
 def _down_backward(ctx, grad_y):
     act, w_down = ctx.saved_tensors
     need = ctx.needs_input_grad
-    d_act, d_w = down_proj_backward(grad_y.contiguous(), act, w_down, need[0], need[1], ctx.weights_out_in)
+    backward = _pick(down_proj_backward, _down_proj_backward, grad_y, act, w_down)
+    d_act, d_w = backward(grad_y.contiguous(), act, w_down, need[0], need[1], ctx.weights_out_in)
     return (d_act if need[0] else None, d_w if need[1] else None, None)
 
 
@@ -205,6 +232,25 @@ def _autocast(dtype, *tensors):
     return tensors
 
 
+def _records_gradient(*tensors: Tensor) -> bool:
+    return torch.is_grad_enabled() and any([t.requires_grad for t in tensors])
+
+
+class _no_autocast:
+    """`with torch.autocast("cuda", enabled=False)`, without its cost when autocast is off anyway."""
+    __slots__ = ("guard",)
+
+    def __enter__(self):
+        self.guard = torch.autocast(device_type="cuda", enabled=False) if torch.is_autocast_enabled("cuda") else None
+        if self.guard is not None:
+            self.guard.__enter__()
+
+    def __exit__(self, *exc):
+        if self.guard is not None:
+            return self.guard.__exit__(*exc)
+        return False
+
+
 def swiglu(x: Tensor, w_gate: Tensor, w_up: Tensor, autocast_dtype: torch.dtype | None = torch.bfloat16,
            recompute: bool = False, weights_out_in: bool = False) -> Tensor:
     """silu(x @ w_gate) * (x @ w_up) with weights laid out [d_model, d_intermediate], or
@@ -212,8 +258,12 @@ def swiglu(x: Tensor, w_gate: Tensor, w_up: Tensor, autocast_dtype: torch.dtype 
     (`weights_out_in=True`), which are read in place."""
     _require_gpu(x, w_gate, w_up)
     x, w_gate, w_up = _autocast(autocast_dtype, x, w_gate, w_up)
+    save = _records_gradient(x, w_gate, w_up)
+    if not save and _unobserved(x, w_gate, w_up):
+        with _no_autocast():
+            return _launch.fused_swiglu_fwd(x, w_gate, w_up, _dtype_of(x), save_preactivations=False,
+                                            weights_out_in=weights_out_in)[0]
     with torch.autocast(device_type="cuda", enabled=False):
-        save = torch.is_grad_enabled() and (x.requires_grad or w_gate.requires_grad or w_up.requires_grad)
         return swiglu_forward(x, w_gate, w_up, save and not recompute, weights_out_in)[0]
 
 
@@ -223,6 +273,9 @@ def down_proj(act: Tensor, w_down: Tensor, autocast_dtype: torch.dtype | None = 
     [d_model, d_intermediate] with `weights_out_in=True`)."""
     _require_gpu(act, w_down)
     act, w_down = _autocast(autocast_dtype, act, w_down)
+    if not _records_gradient(act, w_down) and _unobserved(act, w_down):
+        with _no_autocast():
+            return _launch.down_proj_forward(act, w_down, _dtype_of(act), weights_out_in=weights_out_in)
     with torch.autocast(device_type="cuda", enabled=False):
         return down_proj_forward(act, w_down, weights_out_in)
 
@@ -253,7 +306,8 @@ class _PackedSwiGLU(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w_gate_up, recompute, weights_out_in):
         w_gate, w_up = _halves(w_gate_up, weights_out_in)
-        out, g, u = swiglu_forward(x, w_gate, w_up, not recompute, weights_out_in)
+        forward = _pick(swiglu_forward, _swiglu_forward, x, w_gate, w_up)
+        out, g, u = forward(x, w_gate, w_up, not recompute, weights_out_in)
         ctx.save_for_backward(x, w_gate_up, g, u)
         ctx.weights_out_in = weights_out_in
         return out
@@ -263,8 +317,9 @@ class _PackedSwiGLU(torch.autograd.Function):
         x, w_gate_up, g, u = ctx.saved_tensors
         w_gate, w_up = _halves(w_gate_up, ctx.weights_out_in)
         need_x, need_w = ctx.needs_input_grad[:2]
-        dx, dw, _ = swiglu_backward(grad_out.contiguous(), x, w_gate, w_up, g, u,
-                                    need_x, need_w, need_w, True, ctx.weights_out_in)
+        backward = _pick(swiglu_backward, _swiglu_backward, grad_out, x, w_gate, w_up, g, u)
+        dx, dw, _ = backward(grad_out.contiguous(), x, w_gate, w_up, g, u,
+                             need_x, need_w, need_w, True, ctx.weights_out_in)
         return (dx if need_x else None), (dw if need_w else None), None, None
 
 
@@ -276,8 +331,13 @@ def swiglu_packed(x: Tensor, w_gate_up: Tensor, autocast_dtype: torch.dtype | No
         raise _launch.ShapeError("packed weight must be [d_model, 2*d_intermediate] (or [2*d_intermediate, d_model])")
     _require_gpu(x, w_gate_up)
     x, w_gate_up = _autocast(autocast_dtype, x, w_gate_up)
+    save = _records_gradient(x, w_gate_up)
+    if not save and _unobserved(x, w_gate_up):
+        with _no_autocast():
+            return _launch.fused_swiglu_fwd(x, *_halves(w_gate_up, weights_out_in), _dtype_of(x), save_preactivations=False,
+                                            weights_out_in=weights_out_in)[0]
     with torch.autocast(device_type="cuda", enabled=False):
-        if torch.is_grad_enabled() and (x.requires_grad or w_gate_up.requires_grad):
+        if save:
             return _PackedSwiGLU.apply(x, w_gate_up, recompute, weights_out_in)
         w_gate, w_up = _halves(w_gate_up, weights_out_in)
         return swiglu_forward(x, w_gate, w_up, False, weights_out_in)[0]
