@@ -291,8 +291,8 @@ static double estimate_us(const SkPlan& p, long long M, long long Nh, long long 
 // Nh: columns of each half.  Narrow blocks are taken where the estimate sees them ahead by more than it errs among the
 // launches above, whose times they then beat on average by 31 / 23 / 28 / 21 % (forward, [I, D], up to 16 / 32 / 64 / 128
 // rows), 15 / 16 / 19 / 15 % (down projection, nn.Linear's layout), 5 / 2 / 4 / 12 % and 10 / 9 / 2 / 0 % (the other
-// layout), at most 3 % slower anywhere: 1 x 1024 x 3072 [I, D] 10.5 -> 5.6 us, 16 x 2048 x 4096 19 -> 10, 1 x 4096 x 11008
-// 37 -> 33, its down projection 24 -> 21.  [D, I] weights of more than 150 MB stay on blocks of 128: their rows, one
+// layout), at most 3 % slower anywhere: 1 x 1024 x 3072 [I, D] 10.5 -> 5.6 us, 16 x 2048 x 4096 17.6 -> 9.1, 1 x 4096 x 11008
+// 36.9 -> 33.2, the down projection of 64 x 2048 x 4096 15.4 -> 10.9.  [D, I] weights of more than 150 MB stay on blocks of 128: their rows, one
 // segment per k and block, are then read 15 to 20 % slower in shorter segments.
 static SkPlan choose(long long M, long long Nh, long long K, int cus, bool w_kc, bool plain, long long max_splits) {
   SkPlan best = plan_wide(M, Nh, K, cus, w_kc, plain ? max_splits : 0);
