@@ -7,6 +7,7 @@ same operands, rel-L2 <= 1e-2 (bfloat16, fused_swiglu/test_swiglu.py:20) and <= 
 import pytest
 import torch
 
+from fusedswiglu_amd import _abi
 from fusedswiglu_amd.kernels import _launch
 
 pytestmark = pytest.mark.gpu
@@ -48,3 +49,23 @@ def test_few_tokens_on_narrow_blocks(shape, out_in):
     y, da = _launch.down_proj_forward(a, wd, **kw), _launch.down_proj_input_grad(gy, wd, **kw)
     assert rel(y, a.float() @ wdf) < tol and rel(da, gy.float() @ wdf.t()) < tol
     assert torch.equal(y, _launch.down_proj_forward(a, wd, **kw)) and torch.equal(da, _launch.down_proj_input_grad(gy, wd, **kw))
+
+
+@pytest.mark.parametrize("out_in", [False, True], ids=["DI", "ID"])
+@pytest.mark.parametrize("planes", [0, 1, 2, 3, 5, 16])
+def test_down_projection_within_any_scratch(planes, out_in):
+    """The split of the down projection keeps to the scratch it is given: nothing is written behind `planes` fp32 planes, and
+    the result is the same sum in another order."""
+    T, D, I = 8, 1024, 4096
+    L = _abi.lib()
+    torch.manual_seed(planes)
+    a = torch.randn(T, I, device=DEV).bfloat16()
+    wd = (torch.randn(*((D, I) if out_in else (I, D)), device=DEV) * I ** -0.5).bfloat16()
+    want = a.float() @ (wd.float().t() if out_in else wd.float())
+    y, size = torch.empty(T, D, device=DEV, dtype=torch.bfloat16), planes * T * D * 4
+    ws = torch.full((size + 4096,), 0x5A, device=DEV, dtype=torch.uint8)
+    _abi.check(L.fsw_down_proj_forward(a.data_ptr(), wd.data_ptr(), y.data_ptr(), T, I, D, I, I if out_in else D, D,
+                                       ws.data_ptr() if planes else None, size, _abi.WEIGHTS_OUT_IN if out_in else 0,
+                                       torch.cuda.current_stream().cuda_stream))
+    assert rel(y, want) < TOL[torch.bfloat16]
+    assert bool((ws[size:] == 0x5A).all())
