@@ -174,11 +174,12 @@ def _weight_dims(w: torch.Tensor, weights_out_in: bool) -> Tuple[int, int]:
 
 
 def fused_swiglu_fwd(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, dtype: torch.dtype,
-                     save_preactivations: bool = True, weights_out_in: bool = False
+                     save_preactivations: bool = True, weights_out_in: bool = False, dense_preactivations: bool = False
                      ) -> Tuple[torch.Tensor, Optional[torch.Tensor], Optional[torch.Tensor]]:
     """out = silu(x @ w_gate) * (x @ w_up); returns (out, x@w_gate, x@w_up) like
     kernels_bf16.py:162-206.  With save_preactivations=False the two pre-activation arrays are
-    neither allocated nor written and None is returned for them."""
+    neither allocated nor written and None is returned for them.  On padded copies (below) they are views of padded rows
+    unless `dense_preactivations` asks for contiguous arrays."""
     _require(x.ndim >= 2 and w_up.ndim == 2 and w_gate.ndim == 2,
              "Incorrect number of dimensions for LHS or RHS")
     D, I = _weight_dims(w_up, weights_out_in)
@@ -200,7 +201,7 @@ def fused_swiglu_fwd(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, 
     out_shape = tuple(x.shape[:-1]) + (I,)
     px, pg, pu, ldx, ldw = x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), _ld(x2), _ld(wg)
     if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and T * D * I >= _PAD_MIN_WORK:
-        return _padded_fwd(x2, wg, wu, dtype, out_shape, D, I, save_preactivations, weights_out_in)
+        return _padded_fwd(x2, wg, wu, dtype, out_shape, D, I, save_preactivations, weights_out_in, dense_preactivations)
     out = torch.empty(out_shape, device=dev, dtype=dtype)
     g = torch.empty_like(out) if save_preactivations else None
     u = torch.empty_like(out) if save_preactivations else None
@@ -211,8 +212,9 @@ def fused_swiglu_fwd(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, 
     return out, g, u
 
 
-def _padded_fwd(x2, wg, wu, dtype, out_shape, D, I, save_preactivations, weights_out_in):
-    """fused_swiglu_fwd on padded copies.  The pre-activations stay padded: views of [T, I rounded up to 8]."""
+def _padded_fwd(x2, wg, wu, dtype, out_shape, D, I, save_preactivations, weights_out_in, dense_preactivations):
+    """fused_swiglu_fwd on padded copies.  The pre-activations stay padded, views of [T, I rounded up to 8], unless the
+    caller wants them dense."""
     T, dev = x2.shape[0], x2.device
     with _on_device(dev):
         (x2,), (wg, wu) = _padded_copies(x2), _padded_copies(wg, wu)
@@ -223,6 +225,10 @@ def _padded_fwd(x2, wg, wu, dtype, out_shape, D, I, save_preactivations, weights
             g.data_ptr() if g is not None else None, u.data_ptr() if u is not None else None,
             T, D, I, _ld(x2), _ld(wg), _pad8(I), _code(dtype, weights_out_in, True), _stream_ptr(dev)))
         out = _unpadded(out, I).view(out_shape)
+        if dense_preactivations and g is not None and I & 7:
+            dense = torch.empty((T, I), device=dev, dtype=dtype), torch.empty((T, I), device=dev, dtype=dtype)
+            _repack(g, dense[0], I, False, u, dense[1])
+            return out, dense[0].view(out_shape), dense[1].view(out_shape)
     if g is not None:
         wide = out_shape[:-1] + (_pad8(I),)
         g, u = g.view(wide)[..., :I], u.view(wide)[..., :I]
