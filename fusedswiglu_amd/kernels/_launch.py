@@ -111,6 +111,9 @@ def _code(dtype: torch.dtype, weights_out_in: bool, padded: bool = False) -> int
 # matrix product the edge-shape kernel's fewer launches win: forward / backward at 2^21.5 33 / 56 against 46 / 75 us, at
 # 2^23.5 38 / 79 against 46 / 76, at 2^24.5 39 / 100 against 46 / 77, at 2^25.2 69 / 224 against 46 / 77.
 _PAD_MIN_WORK = 1 << 24
+# The tiled kernels address rows of less than this many elements: operands with a larger pitch are copied as well, and a
+# problem whose padded rows would be longer stays on the edge-shape kernel, which has no such limit.
+_TILED_MAX_LD = 1 << 21
 
 
 def _pad8(n: int) -> int:
@@ -133,7 +136,7 @@ def _repack(src: torch.Tensor, dst: torch.Tensor, cols: int, pad: bool, src1: Op
 def _padded_copies(*ts: torch.Tensor) -> Tuple[torch.Tensor, ...]:
     """[rows, cols] tensors (one, or two with the same shape and row pitch) as padded, aligned copies
     [rows, cols rounded up to 8]; as they are when the tiled kernels can read them directly."""
-    if all(_whole_chunks(t) for t in ts):
+    if all(_whole_chunks(t) and _ld(t) < _TILED_MAX_LD for t in ts):
         return ts
     rows, cols = ts[0].shape
     out = tuple(torch.empty((rows, _pad8(cols)), device=t.device, dtype=t.dtype) for t in ts)
@@ -154,13 +157,13 @@ def _unpadded(t: torch.Tensor, cols: int) -> torch.Tensor:
     return out
 
 
-def pads_rows(x: torch.Tensor, I: int) -> bool:
-    """Whether a problem with this x and dimensions that are not multiples of 8 runs on padded copies."""
-    return x.numel() * I >= _PAD_MIN_WORK
+def pads_rows(T: int, D: int, I: int) -> bool:
+    """Whether a problem of these sizes runs on padded copies if its rows are not whole, aligned 16-byte chunks."""
+    return T * D * I >= _PAD_MIN_WORK and D <= _TILED_MAX_LD - 8 and I <= _TILED_MAX_LD - 8
 
 
 def _wants_padding(T: int, D: int, I: int, *ts: torch.Tensor) -> bool:
-    if T * D * I < _PAD_MIN_WORK:
+    if not pads_rows(T, D, I):
         return False
     bits = D | I
     for t in ts:
@@ -200,7 +203,7 @@ def fused_swiglu_fwd(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, 
     T = x2.shape[0]
     out_shape = tuple(x.shape[:-1]) + (I,)
     px, pg, pu, ldx, ldw = x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), _ld(x2), _ld(wg)
-    if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and T * D * I >= _PAD_MIN_WORK:
+    if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and pads_rows(T, D, I):
         return _padded_fwd(x2, wg, wu, dtype, out_shape, D, I, save_preactivations, weights_out_in, dense_preactivations)
     out = torch.empty(out_shape, device=dev, dtype=dtype)
     g = torch.empty_like(out) if save_preactivations else None
@@ -405,7 +408,7 @@ def swiglu_backward(grad_output: torch.Tensor, x: torch.Tensor, w_gate: torch.Te
         wg, wu = wg.contiguous(), wu.contiguous()
     T = x2.shape[0]
     px, pg, pu, ldx, ldw = x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), _ld(x2), _ld(wg)
-    if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and T * D * I >= _PAD_MIN_WORK:
+    if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and pads_rows(T, D, I):
         grad_xw_up, grad_xw_gate = elementwise_backward(grad_output, xw_gate, xw_up, dtype, padded=True)
         grad_w_up = grad_w_gate = grad_x = None
         if need_weight_grad or need_input_grad:
@@ -460,7 +463,7 @@ def fused_weight_grad(x: torch.Tensor, grad_xw_up: torch.Tensor, grad_xw_gate: t
     I = padded_from or du.shape[1]
     wshape = (I, D) if weights_out_in else (D, I)
     pad = bool(padded_from) or _wants_padding(T, D, I, x2, du, dg) or (
-        out is not None and T * D * I >= _PAD_MIN_WORK and not all(_whole_chunks(t) for t in out))
+        out is not None and pads_rows(T, D, I) and not all(_whole_chunks(t) for t in out))
     if pad and out is None:
         with _on_device(dev):
             (x2,), (du, dg) = _padded_copies(x2), (du, dg) if padded_from else _padded_copies(du, dg)

@@ -1,0 +1,87 @@
+"""Which calls the launchers hand to the library with padded rows: only those that the tiled kernels can address (row pitches
+below 2^21 elements), so that every other call still finds the edge-shape kernel.  Host tensors; the library calls are
+recorded instead of made."""
+import pytest
+import torch
+
+from fusedswiglu_amd import _abi, ops
+from fusedswiglu_amd.kernels import _launch
+
+MAX_LD = 1 << 21
+BF = torch.bfloat16
+# positions of the leading dimensions and of the dtype code in the argument lists of the entry points
+LDS = {"fsw_swiglu_forward": ((9, 10, 11), 12), "fsw_gating_grad_recompute": ((9, 10, 11), 12), "fsw_input_grad": ((8, 9, 10), 13),
+       "fsw_weight_grad": ((8, 9, 10), 13), "fsw_swiglu_backward": ((14, 15, 16, 17), 20),
+       **{f"fsw_down_proj_{k}": ((6, 7, 8), 11) for k in ("forward", "input_grad", "weight_grad")}}
+
+
+class Recorder:
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        def call(*args):
+            if name in LDS:
+                lds, code = LDS[name]
+                self.calls.append((name, [args[i] for i in lds], bool(args[code] & _abi.ROWS_PADDED)))
+            return 0
+        return call
+
+
+@pytest.fixture
+def library(monkeypatch):
+    L = Recorder()
+    monkeypatch.setattr(_launch._abi, "lib", lambda: L)
+    monkeypatch.setattr(_launch, "_stream_ptr", lambda dev: 0)
+    monkeypatch.setattr(_launch, "_check_device", lambda *tensors: tensors[0].device)
+    monkeypatch.setattr(_launch, "_PAD_MIN_WORK", 0)
+    return L
+
+
+def every_launcher(x, wg, wu, wd, dy, dz, oi):
+    kw = dict(dtype=BF, weights_out_in=oi)
+    _, g, u = _launch.fused_swiglu_fwd(x, wg, wu, **kw)
+    _launch.swiglu_backward(dy, x, wg, wu, g, u, **kw)
+    _launch.fused_input_grad(dy, dy, wg, wu, **kw)
+    _launch.fused_weight_grad(x, dy, dy, **kw)
+    _launch.gating_grad_recompute(dy, x, wg, wu, **kw)
+    _launch.down_proj_forward(dy, wd, **kw)
+    _launch.down_proj_input_grad(dz, wd, **kw)
+    _launch.down_proj_weight_grad(dy, dz, **kw)
+    for packed in (False, True):
+        for saved in (g, g.new_empty(0)):
+            ops._swiglu_backward(dy, x, wg, wu, saved, saved, True, True, True, packed, oi)
+
+
+def array(rows, cols, pitch=0, skew=0):
+    """Uninitialised [rows, cols] with the given row pitch, `skew` elements into its allocation."""
+    pitch = pitch or cols
+    return torch.empty((rows - 1) * pitch + cols + skew, dtype=BF).as_strided((rows, cols), (pitch, 1), skew)
+
+
+@pytest.mark.parametrize("oi", [False, True], ids=["DI", "ID"])
+@pytest.mark.parametrize("D,I", [(9, MAX_LD + 3), (3, MAX_LD - 7), (MAX_LD - 1, 5), (3, MAX_LD - 9), (9, 17)], ids=str)
+def test_row_lengths(library, D, I, oi):
+    T = 2
+    w = array(*((I, D) if oi else (D, I)))
+    every_launcher(array(T, D), w, w, array(*((D, I) if oi else (I, D))), array(T, I), array(T, D), oi)
+    fits = (max(D, I) + 7) & ~7 < MAX_LD
+    assert len(library.calls) > 10
+    for name, lds, padded in library.calls:
+        assert padded == fits, name
+        assert not padded or max(lds) < MAX_LD, (name, lds)
+
+
+@pytest.mark.parametrize("oi", [False, True], ids=["DI", "ID"])
+@pytest.mark.parametrize("wide", range(4), ids=["x", "w", "w_down", "dy"])
+def test_row_pitches(library, wide, oi):
+    """One operand in rows of 2^21 elements, the others unaligned."""
+    T, D, I = 3, 16, 24
+    pitch = [MAX_LD if i == wide else 0 for i in range(4)]
+    skew = [0 if p else 1 for p in pitch]
+    x, dy = array(T, D, pitch[0], skew[0]), array(T, I, pitch[3], skew[3])
+    w = array(*((I, D) if oi else (D, I)), pitch[1], skew[1])
+    every_launcher(x, w, w, array(*((D, I) if oi else (I, D)), pitch[2], skew[2]), dy, array(T, D, 0, 1), oi)
+    assert any(padded for _, _, padded in library.calls)
+    for name, lds, padded in library.calls:
+        assert not padded or max(lds) < MAX_LD, (name, lds)
