@@ -62,8 +62,8 @@ inline long long tail_bytes(const TailPlan& t) { return (long long)t.count * t.p
 // Scratch a caller is asked for: enough to split the reduction until whole tiles fill the chip (as far as that pays at
 // 1 us per step and 4 TB/s for the partial tiles), or to split the tail.  Plans take what is offered, up to this or to
 // what plan() wants on top.
-inline int scratch_splits(long long tiles, int steps, double result_elems) {
-  if (tiles >= 1024 || steps < 32) return 1;
+inline SplitPlan scratch_splits(long long tiles, int steps, double result_elems) {
+  if (tiles >= 1024 || steps < 32) return SplitPlan{1, steps};
   auto cost = [&](int s) {
     const double rounds = (double)((tiles * s + kCus - 1) / kCus);
     return rounds * ((double)steps / s + 6.0) * 0.96 + (s > 1 ? 2.0 * s * result_elems * 4.0 / 4.0e6 : 0.0);
@@ -75,7 +75,7 @@ inline int scratch_splits(long long tiles, int steps, double result_elems) {
     const double c = cost(s);
     if (c < best_cost * 0.95) { best_cost = c; best = s; }
   }
-  return split_steps(steps, best).splits;
+  return split_steps(steps, best);
 }
 
 inline int steps_of(int mode, long long K) {
@@ -132,6 +132,21 @@ Plan plan(long long M, long long N, long long K, long long ws_bytes) {
   return best;
 }
 
+// The eight-wave form has tiles of 256 rows (kDwT 128) only and takes the split that scratch was asked for, or none: its
+// operands span 2^31 bytes along the reduction, so few tiles mean a reduction of thousands of steps for each.  Weight
+// gradients of 131072 x 256 x 8192, 524288 x 1024 x 2048 and 2097152 x 256 x 768: 1.1, 3.5 and 1.9 ms split, 2.5, 9.6 and
+// 38 ms on whole tiles.
+template <int MODE>
+Plan plan_eight_waves(long long M, long long N, long long K, long long ws_bytes) {
+  using C = Cfg<MODE>;
+  const int steps = steps_of(MODE, K);
+  const long long tiles = ((M + C::kTileM - 1) / C::kTileM) * ((N + C::kTileN - 1) / C::kTileN);
+  SplitPlan sp{1, steps};
+  if (!C::kForward) sp = scratch_splits(tiles, steps, (double)M * N * C::kResults);
+  if (sp.splits > 1 && (double)sp.splits * M * N * 4 * C::kResults > (double)ws_bytes) sp = SplitPlan{1, steps};
+  return Plan{8, sp.splits, sp.steps_per_split, 0, 0, 1, steps};
+}
+
 // Scratch for a GEMM of the given mode with results `results` x [M, N] and a reduction of K per pass.
 template <int MODE>
 long long workspace_of(long long M, long long N, long long K, bool with_tail = true) {
@@ -140,7 +155,7 @@ long long workspace_of(long long M, long long N, long long K, bool with_tail = t
   const long long tiles = ((M + C::kTileM - 1) / C::kTileM) * ((N + C::kTileN - 1) / C::kTileN);
   const int steps = steps_of(MODE, K);
   const long long plane = M * N * 4 * C::kResults;
-  const int asked = scratch_splits(tiles, steps, (double)M * N * C::kResults);
+  const int asked = scratch_splits(tiles, steps, (double)M * N * C::kResults).splits;
   if (!with_tail) return asked > 1 ? asked * plane : 0;
   const Plan p = plan<MODE>(M, N, K, 1LL << 62);
   return std::max({asked > 1 ? asked * plane : 0LL, p.splits > 1 ? p.splits * plane : 0LL, asked > 1 ? 0LL : tail_bytes(plan_tail(tiles, steps))});
@@ -163,8 +178,7 @@ hipError_t launch_typed(GemmParams g, hipStream_t s, void* ws, long long ws_byte
   // The four-wave form walks an m/n-contiguous operand through 32-bit offsets from its first k-row; larger operands
   // take the eight-wave form (256-row tiles).
   const bool fits = (C::kAKc || (long long)g.K * g.lda * 2 < (1LL << 31)) && (C::kBKc || (long long)g.K * g.ldb * 2 < (1LL << 31));
-  Plan p{8, 1, steps_of(MODE, g.K), 0, 0, 1, 0};
-  if (fits) p = plan<MODE>(g.M, g.N, g.K, ws ? ws_bytes : 0);
+  const Plan p = fits ? plan<MODE>(g.M, g.N, g.K, ws ? ws_bytes : 0) : plan_eight_waves<MODE>(g.M, g.N, g.K, ws ? ws_bytes : 0);
   const int tile_m = C::kTileM * p.mb / 8;
   g.tiles_m = (g.M + tile_m - 1) / tile_m;
   g.tiles_n = (g.N + C::kTileN - 1) / C::kTileN;
