@@ -411,13 +411,11 @@ def swiglu_backward(grad_output: torch.Tensor, x: torch.Tensor, w_gate: torch.Te
     if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and pads_rows(T, D, I):
         grad_xw_up, grad_xw_gate = elementwise_backward(grad_output, xw_gate, xw_up, dtype, padded=True)
         grad_w_up = grad_w_gate = grad_x = None
-        if need_weight_grad or need_input_grad:
-            with _on_device(dev):
-                (x2,), (wg, wu) = _padded_copies(x2), _padded_copies(wg, wu)
-        if need_weight_grad:
-            grad_w_up, grad_w_gate = _padded_weight_grad(x2, grad_xw_up, grad_xw_gate, dtype, D, I, weights_out_in)
-        if need_input_grad:
-            grad_x = _padded_input_grad(grad_xw_gate, grad_xw_up, wg, wu, dtype, D, I, weights_out_in).view(x.shape)
+        with _on_device(dev):
+            if need_weight_grad:
+                grad_w_up, grad_w_gate = _padded_weight_grad(*_padded_copies(x2), grad_xw_up, grad_xw_gate, dtype, D, I, weights_out_in)
+            if need_input_grad:
+                grad_x = _padded_input_grad(grad_xw_gate, grad_xw_up, *_padded_copies(wg, wu), dtype, D, I, weights_out_in).view(x.shape)
         return grad_x, grad_w_gate, grad_w_up
     # the gating gradient indexes flat, dense arrays
     dout, g, u = grad_output.contiguous(), xw_gate.contiguous(), xw_up.contiguous()

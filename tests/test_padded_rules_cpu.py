@@ -85,3 +85,45 @@ def test_row_pitches(library, wide, oi):
     assert any(padded for _, _, padded in library.calls)
     for name, lds, padded in library.calls:
         assert not padded or max(lds) < MAX_LD, (name, lds)
+
+
+@pytest.mark.parametrize("D,I", [(16, 24), (15, 24), (16, 23), (15, 23)], ids=str)
+def test_every_launch_is_made_on_the_operands_device(library, monkeypatch, D, I):
+    """Kernels go to the current device: each library call that takes a stream is made inside the device guard."""
+    inside = []
+
+    class Guard:
+        def __init__(self, dev):
+            pass
+
+        def __enter__(self):
+            inside.append(True)
+
+        def __exit__(self, *exc):
+            inside.pop()
+
+    class Guarded:
+        def __getattr__(self, name):
+            def call(*args):
+                assert inside or name == "fsw_workspace_bytes", f"{name} outside the device guard"
+                return 0
+            return call
+
+    monkeypatch.setattr(_launch, "_on_device", Guard)
+    monkeypatch.setattr(_launch._abi, "lib", Guarded)
+    for oi in (False, True):
+        w = array(*((I, D) if oi else (D, I)))
+        every_launcher(array(3, D), w, w, array(*((D, I) if oi else (I, D))), array(3, I), array(3, D), oi)
+
+
+@pytest.mark.parametrize("need", [(True, False), (False, True), (False, False)], ids=["input", "weights", "none"])
+def test_only_what_a_gradient_reads_is_copied(library, monkeypatch, need):
+    """The padded backward copies x for the weight gradients and the weights for the input gradient."""
+    copied = []
+    repack = _launch._repack
+    monkeypatch.setattr(_launch, "_repack", lambda src, dst, cols, pad, *two: (pad and copied.append(tuple(src.shape)),
+                                                                              repack(src, dst, cols, pad, *two)))
+    T, D, I = 3, 15, 23
+    x, w, y = array(T, D), array(D, I), array(T, I)
+    _launch.swiglu_backward(y, x, w, w, y, y, BF, need_input_grad=need[0], need_weight_grad=need[1])
+    assert copied == [(D, I)] * need[0] + [(T, D)] * need[1]
