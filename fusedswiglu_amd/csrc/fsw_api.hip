@@ -459,7 +459,8 @@ int fsw_input_grad_noalloc(const void* grad_xw_gate, const void* grad_xw_up, con
     return e;
   // only the split reduction of small problems needs its scratch; a large problem whose optional tail split
   // would not fit the buffer simply runs without it
-  const int64_t need = fsw::splitk_workspace_bytes(out_in_of(dtype) ? 4 : 1, T, D, I, /*with_tail=*/false);
+  const int64_t cols = padded_of(dtype) ? fsw::result_cols(D) : D;
+  const int64_t need = fsw::splitk_workspace_bytes(out_in_of(dtype) ? 4 : 1, T, cols, I, /*with_tail=*/false);
   if (need > (int64_t)FSW_NOALLOC_SCRATCH_BYTES)
     return fail(FSW_ERR_SCRATCH_LIMIT,
                 "%s: T=%lld D=%lld I=%lld needs %lld bytes of split-reduction scratch, the built-in buffer holds %lld; "

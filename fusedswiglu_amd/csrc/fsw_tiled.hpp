@@ -147,11 +147,12 @@ Plan plan_eight_waves(long long M, long long N, long long K, long long ws_bytes)
   return Plan{8, sp.splits, sp.steps_per_split, 0, 0, 1, steps};
 }
 
-// Scratch for a GEMM of the given mode with results `results` x [M, N] and a reduction of K per pass.
+// Scratch for a GEMM of the given mode with results `results` x [M, N] and a reduction of K per pass.  with_tail: as a
+// caller is told, enough for whatever plan() may choose and for padded rows; without, the split reduction alone.
 template <int MODE>
 long long workspace_of(long long M, long long N, long long K, bool with_tail = true) {
   using C = Cfg<MODE>;
-  N = result_cols(N);
+  if (with_tail) N = result_cols(N);
   const long long tiles = ((M + C::kTileM - 1) / C::kTileM) * ((N + C::kTileN - 1) / C::kTileN);
   const int steps = steps_of(MODE, K);
   const long long plane = M * N * 4 * C::kResults;
