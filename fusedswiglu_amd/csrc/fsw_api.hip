@@ -332,6 +332,13 @@ int fsw_swiglu_backward(const void* grad_out, const void* xw_gate, const void* x
     if (int e = check_weight_grad_args(fn, x, grad_xw_up, grad_xw_gate, grad_w_up, grad_w_gate, T, D, I, ldx, ldi, ld_dw, dtype))
       return e;
   if (padded) {
+    // the two GEMMs refuse what their kernels cannot take: asked before the first launch
+    fsw::Problem p{};
+    p.x = x; p.wg = w_gate; p.wu = w_up; p.dG = grad_xw_gate; p.dU = grad_xw_up;
+    p.dx = grad_x; p.dWg = grad_w_gate; p.dWu = grad_w_up;
+    p.T = T; p.D = D; p.I = I; p.ldx = ldx; p.ldw = ldw; p.ldo = ldi; p.lddx = ld_dx; p.lddw = ld_dw;
+    p.w_out_in = out_in_of(dtype); p.padded = true;
+    if ((grad_x && !fsw::fast_path_ok_input_grad(p)) || (grad_w_gate && !fsw::fast_path_ok_weight_grad(p))) return not_padded(fn);
     if (int e = fsw_elementwise_backward_rows(grad_out, xw_gate, xw_up, grad_xw_up, grad_xw_gate, T, I, I, ldi, ldi,
                                               elem_of(dtype), stream))
       return e;
