@@ -215,7 +215,8 @@ int fsw_elementwise_backward(const void* grad_out, const void* xw_gate, const vo
   const char* fn = "fsw_elementwise_backward";
   if (!grad_out || !xw_gate || !xw_up || !grad_xw_up || !grad_xw_gate)
     return fail(FSW_ERR_NULL_POINTER, "%s: all five arrays must be non-null", fn);
-  if (!dtype_ok(dtype)) return fail(FSW_ERR_BAD_DTYPE, "%s: dtype %d is neither bf16 (0) nor fp16 (1)", fn, dtype);
+  // (dense arrays of `numel` elements have no rows that could be padded)
+  if (!dtype_ok(dtype) || padded_of(dtype)) return fail(FSW_ERR_BAD_DTYPE, "%s: dtype %d is neither bf16 (0) nor fp16 (1)", fn, dtype);
   dtype = elem_of(dtype);
   if (numel <= 0) return fail(FSW_ERR_BAD_SHAPE, "%s: numel must be positive (got %lld)", fn, (long long)numel);
   if (!al2(grad_out) || !al2(xw_gate) || !al2(xw_up) || !al2(grad_xw_up) || !al2(grad_xw_gate))

@@ -50,3 +50,8 @@ def test_other_entry_points(L, oi):
     assert L.fsw_down_proj_input_grad(P, ODD, P, T, I, D, D8, d8, I8, None, 0, PAD | oi, None) == ALIGNMENT
     assert L.fsw_down_proj_weight_grad(P, P, ODD, T, I, D, I8, D8, d8, None, 0, PAD | oi, None) == ALIGNMENT
     assert b"FSW_ROWS_PADDED" in L.fsw_last_error()
+
+
+def test_dense_gating_gradient_has_no_rows_to_pad(L):
+    """fsw_elementwise_backward takes dense arrays: the flag is refused there, not ignored."""
+    assert L.fsw_elementwise_backward(P, P, P, P, P, 8, PAD, None) == 2
