@@ -460,17 +460,8 @@ def fused_weight_grad(x: torch.Tensor, grad_xw_up: torch.Tensor, grad_xw_gate: t
     T, D = x2.shape
     I = padded_from or du.shape[1]
     wshape = (I, D) if weights_out_in else (D, I)
-    pad = bool(padded_from) or _wants_padding(T, D, I, x2, du, dg) or (
-        out is not None and pads_rows(T, D, I) and not all(_whole_chunks(t) for t in out))
-    if pad and out is None:
-        with _on_device(dev):
-            (x2,), (du, dg) = _padded_copies(x2), (du, dg) if padded_from else _padded_copies(du, dg)
-            return _padded_weight_grad(x2, du, dg, dtype, D, I, weights_out_in)
-    if out is None:
-        grad_w_up = torch.empty(wshape, device=dev, dtype=dtype)
-        grad_w_gate = torch.empty(wshape, device=dev, dtype=dtype)
-    else:
-        grad_w_up, grad_w_gate = out
+    if out is not None:
+        out = grad_w_up, grad_w_gate = tuple(out)
         _require(tuple(grad_w_up.shape) == wshape and tuple(grad_w_gate.shape) == wshape,
                  f"weight-gradient outputs must be {list(wshape)}")
         _require(grad_w_up.dtype == dtype and grad_w_gate.dtype == dtype, f"Expected {dtype} tensors")
@@ -478,10 +469,14 @@ def fused_weight_grad(x: torch.Tensor, grad_xw_up: torch.Tensor, grad_xw_gate: t
         _require(grad_w_up.stride(-1) == 1 and grad_w_gate.stride(-1) == 1 and _ld(grad_w_up) == _ld(grad_w_gate)
                  and _ld(grad_w_up) >= wshape[1],
                  "weight-gradient outputs need unit inner stride and equal row strides")
-        if pad:
-            with _on_device(dev):
-                (x2,), (du, dg) = _padded_copies(x2), (du, dg) if padded_from else _padded_copies(du, dg)
-                return _padded_weight_grad(x2, du, dg, dtype, D, I, weights_out_in, out=(grad_w_up, grad_w_gate))
+    if padded_from or _wants_padding(T, D, I, x2, du, dg) or (
+            out is not None and pads_rows(T, D, I) and not all(_whole_chunks(t) for t in out)):
+        with _on_device(dev):
+            (x2,), (du, dg) = _padded_copies(x2), (du, dg) if padded_from else _padded_copies(du, dg)
+            return _padded_weight_grad(x2, du, dg, dtype, D, I, weights_out_in, out=out)
+    if out is None:
+        grad_w_up = torch.empty(wshape, device=dev, dtype=dtype)
+        grad_w_gate = torch.empty(wshape, device=dev, dtype=dtype)
     with _on_device(dev):
         flag = _abi.WEIGHTS_OUT_IN if weights_out_in else 0
         ws, ws_bytes = _workspace(_abi.STEP_WEIGHT_GRAD | flag, T, D, I, dev)

@@ -127,3 +127,13 @@ def test_only_what_a_gradient_reads_is_copied(library, monkeypatch, need):
     x, w, y = array(T, D), array(D, I), array(T, I)
     _launch.swiglu_backward(y, x, w, w, y, y, BF, need_input_grad=need[0], need_weight_grad=need[1])
     assert copied == [(D, I)] * need[0] + [(T, D)] * need[1]
+
+
+@pytest.mark.parametrize("D,I", [(16, 24), (15, 24), (16, 23)], ids=str)
+@pytest.mark.parametrize("bad", [lambda D, I: torch.empty(D * I, dtype=BF), lambda D, I: torch.empty(D, I + 1, dtype=BF),
+                                 lambda D, I: torch.empty((), dtype=BF), lambda D, I: torch.empty(I, D, dtype=BF).t(),
+                                 lambda D, I: torch.empty(D, I)], ids=["flat", "columns", "scalar", "stride", "type"])
+def test_unfit_weight_gradient_outputs_are_shape_errors(library, D, I, bad):
+    with pytest.raises(_launch.ShapeError):
+        _launch.fused_weight_grad(array(3, D), array(3, I), array(3, I), BF, out=(bad(D, I), bad(D, I)))
+    assert not library.calls
