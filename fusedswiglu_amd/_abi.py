@@ -13,7 +13,7 @@ import threading
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIBRARY_PATH = os.path.join(_CSRC, "libfusedswiglu.so")
-#: machine probes for the benchmark harness: a separate library, not part of the drop-in boundary
+#: machine probes for the benchmark harness and launch plans for the tests: a separate library, not part of the drop-in boundary
 BENCH_LIBRARY_PATH = os.path.join(_CSRC, "libfusedswiglu_bench.so")
 
 DTYPE_BF16 = 0
@@ -51,7 +51,8 @@ EXPORTED_SYMBOLS = (
     "fsw_down_proj_weight_grad",
 )
 #: every symbol include/fusedswiglu_bench.h declares (libfusedswiglu_bench.so)
-BENCH_SYMBOLS = ("fsw_probe_mfma", "fsw_probe_stream_read", "fsw_probe_mfma_mix", "fsw_probe_dma_read")
+BENCH_SYMBOLS = ("fsw_probe_mfma", "fsw_probe_stream_read", "fsw_probe_mfma_mix", "fsw_probe_dma_read", "fsw_plan_tiled",
+                 "fsw_plan_few_tokens")
 
 
 class FusedSwiGLUError(RuntimeError):
@@ -139,7 +140,7 @@ _bench_lib = None
 
 
 def bench_lib() -> ctypes.CDLL:
-    """The probe library of the benchmark harness (include/fusedswiglu_bench.h)."""
+    """The probes and launch plans (include/fusedswiglu_bench.h)."""
     global _bench_lib
     if _bench_lib is not None:
         return _bench_lib
@@ -156,6 +157,9 @@ def bench_lib() -> ctypes.CDLL:
             L.fsw_probe_dma_read.argtypes = [vp, i64, ci, vp]
             L.fsw_probe_mfma_mix.restype = ci
             L.fsw_probe_mfma_mix.argtypes = [ci, ci, ci, vp, i64, vp, vp, ctypes.POINTER(ctypes.c_double)]
+            pi = ctypes.POINTER(ci)
+            L.fsw_plan_tiled.argtypes = [ci, i64, i64, i64, i64, pi, pi, pi]
+            L.fsw_plan_few_tokens.argtypes = [ci, ci, i64, i64, i64, ci, i64, pi, pi, pi, pi]
             _bench_lib = L
     return _bench_lib
 

@@ -1,9 +1,10 @@
 // Two machine probes used by the benchmark to state practical ceilings next to the nominal peaks:
 // a register-only MFMA loop (no memory traffic at all) and a streaming read.  They only enqueue a
-// kernel; the caller times them with events on the same stream.
+// kernel; the caller times them with events on the same stream.  And the plans of the product's launches, for tests.
 #include "../../include/fusedswiglu.h"
 #include "../../include/fusedswiglu_bench.h"
-#include "fsw_common.hpp"
+#include "fsw_skinny_plan.hpp"
+#include "fsw_tiled.hpp"
 
 namespace fsw {
 
@@ -205,6 +206,38 @@ int fsw_probe_dma_read(const void* buf, int64_t bytes, int non_temporal, void* s
   if (non_temporal) fsw::probe_dma_read_kernel<true><<<2048, 256, 0, (hipStream_t)stream>>>((const char*)buf, (unsigned)bytes);
   else fsw::probe_dma_read_kernel<false><<<2048, 256, 0, (hipStream_t)stream>>>((const char*)buf, (unsigned)bytes);
   return hipGetLastError() == hipSuccess ? FSW_OK : FSW_ERR_LAUNCH;
+}
+
+int fsw_plan_tiled(int mode, int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int* blocks, int* splits, int* tail_parts) {
+  if (M <= 0 || N <= 0 || K <= 0 || !blocks || !splits || !tail_parts) return FSW_ERR_BAD_SHAPE;
+  fsw::Plan p;
+  switch (mode) {
+    case fsw::kFwd: p = fsw::plan<fsw::kFwd>(M, N, K, workspace_bytes); break;
+    case fsw::kDx: p = fsw::plan<fsw::kDx>(M, N, K, workspace_bytes); break;
+    case fsw::kDw: p = fsw::plan<fsw::kDw>(M, N, K, workspace_bytes); break;
+    case fsw::kNN: p = fsw::plan<fsw::kNN>(M, N, K, workspace_bytes); break;
+    case fsw::kNT: p = fsw::plan<fsw::kNT>(M, N, K, workspace_bytes); break;
+    case fsw::kTN: p = fsw::plan<fsw::kTN>(M, N, K, workspace_bytes); break;
+    case fsw::kFwdT: p = fsw::plan<fsw::kFwdT>(M, N, K, workspace_bytes); break;
+    case fsw::kDxT: p = fsw::plan<fsw::kDxT>(M, N, K, workspace_bytes); break;
+    case fsw::kDwT: p = fsw::plan<fsw::kDwT>(M, N, K, workspace_bytes); break;
+    default: return FSW_ERR_BAD_SHAPE;
+  }
+  *blocks = p.mb;
+  *splits = p.splits;
+  *tail_parts = p.tail_count > 0 ? p.tail_parts : 1;
+  return FSW_OK;
+}
+
+int fsw_plan_few_tokens(int out_in, int down, int64_t M, int64_t N, int64_t K, int cus, int64_t planes, int* slot, int* blocks,
+                        int* columns, int* splits) {
+  if (M <= 0 || M > 128 || N <= 0 || K <= 0 || cus <= 0 || !slot || !blocks || !columns || !splits) return FSW_ERR_BAD_SHAPE;
+  const fsw::SkPlan p = fsw::choose(M, down ? N / 2 : N, K, cus, out_in != 0, down != 0, down ? planes : 1);
+  *slot = p.slot;
+  *blocks = p.slot == 128 ? (M <= 32 ? 2 : (M <= 64 ? 4 : 8)) : p.mq;
+  *columns = p.bn;
+  *splits = p.splits;
+  return FSW_OK;
 }
 
 }  // extern "C"

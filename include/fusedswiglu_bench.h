@@ -1,5 +1,5 @@
 /*
- * libfusedswiglu_bench -- machine probes for the benchmark harness.  Not part of the drop-in boundary
+ * libfusedswiglu_bench -- machine probes for the benchmark harness and launch plans for the tests.  Not part of the drop-in boundary
  * (include/fusedswiglu.h) and not linked into libfusedswiglu.so: a separate library built from
  * fusedswiglu_amd/csrc/fsw_probe.hip.  Status codes are those of fusedswiglu.h.
  */
@@ -42,6 +42,21 @@ FSW_API int fsw_probe_stream_read(const void* buf, int64_t bytes, void* sink4, v
 FSW_API int fsw_probe_dma_read(const void* buf, int64_t bytes, int non_temporal, void* stream);
 FSW_API int fsw_probe_mfma_mix(int mix, int iters, int workgroups, const void* buf, int64_t bytes, void* sink4,
                        void* stream, double* flop_out);
+
+/*
+ * How the product cuts a problem into workgroups: pure host arithmetic, the functions that its launches use, so that a
+ * test can state which kernel variants its shapes reach.
+ * fsw_plan_tiled: a launch of the tiled kernels with results [M,N] and a reduction of K per pass, in mode 0 .. 8 = forward,
+ * input gradient, weight gradient ([D,I] weights), C = A B, A B^T, A^T B, forward, input gradient, weight gradient ([I,D]
+ * weights).  blocks: 16-row blocks per wave (4 .. 8); splits of the reduction; parts of each tile of the last round (1: whole).
+ * fsw_plan_few_tokens: at most 128 rows, the forward (down 0, N = I) or a down projection (down 1, N result columns, scratch
+ * for `planes` fp32 planes [M,N]) with weights whose reduction index is contiguous (out_in 1) or not, on `cus` compute units.
+ * slot: column width of the variant (16, 32, 64, 128); blocks: its 16-row blocks of x; columns used of each slot; splits.
+ */
+FSW_API int fsw_plan_tiled(int mode, int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int* blocks, int* splits,
+                           int* tail_parts);
+FSW_API int fsw_plan_few_tokens(int out_in, int down, int64_t M, int64_t N, int64_t K, int cus, int64_t planes, int* slot,
+                                int* blocks, int* columns, int* splits);
 
 #ifdef __cplusplus
 }

@@ -2,8 +2,9 @@
 gradient of [I, D] weights) and how often its reduction is split from the shape.  These shapes are small ones at which each
 of the choices is made, with remainders in every direction: per launcher (forward and recomputed gating gradient, input
 gradient, weight gradient, and the three products of the down projection) every row count with and without a split
-reduction.  Whole arrays against fp32 products of the same operands, rel-L2 <= 1e-2 (bfloat16,
-fused_swiglu/test_swiglu.py:20) and <= 5e-3 (float16)."""
+reduction, save those that test_variants_gpu.py adds (test_variants_cpu.py asserts that nothing is left out).
+Whole arrays against fp32 products of the same operands, rel-L2 <= 1e-2 (bfloat16, fused_swiglu/test_swiglu.py:20) and <= 5e-3
+(float16)."""
 import pytest
 import torch
 

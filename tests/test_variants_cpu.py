@@ -1,0 +1,89 @@
+"""Which kernel variants the GPU tests' shapes reach, asked of the functions that plan the launches: every variant that is
+compiled, in both element types.  A change of a rule or of its constants that moves a variant out of the lists fails here."""
+import ctypes
+
+import pytest
+
+import test_narrow_blocks_gpu
+import test_tile_rows_gpu
+import test_variants_gpu
+from fusedswiglu_amd import _abi
+
+CUS = 256
+FWD, DX, DW, NN, NT, TN, FWD_T, DX_T, DW_T = range(9)
+FORWARDS = (FWD, FWD_T)
+
+
+def ask(fn, *args, results):
+    v = [ctypes.c_int() for _ in range(results)]
+    assert fn(*args, *v) == 0
+    return tuple(x.value for x in v)
+
+
+def tiled_variants(T, D, I, oi):
+    """(mode, 16-row blocks per wave, how) of every launcher's tiled launches, as the Python launchers make them"""
+    L, flag = _abi.lib(), _abi.WEIGHTS_OUT_IN if oi else 0
+    scratch = lambda step: L.fsw_workspace_bytes(step | flag, T, D, I)  # noqa: E731
+    launches = [(FWD_T if oi else FWD, T, I, D, 0),                                      # forward, recomputed gating gradient
+                (DX_T if oi else DX, T, D, I, scratch(_abi.STEP_INPUT_GRAD)),
+                (DW_T, I, D, T, scratch(_abi.STEP_WEIGHT_GRAD)) if oi else (DW, D, I, T, scratch(_abi.STEP_WEIGHT_GRAD)),
+                (TN, *((D, I) if oi else (I, D)), T, scratch(_abi.STEP_DOWN_WEIGHT_GRAD))]
+    if T > 128:
+        launches += [(NT if oi else NN, T, D, I, scratch(_abi.STEP_DOWN_FORWARD)),
+                     (NN if oi else NT, T, I, D, scratch(_abi.STEP_DOWN_INPUT_GRAD))]
+    for mode, M, N, K, ws in launches:
+        blocks, splits, tail_parts = ask(_abi.bench_lib().fsw_plan_tiled, mode, M, N, K, ws, results=3)
+        rows = (128 if mode == DW_T else 256) * blocks // 8
+        how = "tail" if tail_parts > 1 else "split" if splits > 1 else "whole"
+        if mode in FORWARDS:
+            how = "one row of tiles" if M <= rows else "whole"
+        yield mode, blocks, how
+
+
+def few_variants(T, D, I, oi):
+    """(reduction contiguous in the weights, column slot, 16-row blocks, down projection, split)"""
+    for down, kc, N, K in ((0, oi, (I + 7) & ~7, D), (1, oi, D, I), (1, not oi, I, D)):
+        if down and (N & 7 or N // 2 % (8 if kc else 64)):
+            continue                                                                     # runs on the tiled kernels
+        slot, blocks, _, splits = ask(_abi.bench_lib().fsw_plan_few_tokens, int(kc), down, T, N, K, CUS, 16, results=4)
+        yield bool(kc), slot, blocks, bool(down), splits > 1
+
+
+def reached():
+    tiled, few = set(), set()
+    for i, shape in enumerate(test_tile_rows_gpu.SHAPES):
+        for oi in (0, 1):
+            tiled |= {(*v, (i + oi) % 2) for v in tiled_variants(*shape, oi)}
+    for T, D, I in test_narrow_blocks_gpu.SHAPES:
+        for oi in (0, 1):
+            few |= {(*v, (T + D // 8) % 2) for v in few_variants(T, D, I, oi)}
+    for case in test_variants_gpu.TILED:
+        tiled |= {(*v, dtype) for v in tiled_variants(*case) for dtype in (0, 1)}
+    for case in test_variants_gpu.FEW:
+        few |= {(*v, dtype) for v in few_variants(*case) for dtype in (0, 1)}
+    return tiled, few
+
+
+@pytest.fixture(scope="module")
+def variants():
+    return reached()
+
+
+def test_tiled_kernels(variants):
+    def ways(mode, b):
+        if mode in FORWARDS:
+            return "whole", "one row of tiles"
+        return ("whole", "split", "tail") if b == 8 else ("whole", "split")
+
+    want = {(mode, b, how, dtype) for mode in range(9) for b in range(4, 9) for how in ways(mode, b) for dtype in (0, 1)}
+    assert variants[0] == want
+
+
+def test_weight_streaming_kernels(variants):
+    """Slots of 16 columns hold up to 64 rows, slots of 64 columns need contiguous reductions and more than 16 rows; blocks of
+    128 columns have room for 32, 64 or 128 rows.  The forward is never split."""
+    blocks = {16: (1, 2, 4), 32: (1, 2, 4, 8), 64: (2, 4, 8), 128: (2, 4, 8)}
+    want = {(kc, slot, b, down, split, dtype) for kc in (False, True) for slot in blocks if kc or slot != 64 for b in blocks[slot]
+            for down in (False, True) for split in (False, True) if down or not split for dtype in (0, 1)}
+    never = {(False, 16, 1, True, False, dtype) for dtype in (0, 1)}                      # a split comes out cheaper there
+    assert variants[1] == want - never
