@@ -27,7 +27,8 @@ PEAK_HBM_GBS = 8000.0      # MI355X HBM3E
 # itself).  The summary is stamped with a hash of the kernel sources it was taken with; when the sources
 # have changed since, `traffic` is reported as null instead of a stale figure.
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "gemm_kernels_c2_bf16.md")
-KERNEL_SOURCES = ("fsw_common.hpp", "fsw_gemm.hpp", "fsw_gemm4.hpp", "fsw_tiled.hpp", "fsw_tiled.hip")
+KERNEL_SOURCES = ("fsw_common.hpp", "fsw_gemm.hpp", "fsw_gemm4.hpp", "fsw_tiled.hpp", "fsw_tiled.hip", "fsw_tiled_dx.hip",
+                  "fsw_tiled_plain.hip")
 
 
 def kernel_source_hash():

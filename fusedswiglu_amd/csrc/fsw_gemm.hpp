@@ -54,7 +54,7 @@ struct GemmParams {
   const void* d0;
   int M, N, K;     // result rows x columns (per result) and reduction length (per pass)
   // rows of a k-contiguous B that exist.  Equal to N, except that N is rounded up to a multiple of 8 when the
-  // caller's rows are padded: the padding columns of a result are written (zeros), the rows of B are not there.
+  // caller's rows are padded: the padding columns of a result are written, the rows of B are not there (zeros).
   int n_rows_b;
   int lda, ldb, ldc;  // leading dimensions in elements
   int tiles_m, tiles_n, group_m;

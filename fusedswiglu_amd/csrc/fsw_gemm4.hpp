@@ -26,7 +26,8 @@
 //                   wave has finished reading pair p out of LDS
 //   gaps  66..109   the 8 loads of that pair of B into pair p's B space
 //   gaps  80..111   fragment reads of step 2p+2 into set 0
-// The rings are 3 pairs of A and 2 of B deep at MB >= 6, 4 and 3 at MB = 4 (Rings4).
+// The rings are 3 pairs of A and 2 of B deep at MB >= 6, 4 and 3 at MB = 4 (Rings4).  A load "of that pair" goes to the pair
+// that the ring is deep enough for: p+2, p+3 for the deeper ones.
 #pragma once
 #include <utility>
 

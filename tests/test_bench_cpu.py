@@ -25,8 +25,8 @@ def test_traffic_is_parsed_from_the_committed_profile():
 
 
 def test_profile_belongs_to_the_current_kernel_sources():
-    """Fails when csrc/fsw_common.hpp, fsw_gemm.hpp or fsw_tiled.hip changed after the counter passes in
-    profiles/gemm_kernels_c2_bf16.md were taken: re-run the passes named there and update the summary."""
+    """Fails when one of bench.KERNEL_SOURCES changed after the counter passes in profiles/gemm_kernels_c2_bf16.md
+    were taken: re-run the passes named there and update the summary."""
     _, stamp = bench.load_profiled_traffic()
     assert stamp == bench.kernel_source_hash()
 
