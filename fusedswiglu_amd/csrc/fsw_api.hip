@@ -71,7 +71,7 @@ const char* fsw_status_string(int status) {
     case FSW_ERR_BAD_DTYPE: return "unsupported dtype";
     case FSW_ERR_BAD_SHAPE: return "bad shape";
     case FSW_ERR_BAD_STRIDE: return "bad leading dimension";
-    case FSW_ERR_ALIGNMENT: return "pointer not 2-byte aligned";
+    case FSW_ERR_ALIGNMENT: return "pointer or leading dimension not aligned";
     case FSW_ERR_LAUNCH: return "kernel launch failed";
     case FSW_ERR_SCRATCH_LIMIT: return "problem needs more scratch than the built-in buffer holds";
     default: return "unknown status";

@@ -15,7 +15,7 @@
  *     arguments are leading dimensions (row pitches) in ELEMENTS.
  *   - Every pointer is a device pointer on the current HIP device.  The caller owns every
  *     buffer; the library never allocates, frees or keeps a pointer after returning.
- *   - `dtype` selects 16-bit storage: FSW_DTYPE_BF16 or FSW_DTYPE_FP16 (optionally | FSW_WEIGHTS_OUT_IN).  Products are
+ *   - `dtype` selects 16-bit storage: FSW_DTYPE_BF16 or FSW_DTYPE_FP16 (optionally | FSW_WEIGHTS_OUT_IN | FSW_ROWS_PADDED).  Products are
  *     accumulated in fp32 on the MFMA units for both (CDNA4 has no fp16-accumulate mode,
  *     so the reference's fp16 "fast accumulation" maps to fp32 accumulation).
  *   - `stream` is a hipStream_t (NULL = the default stream).  Calls only enqueue work; they
@@ -43,7 +43,8 @@ extern "C" {
 #endif
 
 /* major*10000 + minor*100 + patch.
- * 0.4.0: fsw_swiglu_backward (the three backward steps in one call).
+ * 0.4.0: fsw_swiglu_backward (the three backward steps in one call); FSW_ROWS_PADDED, fsw_repack_rows and
+ *        fsw_elementwise_backward_rows.
  * 0.3.0: FSW_WEIGHTS_OUT_IN, the fsw_down_proj_* entry points, fsw_input_grad_noalloc and status 7,
  *        fsw_uses_tiled_kernel answers 2 for the weight-streaming kernels and knows steps 4 / 5 / 6,
  *        fsw_workspace_bytes may ask for up to 64 MiB for large gradient GEMMs (tail split).
@@ -61,9 +62,11 @@ enum { FSW_DTYPE_BF16 = 0, FSW_DTYPE_FP16 = 1 };
 
 /* May be OR-ed into the `dtype` of every entry point that takes leading dimensions and of fsw_swiglu_backward: D and I
  * need not be multiples of 8, but every row of every 16-bit array of the call has room for the next multiple of 8
- * elements - zeros in inputs; in results the kernels write zeros there - every leading dimension is a multiple of 8
- * (below 2^21) and every pointer is 16-byte aligned (else FSW_ERR_ALIGNMENT).  The exception is grad_out of
- * fsw_swiglu_backward, which stays dense, [T,I] with leading dimension I. */
+ * elements, every leading dimension is a multiple of 8 (below 2^21) and every pointer is 16-byte aligned (else
+ * FSW_ERR_ALIGNMENT, with nothing enqueued).  These padding columns take part in the arithmetic: they must be zeros in
+ * inputs, and in results the kernels write what zero columns give: zeros, or NaN in the rows that an infinity or a NaN of
+ * the other operand reaches (pad such a result anew, fsw_repack_rows, before it becomes an input).  The exception is
+ * grad_out of fsw_swiglu_backward, which stays dense, [T,I] with leading dimension I. */
 #define FSW_ROWS_PADDED 0x400
 
 enum {
@@ -72,7 +75,8 @@ enum {
   FSW_ERR_BAD_DTYPE = 2,
   FSW_ERR_BAD_SHAPE = 3,  /* a dimension is <= 0 or exceeds 2^31-1 */
   FSW_ERR_BAD_STRIDE = 4, /* a leading dimension is smaller than the row it describes */
-  FSW_ERR_ALIGNMENT = 5,  /* a pointer is not 2-byte aligned */
+  FSW_ERR_ALIGNMENT = 5,  /* a pointer is not 2-byte aligned; with FSW_ROWS_PADDED, a pointer or a leading dimension is not
+                           * what the flag asks for */
   FSW_ERR_LAUNCH = 6,     /* the HIP runtime refused the launch; see fsw_last_error() */
   FSW_ERR_SCRATCH_LIMIT = 7 /* fsw_input_grad_noalloc: the problem needs more than FSW_NOALLOC_SCRATCH_BYTES */
 };
