@@ -107,7 +107,9 @@ def _code(dtype: torch.dtype, weights_out_in: bool, padded: bool = False) -> int
 # Rows that are not whole 16-byte chunks (a dimension that is not a multiple of 8) or do not start on 16-byte
 # boundaries are copied once into padded rows; the padded results are copied back.  Each copy moves an array once in
 # each direction; the kernels behind it run at 10 to 30 times the rate of the edge-shape kernel (a training step of 2048
-# tokens, 1024 x 2730, bf16: 1716 us on the edge-shape kernel, 237 us on padded copies).  Below this many multiply-adds per
+# tokens, 1024 x 2730, bf16: 1712 us of GPU time on the edge-shape kernel, 134 us on padded copies in 13 launches, whose host
+# time makes it 143 to 255 us of wall time, by the host).  The copies add to a call's peak memory: x and both weights padded,
+# and each result padded until it is copied back (that step 116 -> 125 MB).  Below this many multiply-adds per
 # matrix product the edge-shape kernel's fewer launches win: forward / backward at 2^21.5 33 / 56 against 46 / 75 us, at
 # 2^23.5 38 / 79 against 46 / 76, at 2^24.5 39 / 100 against 46 / 77, at 2^25.2 69 / 224 against 46 / 77.
 _PAD_MIN_WORK = 1 << 24
