@@ -109,10 +109,18 @@ def _code(dtype: torch.dtype, weights_out_in: bool, padded: bool = False) -> int
 # each direction; the kernels behind it run at 10 to 30 times the rate of the edge-shape kernel (a training step of 2048
 # tokens, 1024 x 2730, bf16: 1712 us of GPU time on the edge-shape kernel, 134 us on padded copies in 13 launches, whose host
 # time makes it 143 to 255 us of wall time, by the host).  The copies add to a call's peak memory: x and both weights padded,
-# and each result padded until it is copied back (that step 116 -> 125 MB).  Below this many multiply-adds per
-# matrix product the edge-shape kernel's fewer launches win: forward / backward at 2^21.5 33 / 56 against 46 / 75 us, at
-# 2^23.5 38 / 79 against 46 / 76, at 2^24.5 39 / 100 against 46 / 77, at 2^25.2 69 / 224 against 46 / 77.
+# and each result padded until it is copied back (that step 116 -> 125 MB).  Padding pays from this
+# many multiply-adds per matrix product on (forward / backward, edge kernel against padded: 33 / 56 against 46 / 75 us at
+# 2^21.5, 39 / 100 against 46 / 77 at 2^24.5, 69 / 224 against 46 / 77 at 2^25.2) ...
 _PAD_MIN_WORK = 1 << 24
+# ... if the edge-shape kernel is not done sooner than the copies and their launches.  Its time is a chain of 32-element
+# steps of the reduction, 2.4 us each while its 64 x 64 tiles are no more than 320: padding pays from 4300 steps x tiles per
+# product on (129 .. 4096 tokens, d_model 65 .. 641, d_intermediate 2 .. 4 times that, edge kernel's time over the padded
+# one's at 2500 / 4000 / 4500 / 5000: forward 0.77 / 1.06 / 1.17 / 1.27, with pre-activations 0.70 / 0.96 / 1.07 / 1.16, the
+# down projection and its gradients 0.62 .. 0.67 / 0.84 / 0.98 / 1.05 .. 1.19).  256 x 257 x 693: forward 29 us on the edge
+# kernel, 38 padded; the same at d_model 641 and 1731: 64 and 40.
+_PAD_MIN_STEPS_SHARE = 3900
+
 # The tiled kernels address rows of less than this many elements: operands with a larger pitch are copied as well, and a
 # problem whose padded rows would be longer stays on the edge-shape kernel, which has no such limit.
 _TILED_MAX_LD = 1 << 21
@@ -159,18 +167,27 @@ def _unpadded(t: torch.Tensor, cols: int) -> torch.Tensor:
     return out
 
 
-def pads_rows(T: int, D: int, I: int) -> bool:
-    """Whether a problem of these sizes runs on padded copies if its rows are not whole, aligned 16-byte chunks."""
-    return T * D * I >= _PAD_MIN_WORK and D <= _TILED_MAX_LD - 8 and I <= _TILED_MAX_LD - 8
+def pads_rows(T: int, D: int, I: int, *products: Tuple[int, int, int]) -> bool:
+    """Whether a problem of these sizes runs on padded copies if its rows are not whole, aligned 16-byte chunks.
+    `products`: (rows, columns, reduction) of the matrix products behind the copies."""
+    if T * D * I < _PAD_MIN_WORK or D > _TILED_MAX_LD - 8 or I > _TILED_MAX_LD - 8:
+        return False
+    steps = sum([-(-k // 32) * max(-(-m // 64) * -(-n // 64), 320) for m, n, k in products])
+    return steps >= len(products) * (_PAD_MIN_WORK // _PAD_MIN_STEPS_SHARE)
 
 
-def _wants_padding(T: int, D: int, I: int, *ts: torch.Tensor) -> bool:
-    if not pads_rows(T, D, I):
+def backward_products(T: int, D: int, I: int) -> Tuple[Tuple[int, int, int], Tuple[int, int, int]]:
+    """For pads_rows: the input and the weight gradient (two results, half as long again per step)."""
+    return (T, D, 2 * I), (D, I, T + T // 2)
+
+
+def _wants_padding(T: int, D: int, I: int, product: Tuple[int, int, int], *ts: torch.Tensor) -> bool:
+    if T * D * I < _PAD_MIN_WORK:
         return False
     bits = D | I
     for t in ts:
         bits |= t.shape[1] | _ld(t) | (t.data_ptr() >> 1)  # 16-byte aligned: bits 1 to 3 of the address
-    return bool(bits & 7)
+    return bool(bits & 7) and pads_rows(T, D, I, product)
 
 
 def _weight_dims(w: torch.Tensor, weights_out_in: bool) -> Tuple[int, int]:
@@ -205,7 +222,7 @@ def fused_swiglu_fwd(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, 
     T = x2.shape[0]
     out_shape = tuple(x.shape[:-1]) + (I,)
     px, pg, pu, ldx, ldw = x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), _ld(x2), _ld(wg)
-    if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and pads_rows(T, D, I):
+    if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and pads_rows(T, D, I, (T, I, D)):
         return _padded_fwd(x2, wg, wu, dtype, out_shape, D, I, save_preactivations, weights_out_in, dense_preactivations)
     out = torch.empty(out_shape, device=dev, dtype=dtype)
     g = torch.empty_like(out) if save_preactivations else None
@@ -295,7 +312,7 @@ def gating_grad_recompute(grad_output: torch.Tensor, x: torch.Tensor, w_gate: to
         wg, wu = wg.contiguous(), wu.contiguous()
     T = x2.shape[0]
     dout = _rows(grad_output)
-    if padded or _wants_padding(T, D, I, x2, wg, wu, dout):
+    if padded or _wants_padding(T, D, I, (T, I, D), x2, wg, wu, dout):
         with _on_device(dev):
             (x2,), (wg, wu), (dout,) = _padded_copies(x2), _padded_copies(wg, wu), _padded_copies(dout)
             if _ld(dout) != _pad8(I):
@@ -368,7 +385,7 @@ def fused_input_grad(grad_xw_gate: torch.Tensor, grad_xw_up: torch.Tensor, w_gat
     if _ld(wg) != _ld(wu):
         wg, wu = wg.contiguous(), wu.contiguous()
     T = dg.shape[0]
-    if padded or _wants_padding(T, D, I, dg, du, wg, wu):
+    if padded or _wants_padding(T, D, I, (T, D, 2 * I), dg, du, wg, wu):
         with _on_device(dev):
             dg, du = (dg, du) if padded else _padded_copies(dg, du)
             grad_x = _padded_input_grad(dg, du, *_padded_copies(wg, wu), dtype, D, I, weights_out_in)
@@ -410,7 +427,7 @@ def swiglu_backward(grad_output: torch.Tensor, x: torch.Tensor, w_gate: torch.Te
         wg, wu = wg.contiguous(), wu.contiguous()
     T = x2.shape[0]
     px, pg, pu, ldx, ldw = x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), _ld(x2), _ld(wg)
-    if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and pads_rows(T, D, I):
+    if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and pads_rows(T, D, I, *backward_products(T, D, I)):
         grad_xw_up, grad_xw_gate = elementwise_backward(grad_output, xw_gate, xw_up, dtype, padded=True)
         grad_w_up = grad_w_gate = grad_x = None
         with _on_device(dev):
@@ -471,8 +488,9 @@ def fused_weight_grad(x: torch.Tensor, grad_xw_up: torch.Tensor, grad_xw_gate: t
         _require(grad_w_up.stride(-1) == 1 and grad_w_gate.stride(-1) == 1 and _ld(grad_w_up) == _ld(grad_w_gate)
                  and _ld(grad_w_up) >= wshape[1],
                  "weight-gradient outputs need unit inner stride and equal row strides")
-    if padded_from or _wants_padding(T, D, I, x2, du, dg) or (
-            out is not None and pads_rows(T, D, I) and not all(_whole_chunks(t) for t in out)):
+    product = (D, I, T + T // 2)
+    if padded_from or _wants_padding(T, D, I, product, x2, du, dg) or (
+            out is not None and not all(_whole_chunks(t) for t in out) and pads_rows(T, D, I, product)):
         with _on_device(dev):
             (x2,), (du, dg) = _padded_copies(x2), (du, dg) if padded_from else _padded_copies(du, dg)
             return _padded_weight_grad(x2, du, dg, dtype, D, I, weights_out_in, out=out)
@@ -507,7 +525,7 @@ def down_proj_forward(act: torch.Tensor, w_down: torch.Tensor, dtype: torch.dtyp
     T = a2.shape[0]
     shape = tuple(act.shape[:-1]) + (D,)
     flag = _abi.WEIGHTS_OUT_IN if weights_out_in else 0
-    pad = _wants_padding(T, D, I, a2, w2)
+    pad = _wants_padding(T, D, I, (T, D, I), a2, w2)
     with _on_device(dev):
         if pad:
             (a2,), (w2,) = _padded_copies(a2), _padded_copies(w2)
@@ -530,7 +548,7 @@ def down_proj_input_grad(grad_y: torch.Tensor, w_down: torch.Tensor, dtype: torc
     T = g2.shape[0]
     shape = tuple(grad_y.shape[:-1]) + (I,)
     flag = _abi.WEIGHTS_OUT_IN if weights_out_in else 0
-    pad = _wants_padding(T, D, I, g2, w2)
+    pad = _wants_padding(T, D, I, (T, I, D), g2, w2)
     with _on_device(dev):
         if pad:
             (g2,), (w2,) = _padded_copies(g2), _padded_copies(w2)
@@ -553,7 +571,7 @@ def down_proj_weight_grad(act: torch.Tensor, grad_y: torch.Tensor, dtype: torch.
     D = g2.shape[1]
     rows, cols = (D, I) if weights_out_in else (I, D)
     flag = _abi.WEIGHTS_OUT_IN if weights_out_in else 0
-    pad = _wants_padding(T, D, I, a2, g2)
+    pad = _wants_padding(T, D, I, (I, D, T), a2, g2)
     with _on_device(dev):
         if pad:
             (a2,), (g2,) = _padded_copies(a2), _padded_copies(g2)

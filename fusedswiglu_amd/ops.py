@@ -116,7 +116,8 @@ def _swiglu_backward(grad_out: Tensor, x: Tensor, w_gate: Tensor, w_up: Tensor, 
         return (dx if dx is not None else e, dw_gate if need_w_gate else e.clone(), dw_up if need_w_up else e.clone())
     # rows of I elements that are not whole 16-byte chunks stay padded between the steps of the backward
     I, D = w_gate.shape if oi else w_gate.shape[::-1]
-    padded = bool(I & 7) and _launch.pads_rows(x.numel() // max(D, 1), D, I)
+    T = x.numel() // max(D, 1)
+    padded = bool(I & 7) and _launch.pads_rows(T, D, I, *_launch.backward_products(T, D, I))
     if xw_gate.numel() == 0:
         d_up, d_gate = _launch.gating_grad_recompute(grad_out, x, w_gate, w_up, dtype, weights_out_in=oi, padded=padded)
     else:

@@ -8,9 +8,9 @@ from torch._subclasses.fake_tensor import FakeTensorMode
 from fusedswiglu_amd import ops
 from fusedswiglu_amd.kernels import _launch
 
-SHAPES = [  # x's leading dimensions, D, I: whole 16-byte chunks or not, below and above 2^24 multiply-adds
+SHAPES = [  # x's leading dimensions, D, I: whole 16-byte chunks or not; on the edge-shape kernel, on padded copies, on both
     ((2, 5), 16, 24), ((2, 5), 15, 30), ((3, 512), 128, 136), ((3, 512), 128, 130), ((1536,), 127, 129), ((2, 768), 129, 136),
-    ((1, 1), 4100, 4099),
+    ((2, 260), 520, 522), ((520,), 521, 523), ((520, 1), 521, 528), ((1, 1), 4100, 4099),
 ]
 
 

@@ -29,13 +29,19 @@ class Recorder:
 
 
 @pytest.fixture
-def library(monkeypatch):
+def recorded(monkeypatch):
     L = Recorder()
     monkeypatch.setattr(_launch._abi, "lib", lambda: L)
     monkeypatch.setattr(_launch, "_stream_ptr", lambda dev: 0)
     monkeypatch.setattr(_launch, "_check_device", lambda *tensors: tensors[0].device)
-    monkeypatch.setattr(_launch, "_PAD_MIN_WORK", 0)
     return L
+
+
+@pytest.fixture
+def library(recorded, monkeypatch):
+    """Every size is large enough for padded copies."""
+    monkeypatch.setattr(_launch, "_PAD_MIN_WORK", 0)
+    return recorded
 
 
 def every_launcher(x, wg, wu, wd, dy, dz, oi):
@@ -137,3 +143,35 @@ def test_unfit_weight_gradient_outputs_are_shape_errors(library, D, I, bad):
     with pytest.raises(_launch.ShapeError):
         _launch.fused_weight_grad(array(3, D), array(3, I), array(3, I), BF, out=(bad(D, I), bad(D, I)))
     assert not library.calls
+
+
+@pytest.mark.parametrize("oi", [False, True], ids=["DI", "ID"])
+@pytest.mark.parametrize("T,D,I,padded", [
+    (256, 257, 693, "idb"), (256, 449, 1213, "frideb"), (512, 127, 2731, "iwdgb"), (512, 385, 1039, "iwdgb"),
+    (2048, 511, 1025, "friwdegb"), (128, 2047, 129, "fre"), (64, 257, 771, ""), (2048, 1024, 2730, "friwdegb"),
+    (8, 4097, 11009, "friwdegb"),
+], ids=str)
+def test_short_reductions_stay_on_the_edge_kernel(recorded, T, D, I, padded, oi):
+    """On both sides of the measured line, for each product by itself and for the two of a backward together.  `padded`: f
+    forward, r recomputed gating gradient, i and w input and weight gradient, d, e and g the down projection and its input
+    and weight gradient, b the backward."""
+    kw = dict(dtype=BF, weights_out_in=oi)
+    x, dy, dz = array(T, D), array(T, I), array(T, D)
+    w, wd = array(*((I, D) if oi else (D, I))), array(*((D, I) if oi else (I, D)))
+    for letter, call in (("f", lambda: _launch.fused_swiglu_fwd(x, w, w, **kw)),
+                         ("r", lambda: _launch.gating_grad_recompute(dy, x, w, w, **kw)),
+                         ("i", lambda: _launch.fused_input_grad(dy, dy, w, w, **kw)),
+                         ("w", lambda: _launch.fused_weight_grad(x, dy, dy, **kw)),
+                         ("d", lambda: _launch.down_proj_forward(dy, wd, **kw)),
+                         ("e", lambda: _launch.down_proj_input_grad(dz, wd, **kw)),
+                         ("g", lambda: _launch.down_proj_weight_grad(dy, dz, **kw)),
+                         ("b", lambda: _launch.swiglu_backward(dy, x, w, w, dy, dy, **kw))):
+        recorded.calls.clear()
+        call()
+        flags = {p for _, _, p in recorded.calls}
+        assert flags == {letter in padded}, letter
+    if I & 7 and "b" in padded:                        # a packed backward decides once for all of its steps
+        for saved in (dy, dy.new_empty(0)):
+            recorded.calls.clear()
+            ops._swiglu_backward(dy, x, w, w, saved, saved, True, True, True, True, oi)
+            assert {p for _, _, p in recorded.calls} == {True}

@@ -51,7 +51,7 @@ def check_every_launcher(x, wg, wu, wd, dy, dz, oi):
 @pytest.mark.parametrize("T,D,I", [(5, 9, LD + 3), (5, 7, LD - 7), (5, 7, LD - 9), (3, LD - 1, 9)], ids=str)
 def test_long_unaligned_rows(T, D, I, oi):
     torch.manual_seed(T + D)
-    assert T * D * I >= _launch._PAD_MIN_WORK
+    assert T * D * I >= _launch._PAD_MIN_WORK and (max(D, I) > LD - 8) != _launch.pads_rows(T, D, I, (T, I, D))
     w = lambda std: rand(*((I, D) if oi else (D, I)), std)  # noqa: E731
     check_every_launcher(rand(T, D), w(D ** -0.5), w(D ** -0.5), rand(*((D, I) if oi else (I, D)), I ** -0.5), rand(T, I),
                          rand(T, D), oi)
@@ -60,9 +60,9 @@ def test_long_unaligned_rows(T, D, I, oi):
 @pytest.mark.parametrize("oi", [False, True], ids=["DI", "ID"])
 @pytest.mark.parametrize("wide", range(4), ids=["x", "weights", "w_down", "dy"])
 def test_wide_pitch_beside_unaligned_operands(wide, oi):
-    T, D, I = 133, 264, 520
+    T, D, I = 517, 520, 528
     torch.manual_seed(wide)
-    assert T * D * I >= _launch._PAD_MIN_WORK
+    assert _launch.pads_rows(T, D, I, (T, I, D)) and _launch.pads_rows(T, D, I, (I, D, T))
     where = lambda i: dict(pitch=LD) if i == wide else dict(skew=1)  # noqa: E731
     w = lambda: rand(*((I, D) if oi else (D, I)), D ** -0.5, **where(1))  # noqa: E731
     check_every_launcher(rand(T, D, **where(0)), w(), w(), rand(*((D, I) if oi else (I, D)), I ** -0.5, **where(2)),
