@@ -212,15 +212,15 @@ int fsw_plan_tiled(int mode, int64_t M, int64_t N, int64_t K, int64_t workspace_
   if (M <= 0 || N <= 0 || K <= 0 || !blocks || !splits || !tail_parts) return FSW_ERR_BAD_SHAPE;
   fsw::Plan p;
   switch (mode) {
-    case fsw::kFwd: p = fsw::plan<fsw::kFwd>(M, N, K, workspace_bytes); break;
-    case fsw::kDx: p = fsw::plan<fsw::kDx>(M, N, K, workspace_bytes); break;
-    case fsw::kDw: p = fsw::plan<fsw::kDw>(M, N, K, workspace_bytes); break;
-    case fsw::kNN: p = fsw::plan<fsw::kNN>(M, N, K, workspace_bytes); break;
-    case fsw::kNT: p = fsw::plan<fsw::kNT>(M, N, K, workspace_bytes); break;
-    case fsw::kTN: p = fsw::plan<fsw::kTN>(M, N, K, workspace_bytes); break;
-    case fsw::kFwdT: p = fsw::plan<fsw::kFwdT>(M, N, K, workspace_bytes); break;
-    case fsw::kDxT: p = fsw::plan<fsw::kDxT>(M, N, K, workspace_bytes); break;
-    case fsw::kDwT: p = fsw::plan<fsw::kDwT>(M, N, K, workspace_bytes); break;
+    case fsw::kFwd: p = fsw::plan<fsw::kFwd>(M, N, K, workspace_bytes, fsw::dense_lines<fsw::kFwd>(M, N, K)); break;
+    case fsw::kDx: p = fsw::plan<fsw::kDx>(M, N, K, workspace_bytes, fsw::dense_lines<fsw::kDx>(M, N, K)); break;
+    case fsw::kDw: p = fsw::plan<fsw::kDw>(M, N, K, workspace_bytes, fsw::dense_lines<fsw::kDw>(M, N, K)); break;
+    case fsw::kNN: p = fsw::plan<fsw::kNN>(M, N, K, workspace_bytes, fsw::dense_lines<fsw::kNN>(M, N, K)); break;
+    case fsw::kNT: p = fsw::plan<fsw::kNT>(M, N, K, workspace_bytes, fsw::dense_lines<fsw::kNT>(M, N, K)); break;
+    case fsw::kTN: p = fsw::plan<fsw::kTN>(M, N, K, workspace_bytes, fsw::dense_lines<fsw::kTN>(M, N, K)); break;
+    case fsw::kFwdT: p = fsw::plan<fsw::kFwdT>(M, N, K, workspace_bytes, fsw::dense_lines<fsw::kFwdT>(M, N, K)); break;
+    case fsw::kDxT: p = fsw::plan<fsw::kDxT>(M, N, K, workspace_bytes, fsw::dense_lines<fsw::kDxT>(M, N, K)); break;
+    case fsw::kDwT: p = fsw::plan<fsw::kDwT>(M, N, K, workspace_bytes, fsw::dense_lines<fsw::kDwT>(M, N, K)); break;
     default: return FSW_ERR_BAD_SHAPE;
   }
   *blocks = p.mb;

@@ -17,7 +17,8 @@ namespace fsw {
 //             a last round of r workgroups: its steps at 0.7 + 0.3 r/256 of that (the chip is power limited)
 //   split     5.8 us (second launch, its latency) + 8 bytes per partial element at 6.9 TB/s
 //   floor     operands and results once at 5.5 TB/s
-// step_us etc. are fitted to 6086 measured launches on operands that are not in the caches (six modes, 46 shapes of 129 ..
+// step_us and what lengthens it are given below.
+// The constants are fitted to 6086 measured launches on operands that are not in the caches (six modes, 46 shapes of 129 ..
 // 16384 tokens, d_model 256 .. 8192, every mb and up to 24 splits; fit within 8 %): the plan found is on average 1 %
 // behind the best of those measured.  Against whole tiles of 256 rows only (same shapes, operands cached): forward 20 %,
 // dx 18 %, dW 15 % faster on average; 777 x 4096 x 11008 forward 160 -> 123 us (160-row tiles), 2048 x 2048 x 5632
@@ -83,27 +84,51 @@ inline int steps_of(int mode, long long K) {
   return (mode == kDx || mode == kDxT) ? 2 * ((steps + 1) & ~1) : steps;
 }
 
-// Microseconds of one 32-element step with 16 mb rows per wave, all CUs at work.
+// Whether the rows of A and B are a whole number of 128-byte lines apart.  (Of their pitch alone: where a tensor starts does not
+// change the order of a sum.)
+struct Lines { bool a, b; };
+inline bool whole_lines(long long ld) { return (ld & 63) == 0; }
+// Dense operands: the pitch of each is its contiguous dimension.
 template <int MODE>
-inline double step_us(int mb) {
+Lines dense_lines(long long M, long long N, long long K) {
+  return Lines{whole_lines(result_cols(Cfg<MODE>::kAKc ? K : M)), whole_lines(result_cols(Cfg<MODE>::kBKc ? K : N))};
+}
+
+// Microseconds of one 32-element step with 16 mb rows per wave, `fill` of the CUs at work (1: all of them, power limited).
+// The loads of a step take longer, and low tiles, which have the most of them per row, lose what they gain,
+//  * where the rows of an operand are not whole lines: the 128-byte (KC) or 256-byte (MC) piece of a row touches one more;
+//  * with a single row of tiles: no other workgroup reads the same piece of B, all of it comes from HBM.
+// Without these two the plan was more than 10 % behind the best of all heights and splits at 5.1 % of 6180 problems of up to
+// 160 rows and at 3.2 % of 16144 larger ones whose rows are not whole lines; with them at 2.4 and 1.6 % (whole lines, 48136
+// problems: 0.8 % either way).  Input gradients of 90 x 8184 x 26856 314 -> 202 us, 122 x 8064 x 19776 184 -> 145, 4182 x 1608 x
+// 3288 120 -> 101.  (A table of its own for kDwT at mb = 4, whose rings are shorter, helps operands that are not cached and
+// costs a training step, where they are, 2 to 3 %.)
+template <int MODE>
+inline double step_us(int mb, double fill, long long tiles_m, Lines lines) {
+  using C = Cfg<MODE>;
   constexpr double forward[5] = {0.435, 0.500, 0.588, 0.650, 0.720};
   constexpr double kc_a[5] = {0.431, 0.483, 0.564, 0.618, 0.673};   // kDx*, kNN, kNT
   constexpr double mc_a[5] = {0.428, 0.508, 0.562, 0.638, 0.692};   // kDw*, kTN
-  return (Cfg<MODE>::kForward ? forward : Cfg<MODE>::kAKc ? kc_a : mc_a)[mb - 4];
+  double us = (C::kForward ? forward : C::kAKc ? kc_a : mc_a)[mb - 4] * (0.7 + 0.3 * fill);
+  if (tiles_m == 1) us = std::max(us, mb <= 5 ? 0.34 + 0.30 * fill : 0.45 + 0.26 * fill);
+  if (C::kAKc && !lines.a) us += 0.0125 * mb;
+  if (!lines.b) us += C::kBKc ? 0.1 : 0.045;
+  return us;
 }
 
 template <int MODE>
-Plan plan(long long M, long long N, long long K, long long ws_bytes) {
+Plan plan(long long M, long long N, long long K, long long ws_bytes, Lines lines) {
   using C = Cfg<MODE>;
   const int steps = steps_of(MODE, K);
   const long long tiles_n = (N + C::kTileN - 1) / C::kTileN;
   const double elems = (double)M * N * C::kResults;
   const double bytes = 2.0 * ((double)M * K * (C::kPasses * (C::kDualM ? 2 : 1)) + (double)N * K * (C::kPasses * (C::kDualN ? 2 : 1)) +
                               elems * (C::kForward ? 3 : 1));
-  auto rounds_us = [&](long long wgs, int s, int mb) {
-    const double body = s * step_us<MODE>(mb), edge = 1.3 + 0.68 * mb;
+  auto rounds_us = [&](long long wgs, int s, int mb, long long tiles_m) {
+    const double edge = 1.3 + 0.68 * mb;
     const long long full = wgs / kCus, rest = wgs % kCus;
-    return full * (body + edge) + (rest ? body * (0.7 + 0.3 * rest / kCus) + edge : 0.0);
+    return (full ? full * (s * step_us<MODE>(mb, 1.0, tiles_m, lines) + edge) : 0.0) +
+           (rest ? s * step_us<MODE>(mb, (double)rest / kCus, tiles_m, lines) + edge : 0.0);
   };
   Plan best{8, 1, steps, 0, 0, 1, steps};
   double best_us = 1e30;
@@ -111,8 +136,8 @@ Plan plan(long long M, long long N, long long K, long long ws_bytes) {
     if (us < best_us) { best_us = us; best = p; }
   };
   for (int mb = 8; mb >= 4; mb--) {
-    const long long tile_m = C::kTileM * mb / 8, tiles = (M + tile_m - 1) / tile_m * tiles_n;
-    consider(Plan{mb, 1, steps, 0, 0, 1, steps}, std::max(rounds_us(tiles, steps, mb), bytes / 5.5e6));
+    const long long tile_m = C::kTileM * mb / 8, tiles_m = (M + tile_m - 1) / tile_m, tiles = tiles_m * tiles_n;
+    consider(Plan{mb, 1, steps, 0, 0, 1, steps}, std::max(rounds_us(tiles, steps, mb, tiles_m), bytes / 5.5e6));
     if (C::kForward) continue;
     // splits that leave the chip a third, half or two thirds full (fewer partial tiles) or fill it once, twice or three
     // times; at least 8 steps per workgroup
@@ -122,12 +147,12 @@ Plan plan(long long M, long long N, long long K, long long ws_bytes) {
       const SplitPlan sp = split_steps(steps, (int)s);
       if (sp.splits < 2 || (double)sp.splits * elems * 4 > (double)ws_bytes) continue;
       consider(Plan{mb, sp.splits, sp.steps_per_split, 0, 0, 1, steps},
-               std::max(rounds_us(tiles * sp.splits, sp.steps_per_split, mb), bytes / 5.5e6) + 5.8 + sp.splits * elems * 8 / 6.9e6);
+               std::max(rounds_us(tiles * sp.splits, sp.steps_per_split, mb, tiles_m), bytes / 5.5e6) + 5.8 + sp.splits * elems * 8 / 6.9e6);
     }
     const TailPlan t = plan_tail(tiles, steps);
     if (mb == 8 && t.count > 0 && tail_bytes(t) <= ws_bytes)
       consider(Plan{mb, 1, steps, t.first, t.count, t.parts, t.steps},
-               rounds_us(t.first, steps, mb) + rounds_us((long long)t.count * t.parts, t.steps, mb) + 5.8 + tail_bytes(t) * 2 / 6.9e6);
+               rounds_us(t.first, steps, mb, tiles_m) + rounds_us((long long)t.count * t.parts, t.steps, mb, tiles_m) + 5.8 + tail_bytes(t) * 2 / 6.9e6);
   }
   return best;
 }
@@ -158,7 +183,7 @@ long long workspace_of(long long M, long long N, long long K, bool with_tail = t
   const long long plane = M * N * 4 * C::kResults;
   const int asked = scratch_splits(tiles, steps, (double)M * N * C::kResults).splits;
   if (!with_tail) return asked > 1 ? asked * plane : 0;
-  const Plan p = plan<MODE>(M, N, K, 1LL << 62);
+  const Plan p = plan<MODE>(M, N, K, 1LL << 62, dense_lines<MODE>(M, N, K));
   return std::max({asked > 1 ? asked * plane : 0LL, p.splits > 1 ? p.splits * plane : 0LL, asked > 1 ? 0LL : tail_bytes(plan_tail(tiles, steps))});
 }
 
@@ -179,7 +204,8 @@ hipError_t launch_typed(GemmParams g, hipStream_t s, void* ws, long long ws_byte
   // The four-wave form walks an m/n-contiguous operand through 32-bit offsets from its first k-row; larger operands
   // take the eight-wave form (256-row tiles).
   const bool fits = (C::kAKc || (long long)g.K * g.lda * 2 < (1LL << 31)) && (C::kBKc || (long long)g.K * g.ldb * 2 < (1LL << 31));
-  const Plan p = fits ? plan<MODE>(g.M, g.N, g.K, ws ? ws_bytes : 0) : plan_eight_waves<MODE>(g.M, g.N, g.K, ws ? ws_bytes : 0);
+  const Lines lines{whole_lines(g.lda), whole_lines(g.ldb)};
+  const Plan p = fits ? plan<MODE>(g.M, g.N, g.K, ws ? ws_bytes : 0, lines) : plan_eight_waves<MODE>(g.M, g.N, g.K, ws ? ws_bytes : 0);
   const int tile_m = C::kTileM * p.mb / 8;
   g.tiles_m = (g.M + tile_m - 1) / tile_m;
   g.tiles_n = (g.N + C::kTileN - 1) / C::kTileN;

@@ -87,3 +87,14 @@ def test_weight_streaming_kernels(variants):
             for down in (False, True) for split in (False, True) if down or not split for dtype in (0, 1)}
     never = {(False, 16, 1, True, False, dtype) for dtype in (0, 1)}                      # a split comes out cheaper there
     assert variants[1] == want - never
+
+
+@pytest.mark.parametrize("mode,M,N,K,whole_lines,ragged", [
+    (DX, 4182, 1608, 3288, None, (8, 2)), (DX, 4182, 1600, 3264, (4, 1), None),      # whole low tiles only where rows are lines
+    (DX, 90, 8184, 26856, None, (4, 8)), (DX_T, 122, 8064, 19776, (8, 8), None),     # one row of tiles: all CUs stream B
+], ids=str)
+def test_what_a_step_costs_decides(mode, M, N, K, whole_lines, ragged):
+    """Tile height (16-row blocks per wave) and split where rows are whole 128-byte lines and where they are not."""
+    want = whole_lines or ragged
+    assert (K % 64 == 0) == (whole_lines is not None)
+    assert ask(_abi.bench_lib().fsw_plan_tiled, mode, M, N, K, 1 << 40, results=3)[:2] == want

@@ -12,11 +12,11 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 TOL = {torch.bfloat16: 1e-2, torch.float16: 5e-3}
 TILED = [  # T, D, I, weights_out_in
-    (8260, 16, 3376, 0), (1801, 1832, 7416, 1), (6959, 8, 2920, 1), (8762, 8, 4456, 0), (3251, 4712, 1120, 1),
-    (4768, 1696, 2416, 0), (8516, 4256, 8, 0), (4817, 4344, 4328, 0), (130, 1128, 16392, 0), (5657, 2712, 656, 0),
-    (4148, 2176, 3600, 1), (8258, 1032, 8, 1), (129, 800, 16560, 1), (161, 800, 16560, 0), (161, 800, 16560, 1),
-    (197, 800, 16432, 0), (197, 800, 16432, 1), (226, 800, 16392, 0), (226, 800, 16392, 1), (4368, 3648, 2008, 1),
-    (100, 264, 520, 0), (100, 264, 520, 1),
+    (3376, 4272, 960, 0), (5391, 264, 5496, 0), (652, 4040, 3848, 1), (4610, 4112, 8, 0), (1935, 4224, 2480, 1),
+    (4218, 4304, 4304, 0), (4054, 2344, 544, 1), (3606, 3320, 520, 0), (129, 1128, 16552, 0), (4747, 2872, 896, 1),
+    (4367, 3864, 2160, 1), (135, 800, 16424, 1), (162, 808, 16440, 0), (162, 808, 16440, 1), (202, 800, 16528, 0),
+    (202, 800, 16528, 1), (225, 800, 16488, 0), (225, 800, 16488, 1), (4411, 1608, 1416, 0), (100, 264, 520, 0),
+    (100, 264, 520, 1),
 ]
 FEW = [
     (1, 16, 128, 1), (127, 128, 16, 0), (48, 128, 16, 0), (96, 768, 640, 1), (17, 1024, 784, 0), (63, 896, 4112, 0),
