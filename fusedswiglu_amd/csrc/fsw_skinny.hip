@@ -252,7 +252,7 @@ bool skinny_gemm_ok(const GemmProblem& p) {
 
 long long skinny_gemm_workspace_bytes(int layout, long long M, long long N, long long K) {
   if (layout > 1 || M > kSkMaxRows || M <= 0 || (N & 7) || (N / 2) % (layout == 1 ? 8 : 64)) return 0;
-  const SkPlan pl = choose(M, N / 2, K, cu_count(), layout == 1, true, 16);
+  const SkPlan pl = choose(M, N / 2, K, cu_count(), layout == 1, true, kSkMaxSplits);
   return pl.splits > 1 ? (long long)pl.splits * M * N * 4 : 0;
 }
 

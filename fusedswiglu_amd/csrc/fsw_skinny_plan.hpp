@@ -37,7 +37,7 @@ inline SkPlan plan_wide(long long M, long long Nh, long long K, int cus, bool w_
   const int stages = (int)((K + 63) / 64);
   const long long tiles = (Nh + 127) / 128;
   // a split shorter than 8 stages does not fill the ring
-  const long long splits = std::min({cus / tiles, 16LL, max_splits, (long long)stages / 8});
+  const long long splits = std::min({cus / tiles, max_splits, (long long)stages / 8});
   if (max_splits < 1 || splits <= 1) return SkPlan{128, 0, block_width((int)Nh, cus, w_kc, (int)M), 1, stages};
   const int sps = (int)((stages + splits - 1) / splits);
   return SkPlan{128, 0, 128, (stages + sps - 1) / sps, sps};
@@ -70,7 +70,7 @@ inline double estimate_us(const SkPlan& p, long long M, long long Nh, long long 
 // layout), at most 3 % slower anywhere: 1 x 1024 x 3072 [I, D] 10.5 -> 5.6 us, 16 x 2048 x 4096 17.6 -> 9.1, 1 x 4096 x 11008
 // 36.9 -> 33.2, the down projection of 64 x 2048 x 4096 15.4 -> 10.9.  [D, I] weights of more than 150 MB stay on blocks of 128: their rows, one
 // segment per k and block, are then read 15 to 20 % slower in shorter segments.
-inline SkPlan choose(long long M, long long Nh, long long K, int cus, bool w_kc, bool plain, long long max_splits) {
+inline SkPlan choose_within(long long M, long long Nh, long long K, int cus, bool w_kc, bool plain, long long max_splits) {
   SkPlan best = plan_wide(M, Nh, K, cus, w_kc, plain ? max_splits : 0);
   if (!w_kc && 4.0 * K * Nh > 150e6) return best;
   double best_us = estimate_us(best, M, Nh, K, cus, w_kc);
@@ -98,6 +98,19 @@ inline SkPlan choose(long long M, long long Nh, long long K, int cus, bool w_kc,
     }
   }
   return best;
+}
+
+// Splits of a reduction that scratch for any number of planes may have.
+constexpr long long kSkMaxSplits = 16;
+
+// The launch for scratch of max_splits fp32 planes.  What the workspace query asks for, the plan under no limit, is taken
+// whenever its planes fit.  A search under a limit only finds it by chance: 8 parts of 18 stages are 6 parts of 3, but 6 as a
+// limit rules out 8, and an unsplit plan has won against a split one of 128-column blocks that a call without scratch does
+// not weigh.  One shape in 14 took another plan than the one its scratch was sized for, and 10 % more time on average
+// (50 such shapes): the down projection of 119 x 1280 -> 448 19.3 instead of 9.5 us, of 26 x 1280 -> 256 12.1 instead of 7.8.
+inline SkPlan choose(long long M, long long Nh, long long K, int cus, bool w_kc, bool plain, long long max_splits) {
+  const SkPlan p = choose_within(M, Nh, K, cus, w_kc, plain, kSkMaxSplits);
+  return !plain || p.splits <= max_splits ? p : choose_within(M, Nh, K, cus, w_kc, plain, max_splits);
 }
 
 }  // namespace fsw

@@ -98,3 +98,15 @@ def test_what_a_step_costs_decides(mode, M, N, K, whole_lines, ragged):
     want = whole_lines or ragged
     assert (K % 64 == 0) == (whole_lines is not None)
     assert ask(_abi.bench_lib().fsw_plan_tiled, mode, M, N, K, 1 << 40, results=3)[:2] == want
+
+
+@pytest.mark.parametrize("out_in,M,N,K", [(0, 104, 336, 1272), (1, 92, 384, 1152), (1, 100, 448, 1336), (0, 13, 2856, 1096),
+                                          (1, 50, 23232, 1960), (0, 15, 240, 848)], ids=str)
+def test_few_tokens_plan_fits_its_own_scratch(out_in, M, N, K):
+    """Scratch for just the planes that a plan writes (what fsw_workspace_bytes answers) gives that plan; less gives one that
+    fits it."""
+    few = lambda planes: ask(_abi.bench_lib().fsw_plan_few_tokens, out_in, 1, M, N, K, CUS, planes, results=4)  # noqa: E731
+    free = few(1 << 30)
+    splits = free[3]
+    assert few(splits) == few(16) == free
+    assert all(few(p)[3] <= p for p in range(1, splits))
