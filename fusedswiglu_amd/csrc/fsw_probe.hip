@@ -232,7 +232,8 @@ int fsw_plan_tiled(int mode, int64_t M, int64_t N, int64_t K, int64_t workspace_
 int fsw_plan_few_tokens(int out_in, int down, int64_t M, int64_t N, int64_t K, int cus, int64_t planes, int* slot, int* blocks,
                         int* columns, int* splits) {
   if (M <= 0 || M > 128 || N <= 0 || K <= 0 || cus <= 0 || !slot || !blocks || !columns || !splits) return FSW_ERR_BAD_SHAPE;
-  const fsw::SkPlan p = fsw::choose(M, down ? N / 2 : N, K, cus, out_in != 0, down != 0, down ? planes : 1);
+  const fsw::SkPlan p = fsw::choose(M, down ? N / 2 : N, K, cus, out_in != 0, (out_in ? K : N) % 64 == 0, down != 0,
+                                    down ? planes : 1);
   *slot = p.slot;
   *blocks = p.slot == 128 ? (M <= 32 ? 2 : (M <= 64 ? 4 : 8)) : p.mq;
   *columns = p.bn;

@@ -235,7 +235,7 @@ hipError_t launch_forward_skinny(int dtype, const Problem& p, hipStream_t s) {
   g.a0 = p.x; g.b0 = p.wg; g.b1 = p.wu; g.c0 = p.out; g.c1 = p.g; g.c2 = p.u;
   g.M = (int)p.T; g.N = (int)result_cols(p.I); g.n_rows_b = (int)p.I; g.K = (int)p.D;
   g.lda = (int)p.ldx; g.ldb = (int)p.ldw; g.ldc = (int)p.ldo;
-  const SkPlan pl = choose(g.M, g.N, g.K, cu_count(), p.w_out_in, false, 1);
+  const SkPlan pl = choose(g.M, g.N, g.K, cu_count(), p.w_out_in, g.ldb % 64 == 0, false, 1);
   if (p.w_out_in) return dtype == kDtypeBF16 ? launch_skinny_t<BF16, true>(g, pl, 0, s) : launch_skinny_t<FP16, true>(g, pl, 0, s);
   return dtype == kDtypeBF16 ? launch_skinny_t<BF16, false>(g, pl, 0, s) : launch_skinny_t<FP16, false>(g, pl, 0, s);
 }
@@ -252,7 +252,7 @@ bool skinny_gemm_ok(const GemmProblem& p) {
 
 long long skinny_gemm_workspace_bytes(int layout, long long M, long long N, long long K) {
   if (layout > 1 || M > kSkMaxRows || M <= 0 || (N & 7) || (N / 2) % (layout == 1 ? 8 : 64)) return 0;
-  const SkPlan pl = choose(M, N / 2, K, cu_count(), layout == 1, true, kSkMaxSplits);
+  const SkPlan pl = choose(M, N / 2, K, cu_count(), layout == 1, true, true, kSkMaxSplits);
   return pl.splits > 1 ? (long long)pl.splits * M * N * 4 : 0;
 }
 
@@ -260,7 +260,7 @@ hipError_t launch_gemm_skinny(int dtype, const GemmProblem& p, hipStream_t s, vo
   const bool w_kc = p.layout == 1;
   const long long nh = p.N / 2;
   const long long fit = ws ? ws_bytes / (p.M * p.N * 4) : 1;
-  const SkPlan pl = choose(p.M, nh, p.K, cu_count(), w_kc, true, fit < 1 ? 1 : fit);
+  const SkPlan pl = choose(p.M, nh, p.K, cu_count(), w_kc, true, true, fit < 1 ? 1 : fit);
   GemmParams g{};
   g.a0 = p.a; g.b0 = p.b;
   g.b1 = (const char*)p.b + (w_kc ? (size_t)nh * p.ldb * 2 : (size_t)nh * 2);

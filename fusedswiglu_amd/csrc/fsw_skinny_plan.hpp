@@ -67,12 +67,21 @@ inline double estimate_us(const SkPlan& p, long long M, long long Nh, long long 
 // Nh: columns of each half.  Narrow blocks are taken where the estimate sees them ahead by more than it errs among the
 // launches above, whose times they then beat on average by 31 / 23 / 28 / 21 % (forward, [I, D], up to 16 / 32 / 64 / 128
 // rows), 15 / 16 / 19 / 15 % (down projection, nn.Linear's layout), 5 / 2 / 4 / 12 % and 10 / 9 / 2 / 0 % (the other
-// layout), at most 3 % slower anywhere: 1 x 1024 x 3072 [I, D] 10.5 -> 5.6 us, 16 x 2048 x 4096 17.6 -> 9.1, 1 x 4096 x 11008
+// layout): 1 x 1024 x 3072 [I, D] 10.5 -> 5.6 us, 16 x 2048 x 4096 17.6 -> 9.1, 1 x 4096 x 11008
 // 36.9 -> 33.2, the down projection of 64 x 2048 x 4096 15.4 -> 10.9.  [D, I] weights of more than 150 MB stay on blocks of 128: their rows, one
 // segment per k and block, are then read 15 to 20 % slower in shorter segments.
-inline SkPlan choose_within(long long M, long long Nh, long long K, int cus, bool w_kc, bool plain, long long max_splits) {
+// Outside those launches: whole_lines says that the rows of the weights are a multiple of 128 bytes apart (only the
+// forward's plan asks).  Where the rows of [I, D] weights start between lines, a forward of up to 32 rows stays on blocks of 128 once
+// 32-column blocks need a second round: 64-column blocks then read 4.2 TB/s and the 48 of 128 up to 5 (60 launches of 1 to 32
+// rows, 8200 to 11808 columns: narrow blocks took 1.10 to 1.21 of the time in all but one, 0.99 in that; 1 x 5448 x 11704
+// 60.7 -> 51.3 us).  More rows, one round of 32-column blocks, or the down projections: narrow blocks win there between lines
+// as well.  What is left: a down projection of more than 64 rows with more than 40 MB of weights, reduction contiguous.  The
+// estimate errs both ways there, narrow blocks took 0.84 to 1.24 of the time (geometric mean 1.0), and no simple rule parts them.
+inline SkPlan choose_within(long long M, long long Nh, long long K, int cus, bool w_kc, bool whole_lines, bool plain,
+                            long long max_splits) {
   SkPlan best = plan_wide(M, Nh, K, cus, w_kc, plain ? max_splits : 0);
   if (!w_kc && 4.0 * K * Nh > 150e6) return best;
+  if (w_kc && !plain && !whole_lines && M <= 32 && Nh > 32LL * cus) return best;
   double best_us = estimate_us(best, M, Nh, K, cus, w_kc);
   best_us /= plain ? (M <= 16 ? 1.05 : 1.15) : (w_kc ? 1.10 : 1.0);
   for (int slot = 16; slot <= (w_kc ? 64 : 32); slot *= 2) {
@@ -108,9 +117,10 @@ constexpr long long kSkMaxSplits = 16;
 // limit rules out 8, and an unsplit plan has won against a split one of 128-column blocks that a call without scratch does
 // not weigh.  One shape in 14 took another plan than the one its scratch was sized for, and 10 % more time on average
 // (50 such shapes): the down projection of 119 x 1280 -> 448 19.3 instead of 9.5 us, of 26 x 1280 -> 256 12.1 instead of 7.8.
-inline SkPlan choose(long long M, long long Nh, long long K, int cus, bool w_kc, bool plain, long long max_splits) {
-  const SkPlan p = choose_within(M, Nh, K, cus, w_kc, plain, kSkMaxSplits);
-  return !plain || p.splits <= max_splits ? p : choose_within(M, Nh, K, cus, w_kc, plain, max_splits);
+inline SkPlan choose(long long M, long long Nh, long long K, int cus, bool w_kc, bool whole_lines, bool plain,
+                     long long max_splits) {
+  const SkPlan p = choose_within(M, Nh, K, cus, w_kc, whole_lines, plain, kSkMaxSplits);
+  return !plain || p.splits <= max_splits ? p : choose_within(M, Nh, K, cus, w_kc, whole_lines, plain, max_splits);
 }
 
 }  // namespace fsw

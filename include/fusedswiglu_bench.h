@@ -50,7 +50,7 @@ FSW_API int fsw_probe_mfma_mix(int mix, int iters, int workgroups, const void* b
  * input gradient, weight gradient ([D,I] weights), C = A B, A B^T, A^T B, forward, input gradient, weight gradient ([I,D]
  * weights).  blocks: 16-row blocks per wave (4 .. 8); splits of the reduction; parts of each tile of the last round (1: whole).
  * fsw_plan_few_tokens: at most 128 rows, the forward (down 0, N = I) or a down projection (down 1, N result columns, scratch
- * for `planes` fp32 planes [M,N]) with weights whose reduction index is contiguous (out_in 1) or not, on `cus` compute units.
+ * for `planes` fp32 planes [M,N]) with weights whose reduction index is contiguous (out_in 1) or not, dense, on `cus` compute units.
  * slot: column width of the variant (16, 32, 64, 128); blocks: its 16-row blocks of x; columns used of each slot; splits.
  */
 FSW_API int fsw_plan_tiled(int mode, int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int* blocks, int* splits,

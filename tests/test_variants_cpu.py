@@ -110,3 +110,11 @@ def test_few_tokens_plan_fits_its_own_scratch(out_in, M, N, K):
     splits = free[3]
     assert few(splits) == few(16) == free
     assert all(few(p)[3] <= p for p in range(1, splits))
+
+
+@pytest.mark.parametrize("M,N,K,slot", [
+    (32, 8704, 4160, 64), (32, 8704, 4168, 128), (33, 8704, 4168, 64), (32, 8192, 4168, 32), (1, 11704, 5448, 128)], ids=str)
+def test_narrow_blocks_where_weight_rows_are_not_whole_lines(M, N, K, slot):
+    """The forward's block width: rows of [I, D] weights that start between 128-byte lines are read by blocks of 128 once
+    32-column blocks need a second round, unless there are more than 32 rows of x."""
+    assert ask(_abi.bench_lib().fsw_plan_few_tokens, 1, 0, M, N, K, CUS, 1, results=4)[0] == slot

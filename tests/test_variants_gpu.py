@@ -24,7 +24,7 @@ FEW = [
     (2, 1360, 4104, 1), (24, 1376, 4112, 1), (8, 16, 968, 1), (48, 768, 256, 1), (63, 2768, 8200, 1), (15, 8208, 648, 1),
     (64, 1032, 5632, 1), (64, 1008, 6144, 1), (17, 840, 8272, 0), (32, 7296, 976, 0), (32, 6912, 1040, 0), (63, 8304, 904, 1),
     (2, 968, 8320, 1), (65, 2768, 3112, 1), (31, 1736, 8208, 1), (17, 976, 16432, 0), (63, 976, 16480, 0),
-    (127, 976, 16512, 0), (17, 2768, 14504, 1),
+    (127, 976, 16512, 0), (17, 2768, 14504, 1), (32, 4160, 8704, 1), (32, 4168, 8704, 1), (1, 5448, 11704, 1),
 ]
 
 
