@@ -118,3 +118,9 @@ def test_narrow_blocks_where_weight_rows_are_not_whole_lines(M, N, K, slot):
     """The forward's block width: rows of [I, D] weights that start between 128-byte lines are read by blocks of 128 once
     32-column blocks need a second round, unless there are more than 32 rows of x."""
     assert ask(_abi.bench_lib().fsw_plan_few_tokens, 1, 0, M, N, K, CUS, 1, results=4)[0] == slot
+
+
+@pytest.mark.parametrize("M,N,K,narrow", [(16, 17536, 7232, False), (11, 16640, 6784, False), (11, 8192, 1024, True)], ids=str)
+def test_no_third_round_of_16_columns(M, N, K, narrow):
+    """16-column blocks of a down projection: half of N in two rounds of the chip at most."""
+    assert (ask(_abi.bench_lib().fsw_plan_few_tokens, 1, 1, M, N, K, CUS, 16, results=4)[0] == 16) == narrow
