@@ -154,18 +154,19 @@ constexpr int kMcRowBytes = 256;
 constexpr int kMcPanelBytes = kBK * kMcRowBytes;  // 8 KiB
 
 // ---- XCD-aware tile order -----------------------------------------------------
-// Workgroups are dealt to the 8 XCDs round-robin by launch index.  Re-number them so that each
-// XCD works through one contiguous range of logical tiles, and inside that range walk bands of
-// `group_m` tile-rows column by column: the ~32 tiles an XCD runs at once then share few A and B
-// panels in that XCD's private L2.
+// Workgroups are dealt to the 8 XCDs round-robin by launch index.  Re-number `count` of them so that each
+// XCD works through one contiguous range,
+FSW_DEV int xcd_linear(int bid, int count) {
+  const int q = count >> 3, r = count & 7;
+  const int xcd = bid & 7, i = bid >> 3;
+  return (xcd < r) ? xcd * (q + 1) + i : r * (q + 1) + (xcd - r) * q + i;
+}
+// and inside that range walk bands of `group_m` tile-rows column by column: the ~32 tiles an XCD runs at once
+// then share few A and B panels in that XCD's private L2.
 struct TileCoord {
   int tm, tn;
 };
-FSW_DEV TileCoord xcd_tile_order(int bid, int tiles_m, int tiles_n, int group_m) {
-  const int nt = tiles_m * tiles_n;
-  const int q = nt >> 3, r = nt & 7;
-  const int xcd = bid & 7, i = bid >> 3;
-  const int lin = (xcd < r) ? xcd * (q + 1) + i : r * (q + 1) + (xcd - r) * q + i;
+FSW_DEV TileCoord band_tile(int lin, int tiles_m, int tiles_n, int group_m) {
   const int per_band = group_m * tiles_n;
   const int band = lin / per_band;
   const int first_m = band * group_m;
@@ -175,6 +176,9 @@ FSW_DEV TileCoord xcd_tile_order(int bid, int tiles_m, int tiles_n, int group_m)
   t.tm = first_m + in_band % rows;
   t.tn = in_band / rows;
   return t;
+}
+FSW_DEV TileCoord xcd_tile_order(int bid, int tiles_m, int tiles_n, int group_m) {
+  return band_tile(xcd_linear(bid, tiles_m * tiles_n), tiles_m, tiles_n, group_m);
 }
 
 }  // namespace fsw

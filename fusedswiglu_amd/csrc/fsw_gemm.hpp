@@ -64,6 +64,7 @@ struct GemmParams {
   // to c0/c1.
   float* ws;
   int splits, steps_per_split;
+  int split_per_xcd;  // four-wave kernel: an XCD works on few slices of the reduction (launch_typed in fsw_tiled.hpp), else on all
   // tail split (four-wave kernel, every mode but the forwards, splits == 1): the tiles of the last, partial round
   // of 256 workgroups - launch indices tail_first .. tail_first + tail_count - 1 - are each given to tail_parts
   // workgroups that reduce tail_steps steps (even) and leave an fp32 partial tile in ws[tile][part][kTileFloats];

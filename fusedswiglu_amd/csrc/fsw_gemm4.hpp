@@ -141,17 +141,28 @@ struct Rings4 {
   static_assert(kBytesA + kBytesB <= kLds, "LDS");
 };
 
-template <typename E, int MODE, int MB = 8, bool STREAM_B = false>
-__global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
+template <int MODE, int MB>
+struct Shape4 {
+  static constexpr bool kAKc = Cfg<MODE>::kAKc;
+  // An m-contiguous A of 128 columns fits one panel; otherwise each wave row has a panel (kDwT: a result) of its own.
+  static constexpr bool kOnePanelA = !kAKc && !Cfg<MODE>::kDualM && MB == 4;
+  static constexpr int kLdA = kAKc || kOnePanelA ? MB : 8, kLdB = 8;  // load instructions (4 KiB of the workgroup) per wave and pair
+  using R = Rings4<kLdA>;
+  static constexpr int kLds = R::kBytesA + R::kBytesB;
+};
+
+// The work of workgroup `index` of a launch of p.tiles_m * p.tiles_n * p.splits (and the tail's).  `index` counts the
+// workgroups of this GEMM; index % 8 has to be the XCD that runs it.
+template <typename E, int MODE, int MB, bool STREAM_B>
+FSW_DEV void gemm4_workgroup(const GemmParams& p, const int index, FSW_LDS char* smem) {
   using C = Cfg<MODE>;
+  using S4 = Shape4<MODE, MB>;
   constexpr bool A_KC = C::kAKc, B_KC = C::kBKc;
   constexpr bool B_INTER = (MODE == kFwdT);
   constexpr int TM = C::kTileM * MB / 8, TN = C::kTileN;
-  // An m-contiguous A of 128 columns fits one panel; otherwise each wave row has a panel (kDwT: a result) of its own.
-  constexpr bool kOnePanelA = !A_KC && !C::kDualM && MB == 4;
-  constexpr int kLdA = A_KC || kOnePanelA ? MB : 8, kLdB = 8;  // load instructions (4 KiB of the workgroup) per wave and pair
-  using R = Rings4<kLdA>;
-  __shared__ __attribute__((aligned(1024))) char smem[R::kBytesA + R::kBytesB];
+  constexpr bool kOnePanelA = S4::kOnePanelA;
+  constexpr int kLdA = S4::kLdA, kLdB = S4::kLdB;
+  using R = typename S4::R;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -160,12 +171,23 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
 
   const int ntiles = p.tiles_m * p.tiles_n;
   // a workgroup of the tail split: part `tail_part` of the tile with launch index tail_first + tail_tile
-  const bool in_tail = !C::kForward && p.tail_count > 0 && (int)blockIdx.x >= p.tail_first;
-  const int tail_part = in_tail ? ((int)blockIdx.x - p.tail_first) / p.tail_count : 0;
-  const int tail_tile = in_tail ? ((int)blockIdx.x - p.tail_first) % p.tail_count : 0;
-  const int split = (C::kForward || in_tail) ? 0 : (int)(blockIdx.x / ntiles);
-  const int tile_index = in_tail ? p.tail_first + tail_tile : (int)(blockIdx.x - split * ntiles);
-  const TileCoord tc = xcd_tile_order(tile_index, p.tiles_m, p.tiles_n, p.group_m);
+  const bool in_tail = !C::kForward && p.tail_count > 0 && index >= p.tail_first;
+  const int tail_part = in_tail ? (index - p.tail_first) / p.tail_count : 0;
+  const int tail_tile = in_tail ? (index - p.tail_first) % p.tail_count : 0;
+  int split = 0, lin;  // which slice of the reduction, and which tile in the order of band_tile
+  if (in_tail) {
+    lin = xcd_linear(p.tail_first + tail_tile, ntiles);
+  } else if (C::kForward || p.splits == 1) {
+    lin = xcd_linear(index, ntiles);
+  } else if (p.split_per_xcd) {
+    lin = xcd_linear(index, ntiles * p.splits);
+    split = lin / ntiles;
+    lin -= split * ntiles;
+  } else {
+    split = index / ntiles;
+    lin = xcd_linear(index - split * ntiles, ntiles);
+  }
+  const TileCoord tc = band_tile(lin, p.tiles_m, p.tiles_n, p.group_m);
   const int m0 = tc.tm * TM;
   const int n0 = tc.tn * TN;
 
@@ -175,7 +197,7 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
   const int kbase = in_tail ? tail_part * p.tail_steps : split * p.steps_per_split;
   const int kt_total = C::kForward ? kt_all : min(in_tail ? p.tail_steps : p.steps_per_split, kt_all - kbase);
 
-  const unsigned smem_a = (unsigned)(uintptr_t)(FSW_LDS char*)smem;
+  const unsigned smem_a = (unsigned)(uintptr_t)smem;
   const unsigned smem_b = smem_a + R::kBytesA;
 
   Loader4 la, lb;
@@ -324,7 +346,7 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
     rd_a[h] = A_KC ? kc_lane + wm * (16 * MB * 128) : mc_lane + (kOnePanelA ? h : h * 2 + wm) * kMcPanelBytes;
     rd_b[h] = B_KC ? kc_lane + wn * 128 * 128 : mc_lane + h * kMcSlotBytes;
   }
-  const FSW_LDS char* lds0 = (const FSW_LDS char*)smem;
+  const FSW_LDS char* lds0 = smem;
   // Read slot r of a step: fragment r >> 1 (0..MB-1 of A, then 0..7 of B).  A KC fragment is one
   // ds_read_b128 in the even slot; an MC fragment is two transposing reads, one per slot (two LDS reads behind
   // the same MFMA cost four times what they cost one MFMA apart).
@@ -512,8 +534,14 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
     }
     return;
   }
-  store_tile<E, MODE, MB, true>(p, acc, (FSW_LDS char*)smem + wave * (2 * 32 * 128), lane, row_base, col_of_half(0),
+  store_tile<E, MODE, MB, true>(p, acc, smem + wave * (2 * 32 * 128), lane, row_base, col_of_half(0),
                                col_of_half(1), result_of_half(0), result_of_half(1));
+}
+
+template <typename E, int MODE, int MB = 8, bool STREAM_B = false>
+__global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
+  __shared__ __attribute__((aligned(1024))) char smem[Shape4<MODE, MB>::kLds];
+  gemm4_workgroup<E, MODE, MB, STREAM_B>(p, blockIdx.x, (FSW_LDS char*)smem);
 }
 
 // Results of the tail tiles: out[tile] = round(sum over parts of ws[tile][part]), fixed order.  One workgroup of

@@ -187,6 +187,15 @@ long long workspace_of(long long M, long long N, long long K, bool with_tail = t
   return std::max({asked > 1 ? asked * plane : 0LL, p.splits > 1 ? p.splits * plane : 0LL, asked > 1 ? 0LL : tail_bytes(plan_tail(tiles, steps))});
 }
 
+// Which slices of a split reduction an XCD works on.  All tiles of a slice read the same k-elements, so an XCD that has few
+// slices and many of their tiles fetches far less into its L2 than one that has a few tiles of every slice: 16384 x 256 x 768
+// weight gradient (12 tiles x 20 slices) with its reduce 34.0 -> 27.3 us, 1024 x 1024 x 4096 input gradient 31.0 -> 28.2, the
+// down projection of 777 x 11008 -> 4096 83.1 -> 79.5.  Short slices that leave a fifth of the CUs or more without work are
+// the exception: they are over before any rate counts, and tiles that all wait for the same lines at once take longer to
+// start (120 random problems of 130 to 16384 tokens: 1 to 16 % longer in 26 of the 43 such, 1.03 on average; the other 77
+// take 0.962, the worst of them 1.025).
+inline bool split_per_xcd(long long workgroups, int steps) { return steps >= 24 || workgroups > 204; }
+
 template <typename E, int MODE, bool STREAM>
 void launch4(const GemmParams& g, int mb, unsigned grid, hipStream_t s) {
   switch (mb) {
@@ -214,6 +223,7 @@ hipError_t launch_typed(GemmParams g, hipStream_t s, void* ws, long long ws_byte
   // the B panels stream past: 8 tile-rows up to K = 4096, 4 beyond (measured at K = 8192: 4 % faster).
   g.group_m = g.K > 4096 ? 4 : 8;
   g.ws = (float*)ws; g.splits = p.splits; g.steps_per_split = p.steps_per_split;
+  g.split_per_xcd = split_per_xcd((long long)g.tiles_m * g.tiles_n * p.splits, p.steps_per_split);
   g.tail_first = p.tail_first; g.tail_count = p.tail_count; g.tail_parts = p.tail_parts; g.tail_steps = p.tail_steps;
   const long long tiles = (long long)g.tiles_m * g.tiles_n;
   const long long grid = p.tail_count > 0 ? p.tail_first + (long long)p.tail_count * p.tail_parts : tiles * p.splits;
