@@ -22,9 +22,9 @@ DTYPE_FP16 = 1
 WEIGHTS_OUT_IN = 0x100
 #: OR-ed into a dtype code: rows are padded to a multiple of 8 elements (FSW_ROWS_PADDED)
 ROWS_PADDED = 0x400
-STEP_DOWN_FORWARD, STEP_DOWN_INPUT_GRAD, STEP_DOWN_WEIGHT_GRAD = 4, 5, 6
+STEP_DOWN_FORWARD, STEP_DOWN_INPUT_GRAD, STEP_DOWN_WEIGHT_GRAD, STEP_DOWN_BACKWARD = 4, 5, 6, 8
 
-STEP_FORWARD, STEP_INPUT_GRAD, STEP_WEIGHT_GRAD = 0, 1, 2
+STEP_FORWARD, STEP_INPUT_GRAD, STEP_WEIGHT_GRAD, STEP_GRADIENTS = 0, 1, 2, 7
 
 #: size of the scratch built into the library for fsw_input_grad_noalloc (FSW_NOALLOC_SCRATCH_BYTES)
 NOALLOC_SCRATCH_BYTES = 32 << 20
@@ -45,14 +45,16 @@ EXPORTED_SYMBOLS = (
     "fsw_input_grad",
     "fsw_input_grad_noalloc",
     "fsw_weight_grad",
+    "fsw_swiglu_gradients",
     "fsw_swiglu_backward",
     "fsw_down_proj_forward",
     "fsw_down_proj_input_grad",
     "fsw_down_proj_weight_grad",
+    "fsw_down_proj_backward",
 )
 #: every symbol include/fusedswiglu_bench.h declares (libfusedswiglu_bench.so)
 BENCH_SYMBOLS = ("fsw_probe_mfma", "fsw_probe_stream_read", "fsw_probe_mfma_mix", "fsw_probe_dma_read", "fsw_plan_tiled",
-                 "fsw_plan_few_tokens")
+                 "fsw_plan_pair", "fsw_plan_few_tokens")
 
 
 class FusedSwiGLUError(RuntimeError):
@@ -125,11 +127,15 @@ def lib() -> ctypes.CDLL:
         L.fsw_input_grad_noalloc.argtypes = [vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, ci, vp]
         L.fsw_weight_grad.restype = ci
         L.fsw_weight_grad.argtypes = [vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, vp, i64, ci, vp]
+        L.fsw_swiglu_gradients.restype = ci
+        L.fsw_swiglu_gradients.argtypes = [vp] * 8 + [i64] * 8 + [vp, i64, ci, vp]
         L.fsw_swiglu_backward.restype = ci
         L.fsw_swiglu_backward.argtypes = [vp] * 11 + [i64] * 7 + [vp, i64, ci, vp]
         for name in ("fsw_down_proj_forward", "fsw_down_proj_input_grad", "fsw_down_proj_weight_grad"):
             getattr(L, name).restype = ci
             getattr(L, name).argtypes = [vp, vp, vp, i64, i64, i64, i64, i64, i64, vp, i64, ci, vp]
+        L.fsw_down_proj_backward.restype = ci
+        L.fsw_down_proj_backward.argtypes = [vp] * 5 + [i64] * 8 + [vp, i64, ci, vp]
         L.fsw_workspace_bytes.restype = i64
         L.fsw_workspace_bytes.argtypes = [ci, i64, i64, i64]
         _lib = L
@@ -159,6 +165,7 @@ def bench_lib() -> ctypes.CDLL:
             L.fsw_probe_mfma_mix.argtypes = [ci, ci, ci, vp, i64, vp, vp, ctypes.POINTER(ctypes.c_double)]
             pi = ctypes.POINTER(ci)
             L.fsw_plan_tiled.argtypes = [ci, i64, i64, i64, i64, pi, pi, pi]
+            L.fsw_plan_pair.argtypes = [ci, ci, i64, i64, i64, pi, pi, pi, pi]
             L.fsw_plan_few_tokens.argtypes = [ci, ci, i64, i64, i64, ci, i64, pi, pi, pi, pi]
             _bench_lib = L
     return _bench_lib

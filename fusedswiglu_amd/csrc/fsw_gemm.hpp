@@ -612,16 +612,13 @@ __global__ __launch_bounds__(kThreads) void fsw_gemm_kernel(GemmParams p) {
                                 col_of_half(1), result_of_half(0), result_of_half(1));
 }
 
-// out_r[i] = round(sum over s of ws[r][s][i]), i < n, fixed order: deterministic.  n is a multiple of 4.
-// blockIdx.y = result r (the weight gradients come in pairs): one launch for both.
+// out[i .. i+3] = round(sum over s of ws[s][i .. i+3]) for this thread's i = 4 * thread < n, fixed order: deterministic.  n is a
+// multiple of 4, the result has N columns and ldc elements from row to row.
 template <typename E>
-__global__ __launch_bounds__(256) void fsw_splitk_reduce_kernel(const float* __restrict__ ws, unsigned short* __restrict__ out0,
-                                                                unsigned short* __restrict__ out1, size_t n, int splits,
-                                                                int N, int ldc) {
-  const size_t i4 = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+FSW_DEV void reduce_planes(const float* __restrict__ ws, unsigned short* __restrict__ out, size_t thread, size_t n, int splits,
+                           int N, int ldc) {
+  const size_t i4 = thread * 4;
   if (i4 >= n) return;
-  ws += (size_t)blockIdx.y * splits * n;
-  unsigned short* out = blockIdx.y ? out1 : out0;
   // Loads of eight partials at a time: one after the other, each add waits for its own trip to memory (16 planes of
   // 1 x 4096: 5.4 us).  The order of the sum is the same.
   f32x4 a{-0.f, -0.f, -0.f, -0.f};
@@ -639,6 +636,14 @@ __global__ __launch_bounds__(256) void fsw_splitk_reduce_kernel(const float* __r
   v.x = E::pack2(a.x, a.y);
   v.y = E::pack2(a.z, a.w);
   *(u32x2*)(out + m * (size_t)ldc + c) = v;
+}
+// blockIdx.y = result (the weight gradients come in pairs): one launch for both.
+template <typename E>
+__global__ __launch_bounds__(256) void fsw_splitk_reduce_kernel(const float* __restrict__ ws, unsigned short* __restrict__ out0,
+                                                                unsigned short* __restrict__ out1, size_t n, int splits,
+                                                                int N, int ldc) {
+  reduce_planes<E>(ws + (size_t)blockIdx.y * splits * n, blockIdx.y ? out1 : out0, (size_t)blockIdx.x * blockDim.x + threadIdx.x,
+                   n, splits, N, ldc);
 }
 
 }  // namespace fsw

@@ -544,6 +544,39 @@ __global__ __launch_bounds__(kThreads4) void fsw_gemm4_kernel(GemmParams p) {
   gemm4_workgroup<E, MODE, MB, STREAM_B>(p, blockIdx.x, (FSW_LDS char*)smem);
 }
 
+// Two GEMMs that wait for the same operands - the weight and the input gradient - in one launch.  Each alone leaves its last
+// round of workgroups part empty and pays for its own start and end; here the workgroups of the second take the CUs that the
+// first leaves (plan_pair() in fsw_tiled.hpp: when, at which tile heights, and figures).  w and x have ranges of the launch
+// index that start at multiples of 8, so that index % 8 is the XCD within each.
+struct PairParams {
+  GemmParams w, x;
+  int w_first, w_count, x_first, x_count;
+};
+template <typename E, int MODE_W, int MB_W, int MODE_X, int MB_X>
+__global__ __launch_bounds__(kThreads4) void fsw_gemm4_pair_kernel(PairParams p) {
+  constexpr int kLdsW = Shape4<MODE_W, MB_W>::kLds, kLdsX = Shape4<MODE_X, MB_X>::kLds;
+  __shared__ __attribute__((aligned(1024))) char smem[kLdsW > kLdsX ? kLdsW : kLdsX];
+  const int iw = (int)blockIdx.x - p.w_first, ix = (int)blockIdx.x - p.x_first;
+  if (iw >= 0 && iw < p.w_count) gemm4_workgroup<E, MODE_W, MB_W, false>(p.w, iw, (FSW_LDS char*)smem);
+  else if (ix >= 0 && ix < p.x_count) gemm4_workgroup<E, MODE_X, MB_X, false>(p.x, ix, (FSW_LDS char*)smem);
+}
+
+// The partial planes of both, added up by one launch: workgroups 0 .. w_blocks - 1 for each of the two weight gradients, the
+// rest for the input gradient.  A GEMM that was not split has no workgroups here.
+template <typename E, int RESULTS_W>
+__global__ __launch_bounds__(256) void fsw_pair_reduce_kernel(PairParams p, int w_blocks) {
+  int b = blockIdx.x;
+  if (b < RESULTS_W * w_blocks) {
+    const int r = b / w_blocks;
+    const size_t n = (size_t)p.w.M * p.w.N;
+    reduce_planes<E>(p.w.ws + (size_t)r * p.w.splits * n, (unsigned short*)(r ? p.w.c1 : p.w.c0),
+                     (size_t)(b - r * w_blocks) * 256 + threadIdx.x, n, p.w.splits, p.w.N, p.w.ldc);
+  } else {
+    b -= RESULTS_W * w_blocks;
+    reduce_planes<E>(p.x.ws, (unsigned short*)p.x.c0, (size_t)b * 256 + threadIdx.x, (size_t)p.x.M * p.x.N, p.x.splits, p.x.N, p.x.ldc);
+  }
+}
+
 // Results of the tail tiles: out[tile] = round(sum over parts of ws[tile][part]), fixed order.  One workgroup of
 // 256 threads per 32 rows x 256 floats of a tile (blockIdx.y = tail tile, blockIdx.x = slice of its 2*TM*TN / 8192).
 template <typename E, int MODE>

@@ -38,6 +38,10 @@ bool fast_path_ok_gemm(const GemmProblem& p);
 hipError_t launch_gemm_fast(int dtype, const GemmProblem& p, hipStream_t s, void* ws, long long ws_bytes);
 hipError_t launch_gemm_generic(int dtype, const GemmProblem& p, hipStream_t s);
 long long gemm_workspace_bytes(int layout, long long M, long long N, long long K);
+// The two gradients of the down projection, w (layout 2) and x (layout 0 or 1), as launch_grads_pair below.
+hipError_t launch_gemm_pair(int dtype, const GemmProblem& w, const GemmProblem& x, hipStream_t s, void* ws, long long ws_bytes, bool* done);
+// Scratch for both: at least what either asks for.
+long long gemm_pair_workspace_bytes(const GemmProblem& w, const GemmProblem& x);
 
 // Tiled direct-to-LDS MFMA kernels: need every dimension and leading dimension to be a multiple
 // of 8 elements and every pointer 16-byte aligned.
@@ -47,7 +51,10 @@ bool fast_path_ok_weight_grad(const Problem& p);
 hipError_t launch_forward_fast(int dtype, const Problem& p, hipStream_t s);
 hipError_t launch_input_grad_fast(int dtype, const Problem& p, hipStream_t s, void* ws, long long ws_bytes);
 hipError_t launch_weight_grad_fast(int dtype, const Problem& p, hipStream_t s, void* ws, long long ws_bytes);
-// Bytes of fp32 scratch that let small input-grad (step 1; 4 for [I,D] weights) / weight-grad (step 2; 5)
+// Both of them in one launch where that is faster and the scratch holds the partial planes of both (*done; else nothing has
+// been enqueued); the same bits as from two.
+hipError_t launch_grads_pair(int dtype, const Problem& p, hipStream_t s, void* ws, long long ws_bytes, bool* done);
+// Bytes of fp32 scratch that let small input-grad (step 1; 4 for [I,D] weights) / weight-grad (step 2; 5; both: 7; 8)
 // problems split their reduction and, with_tail, large ones share the tiles of a short last round (at most
 // 64 MiB; without that scratch they run exactly as before).
 long long splitk_workspace_bytes(int step, long long T, long long D, long long I, bool with_tail = true);

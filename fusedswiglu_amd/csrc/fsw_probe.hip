@@ -229,6 +229,31 @@ int fsw_plan_tiled(int mode, int64_t M, int64_t N, int64_t K, int64_t workspace_
   return FSW_OK;
 }
 
+int fsw_plan_pair(int out_in, int down, int64_t T, int64_t D, int64_t I, int* blocks_w, int* blocks_x, int* splits_w, int* splits_x) {
+  constexpr int64_t kMax = (1LL << 31) - 8;
+  if (T <= 0 || D <= 0 || I <= 0 || T >= kMax || D >= kMax || I >= kMax || !blocks_w || !blocks_x || !splits_w || !splits_x) return FSW_ERR_BAD_SHAPE;
+  constexpr long long kScratch = 1LL << 62;
+  const int64_t d8 = fsw::result_cols(D), i8 = fsw::result_cols(I);
+  fsw::PairPlan pl;
+  if (down) {
+    const fsw::GemmParams x = fsw::gemm_params({nullptr, nullptr, nullptr, T, I, D, d8, out_in ? i8 : d8, i8, out_in ? 0 : 1, false});
+    const fsw::GemmParams w = out_in ? fsw::gemm_params({nullptr, nullptr, nullptr, D, I, T, d8, i8, i8, 2, false})
+                                     : fsw::gemm_params({nullptr, nullptr, nullptr, I, D, T, i8, d8, d8, 2, false});
+    pl = out_in ? fsw::plan_pair<fsw::kTN, fsw::kNN>(w, x, kScratch) : fsw::plan_pair<fsw::kTN, fsw::kNT>(w, x, kScratch);
+  } else {
+    fsw::Problem p{};
+    p.T = T; p.D = D; p.I = I; p.w_out_in = out_in != 0;
+    p.ldx = p.lddx = d8; p.ldo = i8; p.ldw = p.lddw = out_in ? d8 : i8;
+    const fsw::GemmParams w = fsw::weight_grad_params(p), x = fsw::input_grad_params(p);
+    pl = out_in ? fsw::plan_pair<fsw::kDwT, fsw::kDxT>(w, x, kScratch) : fsw::plan_pair<fsw::kDw, fsw::kDx>(w, x, kScratch);
+  }
+  *blocks_w = pl.w.mb;
+  *blocks_x = pl.x.mb;
+  *splits_w = pl.w.splits;
+  *splits_x = pl.x.splits;
+  return FSW_OK;
+}
+
 int fsw_plan_few_tokens(int out_in, int down, int64_t M, int64_t N, int64_t K, int cus, int64_t planes, int* slot, int* blocks,
                         int* columns, int* splits) {
   if (M <= 0 || M > 128 || N <= 0 || K <= 0 || cus <= 0 || !slot || !blocks || !columns || !splits) return FSW_ERR_BAD_SHAPE;

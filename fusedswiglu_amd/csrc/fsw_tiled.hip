@@ -44,6 +44,19 @@ long long splitk_workspace_bytes(int step, long long T, long long D, long long I
     case 2: return workspace_of<kDw>(D, I, T, with_tail);    // weight_grad: results 2 x [D, I], reduction over T
     case 4: return workspace_of<kDxT>(T, D, I, with_tail);   // the same two for [I, D] weights
     case 5: return workspace_of<kDwT>(I, D, T, with_tail);
+    case 7:                                                  // both, one after the other or in one launch
+    case 8: {
+      const bool oi = step == 8;
+      const long long one = std::max(splitk_workspace_bytes(oi ? 4 : 1, T, D, I), splitk_workspace_bytes(oi ? 5 : 2, T, D, I));
+      if (std::max({T, D, I}) >= (1LL << 31) - 8) return one;
+      Problem p{};
+      p.T = T; p.D = D; p.I = I; p.w_out_in = oi;
+      p.ldx = p.lddx = result_cols(D);
+      p.ldo = result_cols(I);
+      p.ldw = p.lddw = oi ? result_cols(D) : result_cols(I);
+      const GemmParams w = weight_grad_params(p), x = input_grad_params(p);
+      return std::max(one, oi ? pair_workspace<kDwT, kDxT>(w, x) : pair_workspace<kDw, kDx>(w, x));
+    }
     default: return 0;
   }
 }
@@ -57,17 +70,8 @@ hipError_t launch_forward_fast(int dtype, const Problem& p, hipStream_t s) {
 }
 
 hipError_t launch_weight_grad_fast(int dtype, const Problem& p, hipStream_t s, void* ws, long long ws_bytes) {
-  GemmParams g{};
-  if (p.w_out_in) {  // dWg [I,D] = dG^T x: the two results share the B tile (x)
-    g.a0 = p.dG; g.a1 = p.dU; g.b0 = p.x; g.c0 = p.dWg; g.c1 = p.dWu;
-    g.M = (int)p.I; g.N = (int)result_cols(p.D); g.n_rows_b = (int)p.D; g.K = (int)p.T;
-    g.lda = (int)p.ldo; g.ldb = (int)p.ldx; g.ldc = (int)p.lddw;
-    return launch<kDwT>(dtype, g, s, ws, ws_bytes);
-  }
-  g.a0 = p.x; g.b0 = p.dG; g.b1 = p.dU; g.c0 = p.dWg; g.c1 = p.dWu;
-  g.M = (int)p.D; g.N = (int)result_cols(p.I); g.n_rows_b = (int)p.I; g.K = (int)p.T;
-  g.lda = (int)p.ldx; g.ldb = (int)p.ldo; g.ldc = (int)p.lddw;
-  return launch<kDw>(dtype, g, s, ws, ws_bytes);
+  const GemmParams g = weight_grad_params(p);
+  return p.w_out_in ? launch<kDwT>(dtype, g, s, ws, ws_bytes) : launch<kDw>(dtype, g, s, ws, ws_bytes);
 }
 
 }  // namespace fsw

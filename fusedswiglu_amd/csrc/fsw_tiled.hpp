@@ -27,6 +27,7 @@ struct Plan {
   int mb;                       // 16-row blocks per wave
   int splits, steps_per_split;  // splits == 1: whole reduction
   int tail_first, tail_count, tail_parts, tail_steps;  // tail split (GemmParams); tail_count == 0: off
+  double us;                    // the estimate
 };
 
 constexpr long long kCus = 256;
@@ -130,14 +131,14 @@ Plan plan(long long M, long long N, long long K, long long ws_bytes, Lines lines
     return (full ? full * (s * step_us<MODE>(mb, 1.0, tiles_m, lines) + edge) : 0.0) +
            (rest ? s * step_us<MODE>(mb, (double)rest / kCus, tiles_m, lines) + edge : 0.0);
   };
-  Plan best{8, 1, steps, 0, 0, 1, steps};
-  double best_us = 1e30;
-  auto consider = [&](const Plan& p, double us) {
-    if (us < best_us) { best_us = us; best = p; }
+  Plan best{8, 1, steps, 0, 0, 1, steps, 1e30};
+  auto consider = [&](Plan p, double us) {
+    p.us = us;
+    if (us < best.us) best = p;
   };
   for (int mb = 8; mb >= 4; mb--) {
     const long long tile_m = C::kTileM * mb / 8, tiles_m = (M + tile_m - 1) / tile_m, tiles = tiles_m * tiles_n;
-    consider(Plan{mb, 1, steps, 0, 0, 1, steps}, std::max(rounds_us(tiles, steps, mb, tiles_m), bytes / 5.5e6));
+    consider(Plan{mb, 1, steps, 0, 0, 1, steps, 0}, std::max(rounds_us(tiles, steps, mb, tiles_m), bytes / 5.5e6));
     if (C::kForward) continue;
     // splits that leave the chip a third, half or two thirds full (fewer partial tiles) or fill it once, twice or three
     // times; at least 8 steps per workgroup
@@ -146,12 +147,12 @@ Plan plan(long long M, long long N, long long K, long long ws_bytes, Lines lines
       if (s < 2) continue;
       const SplitPlan sp = split_steps(steps, (int)s);
       if (sp.splits < 2 || (double)sp.splits * elems * 4 > (double)ws_bytes) continue;
-      consider(Plan{mb, sp.splits, sp.steps_per_split, 0, 0, 1, steps},
+      consider(Plan{mb, sp.splits, sp.steps_per_split, 0, 0, 1, steps, 0},
                std::max(rounds_us(tiles * sp.splits, sp.steps_per_split, mb, tiles_m), bytes / 5.5e6) + 5.8 + sp.splits * elems * 8 / 6.9e6);
     }
     const TailPlan t = plan_tail(tiles, steps);
     if (mb == 8 && t.count > 0 && tail_bytes(t) <= ws_bytes)
-      consider(Plan{mb, 1, steps, t.first, t.count, t.parts, t.steps},
+      consider(Plan{mb, 1, steps, t.first, t.count, t.parts, t.steps, 0},
                rounds_us(t.first, steps, mb, tiles_m) + rounds_us((long long)t.count * t.parts, t.steps, mb, tiles_m) + 5.8 + tail_bytes(t) * 2 / 6.9e6);
   }
   return best;
@@ -169,7 +170,7 @@ Plan plan_eight_waves(long long M, long long N, long long K, long long ws_bytes)
   SplitPlan sp{1, steps};
   if (!C::kForward) sp = scratch_splits(tiles, steps, (double)M * N * C::kResults);
   if (sp.splits > 1 && (double)sp.splits * M * N * 4 * C::kResults > (double)ws_bytes) sp = SplitPlan{1, steps};
-  return Plan{8, sp.splits, sp.steps_per_split, 0, 0, 1, steps};
+  return Plan{8, sp.splits, sp.steps_per_split, 0, 0, 1, steps, 0};
 }
 
 // Scratch for a GEMM of the given mode with results `results` x [M, N] and a reduction of K per pass.  with_tail: as a
@@ -207,26 +208,40 @@ void launch4(const GemmParams& g, int mb, unsigned grid, hipStream_t s) {
   }
 }
 
-template <typename E, int MODE>
-hipError_t launch_typed(GemmParams g, hipStream_t s, void* ws, long long ws_bytes) {
+// Whether the four-wave form can address the operands: it walks an m/n-contiguous one through 32-bit offsets from its first
+// k-row.  Larger ones take the eight-wave form (256-row tiles).
+template <int MODE>
+bool fits_four_waves(const GemmParams& g) {
   using C = Cfg<MODE>;
-  // The four-wave form walks an m/n-contiguous operand through 32-bit offsets from its first k-row; larger operands
-  // take the eight-wave form (256-row tiles).
-  const bool fits = (C::kAKc || (long long)g.K * g.lda * 2 < (1LL << 31)) && (C::kBKc || (long long)g.K * g.ldb * 2 < (1LL << 31));
-  const Lines lines{whole_lines(g.lda), whole_lines(g.ldb)};
-  const Plan p = fits ? plan<MODE>(g.M, g.N, g.K, ws ? ws_bytes : 0, lines) : plan_eight_waves<MODE>(g.M, g.N, g.K, ws ? ws_bytes : 0);
+  return (C::kAKc || (long long)g.K * g.lda * 2 < (1LL << 31)) && (C::kBKc || (long long)g.K * g.ldb * 2 < (1LL << 31));
+}
+template <int MODE>
+Lines lines_of(const GemmParams& g) { return Lines{whole_lines(g.lda), whole_lines(g.ldb)}; }
+
+// Returns the workgroups of the launch.
+template <int MODE>
+long long set_plan(GemmParams& g, const Plan& p, void* ws) {
+  using C = Cfg<MODE>;
   const int tile_m = C::kTileM * p.mb / 8;
   g.tiles_m = (g.M + tile_m - 1) / tile_m;
   g.tiles_n = (g.N + C::kTileN - 1) / C::kTileN;
-  // Height of the bands of tile-rows an XCD walks (xcd_tile_order).  The A panels of the 8 bands in
+  // Height of the bands of tile-rows an XCD walks (band_tile).  The A panels of the 8 bands in
   // flight (8 XCDs x group_m panels of 256 rows x K) should stay in the 256 MB memory-side cache while
   // the B panels stream past: 8 tile-rows up to K = 4096, 4 beyond (measured at K = 8192: 4 % faster).
   g.group_m = g.K > 4096 ? 4 : 8;
   g.ws = (float*)ws; g.splits = p.splits; g.steps_per_split = p.steps_per_split;
-  g.split_per_xcd = split_per_xcd((long long)g.tiles_m * g.tiles_n * p.splits, p.steps_per_split);
   g.tail_first = p.tail_first; g.tail_count = p.tail_count; g.tail_parts = p.tail_parts; g.tail_steps = p.tail_steps;
   const long long tiles = (long long)g.tiles_m * g.tiles_n;
-  const long long grid = p.tail_count > 0 ? p.tail_first + (long long)p.tail_count * p.tail_parts : tiles * p.splits;
+  g.split_per_xcd = split_per_xcd(tiles * p.splits, p.steps_per_split);
+  return p.tail_count > 0 ? p.tail_first + (long long)p.tail_count * p.tail_parts : tiles * p.splits;
+}
+
+template <typename E, int MODE>
+hipError_t launch_typed(GemmParams g, hipStream_t s, void* ws, long long ws_bytes) {
+  using C = Cfg<MODE>;
+  const bool fits = fits_four_waves<MODE>(g);
+  const Plan p = fits ? plan<MODE>(g.M, g.N, g.K, ws ? ws_bytes : 0, lines_of<MODE>(g)) : plan_eight_waves<MODE>(g.M, g.N, g.K, ws ? ws_bytes : 0);
+  const long long grid = set_plan<MODE>(g, p, ws);
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
   // a forward with a single row of tiles reads every weight byte exactly once: stream them past the caches
   const bool stream = C::kForward && g.tiles_m == 1;
@@ -259,6 +274,150 @@ hipError_t launch_typed(GemmParams g, hipStream_t s, void* ws, long long ws_byte
 template <int MODE>
 hipError_t launch(int dtype, const GemmParams& g, hipStream_t s, void* ws = nullptr, long long ws_bytes = 0) {
   return dtype == kDtypeBF16 ? launch_typed<BF16, MODE>(g, s, ws, ws_bytes) : launch_typed<FP16, MODE>(g, s, ws, ws_bytes);
+}
+
+// ---- both gradients in one launch -----------------------------------------------------------------------------------
+// The weight and the input gradient wait for the same gating gradients, and on problems of a few rounds each alone leaves much
+// of its last round empty: at 8192 x 256 x 768 156 and 64 workgroups on 256 CUs, one after the other.  In one launch the second
+// GEMM's workgroups start on the CUs that the first leaves, higher tiles (which cost less per row) fill the chip together, and
+// start, end and the sum of partial planes are paid once.  The whole backward behind a forward, gating gradient included, two
+// launches -> one: 8192 x 256 x 768 54.3 -> 43.9 us, 2048 x 512 x 1536 50.8 -> 37.5, 2048 x 1024 x 2736 80.5 -> 65.1, 8192 x 1024 x
+// 3072 223 -> 204; 120 random steps of 256 to 32768 tokens, d_model 256 to 8192: 0.89 of the time on average, 0.59 the best.
+// Large problems, whose last round is a small part of the launch, stay at two launches (plan_pair's margin).  The two gradients
+// of the down projection wait for the same operand as well.
+// The operands of a gradient GEMM from a Problem; mode kDw / kDwT and kDx / kDxT by the layout of the weights.
+inline GemmParams weight_grad_params(const Problem& p) {
+  GemmParams g{};
+  if (p.w_out_in) {  // dWg [I,D] = dG^T x: the two results share the B tile (x)
+    g.a0 = p.dG; g.a1 = p.dU; g.b0 = p.x; g.c0 = p.dWg; g.c1 = p.dWu;
+    g.M = (int)p.I; g.N = (int)result_cols(p.D); g.n_rows_b = (int)p.D; g.K = (int)p.T;
+    g.lda = (int)p.ldo; g.ldb = (int)p.ldx; g.ldc = (int)p.lddw;
+    return g;
+  }
+  g.a0 = p.x; g.b0 = p.dG; g.b1 = p.dU; g.c0 = p.dWg; g.c1 = p.dWu;
+  g.M = (int)p.D; g.N = (int)result_cols(p.I); g.n_rows_b = (int)p.I; g.K = (int)p.T;
+  g.lda = (int)p.ldx; g.ldb = (int)p.ldo; g.ldc = (int)p.lddw;
+  return g;
+}
+inline GemmParams input_grad_params(const Problem& p) {
+  GemmParams g{};
+  g.a0 = p.dG; g.a1 = p.dU; g.b0 = p.wg; g.b1 = p.wu; g.c0 = p.dx;
+  g.M = (int)p.T; g.N = (int)result_cols(p.D); g.n_rows_b = (int)p.D; g.K = (int)p.I;
+  g.lda = (int)p.ldo; g.ldb = (int)p.ldw; g.ldc = (int)p.lddx;
+  return g;
+}
+
+inline GemmParams gemm_params(const GemmProblem& p) {
+  GemmParams g{};
+  g.a0 = p.a; g.b0 = p.b; g.c0 = p.c;
+  g.M = (int)p.M; g.N = (int)result_cols(p.N); g.n_rows_b = (int)p.N; g.K = (int)p.K;
+  g.lda = (int)p.lda; g.ldb = (int)p.ldb; g.ldc = (int)p.ldc;
+  return g;
+}
+
+struct PairPlan {
+  Plan w, x;      // w.mb == 0: two launches are better
+  bool x_first;   // the longer workgroups first
+  double us;
+};
+// Tile heights (16-row blocks per wave of w, of x) that the pair kernel is built for: of all 25 combinations these give up 1 %
+// of the backward's time on average, four of them 2 % more.
+constexpr int kPairHeights[][2] = {{8, 8}, {8, 4}, {4, 8}, {4, 4}, {5, 5}, {7, 8}, {8, 7}};
+
+// Microseconds of na workgroups of ta each and, behind them, nb of tb each, tb <= ta, on all CUs: a workgroup starts on the
+// first CU that is free.
+inline double two_jobs_us(long long na, double ta, long long nb, double tb) {
+  const long long late = na % kCus, early = kCus - late;  // CUs that are free after `full` rounds of a, and one round later
+  const double t_early = na / kCus * ta, t_late = t_early + ta;
+  if (nb == 0) return late ? t_late : t_early;
+  // each early CU takes e workgroups of b and each late one l: the smallest end that has room for nb
+  long long e = std::max(0LL, nb / kCus - 1);
+  for (;; e++) {
+    const double end = t_early + e * tb;
+    const long long l = end > t_late ? (long long)((end - t_late) / tb) : 0;
+    if (e * early + l * late >= nb) return std::max(end, late ? t_late : 0.0);
+    const double end_late = t_late + (l + 1) * tb;  // before the early CUs end another one
+    if (late && end_late < end + tb && e * early + (l + 1) * late >= nb) return std::max(end_late, t_late);
+  }
+}
+
+// Bytes of a plan's fp32 partial planes.
+template <int MODE>
+double plane_bytes(const Plan& p, const GemmParams& g) {
+  return p.splits > 1 ? 4.0 * p.splits * Cfg<MODE>::kResults * g.M * g.N : 0.0;
+}
+
+template <int MODE_W, int MODE_X>
+PairPlan plan_pair(const GemmParams& w, const GemmParams& x, long long ws_bytes) {
+  PairPlan none{}, best{};
+  const Lines lw = lines_of<MODE_W>(w), lx = lines_of<MODE_X>(x);
+  // The splits are those of two launches, so that a sum is made of the same parts in either case.
+  const Plan pw = plan<MODE_W>(w.M, w.N, w.K, ws_bytes, lw), px = plan<MODE_X>(x.M, x.N, x.K, ws_bytes, lx);
+  if (pw.tail_count > 0 || px.tail_count > 0) return none;
+  const double planes = plane_bytes<MODE_W>(pw, w) + plane_bytes<MODE_X>(px, x);
+  if (planes > (double)ws_bytes) return none;
+  best.us = 0.97 * (pw.us + px.us + 1.0);  // (a predicted gain below that came out between -3 and +1 %)
+  const double reduce = planes > 0 ? 5.8 + planes * 2 / 6.9e6 : 0.0;
+  for (const auto& mb : kPairHeights) {
+    const long long rows_w = Cfg<MODE_W>::kTileM * mb[0] / 8, rows_x = Cfg<MODE_X>::kTileM * mb[1] / 8;
+    const long long tm_w = (w.M + rows_w - 1) / rows_w, tm_x = (x.M + rows_x - 1) / rows_x;
+    const long long nw = tm_w * ((w.N + Cfg<MODE_W>::kTileN - 1) / Cfg<MODE_W>::kTileN) * pw.splits;
+    const long long nx = tm_x * ((x.N + Cfg<MODE_X>::kTileN - 1) / Cfg<MODE_X>::kTileN) * px.splits;
+    const double tw = pw.steps_per_split * step_us<MODE_W>(mb[0], 1.0, tm_w, lw) + 1.3 + 0.68 * mb[0];
+    const double tx = px.steps_per_split * step_us<MODE_X>(mb[1], 1.0, tm_x, lx) + 1.3 + 0.68 * mb[1];
+    const double work = (nw * tw + nx * tx) / kCus;
+    if (work + reduce >= best.us || nw + nx > (1LL << 30)) continue;
+    const double end = tx > tw ? two_jobs_us(nx, tx, nw, tw) : two_jobs_us(nw, tw, nx, tx);
+    const double us = end * (0.7 + 0.3 * work / end) + reduce;
+    if (us < best.us) {
+      best = PairPlan{pw, px, tx > tw, us};
+      best.w.mb = mb[0];
+      best.x.mb = mb[1];
+    }
+  }
+  return best;
+}
+
+// Scratch for the partial planes of both in one launch, 0 if they would not share one.
+template <int MODE_W, int MODE_X>
+long long pair_workspace(const GemmParams& w, const GemmParams& x) {
+  if (!fits_four_waves<MODE_W>(w) || !fits_four_waves<MODE_X>(x)) return 0;
+  const PairPlan pl = plan_pair<MODE_W, MODE_X>(w, x, 1LL << 62);
+  return pl.w.mb == 0 ? 0 : (long long)(plane_bytes<MODE_W>(pl.w, w) + plane_bytes<MODE_X>(pl.x, x));
+}
+
+template <typename E, int MODE_W, int MODE_X, int I = 0>
+void launch_pair_kernel(const PairParams& p, int mb_w, int mb_x, unsigned grid, hipStream_t s) {
+  if constexpr (I < (int)(sizeof(kPairHeights) / sizeof(kPairHeights[0]))) {
+    constexpr int W = kPairHeights[I][0], X = kPairHeights[I][1];
+    if (mb_w == W && mb_x == X) fsw_gemm4_pair_kernel<E, MODE_W, W, MODE_X, X><<<grid, kThreads4, 0, s>>>(p);
+    else launch_pair_kernel<E, MODE_W, MODE_X, I + 1>(p, mb_w, mb_x, grid, s);
+  }
+}
+
+// *done: whether the pair took the launch; if not, nothing has been enqueued.
+template <typename E, int MODE_W, int MODE_X>
+hipError_t launch_pair(GemmParams w, GemmParams x, hipStream_t s, void* ws, long long ws_bytes, bool* done) {
+  *done = false;
+  if (!fits_four_waves<MODE_W>(w) || !fits_four_waves<MODE_X>(x)) return hipSuccess;
+  const PairPlan pl = plan_pair<MODE_W, MODE_X>(w, x, ws ? ws_bytes : 0);
+  if (pl.w.mb == 0) return hipSuccess;
+  PairParams p{};
+  const size_t floats_w = (size_t)plane_bytes<MODE_W>(pl.w, w) / 4;
+  p.w_count = (int)set_plan<MODE_W>(w, pl.w, ws);
+  p.x_count = (int)set_plan<MODE_X>(x, pl.x, (float*)ws + floats_w);
+  p.w = w;
+  p.x = x;
+  p.w_first = pl.x_first ? (p.x_count + 7) & ~7 : 0;
+  p.x_first = pl.x_first ? 0 : (p.w_count + 7) & ~7;
+  const unsigned grid = (unsigned)std::max(p.w_first + p.w_count, p.x_first + p.x_count);
+  *done = true;
+  launch_pair_kernel<E, MODE_W, MODE_X>(p, pl.w.mb, pl.x.mb, grid, s);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || (w.splits == 1 && x.splits == 1)) return e;
+  auto blocks = [](const GemmParams& g) { return g.splits > 1 ? (unsigned)(((size_t)g.M * g.N / 4 + 255) / 256) : 0u; };
+  fsw_pair_reduce_kernel<E, Cfg<MODE_W>::kResults><<<Cfg<MODE_W>::kResults * blocks(w) + blocks(x), 256, 0, s>>>(p, (int)blocks(w));
+  return hipGetLastError();
 }
 
 }  // namespace fsw

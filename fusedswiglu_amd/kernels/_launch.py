@@ -366,6 +366,25 @@ def _padded_weight_grad(x2, du, dg, dtype, D, I, weights_out_in, out=None) -> Tu
     return out
 
 
+def _padded_gradients(x2, wg, wu, dg, du, dtype, D, I, weights_out_in, out=None):
+    """(dense [T, D] input gradient, grad_w_up, grad_w_gate) from operands with padded rows, the weight gradients dense or in
+    the two arrays of `out` (current device: theirs)."""
+    T, dev = dg.shape[0], dg.device
+    rows, cols = (I, D) if weights_out_in else (D, I)
+    grad_w_up, grad_w_gate, grad_x = _padded_result(rows, cols, x2), _padded_result(rows, cols, x2), _padded_result(T, D, dg)
+    ws, ws_bytes = _workspace(_abi.STEP_GRADIENTS | (_abi.WEIGHTS_OUT_IN if weights_out_in else 0), T, D, I, dev)
+    _abi.check(_abi.lib().fsw_swiglu_gradients(
+        x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), dg.data_ptr(), du.data_ptr(), grad_x.data_ptr(), grad_w_gate.data_ptr(),
+        grad_w_up.data_ptr(), T, D, I, _ld(x2), _ld(wg), _ld(dg), _pad8(D), _pad8(cols),
+        ws.data_ptr() if ws is not None else None, ws_bytes, _code(dtype, weights_out_in, True), _stream_ptr(dev)))
+    if out is None and cols % 8 == 0:
+        return _unpadded(grad_x, D), grad_w_up, grad_w_gate
+    if out is None:
+        out = tuple(torch.empty((rows, cols), device=dev, dtype=dtype) for _ in range(2))
+    _repack(grad_w_up, out[0], cols, False, grad_w_gate, out[1])
+    return _unpadded(grad_x, D), *out
+
+
 def fused_input_grad(grad_xw_gate: torch.Tensor, grad_xw_up: torch.Tensor, w_gate: torch.Tensor,
                      w_up: torch.Tensor, dtype: torch.dtype, weights_out_in: bool = False,
                      padded: bool = False) -> torch.Tensor:
@@ -401,6 +420,42 @@ def fused_input_grad(grad_xw_gate: torch.Tensor, grad_xw_up: torch.Tensor, w_gat
     return grad_x
 
 
+def _padded_backward(dout, x2, wg, wu, g, u, x_shape, dtype, D, I, need_input_grad, need_weight_grad, weights_out_in):
+    """swiglu_backward on padded copies of x (for the weight gradients) and the weights (for the input gradient)."""
+    T, dev = dout.shape[0], dout.device
+    rows, cols = (I, D) if weights_out_in else (D, I)
+    with _on_device(dev):
+        L = _abi.lib()
+        grad_x = grad_w_gate = grad_w_up = None
+        step = _abi.STEP_GRADIENTS
+        if need_weight_grad:
+            (x2,) = _padded_copies(x2)
+            grad_w_gate, grad_w_up = _padded_result(rows, cols, x2), _padded_result(rows, cols, x2)
+        else:
+            step = _abi.STEP_INPUT_GRAD
+        if need_input_grad:
+            wg, wu = _padded_copies(wg, wu)
+            grad_x = _padded_result(T, D, g)
+        else:
+            step = _abi.STEP_WEIGHT_GRAD
+        grad_xw_gate, grad_xw_up = _padded_result(T, I, g), _padded_result(T, I, g)
+        ws, ws_bytes = (_workspace(step | (_abi.WEIGHTS_OUT_IN if weights_out_in else 0), T, D, I, dev)
+                        if need_input_grad or need_weight_grad else (None, 0))
+        _abi.check(L.fsw_swiglu_backward(
+            dout.data_ptr(), g.data_ptr(), u.data_ptr(), x2.data_ptr(), wg.data_ptr(), wu.data_ptr(),
+            grad_xw_gate.data_ptr(), grad_xw_up.data_ptr(), grad_x.data_ptr() if need_input_grad else None,
+            grad_w_gate.data_ptr() if need_weight_grad else None, grad_w_up.data_ptr() if need_weight_grad else None,
+            T, D, I, _ld(x2), _ld(wg), _pad8(D), _pad8(cols), ws.data_ptr() if ws is not None else None, ws_bytes,
+            _code(dtype, weights_out_in, True), _stream_ptr(dev)))
+        if need_input_grad:
+            grad_x = _unpadded(grad_x, D).view(x_shape)
+        if need_weight_grad and cols & 7:
+            padded = grad_w_gate, grad_w_up
+            grad_w_gate, grad_w_up = (torch.empty((rows, cols), device=dev, dtype=dtype) for _ in range(2))
+            _repack(padded[0], grad_w_gate, cols, False, padded[1], grad_w_up)
+    return grad_x, grad_w_gate, grad_w_up
+
+
 def swiglu_backward(grad_output: torch.Tensor, x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor,
                     xw_gate: torch.Tensor, xw_up: torch.Tensor, dtype: torch.dtype, need_input_grad: bool = True,
                     need_weight_grad: bool = True, weights_out_in: bool = False
@@ -428,9 +483,18 @@ def swiglu_backward(grad_output: torch.Tensor, x: torch.Tensor, w_gate: torch.Te
     T = x2.shape[0]
     px, pg, pu, ldx, ldw = x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), _ld(x2), _ld(wg)
     if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and pads_rows(T, D, I, *backward_products(T, D, I)):
+        g, u = _rows(xw_gate), _rows(xw_up)
+        if g.stride(0) == u.stride(0) == _pad8(I) and not (g.data_ptr() | u.data_ptr()) & 15:
+            # pre-activations in padded rows, as fused_swiglu_fwd keeps them: the one call takes them as they are
+            return _padded_backward(_rows(grad_output.contiguous()), x2, wg, wu, g, u, x.shape, dtype, D, I, need_input_grad,
+                                    need_weight_grad, weights_out_in)
         grad_xw_up, grad_xw_gate = elementwise_backward(grad_output, xw_gate, xw_up, dtype, padded=True)
         grad_w_up = grad_w_gate = grad_x = None
         with _on_device(dev):
+            if need_weight_grad and need_input_grad:
+                grad_x, grad_w_up, grad_w_gate = fused_gradients(x2, wg, wu, grad_xw_up, grad_xw_gate, dtype,
+                                                                 weights_out_in=weights_out_in, padded_from=I)
+                return grad_x.view(x.shape), grad_w_gate, grad_w_up
             if need_weight_grad:
                 grad_w_up, grad_w_gate = _padded_weight_grad(*_padded_copies(x2), grad_xw_up, grad_xw_gate, dtype, D, I, weights_out_in)
             if need_input_grad:
@@ -445,8 +509,9 @@ def swiglu_backward(grad_output: torch.Tensor, x: torch.Tensor, w_gate: torch.Te
     with _on_device(dev):
         L = _abi.lib()
         flag = _abi.WEIGHTS_OUT_IN if weights_out_in else 0
-        nbytes = max(int(L.fsw_workspace_bytes(_abi.STEP_INPUT_GRAD | flag, T, D, I)) if need_input_grad else 0,
-                     int(L.fsw_workspace_bytes(_abi.STEP_WEIGHT_GRAD | flag, T, D, I)) if need_weight_grad else 0)
+        step = (_abi.STEP_GRADIENTS if need_input_grad and need_weight_grad
+                else _abi.STEP_INPUT_GRAD if need_input_grad else _abi.STEP_WEIGHT_GRAD)
+        nbytes = int(L.fsw_workspace_bytes(step | flag, T, D, I)) if need_input_grad or need_weight_grad else 0
         ws = torch.empty(nbytes, device=dev, dtype=torch.uint8) if nbytes > 0 else None
         ld_dw = w_gate.shape[1]
         _abi.check(L.fsw_swiglu_backward(
@@ -505,6 +570,50 @@ def fused_weight_grad(x: torch.Tensor, grad_xw_up: torch.Tensor, grad_xw_gate: t
             T, D, I, _ld(x2), _ld(du), _ld(grad_w_up), ws.data_ptr() if ws is not None else None, ws_bytes,
             _code(dtype, weights_out_in), _stream_ptr(dev)))
     return grad_w_up, grad_w_gate
+
+
+def fused_gradients(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, grad_xw_up: torch.Tensor,
+                    grad_xw_gate: torch.Tensor, dtype: torch.dtype, out: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
+                    weights_out_in: bool = False, padded_from: Optional[int] = None
+                    ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(grad_x, grad_w_up, grad_w_gate): fused_input_grad and fused_weight_grad of the same gating gradients, same arguments
+    and bits, in one launch where that is faster."""
+    D, I = _weight_dims(w_gate, weights_out_in)
+    x2, wg, wu, du, dg = _rows(x), _rows(w_gate), _rows(w_up), _rows(grad_xw_up), _rows(grad_xw_gate)
+    T, dev = x2.shape[0], x.device
+    cols, ldw, ldg = _pad8(I) if padded_from else I, _ld(wg), _ld(dg)
+    # what is not plain - operands that want copies, other sizes, types or devices - is left to the two launchers and their checks
+    plain = (dev.type == "cuda" and w_gate.device == w_up.device == grad_xw_up.device == grad_xw_gate.device == dev
+             and x.dtype == w_gate.dtype == w_up.dtype == grad_xw_up.dtype == grad_xw_gate.dtype == dtype
+             and x2.shape[1] == D and wg.shape == wu.shape and dg.shape == du.shape == (T, cols) and T > 0 and D > 0 and I > 0
+             and _ld(wu) == ldw and _ld(du) == ldg)
+    if plain and padded_from:
+        plain = padded_from == I
+    elif plain:
+        ldx = _ld(x2)
+        plain = not ((D | I | ldx | ldw | ldg) & 7 or (x2.data_ptr() | wg.data_ptr() | wu.data_ptr() | dg.data_ptr() | du.data_ptr()) & 15
+                     or max(ldx, ldw, ldg) >= _TILED_MAX_LD)
+    if plain and out is not None:
+        plain = all([t.shape == w_gate.shape and t.dtype == dtype and t.device == dev and t.stride(-1) == 1
+                     and _ld(t) == _ld(out[0]) >= t.shape[1] and (padded_from or _whole_chunks(t)) for t in out])
+    if not plain:
+        grad_w_up, grad_w_gate = fused_weight_grad(x, grad_xw_up, grad_xw_gate, dtype, out=out, weights_out_in=weights_out_in,
+                                                   padded_from=padded_from)
+        return (fused_input_grad(grad_xw_gate, grad_xw_up, w_gate, w_up, dtype, weights_out_in=weights_out_in,
+                                 padded=padded_from is not None), grad_w_up, grad_w_gate)
+    with _on_device(dev):
+        if padded_from:
+            (x2,), (wg, wu) = _padded_copies(x2), _padded_copies(wg, wu)
+            grad_x, grad_w_up, grad_w_gate = _padded_gradients(x2, wg, wu, dg, du, dtype, D, I, weights_out_in, out=out)
+            return grad_x.view(tuple(grad_xw_gate.shape[:-1]) + (D,)), grad_w_up, grad_w_gate
+        grad_x = torch.empty(tuple(grad_xw_gate.shape[:-1]) + (D,), device=dev, dtype=dtype)
+        grad_w_up, grad_w_gate = out if out is not None else (torch.empty(w_gate.shape, device=dev, dtype=dtype) for _ in range(2))
+        ws, ws_bytes = _workspace(_abi.STEP_GRADIENTS | (_abi.WEIGHTS_OUT_IN if weights_out_in else 0), T, D, I, dev)
+        _abi.check(_abi.lib().fsw_swiglu_gradients(
+            x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), dg.data_ptr(), du.data_ptr(), grad_x.data_ptr(), grad_w_gate.data_ptr(),
+            grad_w_up.data_ptr(), T, D, I, _ld(x2), _ld(wg), _ld(dg), D, _ld(grad_w_up),
+            ws.data_ptr() if ws is not None else None, ws_bytes, _code(dtype, weights_out_in), _stream_ptr(dev)))
+    return grad_x, grad_w_up, grad_w_gate
 
 
 # ---- the down projection that follows the SwiGLU (w_down [I, D]; [D, I] with weights_out_in) ----
@@ -581,6 +690,32 @@ def down_proj_weight_grad(act: torch.Tensor, grad_y: torch.Tensor, dtype: torch.
             a2.data_ptr(), g2.data_ptr(), grad_w.data_ptr(), T, I, D, _ld(a2), _ld(g2), grad_w.shape[1],
             ws.data_ptr() if ws is not None else None, ws_bytes, _code(dtype, weights_out_in, pad), _stream_ptr(dev)))
         return _unpadded(grad_w, cols) if pad else grad_w
+
+
+def down_proj_backward(grad_y: torch.Tensor, act: torch.Tensor, w_down: torch.Tensor, dtype: torch.dtype,
+                       weights_out_in: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(grad_act, grad_w_down): down_proj_input_grad and down_proj_weight_grad, same bits, in one launch where that is
+    faster."""
+    I, D = _down_dims(w_down, weights_out_in)
+    a2, g2, w2 = _rows(act), _rows(grad_y), _rows(w_down)
+    T, dev = g2.shape[0], act.device
+    lda, ldg, ldw = _ld(a2), _ld(g2), _ld(w2)
+    # what is not plain is left to the two launchers, their copies and their checks
+    if not (dev.type == "cuda" and grad_y.device == w_down.device == dev and act.dtype == grad_y.dtype == w_down.dtype == dtype
+            and g2.shape[1] == D and a2.shape == (T, I) and act.shape[:-1] == grad_y.shape[:-1] and T > 0 and D > 0 and I > 0
+            and not ((D | I | lda | ldg | ldw) & 7 or (a2.data_ptr() | g2.data_ptr() | w2.data_ptr()) & 15)
+            and max(lda, ldg, ldw) < _TILED_MAX_LD):
+        return (down_proj_input_grad(grad_y, w_down, dtype, weights_out_in=weights_out_in),
+                down_proj_weight_grad(act, grad_y, dtype, weights_out_in=weights_out_in))
+    with _on_device(dev):
+        grad_act = torch.empty(tuple(grad_y.shape[:-1]) + (I,), device=dev, dtype=dtype)
+        grad_w = torch.empty(w_down.shape, device=dev, dtype=dtype)
+        ws, ws_bytes = _workspace(_abi.STEP_DOWN_BACKWARD | (_abi.WEIGHTS_OUT_IN if weights_out_in else 0), T, D, I, dev)
+        _abi.check(_abi.lib().fsw_down_proj_backward(
+            a2.data_ptr(), g2.data_ptr(), w2.data_ptr(), grad_act.data_ptr(), grad_w.data_ptr(), T, I, D, _ld(a2), _ld(g2),
+            _ld(w2), I, w_down.shape[1], ws.data_ptr() if ws is not None else None, ws_bytes, _code(dtype, weights_out_in),
+            _stream_ptr(dev)))
+    return grad_act, grad_w
 
 
 def fused_bmm(x_t: torch.Tensor, grad_xw_up: torch.Tensor, grad_xw_gate: torch.Tensor,

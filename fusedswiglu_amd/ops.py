@@ -124,26 +124,25 @@ def _swiglu_backward(grad_out: Tensor, x: Tensor, w_gate: Tensor, w_up: Tensor, 
         d_up, d_gate = _launch.elementwise_backward(grad_out, xw_gate, xw_up, dtype, padded=padded)
     padded_from = I if padded else None
     dx = dw_gate = dw_up = None
-    # the weight gradient first: the input gradient then finds d_gate and d_up in the memory-side cache
-    if need_w_gate or need_w_up:
-        if packed and oi:
-            I, D = w_gate.shape
-            dw_gate = torch.empty((2 * I, D), device=x.device, dtype=dtype)
-            _launch.fused_weight_grad(x, d_up, d_gate, dtype, out=(dw_gate[I:], dw_gate[:I]), weights_out_in=True,
-                                      padded_from=padded_from)
-        elif packed:
-            D, I = w_gate.shape
-            dw_gate = torch.empty((D, 2 * I), device=x.device, dtype=dtype)
-            _launch.fused_weight_grad(x, d_up, d_gate, dtype, out=(dw_gate[:, I:], dw_gate[:, :I]),
-                                      padded_from=padded_from)
-        else:
-            dw_up, dw_gate = _launch.fused_weight_grad(x, d_up, d_gate, dtype, weights_out_in=oi, padded_from=padded_from)
-            if not need_w_gate:
-                dw_gate = None
-            if not need_w_up:
-                dw_up = None
-    if need_x:
-        dx = _launch.fused_input_grad(d_gate, d_up, w_gate, w_up, dtype, weights_out_in=oi, padded=padded).view(x.shape)
+    need_w = need_w_gate or need_w_up
+    out = None
+    if need_w and packed:
+        # the two halves of one packed array
+        dw_gate = torch.empty((2 * I, D) if oi else (D, 2 * I), device=x.device, dtype=dtype)
+        out = (dw_gate[I:], dw_gate[:I]) if oi else (dw_gate[:, I:], dw_gate[:, :I])
+    if need_x and need_w:
+        dx, dw_up, half = _launch.fused_gradients(x, w_gate, w_up, d_up, d_gate, dtype, out=out, weights_out_in=oi,
+                                                  padded_from=padded_from)
+    elif need_w:
+        dw_up, half = _launch.fused_weight_grad(x, d_up, d_gate, dtype, out=out, weights_out_in=oi, padded_from=padded_from)
+    elif need_x:
+        dx = _launch.fused_input_grad(d_gate, d_up, w_gate, w_up, dtype, weights_out_in=oi, padded=padded)
+    if packed or not need_w_up:
+        dw_up = None
+    if not packed and need_w_gate:
+        dw_gate = half
+    if dx is not None:
+        dx = dx.view(x.shape)
     return (dx if dx is not None else e, dw_gate if dw_gate is not None else e.clone(),
             dw_up if dw_up is not None else e.clone())
 
@@ -201,6 +200,8 @@ def _down_proj_backward(grad_y: Tensor, act: Tensor, w_down: Tensor, need_act: b
     if grad_y.dtype != dtype:
         grad_y = grad_y.to(dtype)
     e = _empty(act)
+    if need_act and need_w:
+        return _launch.down_proj_backward(grad_y, act, w_down, dtype, weights_out_in=weights_out_in)
     d_act = _launch.down_proj_input_grad(grad_y, w_down, dtype, weights_out_in=weights_out_in) if need_act else e
     d_w = _launch.down_proj_weight_grad(act, grad_y, dtype, weights_out_in=weights_out_in) if need_w else e.clone()
     return d_act, d_w

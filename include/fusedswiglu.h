@@ -43,8 +43,8 @@ extern "C" {
 #endif
 
 /* major*10000 + minor*100 + patch.
- * 0.4.0: fsw_swiglu_backward (the three backward steps in one call); FSW_ROWS_PADDED, fsw_repack_rows and
- *        fsw_elementwise_backward_rows.
+ * 0.4.0: fsw_swiglu_backward (the three backward steps in one call), fsw_swiglu_gradients, fsw_down_proj_backward
+ *        and steps 7 and 8 of fsw_workspace_bytes; FSW_ROWS_PADDED, fsw_repack_rows and fsw_elementwise_backward_rows.
  * 0.3.0: FSW_WEIGHTS_OUT_IN, the fsw_down_proj_* entry points, fsw_input_grad_noalloc and status 7,
  *        fsw_uses_tiled_kernel answers 2 for the weight-streaming kernels and knows steps 4 / 5 / 6,
  *        fsw_workspace_bytes may ask for up to 64 MiB for large gradient GEMMs (tail split).
@@ -156,8 +156,8 @@ FSW_API int fsw_gating_grad_recompute(const void* x, const void* w_gate, const v
  * workgroups use it the same way for the tiles of that round only (at most 64 MiB).  The few-token down
  * projection plans its split with the compute-unit count of the current device: query and call with the
  * same device current.  fsw_workspace_bytes gives a sufficient size for
- * step 1 (input_grad), 2 (weight_grad), 4 / 5 / 6 (down projection forward / input grad / weight grad),
- * each optionally | FSW_WEIGHTS_OUT_IN; with workspace == NULL or a smaller size the call still
+ * step 1 (input_grad), 2 (weight_grad), 7 (fsw_swiglu_gradients and fsw_swiglu_backward, at least the larger of the two),
+ * 4 / 5 / 6 / 8 (down projection forward / input grad / weight grad / fsw_down_proj_backward), each optionally | FSW_WEIGHTS_OUT_IN; with workspace == NULL or a smaller size the call still
  * works, just without the split.
  */
 FSW_API int64_t fsw_workspace_bytes(int step, int64_t T, int64_t D, int64_t I);
@@ -205,15 +205,27 @@ FSW_API int fsw_weight_grad(const void* x, const void* grad_xw_up, const void* g
                     int dtype, void* stream);
 
 /*
+ * fsw_weight_grad and fsw_input_grad of the same gating gradients in one call.  Where both are small enough to leave CUs
+ * without work they share one launch, which needs `workspace` to hold the partial tiles of both
+ * (fsw_workspace_bytes(7, ...)); the results have the same bits as from the two calls with scratch of the sizes they ask for.
+ *   x, grad_x [T,D] (ldx, ld_dx)   w_gate, w_up (ldw)   grad_xw_gate, grad_xw_up [T,I] (ldo)   grad_w_gate, grad_w_up (ld_dw)
+ */
+FSW_API int fsw_swiglu_gradients(const void* x, const void* w_gate, const void* w_up, const void* grad_xw_gate,
+                         const void* grad_xw_up, void* grad_x, void* grad_w_gate, void* grad_w_up, int64_t T, int64_t D,
+                         int64_t I, int64_t ldx, int64_t ldw, int64_t ldo, int64_t ld_dx, int64_t ld_dw, void* workspace,
+                         int64_t workspace_bytes, int dtype, void* stream);
+
+/*
  * The whole backward of the path in one call: the body of FusedSwiGLU.backward (fused_swiglu/swiglu.py:34-58).
- * Exactly fsw_elementwise_backward, then fsw_weight_grad (if the two weight gradients are given), then fsw_input_grad
- * (if grad_x is given), enqueued on `stream` in that order - for hosts where three calls through a foreign-function
- * interface cost more than the small kernels they launch.
+ * fsw_elementwise_backward, then fsw_weight_grad (if the two weight gradients are given) and fsw_input_grad (if grad_x is
+ * given), both together as in fsw_swiglu_gradients, enqueued on `stream` - for hosts where three calls through a
+ * foreign-function interface cost more than the small kernels they launch.  The same bits as from the three calls.
  *   grad_out, xw_gate, xw_up, grad_xw_gate, grad_xw_up [T,I] dense (leading dimension I)
  *   x [T,D] (ldx)   w_gate, w_up (ldw)   grad_x [T,D] (ld_dx)   grad_w_gate, grad_w_up (ld_dw)
  * grad_xw_gate and grad_xw_up are results too (the gating gradients), always written.  grad_x may be NULL, and
- * grad_w_gate / grad_w_up both NULL: that gradient is skipped (ctx.needs_input_grad).  `workspace` is used by the
- * two GEMMs one after the other: the larger of fsw_workspace_bytes(1, ...) and fsw_workspace_bytes(2, ...) serves both.
+ * grad_w_gate / grad_w_up both NULL: that gradient is skipped (ctx.needs_input_grad).  The larger of
+ * fsw_workspace_bytes(1, ...) and fsw_workspace_bytes(2, ...) serves both GEMMs one after the other, fsw_workspace_bytes(7, ...)
+ * in one launch as well.
  */
 FSW_API int fsw_swiglu_backward(const void* grad_out, const void* xw_gate, const void* xw_up, const void* x,
                         const void* w_gate, const void* w_up, void* grad_xw_gate, void* grad_xw_up, void* grad_x,
@@ -245,6 +257,14 @@ FSW_API int fsw_down_proj_input_grad(const void* grad_y, const void* w_down, voi
 FSW_API int fsw_down_proj_weight_grad(const void* act, const void* grad_y, void* grad_w_down, int64_t T, int64_t I,
                                       int64_t D, int64_t ld_act, int64_t ldy, int64_t ld_dw, void* workspace,
                                       int64_t workspace_bytes, int dtype, void* stream);
+
+/*
+ * Both gradients in one call: fsw_down_proj_input_grad and fsw_down_proj_weight_grad, in one launch where that is faster
+ * and `workspace` holds the partial tiles of both (step 8 of fsw_workspace_bytes); the same bits as from the two calls.
+ */
+FSW_API int fsw_down_proj_backward(const void* act, const void* grad_y, const void* w_down, void* grad_act, void* grad_w_down,
+                                   int64_t T, int64_t I, int64_t D, int64_t ld_act, int64_t ldy, int64_t ldw, int64_t ld_dact,
+                                   int64_t ld_dw, void* workspace, int64_t workspace_bytes, int dtype, void* stream);
 
 #ifdef __cplusplus
 }

@@ -55,6 +55,10 @@ FSW_API int fsw_probe_mfma_mix(int mix, int iters, int workgroups, const void* b
  */
 FSW_API int fsw_plan_tiled(int mode, int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int* blocks, int* splits,
                            int* tail_parts);
+/* fsw_plan_pair: the two gradients of the SwiGLU (down 0) or of the down projection (down 1) with dense operands and scratch
+ * without limit.  blocks_w, blocks_x: 16-row blocks per wave of the weight and the input gradient in their one launch, both 0 where
+ * they take two; splits_w, splits_x: of their reductions. */
+FSW_API int fsw_plan_pair(int out_in, int down, int64_t T, int64_t D, int64_t I, int* blocks_w, int* blocks_x, int* splits_w, int* splits_x);
 FSW_API int fsw_plan_few_tokens(int out_in, int down, int64_t M, int64_t N, int64_t K, int cus, int64_t planes, int* slot,
                                 int* blocks, int* columns, int* splits);
 
