@@ -50,25 +50,30 @@ FSW_DEV void store_few(const GemmParams& p, int plain, int split, int m, int n, 
   }
 }
 
-// MQ: 16-row blocks of x (T <= 16 MQ).  BN: columns of both weight matrices a workgroup has room for.
-// A stage is SK k-elements in blocks of 64: x, 16 MQ rows of one 128-byte line each, then the weights,
+// MQ: 16-row blocks of x (T <= 16 MQ; 0: T <= 8).  BN: columns of both weight matrices a workgroup has room for.
+// A stage is SK k-elements in blocks of 64: x, 16 MQ (8) rows of one 128-byte line each, then the weights,
 //   [I, D]: BN gate rows and BN up rows, one line each;   [D, I]: 64 k-rows x 2 BN bytes of Wg, then of Wu.
 // The ring holds as many stages as fit into 160 KiB; four waves share it, wave w working on columns
 // 16 (w % (BN / 16)).. and on every (64 / BN)th group of 32 k-elements; partial sums meet in LDS at the end.
+// BN = 8 ([I, D] only, T <= 16): the 16 rows of an MFMA operand are 8 gate and 8 up rows, so a short result has twice the
+// workgroups without an LDS slot, a line of x or an MFMA that is half empty.
 template <int MQ, int BN>
 struct NarrowCfg {
-  static constexpr int SK = BN == 16 || (BN == 32 && MQ == 1) ? 128 : 64;
+  static constexpr int SK = MQ == 0 ? 256 : BN <= 16 || (BN == 32 && MQ == 1) ? 128 : 64;
   static constexpr int kBlocks = SK / 64;
-  static constexpr int kXBlock = 16 * MQ * 128, kWBlock = 2 * BN * 128;  // bytes per 64 k-elements
+  static constexpr int kXRows = MQ == 0 ? 8 : 16 * MQ, kQ = MQ == 0 ? 1 : MQ;
+  static constexpr int kXBlock = kXRows * 128, kWBlock = 2 * BN * 128;  // bytes per 64 k-elements
   static constexpr int kXBytes = kBlocks * kXBlock;
   static constexpr int kStage = kBlocks * (kXBlock + kWBlock);
   static constexpr int kStages = (160 * 1024) / kStage;
   static constexpr int kXLoads = kXBytes / 4096, kWLoads = kBlocks * kWBlock / 4096;  // per wave
   static constexpr int kPerStage = kXLoads + kWLoads;
-  static constexpr int kColGroups = BN / 16, kKWays = 4 / kColGroups;
+  static constexpr int kFrags = BN == 8 ? 1 : 2;  // weight operands per 16 columns: gate and up, or both in one
+  static constexpr int kColGroups = BN == 8 ? 1 : BN / 16, kKWays = 4 / kColGroups;
   static constexpr int kSteps = SK / 32 / kKWays;  // groups of 32 k-elements per wave and stage
-  static_assert(kXLoads > 0 && kXBytes % 4096 == 0 && kWLoads > 0 && kSteps > 0 && kStages >= 3, "");
+  static_assert(kXLoads > 0 && kXBytes % 4096 == 0 && kWLoads > 0 && kBlocks * kWBlock % 4096 == 0 && kSteps > 0 && kStages >= 3, "");
   static_assert((kStages - 2) * kPerStage < 64, "vmcnt is 6 bits");
+  static_assert(BN != 8 || MQ <= 1, "");
 };
 
 // [D, I] weights, a panel of k-rows x 2 BN bytes.  The transposing read takes 32 bytes (16 columns) of four
@@ -106,7 +111,7 @@ __global__ __launch_bounds__(kSkThreads) void fsw_narrow_kernel(GemmParams p, Sk
   const char* w_base[C::kWLoads];
 #pragma unroll
   for (int j = 0; j < C::kXLoads; j++) {
-    const int idx = wave + 4 * j, kb = idx / (2 * MQ), row = 8 * (idx % (2 * MQ)) + (lane >> 3);
+    const int idx = wave + 4 * j, kb = idx / (C::kXRows / 8), row = 8 * (idx % (C::kXRows / 8)) + (lane >> 3);
     const int k = kb * 64 + ((lane & 7) ^ ((row >> 1) & 7)) * 8;
     x_off[j] = (unsigned)row * (unsigned)p.lda * 2u + k * 2u;
     x_klim[j] = row < p.M ? k_end - k : -0x40000000;
@@ -118,7 +123,7 @@ __global__ __launch_bounds__(kSkThreads) void fsw_narrow_kernel(GemmParams p, Sk
     w_base[j] = (const char*)(up ? p.b1 : p.b0) + (W_KC ? (size_t)n0 * p.ldb * 2 : (size_t)n0 * 2);
     if constexpr (W_KC) {
       const int row = 8 * ii + (lane >> 3);
-      const int k = kb * 64 + ((lane & 7) ^ ((row >> 1) & 7)) * 8;
+      const int k = kb * 64 + ((lane & 7) ^ (((row + up * BN) >> 1) & 7)) * 8;  // (up * BN + row of the area)
       w_off[j] = (unsigned)row * (unsigned)p.ldb * 2u + k * 2u;
       w_klim[j] = row < bn && n0 + row < p.n_rows_b ? k_end - k : -0x40000000;
     } else {
@@ -143,20 +148,20 @@ __global__ __launch_bounds__(kSkThreads) void fsw_narrow_kernel(GemmParams p, Sk
                            st + C::kXBytes + (wave + 4 * j) * 1024);
   };
   const int cg = wave % C::kColGroups, kw = wave / C::kColGroups;
-  f32x4 acc[2][MQ];
+  f32x4 acc[C::kFrags][C::kQ];
 #pragma unroll
-  for (int h = 0; h < 2; h++)
+  for (int h = 0; h < C::kFrags; h++)
 #pragma unroll
-    for (int q = 0; q < MQ; q++) acc[h][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int q = 0; q < C::kQ; q++) acc[h][q] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto multiply = [&](const FSW_LDS char* st) {
 #pragma unroll
     for (int i = 0; i < C::kSteps; i++) {
       const int step = kw + i * C::kKWays, kb = step >> 1, half = step & 1;
       const FSW_LDS char* sx = st + kb * C::kXBlock;
       const FSW_LDS char* sw = st + C::kXBytes + kb * C::kWBlock;
-      i16x8 fw[2], fx[MQ];
+      i16x8 fw[C::kFrags], fx[C::kQ];
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
+      for (int h = 0; h < C::kFrags; h++) {
         if constexpr (W_KC) {
           fw[h] = read_frag_kc16(sw, h * BN + cg * 16, half, lane);
         } else {
@@ -168,12 +173,13 @@ __global__ __launch_bounds__(kSkThreads) void fsw_narrow_kernel(GemmParams p, Sk
           fw[h] = i16x8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
         }
       }
+      // (8 rows of x: the other 8 columns of the MFMA's result repeat them and go nowhere)
 #pragma unroll
-      for (int q = 0; q < MQ; q++) fx[q] = read_frag_kc16(sx, q * 16, half, lane);
+      for (int q = 0; q < C::kQ; q++) fx[q] = read_frag_kc16(sx, q * 16, half, MQ == 0 ? lane & ~8 : lane);
 #pragma unroll
-      for (int q = 0; q < MQ; q++)
+      for (int q = 0; q < C::kQ; q++)
 #pragma unroll
-        for (int h = 0; h < 2; h++) acc[h][q] = E::mfma16(fw[h], fx[q], acc[h][q]);
+        for (int h = 0; h < C::kFrags; h++) acc[h][q] = E::mfma16(fw[h], fx[q], acc[h][q]);
     }
   };
 
@@ -190,36 +196,44 @@ __global__ __launch_bounds__(kSkThreads) void fsw_narrow_kernel(GemmParams p, Sk
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the zero-filling loads past the end too
 
+  constexpr int F = C::kFrags, Q = C::kQ;
   if constexpr (C::kKWays > 1) {
-    static_assert((C::kKWays - 1) * C::kColGroups * 64 * 2 * MQ * 16 <= C::kStages * C::kStage, "");
+    static_assert((C::kKWays - 1) * C::kColGroups * 64 * F * Q * 16 <= C::kStages * C::kStage, "");
     FSW_LDS f32x4* part = (FSW_LDS f32x4*)smem;
     if (kw > 0) {
 #pragma unroll
-      for (int h = 0; h < 2; h++)
+      for (int h = 0; h < F; h++)
 #pragma unroll
-        for (int q = 0; q < MQ; q++) part[(((wave - C::kColGroups) * 2 + h) * MQ + q) * 64 + lane] = acc[h][q];
+        for (int q = 0; q < Q; q++) part[(((wave - C::kColGroups) * F + h) * Q + q) * 64 + lane] = acc[h][q];
     }
     __syncthreads();
     if (kw > 0) return;
 #pragma unroll
     for (int w = 1; w < C::kKWays; w++)
 #pragma unroll
-      for (int h = 0; h < 2; h++)
+      for (int h = 0; h < F; h++)
 #pragma unroll
-        for (int q = 0; q < MQ; q++) {
-          const f32x4 b = part[((((w - 1) * C::kColGroups + cg) * 2 + h) * MQ + q) * 64 + lane];
+        for (int q = 0; q < Q; q++) {
+          const f32x4 b = part[((((w - 1) * C::kColGroups + cg) * F + h) * Q + q) * 64 + lane];
           acc[h][q].x += b.x; acc[h][q].y += b.y; acc[h][q].z += b.z; acc[h][q].w += b.w;
         }
   }
-  // acc[h][q][r] of lane l: row 16 q + (l & 15), column n0 + 16 cg + 4 (l >> 4) + r
+  // acc[h][q][r] of lane l: row 16 q + (l & 15), column n0 + 16 cg + 4 (l >> 4) + r; BN = 8: gate in lanes 0-31, the up
+  // column of lane l in lane l + 32
+  f32x4 up[Q];
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    if constexpr (F == 2) up[q] = acc[F - 1][q];
+    else up[q] = f32x4{__shfl_xor(acc[0][q].x, 32), __shfl_xor(acc[0][q].y, 32), __shfl_xor(acc[0][q].z, 32), __shfl_xor(acc[0][q].w, 32)};
+  }
   const int nc = cg * 16 + 4 * (lane >> 4), n = n0 + nc;
   if (nc >= bn || n >= p.N) return;
 #pragma unroll
-  for (int q = 0; q < MQ; q++) {
+  for (int q = 0; q < Q; q++) {
     const int m = q * 16 + (lane & 15);
     if (m >= p.M) continue;
     const float g[4] = {acc[0][q].x, acc[0][q].y, acc[0][q].z, acc[0][q].w};
-    const float u[4] = {acc[1][q].x, acc[1][q].y, acc[1][q].z, acc[1][q].w};
+    const float u[4] = {up[q].x, up[q].y, up[q].z, up[q].w};
     store_few<E>(p, a.plain, split, m, n, g, u);
   }
 }

@@ -202,6 +202,13 @@ template <typename E, bool W_KC>
 static hipError_t launch_skinny_t(const GemmParams& g, const SkPlan& pl, int plain, hipStream_t s) {
   const SkArgs a{pl.bn, plain, pl.splits, pl.stages_per_split};
   const dim3 grid((unsigned)((g.N + a.bn - 1) / a.bn), (unsigned)a.splits);
+  if constexpr (W_KC) {
+    if (pl.paired) {
+      if (g.M <= 8) fsw_narrow_kernel<E, 0, 8, true><<<grid, kSkThreads, 0, s>>>(g, a);
+      else fsw_narrow_kernel<E, 1, 8, true><<<grid, kSkThreads, 0, s>>>(g, a);
+      return hipGetLastError();
+    }
+  }
   switch (pl.slot * 16 + pl.mq) {
 #define FSW_NARROW(SLOT, MQ) case SLOT * 16 + MQ: fsw_narrow_kernel<E, MQ, SLOT, W_KC><<<grid, kSkThreads, 0, s>>>(g, a); break
     FSW_NARROW(16, 1);

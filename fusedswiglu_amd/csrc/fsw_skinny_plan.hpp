@@ -26,8 +26,10 @@ inline int block_width(int N, int cus, bool w_kc, int bm) {
 }
 
 // A launch: column blocks of `slot` = 128 (fsw_skinny_forward_kernel) or 16, 32, 64 columns (fsw_narrow_kernel; mq
-// 16-row blocks of x), of which bn are used, times k-splits.
-struct SkPlan { int slot, mq, bn, splits, stages_per_split; };
+// 16-row blocks of x), of which bn are used, times k-splits.  paired: 8 columns whose gate and up rows share a slot of 16.
+struct SkPlan { int slot, mq, bn, splits, stages_per_split; bool paired; };
+// k-elements of a stage of the narrow kernel (NarrowCfg)
+inline int narrow_stage(int slot, int mq, bool paired, long long M) { return paired ? (M <= 8 ? 256 : 128) : slot == 16 || (slot == 32 && mq == 1) ? 128 : 64; }
 
 // Blocks of 128 columns for the down projection: full blocks and as many k-splits as fit into one round of workgroups
 // (measured at N = 8192, K = 28672: 32 blocks x 8 splits beat every narrower block with fewer splits in this kernel,
@@ -38,9 +40,9 @@ inline SkPlan plan_wide(long long M, long long Nh, long long K, int cus, bool w_
   const long long tiles = (Nh + 127) / 128;
   // a split shorter than 8 stages does not fill the ring
   const long long splits = std::min({cus / tiles, max_splits, (long long)stages / 8});
-  if (max_splits < 1 || splits <= 1) return SkPlan{128, 0, block_width((int)Nh, cus, w_kc, (int)M), 1, stages};
+  if (max_splits < 1 || splits <= 1) return SkPlan{128, 0, block_width((int)Nh, cus, w_kc, (int)M), 1, stages, false};
   const int sps = (int)((stages + splits - 1) / splits);
-  return SkPlan{128, 0, 128, (stages + sps - 1) / sps, sps};
+  return SkPlan{128, 0, 128, (stages + sps - 1) / sps, sps, false};
 }
 
 // Microseconds of a launch by what it moves, fitted to 9700 measured launches with weights that are not in the caches (1 to
@@ -52,11 +54,11 @@ inline SkPlan plan_wide(long long M, long long Nh, long long K, int cus, bool w_
 inline double estimate_us(const SkPlan& p, long long M, long long Nh, long long K, int cus, bool w_kc) {
   const bool wide = p.slot == 128;
   const long long wgs = (Nh + p.bn - 1) / p.bn * p.splits, rounds = (wgs + cus - 1) / cus;
-  const int x_rows = !wide ? 16 * p.mq : (M <= 32 ? 32 : (M <= 64 ? 64 : 128));
-  const double stage = p.slot == 16 || (p.slot == 32 && p.mq == 1) ? 128 : 64;
+  const int x_rows = p.paired && M <= 8 ? 8 : !wide ? 16 * p.mq : (M <= 32 ? 32 : (M <= 64 ? 64 : 128));
+  const double stage = wide ? 64 : narrow_stage(p.slot, p.mq, p.paired, M);
   const double k64 = (double)rounds * p.stages_per_split * stage / 64;  // 64-element blocks a CU goes through
   const double lines = w_kc || p.slot >= 64 ? 1 : 64 / p.slot;
-  const double useful = k64 * p.bn * 256 * lines, fill = k64 * (256 * p.slot * lines + 128 * x_rows);
+  const double useful = k64 * p.bn * 256 * lines, fill = k64 * (256 * (p.paired ? p.bn : p.slot) * lines + 128 * x_rows);
   const double cu_rate = w_kc ? (wide ? 26e3 : 49e3) : (wide ? 30e3 : 36e3), fill_rate = w_kc ? (wide ? 62e3 : 50e3) : (wide ? 55e3 : 47e3);
   const double start = w_kc ? (wide ? 0.6 : 4.2) : (wide ? 1.2 : 4.3), round = wide ? 2.0 : (w_kc ? 1.3 : 0.0);
   double us = std::max({4.0 * K * Nh / 6.0e6, useful / cu_rate, fill / fill_rate}) + start + round * (rounds - 1);
@@ -77,6 +79,11 @@ inline double estimate_us(const SkPlan& p, long long M, long long Nh, long long 
 // 60.7 -> 51.3 us).  More rows, one round of 32-column blocks, or the down projections: narrow blocks win there between lines
 // as well.  What is left: a down projection of more than 64 rows with more than 40 MB of weights, reduction contiguous.  The
 // estimate errs both ways there, narrow blocks took 0.84 to 1.24 of the time (geometric mean 1.0), and no simple rule parts them.
+// 8-column blocks whose gate and up rows share the 16 rows of an MFMA operand ([I, D], up to 16 rows; NarrowCfg): twice the
+// workgroups of 16-column blocks and no half-empty slots, and a result of up to 4096 columns needs neither parts nor the launch
+// that adds them.  Against what was chosen before (1 to 16 rows, nn.Linear's layout, 70 random down projections): 0.951 of the time
+// on average, worst 1.05, best 0.74; 1 x 11008 -> 4096 20.7 -> 18.9 us, 4 x 8704 -> 4096 18.7 -> 14.8, 1 x 9408 -> 2688 15.5 -> 12.5,
+// the input gradient of 2 x 3328 x 1152 in the other layout 5.6 -> 4.8.
 inline SkPlan choose_within(long long M, long long Nh, long long K, int cus, bool w_kc, bool whole_lines, bool plain,
                             long long max_splits) {
   SkPlan best = plan_wide(M, Nh, K, cus, w_kc, plain ? max_splits : 0);
@@ -90,20 +97,27 @@ inline SkPlan choose_within(long long M, long long Nh, long long K, int cus, boo
     // a third round of 16-column blocks: 1 to 29 % longer than blocks of 64 or 128 in 11 of 12 down projections of up to 16 rows
     // (16 x 7232 -> 17536 56.3 -> 43.6 us; 6 x 7760 -> 17520 67.0 -> 69.7)
     if (slot == 16 && (mq > 4 || (w_kc && Nh > 32LL * cus))) continue;
-    const int stage = slot == 16 || (slot == 32 && mq == 1) ? 128 : 64;
-    const int stages = (int)((K + stage - 1) / stage);
     // widths: the whole slot; rows of [I, D] weights are lines of their own, so also what fills 1 .. 5 rounds, and 8
     // columns for short results
     for (int i = 0; i <= (w_kc ? 6 : 0); i++) {
       const int bn = i == 0 ? slot : (i == 6 ? 8 : (int)(((Nh + cus * i - 1) / (cus * i) + 3) & ~3LL));
+      const bool paired = w_kc && bn == 8 && mq == 1;
       if (bn > slot || bn < slot / 2 || (i == 6 && !plain)) continue;
+      const int stage = narrow_stage(slot, mq, paired, M), stages = (int)((K + stage - 1) / stage);
       const long long blocks = (Nh + bn - 1) / bn;
       for (int splits : {1, 2, 3, 4, 6, 8}) {
-        if (splits > 1 && (!plain || splits > max_splits || blocks * splits > 560 || K < 128 * splits)) break;
+        // (8-column blocks in parts: no faster than whole in 40 of 42 launches, for all their scratch and the second launch)
+        if (splits > 1 && (!plain || paired || splits > max_splits || blocks * splits > 560 || K < 128 * splits)) break;
         if (blocks * splits < (splits > 1 ? 48 : 40)) continue;
         const int sps = (stages + splits - 1) / splits;
-        const SkPlan pl{slot, mq, bn, (stages + sps - 1) / sps, sps};
-        const double us = estimate_us(pl, M, Nh, K, cus, w_kc);
+        const SkPlan pl{slot, mq, bn, (stages + sps - 1) / sps, sps, paired};
+        // (x rows that are there cost more than those that zero-fill: 12 x 5440 -> 1984 10.3 us, paired 10.9; 6 x 9472 -> 2560 13.8
+        // and 14.6)
+        double us = estimate_us(pl, M, Nh, K, cus, w_kc) * (!paired || M <= 4 ? 1.0 : M <= 8 ? 1.04 : 1.08);
+        // One full round of 8-column blocks against split blocks of 128: 3 us more than the estimate knows, for the start of many
+        // short parts and, between lines, for their rows (1 / 8 / 16 x 11008 -> 4096 20.7 -> 18.8, 21.4 -> 19.9, 23.0 -> 21.8 us,
+        // 4 x 12976 -> 4032 30.4 -> 22.6)
+        if (paired && splits == 1 && blocks <= cus && 8 * blocks >= 7LL * cus && best.slot == 128 && best.splits > 1) us -= 3.0;
         if (us < best_us) { best_us = us; best = pl; }
       }
     }
