@@ -96,12 +96,11 @@ class SwiGLU(nn.Module):
         return tuple(out)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        dtype = next(self.parameters()).dtype
         if self.packed:
-            return ops.swiglu_packed(x, self.w_gate_up, autocast_dtype=dtype, recompute=self.recompute,
-                                     weights_out_in=self.weights_out_in)
-        return ops.swiglu(x, self.w_gate, self.w_up, autocast_dtype=dtype, recompute=self.recompute,
-                          weights_out_in=self.weights_out_in)
+            w = self.w_gate_up
+            return ops.swiglu_packed(x, w, autocast_dtype=w.dtype, recompute=self.recompute, weights_out_in=self.weights_out_in)
+        w = self.w_gate
+        return ops.swiglu(x, w, self.w_up, autocast_dtype=w.dtype, recompute=self.recompute, weights_out_in=self.weights_out_in)
 
     def extra_repr(self) -> str:
         return (f"d_model={self.d_model}, d_intermediate={self.d_intermediate}, packed={self.packed}, "
@@ -146,5 +145,5 @@ class SwiGLUMLP(nn.Module):
         return m
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return ops.down_proj(self.swiglu(x), self.w_down, autocast_dtype=self.w_down.dtype,
-                             weights_out_in=self.weights_out_in)
+        w = self.w_down
+        return ops.down_proj(self.swiglu(x), w, autocast_dtype=w.dtype, weights_out_in=self.weights_out_in)

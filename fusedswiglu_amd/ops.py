@@ -30,6 +30,7 @@ from typing import Tuple
 import torch
 from torch import Tensor
 
+from . import _host
 from .kernels import _launch
 
 _SUPPORTED = (torch.bfloat16, torch.float16)
@@ -145,6 +146,29 @@ def _swiglu_backward(grad_out: Tensor, x: Tensor, w_gate: Tensor, w_up: Tensor, 
         dx = dx.view(x.shape)
     return (dx if dx is not None else e, dw_gate if dw_gate is not None else e.clone(),
             dw_up if dw_up is not None else e.clone())
+
+
+def _general_backward(grad_out, x, w_gate, w_up, xw_gate, xw_up, need_x, need_w_gate, need_w_up, packed, weights_out_in, operator):
+    """A backward pass of the native path's autograd node that is not plain: pre-activations as that path keeps them (None:
+    recomputed; or [tokens, I rounded up to 8]), a packed weight in one piece; None for what is not needed."""
+    if packed:
+        w_gate, w_up = _halves(w_gate, weights_out_in)
+        need_w_up = need_w_gate
+    if xw_gate is None:
+        xw_gate = xw_up = _empty(x)
+    else:
+        wide = tuple(grad_out.shape[:-1]) + (xw_gate.shape[-1],)
+        xw_gate, xw_up = (t.view(wide)[..., :grad_out.shape[-1]] for t in (xw_gate, xw_up))
+    backward = _pick(swiglu_backward, _swiglu_backward, grad_out, x, w_gate, w_up, xw_gate, xw_up) if operator else _swiglu_backward
+    dx, dw_gate, dw_up = backward(grad_out.contiguous(), x, w_gate, w_up, xw_gate, xw_up, need_x, need_w_gate, need_w_up, packed,
+                                  weights_out_in)
+    return dx if need_x else None, dw_gate if need_w_gate else None, dw_up if need_w_up and not packed else None
+
+
+def _general_down_backward(grad_y, act, w_down, need_act, need_w, weights_out_in):
+    backward = _pick(down_proj_backward, _down_proj_backward, grad_y, act, w_down)
+    d_act, d_w = backward(grad_y.contiguous(), act, w_down, need_act, need_w, weights_out_in)
+    return d_act if need_act else None, d_w if need_w else None
 
 
 swiglu_backward = torch.library.custom_op("fusedswiglu_amd::swiglu_backward", mutates_args=(), device_types="cuda")(_swiglu_backward)
@@ -264,6 +288,10 @@ def swiglu(x: Tensor, w_gate: Tensor, w_up: Tensor, autocast_dtype: torch.dtype 
     """silu(x @ w_gate) * (x @ w_up) with weights laid out [d_model, d_intermediate], or
     silu(x @ w_gate.T) * (x @ w_up.T) with nn.Linear-style [d_intermediate, d_model] weights
     (`weights_out_in=True`), which are read in place."""
+    if not torch.compiler.is_compiling():
+        out = _host.swiglu(x, w_gate, w_up, -1, bool(recompute), bool(weights_out_in), True)
+        if out is not None:
+            return out
     _require_gpu(x, w_gate, w_up)
     x, w_gate, w_up = _autocast(autocast_dtype, x, w_gate, w_up)
     save = _records_gradient(x, w_gate, w_up)
@@ -279,6 +307,10 @@ def down_proj(act: Tensor, w_down: Tensor, autocast_dtype: torch.dtype | None = 
               weights_out_in: bool = False) -> Tensor:
     """act @ w_down with w_down [d_intermediate, d_model] (act @ w_down.T for nn.Linear-style
     [d_model, d_intermediate] with `weights_out_in=True`)."""
+    if not torch.compiler.is_compiling():
+        y = _host.down_proj(act, w_down, bool(weights_out_in))
+        if y is not None:
+            return y
     _require_gpu(act, w_down)
     act, w_down = _autocast(autocast_dtype, act, w_down)
     if not _records_gradient(act, w_down) and _unobserved(act, w_down):
@@ -335,6 +367,10 @@ def swiglu_packed(x: Tensor, w_gate_up: Tensor, autocast_dtype: torch.dtype | No
                   recompute: bool = False, weights_out_in: bool = False) -> Tensor:
     """SwiGLU with a packed weight [d_model, 2*d_intermediate] = [w_gate | w_up] (or, with
     `weights_out_in`, [2*d_intermediate, d_model] = gate rows then up rows)."""
+    if not torch.compiler.is_compiling():
+        out = _host.swiglu(x, w_gate_up, None, -1, bool(recompute), bool(weights_out_in), True)
+        if out is not None:
+            return out
     if w_gate_up.ndim != 2 or w_gate_up.shape[0 if weights_out_in else 1] % 2:
         raise _launch.ShapeError("packed weight must be [d_model, 2*d_intermediate] (or [2*d_intermediate, d_model])")
     _require_gpu(x, w_gate_up)

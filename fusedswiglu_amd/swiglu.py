@@ -7,10 +7,11 @@ same autocast behaviour (inputs are cast to bfloat16 only under torch.autocast),
 import torch
 from torch.autograd import Function
 
-from . import _function
+from . import _abi, _function, _host
 from .kernels import kernels_bf16 as _kernels
 
 _DTYPE = torch.bfloat16
+_CODE = _abi.DTYPE_BF16
 
 
 class FusedSwiGLU(Function):
@@ -26,6 +27,11 @@ class FusedSwiGLU(Function):
 
     @classmethod
     def apply(cls, input, weight_gate, weight_up):
+        # a plain call, in native code (a subclass may have a forward or backward of its own)
+        if cls is FusedSwiGLU and not torch.compiler.is_compiling():
+            out = _host.swiglu(input, weight_gate, weight_up, _CODE)
+            if out is not None:
+                return out
         # no gradient can flow: skip the autograd node and the two pre-activation stores
         if not _function.wants_grad(input, weight_gate, weight_up):
             return _function.forward_inference(_kernels, _DTYPE, input, weight_gate, weight_up)

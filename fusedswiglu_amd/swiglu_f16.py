@@ -7,10 +7,11 @@ only for compatibility."""
 import torch
 from torch.autograd import Function
 
-from . import _function
+from . import _abi, _function, _host
 from .kernels import kernels_fp16 as _kernels
 
 _DTYPE = torch.float16
+_CODE = _abi.DTYPE_FP16
 
 
 class FastAccumFusedSwiGLU(Function):
@@ -26,6 +27,11 @@ class FastAccumFusedSwiGLU(Function):
 
     @classmethod
     def apply(cls, input, weight_gate, weight_up):
+        # a plain call, in native code (a subclass may have a forward or backward of its own)
+        if cls is FastAccumFusedSwiGLU and not torch.compiler.is_compiling():
+            out = _host.swiglu(input, weight_gate, weight_up, _CODE)
+            if out is not None:
+                return out
         if not _function.wants_grad(input, weight_gate, weight_up):
             return _function.forward_inference(_kernels, _DTYPE, input, weight_gate, weight_up)
         return super().apply(input, weight_gate, weight_up)
