@@ -40,7 +40,9 @@ EXPORTED_SYMBOLS = (
     "fsw_swiglu_forward",
     "fsw_elementwise_backward",
     "fsw_elementwise_backward_rows",
+    "fsw_elementwise_backward_group",
     "fsw_repack_rows",
+    "fsw_repack_group",
     "fsw_gating_grad_recompute",
     "fsw_input_grad",
     "fsw_input_grad_noalloc",
@@ -55,6 +57,12 @@ EXPORTED_SYMBOLS = (
 #: every symbol include/fusedswiglu_bench.h declares (libfusedswiglu_bench.so)
 BENCH_SYMBOLS = ("fsw_probe_mfma", "fsw_probe_stream_read", "fsw_probe_mfma_mix", "fsw_probe_dma_read", "fsw_plan_tiled",
                  "fsw_plan_pair", "fsw_plan_few_tokens")
+
+
+class RowCopy(ctypes.Structure):
+    """fsw_row_copy"""
+    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("rows", ctypes.c_int64), ("cols", ctypes.c_int64),
+                ("ld_src", ctypes.c_int64), ("ld_dst", ctypes.c_int64), ("pad", ctypes.c_int)]
 
 
 class FusedSwiGLUError(RuntimeError):
@@ -119,6 +127,10 @@ def lib() -> ctypes.CDLL:
         L.fsw_elementwise_backward_rows.argtypes = [vp] * 5 + [i64] * 5 + [ci, vp]
         L.fsw_repack_rows.restype = ci
         L.fsw_repack_rows.argtypes = [vp] * 4 + [i64] * 4 + [ci, vp]
+        L.fsw_repack_group.restype = ci
+        L.fsw_repack_group.argtypes = [ctypes.POINTER(RowCopy), ci, vp]
+        L.fsw_elementwise_backward_group.restype = ci
+        L.fsw_elementwise_backward_group.argtypes = [vp] * 5 + [i64] * 5 + [ctypes.POINTER(RowCopy), ci, ci, vp]
         L.fsw_gating_grad_recompute.restype = ci
         L.fsw_gating_grad_recompute.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, ci, vp]
         L.fsw_input_grad.restype = ci

@@ -196,23 +196,43 @@ int fsw_gating_grad_recompute(const void* x, const void* w_gate, const void* w_u
   return launched(fn, fsw::launch_forward_generic(dtype, p, s));
 }
 
+static int check_copy(const char* fn, const fsw_row_copy& c) {
+  if (!c.src || !c.dst) return fail(FSW_ERR_NULL_POINTER, "%s: source and destination must be non-null", fn);
+  if (c.rows <= 0 || c.cols <= 0 || c.rows > 0x7fffffffLL || c.cols > 0x7fffffffLL - 8)
+    return fail(FSW_ERR_BAD_SHAPE, "%s: rows and columns must be positive and below 2^31 (rows=%lld cols=%lld)", fn, (long long)c.rows, (long long)c.cols);
+  if (int e = check_ld(fn, "ld_src", c.ld_src, c.cols)) return e;
+  if (int e = check_ld(fn, "ld_dst", c.ld_dst, c.cols, c.pad != 0)) return e;
+  if (!al2(c.src) || !al2(c.dst)) return fail(FSW_ERR_ALIGNMENT, "%s: pointers must be 2-byte aligned", fn);
+  return FSW_OK;
+}
+static int run_row_group(const char* fn, int dtype, const fsw::GatingRows* gating, const fsw_row_copy* copies, int count, void* stream) {
+  fsw::RowCopy c[fsw::kMaxRowCopies];
+  static_assert(fsw::kMaxRowCopies == FSW_MAX_ROW_COPIES, "the header's limit");
+  if (count < 0 || count > FSW_MAX_ROW_COPIES) return fail(FSW_ERR_BAD_SHAPE, "%s: 0 to %d copies, got %d", fn, FSW_MAX_ROW_COPIES, count);
+  if (count > 0 && !copies) return fail(FSW_ERR_NULL_POINTER, "%s: copies must be non-null", fn);
+  for (int i = 0; i < count; i++) {
+    if (int e = check_copy(fn, copies[i])) return e;
+    c[i] = fsw::RowCopy{copies[i].src, copies[i].dst, copies[i].rows, copies[i].cols, copies[i].ld_src, copies[i].ld_dst, copies[i].pad != 0};
+  }
+  return launched(fn, fsw::launch_row_group(dtype, gating, c, count, (hipStream_t)stream));
+}
+
 int fsw_repack_rows(const void* src0, void* dst0, const void* src1, void* dst1, int64_t rows, int64_t cols, int64_t ld_src,
                     int64_t ld_dst, int pad, void* stream) {
   const char* fn = "fsw_repack_rows";
   if (!src0 || !dst0 || (src1 == nullptr) != (dst1 == nullptr))
     return fail(FSW_ERR_NULL_POINTER, "%s: src0 and dst0 must be non-null, src1 and dst1 both given or both null", fn);
-  if (rows <= 0 || cols <= 0 || rows > 0x7fffffffLL || cols > 0x7fffffffLL - 8)
-    return fail(FSW_ERR_BAD_SHAPE, "%s: rows and columns must be positive and below 2^31 (rows=%lld cols=%lld)", fn, (long long)rows, (long long)cols);
-  if (int e = check_ld(fn, "ld_src", ld_src, cols)) return e;
-  if (int e = check_ld(fn, "ld_dst", ld_dst, cols, pad != 0)) return e;
-  if (!al2(src0) || !al2(dst0) || !al2(src1) || !al2(dst1)) return fail(FSW_ERR_ALIGNMENT, "%s: pointers must be 2-byte aligned", fn);
-  return launched(fn, fsw::launch_repack(src0, dst0, src1, dst1, rows, cols, ld_src, ld_dst, pad != 0, (hipStream_t)stream));
+  const fsw_row_copy c[2] = {{src0, dst0, rows, cols, ld_src, ld_dst, pad}, {src1, dst1, rows, cols, ld_src, ld_dst, pad}};
+  return run_row_group(fn, fsw::kDtypeBF16, nullptr, c, src1 ? 2 : 1, stream);
 }
 
-int fsw_elementwise_backward_rows(const void* grad_out, const void* xw_gate, const void* xw_up, void* grad_xw_up,
-                                  void* grad_xw_gate, int64_t T, int64_t I, int64_t ld_grad_out, int64_t ld_xw, int64_t ld_grad,
-                                  int dtype, void* stream) {
-  const char* fn = "fsw_elementwise_backward_rows";
+int fsw_repack_group(const fsw_row_copy* copies, int count, void* stream) {
+  return run_row_group("fsw_repack_group", fsw::kDtypeBF16, nullptr, copies, count, stream);
+}
+
+static int elementwise_rows(const char* fn, const void* grad_out, const void* xw_gate, const void* xw_up, void* grad_xw_up,
+                            void* grad_xw_gate, int64_t T, int64_t I, int64_t ld_grad_out, int64_t ld_xw, int64_t ld_grad,
+                            const fsw_row_copy* copies, int count, int dtype, void* stream) {
   if (!grad_out || !xw_gate || !xw_up || !grad_xw_up || !grad_xw_gate)
     return fail(FSW_ERR_NULL_POINTER, "%s: all five arrays must be non-null", fn);
   if (!dtype_ok(dtype)) return fail(FSW_ERR_BAD_DTYPE, "%s: dtype %d is neither bf16 (0) nor fp16 (1)", fn, dtype);
@@ -223,8 +243,22 @@ int fsw_elementwise_backward_rows(const void* grad_out, const void* xw_gate, con
   if (!al2(grad_out) || !al2(xw_gate) || !al2(xw_up)) return fail(FSW_ERR_ALIGNMENT, "%s: pointers must be 2-byte aligned", fn);
   if ((((uintptr_t)grad_xw_up | (uintptr_t)grad_xw_gate) & 15) || (ld_grad & 7))
     return fail(FSW_ERR_ALIGNMENT, "%s: the rows of the results must be 16-byte aligned", fn);
-  return launched(fn, fsw::launch_elementwise_rows(elem_of(dtype), grad_out, ld_grad_out, xw_gate, xw_up, ld_xw, grad_xw_up,
-                                                   grad_xw_gate, ld_grad, T, I, (hipStream_t)stream));
+  const fsw::GatingRows g{grad_out, xw_gate, xw_up, grad_xw_up, grad_xw_gate, T, I, ld_grad_out, ld_xw, ld_grad};
+  return run_row_group(fn, elem_of(dtype), &g, copies, count, stream);
+}
+
+int fsw_elementwise_backward_rows(const void* grad_out, const void* xw_gate, const void* xw_up, void* grad_xw_up,
+                                  void* grad_xw_gate, int64_t T, int64_t I, int64_t ld_grad_out, int64_t ld_xw, int64_t ld_grad,
+                                  int dtype, void* stream) {
+  return elementwise_rows("fsw_elementwise_backward_rows", grad_out, xw_gate, xw_up, grad_xw_up, grad_xw_gate, T, I, ld_grad_out, ld_xw,
+                          ld_grad, nullptr, 0, dtype, stream);
+}
+
+int fsw_elementwise_backward_group(const void* grad_out, const void* xw_gate, const void* xw_up, void* grad_xw_up,
+                                   void* grad_xw_gate, int64_t T, int64_t I, int64_t ld_grad_out, int64_t ld_xw, int64_t ld_grad,
+                                   const fsw_row_copy* copies, int count, int dtype, void* stream) {
+  return elementwise_rows("fsw_elementwise_backward_group", grad_out, xw_gate, xw_up, grad_xw_up, grad_xw_gate, T, I, ld_grad_out, ld_xw,
+                          ld_grad, copies, count, dtype, stream);
 }
 
 int fsw_elementwise_backward(const void* grad_out, const void* xw_gate, const void* xw_up,

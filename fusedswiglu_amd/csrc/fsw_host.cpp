@@ -151,34 +151,46 @@ struct Call {  // what every library call of one pass shares
     *bytes = fsw_workspace_bytes(step | (dtype & FSW_WEIGHTS_OUT_IN), T, D, I);
     return *bytes > 0 ? at::empty({*bytes}, options.dtype(at::kByte)) : Tensor();
   }
-  void repack(uintptr_t s0, void* d0, uintptr_t s1, void* d1, int64_t rows, int64_t cols, int64_t ld_src, int64_t ld_dst, bool pad) const {
-    check(fsw_repack_rows(reinterpret_cast<void*>(s0), d0, reinterpret_cast<void*>(s1), d1, rows, cols, ld_src, ld_dst, pad, stream));
-  }
 };
 void* ptr(uintptr_t p) { return reinterpret_cast<void*>(p); }
 void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
+// Copies between row pitches that go into one launch; the arrays outlive it.
+struct Copies {
+  fsw_row_copy copy[FSW_MAX_ROW_COPIES];
+  int count = 0;
+  void add(uintptr_t src, uintptr_t dst, int64_t rows, int64_t cols, int64_t ld_src, int64_t ld_dst, bool pad) {
+    TORCH_INTERNAL_ASSERT(count < FSW_MAX_ROW_COPIES);
+    copy[count++] = {ptr(src), ptr(dst), rows, cols, ld_src, ld_dst, pad};
+  }
+  void run(const Call& c) {
+    if (count > 0) check(fsw_repack_group(copy, count, c.stream));
+    count = 0;
+  }
+};
+
 // Padded copies of rows the tiled kernels cannot read as they are (`keep` holds them), and of the two weights together.
-void pad_rows(const Call& c, Rows& r, Tensor& keep) {
+void pad_rows(const Call& c, Rows& r, Tensor& keep, Copies& todo) {
   if (whole_chunks(r) && r.ld < g_max_ld) return;
   keep = c.empty({r.rows, pad8(r.cols)});
-  c.repack(r.p, ptr(keep), 0, nullptr, r.rows, r.cols, r.ld, pad8(r.cols), true);
+  todo.add(r.p, addr(keep), r.rows, r.cols, r.ld, pad8(r.cols), true);
   r.p = addr(keep);
   r.ld = pad8(r.cols);
 }
-void pad_weights(const Call& c, Weights& w, Tensor (&keep)[2]) {
+void pad_weights(const Call& c, Weights& w, Tensor (&keep)[2], Copies& todo) {
   if (w.whole() && w.ld < g_max_ld) return;
   for (auto& k : keep) k = c.empty({w.rows(), pad8(w.cols())});
-  c.repack(w.pg, ptr(keep[0]), w.pu, ptr(keep[1]), w.rows(), w.cols(), w.ld, pad8(w.cols()), true);
+  todo.add(w.pg, addr(keep[0]), w.rows(), w.cols(), w.ld, pad8(w.cols()), true);
+  todo.add(w.pu, addr(keep[1]), w.rows(), w.cols(), w.ld, pad8(w.cols()), true);
   w.pg = addr(keep[0]);
   w.pu = addr(keep[1]);
   w.ld = pad8(w.cols());
 }
 // The dense array of the given shape from a result whose rows are padded (as it is if they are not).
-Tensor dense(const Call& c, const Tensor& padded, int64_t cols, at::IntArrayRef shape) {
+Tensor dense(const Call& c, const Tensor& padded, int64_t cols, at::IntArrayRef shape, Copies& todo) {
   if (padded.size(-1) == cols) return padded;
   Tensor out = c.empty(shape);
-  c.repack(addr(padded), ptr(out), 0, nullptr, padded.size(0), cols, padded.size(1), cols, false);
+  todo.add(addr(padded), addr(out), padded.size(0), cols, padded.size(1), cols, false);
   return out;
 }
 
@@ -203,8 +215,10 @@ void run_forward(const Tensor& x, Weights w, bool save, Tensor& out, Tensor& g, 
   const Call c(x, w.out_in, padded);
   Tensor keep_x, keep_w[2];
   if (padded) {
-    pad_rows(c, rx, keep_x);
-    pad_weights(c, w, keep_w);
+    Copies todo;
+    pad_rows(c, rx, keep_x, todo);
+    pad_weights(c, w, keep_w, todo);
+    todo.run(c);
   }
   const int64_t ldo = padded ? pad8(I) : I;
   const auto shape = with_last(x, I);
@@ -216,7 +230,12 @@ void run_forward(const Tensor& x, Weights w, bool save, Tensor& out, Tensor& g, 
     u = c.empty(result);
   }
   check(fsw_swiglu_forward(ptr(rx.p), ptr(w.pg), ptr(w.pu), ptr(out), ptr(g), ptr(u), T, D, I, rx.ld, w.ld, ldo, c.dtype, c.stream));
-  if (padded) out = dense(c, out, I, shape);
+  if (padded) {
+    Copies todo;
+    const Tensor result_rows = out;
+    out = dense(c, result_rows, I, shape, todo);
+    todo.run(c);
+  }
 }
 
 // The gradients that are asked for, or false for a call that is not plain.  Without g and u the pre-activations are recomputed.
@@ -237,8 +256,9 @@ bool run_backward(const Tensor& grad, const Tensor& x, Weights w, const Tensor& 
   const Call c(x, w.out_in, padded);
   const Tensor dout = grad.contiguous();
   Tensor keep_x, keep_w[2], keep_d;
-  if (padded && (need_w || recompute)) pad_rows(c, rx, keep_x);
-  if (padded && (need_x || recompute)) pad_weights(c, w, keep_w);
+  Copies todo;  // (what the gradients read: goes with the gating gradient)
+  if (padded && (need_w || recompute)) pad_rows(c, rx, keep_x, todo);
+  if (padded && (need_x || recompute)) pad_weights(c, w, keep_w, todo);
   const Tensor dG = c.empty({T, ldi}), dU = c.empty({T, ldi});
   const int64_t rows = w.rows(), cols = w.cols(), ldx = padded ? pad8(D) : D;
   // results: dense, or padded and made dense at the end; the halves of a packed gradient lie in one array
@@ -263,14 +283,21 @@ bool run_backward(const Tensor& grad, const Tensor& x, Weights w, const Tensor& 
   int64_t bytes = 0;
   Tensor ws;
   if (need_x || need_w) ws = c.scratch(need_x && need_w ? 7 : need_x ? 1 : 2, T, D, I, &bytes);
-  if (!recompute) {
+  if (!recompute && !padded) {
     check(fsw_swiglu_backward(ptr(dout), ptr(g), ptr(u), ptr(rx.p), ptr(w.pg), ptr(w.pu), ptr(dG), ptr(dU), ptr(dx), dwg, dwu, T, D, I,
                               rx.ld, w.ld, ldx, ld_dw, ptr(ws), bytes, c.dtype, c.stream));
   } else {
-    Rows rd;
-    rd.rows = T, rd.cols = rd.ld = I, rd.p = addr(dout);
-    if (padded) pad_rows(c, rd, keep_d);
-    check(fsw_gating_grad_recompute(ptr(rx.p), ptr(w.pg), ptr(w.pu), ptr(rd.p), ptr(dU), ptr(dG), T, D, I, rx.ld, w.ld, ldi, c.dtype, c.stream));
+    if (recompute) {
+      Rows rd;
+      rd.rows = T, rd.cols = rd.ld = I, rd.p = addr(dout);
+      if (padded) pad_rows(c, rd, keep_d, todo);
+      todo.run(c);
+      check(fsw_gating_grad_recompute(ptr(rx.p), ptr(w.pg), ptr(w.pu), ptr(rd.p), ptr(dU), ptr(dG), T, D, I, rx.ld, w.ld, ldi, c.dtype, c.stream));
+    } else {
+      check(fsw_elementwise_backward_group(ptr(dout), ptr(g), ptr(u), ptr(dU), ptr(dG), T, I, I, ldi, ldi, todo.copy, todo.count,
+                                           c.dtype & ~(FSW_WEIGHTS_OUT_IN | FSW_ROWS_PADDED), c.stream));
+      todo.count = 0;
+    }
     if (need_x && need_w)
       check(fsw_swiglu_gradients(ptr(rx.p), ptr(w.pg), ptr(w.pu), ptr(dG), ptr(dU), ptr(dx), dwg, dwu, T, D, I, rx.ld, w.ld, ldi, ldx, ld_dw,
                                  ptr(ws), bytes, c.dtype, c.stream));
@@ -279,19 +306,21 @@ bool run_backward(const Tensor& grad, const Tensor& x, Weights w, const Tensor& 
     else if (need_x)
       check(fsw_input_grad(ptr(dG), ptr(dU), ptr(w.pg), ptr(w.pu), ptr(dx), T, D, I, ldi, w.ld, ldx, ptr(ws), bytes, c.dtype, c.stream));
   }
-  if (need_x) dx = dense(c, dx, D, x.sizes());
+  const Tensor dx_rows = dx;  // (held until the copies are enqueued)
+  if (need_x) dx = dense(c, dx_rows, D, x.sizes(), todo);
   if (need_w) {
     if (w.packed && padded) {
-      c.repack(addr(pg), ptr(p_dwg), addr(pu), ptr(p_dwu), rows, cols, ld_dw, dw_gate.size(1), false);
+      todo.add(addr(pg), p_dwg, rows, cols, ld_dw, dw_gate.size(1), false);
+      todo.add(addr(pu), p_dwu, rows, cols, ld_dw, dw_gate.size(1), false);
     } else if (!w.packed && ld_dw != cols) {
-      dw_gate = c.empty({rows, cols});
-      dw_up = c.empty({rows, cols});
-      c.repack(addr(pg), ptr(dw_gate), addr(pu), ptr(dw_up), rows, cols, ld_dw, cols, false);
+      dw_gate = dense(c, pg, cols, {rows, cols}, todo);
+      dw_up = dense(c, pu, cols, {rows, cols}, todo);
     } else if (!w.packed) {
       dw_gate = pg;
       dw_up = pu;
     }
   }
+  todo.run(c);
   return true;
 }
 

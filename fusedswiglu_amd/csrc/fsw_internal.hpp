@@ -74,17 +74,26 @@ hipError_t launch_forward_generic(int dtype, const Problem& p, hipStream_t s);
 hipError_t launch_input_grad_generic(int dtype, const Problem& p, hipStream_t s);
 hipError_t launch_weight_grad_generic(int dtype, const Problem& p, hipStream_t s);
 
-// [rows, cols] from one row pitch to another (elements of 16 bits), two arrays at most; with `pad`, the columns up to the
-// next multiple of 8 are set to zero.
-hipError_t launch_repack(const void* src0, void* dst0, const void* src1, void* dst1, long long rows, long long cols,
-                         long long ld_src, long long ld_dst, bool pad, hipStream_t s);
+// [rows, cols] from one row pitch to another (elements of 16 bits); with `pad`, the columns up to the next multiple of 8 are
+// set to zero.
+struct RowCopy {
+  const void* src;
+  void* dst;
+  long long rows, cols, ld_src, ld_dst;
+  bool pad;
+};
+constexpr int kMaxRowCopies = 4;
+// The gating gradient on rows: dout [rows, cols] (ld_dout), g, u (ld_gu) -> dU, dG (ld_out, 16-byte aligned rows, columns up to
+// the next multiple of 8 set to zero).
+struct GatingRows {
+  const void *dout, *g, *u;
+  void *dU, *dG;
+  long long rows, cols, ld_dout, ld_gu, ld_out;
+};
+// Both (gating may be null), in one launch; no array may be the result of another.
+hipError_t launch_row_group(int dtype, const GatingRows* gating, const RowCopy* copies, int n, hipStream_t s);
 
 hipError_t launch_elementwise(int dtype, const void* dout, const void* g, const void* u, void* dU,
                               void* dG, size_t n, hipStream_t stream);
-
-// The same on rows: dout [rows, cols] (ld_in), g, u (ld_gu) -> dU, dG (ld_out, 16-byte aligned rows, columns up to the next
-// multiple of 8 set to zero).
-hipError_t launch_elementwise_rows(int dtype, const void* dout, long long ld_dout, const void* g, const void* u, long long ld_gu,
-                                   void* dU, void* dG, long long ld_out, long long rows, long long cols, hipStream_t stream);
 
 }  // namespace fsw

@@ -107,8 +107,8 @@ def _code(dtype: torch.dtype, weights_out_in: bool, padded: bool = False) -> int
 # Rows that are not whole 16-byte chunks (a dimension that is not a multiple of 8) or do not start on 16-byte
 # boundaries are copied once into padded rows; the padded results are copied back.  Each copy moves an array once in
 # each direction; the kernels behind it run at 10 to 30 times the rate of the edge-shape kernel (a training step of 2048
-# tokens, 1024 x 2730, bf16: 1712 us of GPU time on the edge-shape kernel, 134 us on padded copies in 13 launches, whose host
-# time makes it 143 to 255 us of wall time, by the host).  The copies add to a call's peak memory: x and both weights padded,
+# tokens, 1024 x 2730, bf16: 1712 us of GPU time on the edge-shape kernel, 115 us on padded copies, in 7 launches from native
+# code; from here, with a launch per array shape and its checks in Python, the host makes it 240 us).  The copies add to a call's peak memory: x and both weights padded,
 # and each result padded until it is copied back (that step 116 -> 125 MB).  Padding pays from this
 # many multiply-adds per matrix product on (forward / backward, edge kernel against padded: 33 / 56 against 46 / 75 us at
 # 2^21.5, 39 / 100 against 46 / 77 at 2^24.5, 69 / 224 against 46 / 77 at 2^25.2) ...

@@ -44,7 +44,8 @@ extern "C" {
 
 /* major*10000 + minor*100 + patch.
  * 0.4.0: fsw_swiglu_backward (the three backward steps in one call), fsw_swiglu_gradients, fsw_down_proj_backward
- *        and steps 7 and 8 of fsw_workspace_bytes; FSW_ROWS_PADDED, fsw_repack_rows and fsw_elementwise_backward_rows.
+ *        and steps 7 and 8 of fsw_workspace_bytes; FSW_ROWS_PADDED, fsw_repack_rows / _group and
+ *        fsw_elementwise_backward_rows / _group.
  * 0.3.0: FSW_WEIGHTS_OUT_IN, the fsw_down_proj_* entry points, fsw_input_grad_noalloc and status 7,
  *        fsw_uses_tiled_kernel answers 2 for the weight-streaming kernels and knows steps 4 / 5 / 6,
  *        fsw_workspace_bytes may ask for up to 64 MiB for large gradient GEMMs (tail split).
@@ -134,6 +135,21 @@ FSW_API int fsw_elementwise_backward_rows(const void* grad_out, const void* xw_g
  */
 FSW_API int fsw_repack_rows(const void* src0, void* dst0, const void* src1, void* dst1, int64_t rows, int64_t cols,
                             int64_t ld_src, int64_t ld_dst, int pad, void* stream);
+
+/* The same for up to FSW_MAX_ROW_COPIES arrays of any shapes in one launch; no array may be the destination of another. */
+#define FSW_MAX_ROW_COPIES 4
+typedef struct fsw_row_copy {
+  const void* src;
+  void* dst;
+  int64_t rows, cols, ld_src, ld_dst;
+  int pad;
+} fsw_row_copy;
+FSW_API int fsw_repack_group(const fsw_row_copy* copies, int count, void* stream);
+
+/* fsw_elementwise_backward_rows and, in the same launch, `count` copies that touch none of its arrays. */
+FSW_API int fsw_elementwise_backward_group(const void* grad_out, const void* xw_gate, const void* xw_up, void* grad_xw_up,
+                                           void* grad_xw_gate, int64_t T, int64_t I, int64_t ld_grad_out, int64_t ld_xw,
+                                           int64_t ld_grad, const fsw_row_copy* copies, int count, int dtype, void* stream);
 
 /*
  * Gating gradient without saved pre-activations: recomputes g = x Wg and u = x Wu (fp32, never
