@@ -168,6 +168,7 @@ int fsw_swiglu_forward(const void* x, const void* w_gate, const void* w_up, void
   if (fsw::skinny_forward_ok(p)) return launched(fn, fsw::launch_forward_skinny(dtype, p, s));
   if (fsw::fast_path_ok_forward(p)) return launched(fn, fsw::launch_forward_fast(dtype, p, s));
   if (padded) return not_padded(fn);
+  if (fsw::stream_unaligned_ok(p)) return launched(fn, fsw::launch_forward_unaligned(dtype, p, s));
   return launched(fn, fsw::launch_forward_generic(dtype, p, s));
 }
 

@@ -62,6 +62,9 @@ long long splitk_workspace_bytes(int step, long long T, long long D, long long I
 // Weight-streaming forward for T <= 128 tokens (same eligibility as the tiled forward otherwise).
 bool skinny_forward_ok(const Problem& p);
 hipError_t launch_forward_skinny(int dtype, const Problem& p, hipStream_t s);
+// The forward for T <= 128 on rows of any length, pitch and 2-byte alignment.
+bool stream_unaligned_ok(const Problem& p);
+hipError_t launch_forward_unaligned(int dtype, const Problem& p, hipStream_t s);
 
 // The same kernel as a plain GEMM for the down projection of few tokens (layouts 0 and 1, M <= 128, N even and
 // its half aligned); splits the reduction into the caller's scratch when column blocks alone leave CUs idle.

@@ -89,10 +89,32 @@ FSW_DEV int narrow_piece(int r, int b) {
   return b ^ ((r >> 1) & 1) ^ (((r >> 3) & 1) << 1);
 }
 
-template <typename E, int MQ, int BN, bool W_KC>
+// Eight elements at any 2-byte aligned address; all of them, or the first `left` with zeros behind.
+struct __attribute__((packed, aligned(2))) AnyChunk { u32x4 v; };
+FSW_DEV u32x4 load_any(const char* p) { return ((const AnyChunk*)p)->v; }
+FSW_DEV u32x4 load_any(const char* p, int left) {
+  if (left >= 8) return load_any(p);
+  u32x4 r{0, 0, 0, 0};
+#pragma unroll
+  for (int e = 0; e < 7; e++)
+    if (e < left) r[e >> 1] |= (unsigned)((const unsigned short*)p)[e] << (16 * (e & 1));
+  return r;
+}
+
+// UNALIGNED: rows of any length, pitch and 2-byte alignment, which the direct loads to LDS do not take (forward only, bn = BN,
+// one split, N >= 8).  The stages go through registers, kAhead of them in flight, into two LDS slots of the same format.  Every
+// stage but the last is loaded without a bounds check: rows of x and of [I, D] weights that do not exist are read from the last
+// one that does, as are [D, I] columns from the last chunk, whose end reaches into the next row; what they give is in rows and
+// columns that are not stored.  The last stage is checked chunk by chunk, and those that end inside go element by element.
+// Bound: HBM for few rows of x (8190 x 20001 [I, D], 1 / 16 tokens: 5.2 / 4.7 TB/s), with more rows the copies of x in every
+// workgroup, and for [D, I] weights their 64-byte row segments, which straddle lines (3.7 / 3.4 TB/s).  Padded copies of the
+// weights and the aligned kernels move the weights three times: 405 / 407 and 368 / 369 us there, 126 / 141 and 178 / 193 here;
+// one of 1 token that stays on the edge-shape kernel, 2047 x 5461: 309 and 353 us, 15 and 17 here.
+template <typename E, int MQ, int BN, bool W_KC, bool UNALIGNED = false>
 __global__ __launch_bounds__(kSkThreads) void fsw_narrow_kernel(GemmParams p, SkArgs a) {
   using C = NarrowCfg<MQ, BN>;
-  __shared__ __attribute__((aligned(1024))) char smem[C::kStages * C::kStage];
+  constexpr int kSlots = UNALIGNED ? 2 : C::kStages;
+  __shared__ __attribute__((aligned(1024))) char smem[kSlots * C::kStage];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Neighbouring column blocks go to the same XCD: [D, I] blocks narrower than 64 columns share 128-byte lines in its L2.
@@ -183,22 +205,113 @@ __global__ __launch_bounds__(kSkThreads) void fsw_narrow_kernel(GemmParams p, Sk
     }
   };
 
+  if constexpr (UNALIGNED) {
+    constexpr int kAhead = MQ == 8 ? 3 : 4;  // (a stage with 128 rows of x is 96 bytes per lane)
+    const char *x_ptr[C::kXLoads], *w_ptr[C::kWLoads];
+    int x_k[C::kXLoads], w_left[C::kWLoads];  // last stage: k-element of the chunk; columns from the chunk on ([D, I])
+    bool x_there[C::kXLoads], w_there[C::kWLoads];
+    int w_k[C::kWLoads];
 #pragma unroll
-  for (int s = 0; s < C::kStages - 1; s++) issue(s, smem_addr + s * C::kStage);
-  unsigned cur = 0, prev = (C::kStages - 1) * C::kStage;
-  for (int s = 0; s < st_total; s++) {
-    // this wave's loads of stage s and its fragment reads of stage s - 1 are complete; behind the barrier everyone's are
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((C::kStages - 2) * C::kPerStage) : "memory");
-    issue(s + C::kStages - 1, smem_addr + prev);
-    multiply(smem_l + cur);
-    prev = cur;
-    cur = cur + C::kStage == C::kStages * C::kStage ? 0 : cur + C::kStage;
+    for (int j = 0; j < C::kXLoads; j++) {
+      const int idx = wave + 4 * j, kb = idx / (C::kXRows / 8), row = 8 * (idx % (C::kXRows / 8)) + (lane >> 3);
+      x_k[j] = kb * 64 + ((lane & 7) ^ ((row >> 1) & 7)) * 8;
+      x_there[j] = row < p.M;
+      x_ptr[j] = (const char*)p.a0 + ((size_t)min(row, p.M - 1) * p.lda + x_k[j]) * 2;
+    }
+#pragma unroll
+    for (int j = 0; j < C::kWLoads; j++) {
+      const int idx = wave + 4 * j, kb = idx / (BN / 4), i = idx % (BN / 4);
+      const int up = i / (BN / 8), ii = i % (BN / 8);
+      const char* base = (const char*)(up ? p.b1 : p.b0);
+      if constexpr (W_KC) {
+        const int row = 8 * ii + (lane >> 3);
+        w_k[j] = kb * 64 + ((lane & 7) ^ (((row + up * BN) >> 1) & 7)) * 8;
+        w_there[j] = n0 + row < p.N;
+        w_left[j] = 8;
+        w_ptr[j] = base + ((size_t)min(n0 + row, p.N - 1) * p.ldb + w_k[j]) * 2;
+      } else {
+        constexpr int kChunks = BN / 8;
+        const int row = narrow_place<BN>(ii * (64 / kChunks) + lane / kChunks), chunk = lane % kChunks;
+        const int col = n0 + narrow_piece<BN>(row, chunk >> 1) * 16 + (chunk & 1) * 8;
+        w_k[j] = kb * 64 + row;
+        w_there[j] = col < p.N;
+        w_left[j] = p.N - col;
+        w_ptr[j] = base + ((size_t)w_k[j] * p.ldb + min(col, (p.N - 1) & ~7)) * 2;
+      }
+    }
+    const int last = st_total - 1;
+    auto put = [&](int s, const u32x4 (&x)[C::kXLoads], const u32x4 (&w)[C::kWLoads]) {
+      FSW_LDS char* st = (FSW_LDS char*)smem + (s & 1) * C::kStage;
+#pragma unroll
+      for (int j = 0; j < C::kXLoads; j++) *(FSW_LDS u32x4*)(st + (wave + 4 * j) * 1024 + lane * 16) = x[j];
+#pragma unroll
+      for (int j = 0; j < C::kWLoads; j++) *(FSW_LDS u32x4*)(st + C::kXBytes + (wave + 4 * j) * 1024 + lane * 16) = w[j];
+    };
+    // The stage is in its slot: the slot's next writer is two stages on, behind the barrier that follows these reads.
+    // (__syncthreads() might wait for the loads ahead as well)
+    auto take = [&](int s) {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      multiply(smem_l + (s & 1) * C::kStage);
+    };
+    if (last > 0) {
+      u32x4 rx[kAhead][C::kXLoads], rw[kAhead][C::kWLoads];
+      // Loads of the main loop are unconditional, stages past the end once more the one before the last: behind a load that
+      // may not have been issued the compiler can only wait for all of them.
+      auto fetch = [&](int s, u32x4 (&x)[C::kXLoads], u32x4 (&w)[C::kWLoads]) {
+        s = min(s, last - 1);
+#pragma unroll
+        for (int j = 0; j < C::kXLoads; j++) x[j] = load_any(x_ptr[j] + (size_t)s * (2 * C::SK));
+#pragma unroll
+        for (int j = 0; j < C::kWLoads; j++) w[j] = load_any(w_ptr[j] + (size_t)s * w_kstep);
+      };
+      static_for<kAhead>([&](auto i) { fetch(decltype(i)::value, rx[decltype(i)::value], rw[decltype(i)::value]); });
+      int s0 = 0;
+      for (; s0 + kAhead <= last; s0 += kAhead) {
+        static_for<kAhead>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          put(s0 + i, rx[i], rw[i]);
+          fetch(s0 + i + kAhead, rx[i], rw[i]);
+          take(s0 + i);
+        });
+      }
+      static_for<kAhead - 1>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        if (s0 + i < last) {
+          put(s0 + i, rx[i], rw[i]);
+          take(s0 + i);
+        }
+      });
+    }
+    u32x4 x[C::kXLoads], w[C::kWLoads];
+    const int k0 = last * C::SK;
+#pragma unroll
+    for (int j = 0; j < C::kXLoads; j++) x[j] = load_any(x_ptr[j] + (size_t)k0 * 2, x_there[j] ? p.K - k0 - x_k[j] : 0);
+#pragma unroll
+    for (int j = 0; j < C::kWLoads; j++) {
+      const int k_left = w_there[j] ? p.K - k0 - w_k[j] : 0;
+      w[j] = load_any(w_ptr[j] + (size_t)last * w_kstep, W_KC ? k_left : k_left > 0 ? w_left[j] : 0);
+    }
+    put(last, x, w);
+    take(last);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  } else {
+#pragma unroll
+    for (int s = 0; s < C::kStages - 1; s++) issue(s, smem_addr + s * C::kStage);
+    unsigned cur = 0, prev = (C::kStages - 1) * C::kStage;
+    for (int s = 0; s < st_total; s++) {
+      // this wave's loads of stage s and its fragment reads of stage s - 1 are complete; behind the barrier everyone's are
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((C::kStages - 2) * C::kPerStage) : "memory");
+      issue(s + C::kStages - 1, smem_addr + prev);
+      multiply(smem_l + cur);
+      prev = cur;
+      cur = cur + C::kStage == C::kStages * C::kStage ? 0 : cur + C::kStage;
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the zero-filling loads past the end too
   }
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the zero-filling loads past the end too
 
   constexpr int F = C::kFrags, Q = C::kQ;
   if constexpr (C::kKWays > 1) {
-    static_assert((C::kKWays - 1) * C::kColGroups * 64 * F * Q * 16 <= C::kStages * C::kStage, "");
+    static_assert((C::kKWays - 1) * C::kColGroups * 64 * F * Q * 16 <= kSlots * C::kStage, "");
     FSW_LDS f32x4* part = (FSW_LDS f32x4*)smem;
     if (kw > 0) {
 #pragma unroll
@@ -234,7 +347,20 @@ __global__ __launch_bounds__(kSkThreads) void fsw_narrow_kernel(GemmParams p, Sk
     if (m >= p.M) continue;
     const float g[4] = {acc[0][q].x, acc[0][q].y, acc[0][q].z, acc[0][q].w};
     const float u[4] = {up[q].x, up[q].y, up[q].z, up[q].w};
-    store_few<E>(p, a.plain, split, m, n, g, u);
+    if constexpr (UNALIGNED) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        if (n + e >= p.N) break;
+        const size_t o = (size_t)m * p.ldc + n + e;
+        ((unsigned short*)p.c0)[o] = E::from_float(silu_mul(g[e], u[e]));
+        if (p.c1) {
+          ((unsigned short*)p.c1)[o] = E::from_float(g[e]);
+          ((unsigned short*)p.c2)[o] = E::from_float(u[e]);
+        }
+      }
+    } else {
+      store_few<E>(p, a.plain, split, m, n, g, u);
+    }
   }
 }
 

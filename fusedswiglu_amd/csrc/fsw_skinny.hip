@@ -247,6 +247,35 @@ hipError_t launch_forward_skinny(int dtype, const Problem& p, hipStream_t s) {
   return dtype == kDtypeBF16 ? launch_skinny_t<BF16, false>(g, pl, 0, s) : launch_skinny_t<FP16, false>(g, pl, 0, s);
 }
 
+// ---- the forward for few tokens on rows that are not whole 16-byte chunks --------------------------------------------------
+bool stream_unaligned_ok(const Problem& p) {
+  return p.T <= kSkMaxRows && p.I >= 8 && !p.padded && p.D < (1LL << 30) && p.I < (1LL << 30) && p.ldx < (1LL << 31) && p.ldw < (1LL << 31) && p.ldo < (1LL << 31);
+}
+
+template <typename E, bool W_KC>
+static hipError_t launch_unaligned_t(const GemmParams& g, hipStream_t s) {
+  constexpr int BN = 32;
+  auto go = [&](auto mq) {
+    constexpr int MQ = decltype(mq)::value;
+    const SkArgs a{BN, 0, 1, (g.K + NarrowCfg<MQ, BN>::SK - 1) / NarrowCfg<MQ, BN>::SK};
+    fsw_narrow_kernel<E, MQ, BN, W_KC, true><<<dim3((unsigned)((g.N + BN - 1) / BN)), kSkThreads, 0, s>>>(g, a);
+    return hipGetLastError();
+  };
+  if (g.M <= 16) return go(std::integral_constant<int, 1>{});
+  if (g.M <= 32) return go(std::integral_constant<int, 2>{});
+  if (g.M <= 64) return go(std::integral_constant<int, 4>{});
+  return go(std::integral_constant<int, 8>{});
+}
+
+hipError_t launch_forward_unaligned(int dtype, const Problem& p, hipStream_t s) {
+  GemmParams g{};
+  g.a0 = p.x; g.b0 = p.wg; g.b1 = p.wu; g.c0 = p.out; g.c1 = p.g; g.c2 = p.u;
+  g.M = (int)p.T; g.N = g.n_rows_b = (int)p.I; g.K = (int)p.D;
+  g.lda = (int)p.ldx; g.ldb = (int)p.ldw; g.ldc = (int)p.ldo;
+  if (p.w_out_in) return dtype == kDtypeBF16 ? launch_unaligned_t<BF16, true>(g, s) : launch_unaligned_t<FP16, true>(g, s);
+  return dtype == kDtypeBF16 ? launch_unaligned_t<BF16, false>(g, s) : launch_unaligned_t<FP16, false>(g, s);
+}
+
 // ---- the down projection for few tokens: y [M, N] = a [M, K] W, W stored [K, N] (layout 0) or [N, K] (layout 1)
 // The same kernel with W's two column halves in the places of Wg and Wu.  N is short and K long here (D and I
 // of the SwiGLU), so column blocks alone do not fill the chip: the reduction is split as well, the fp32 partial

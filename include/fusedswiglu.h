@@ -26,7 +26,8 @@
  *   - Operands whose dimensions and leading dimensions are multiples of 8 elements and whose
  *     pointers are 16-byte aligned run on the tiled direct-to-LDS MFMA kernels, and so does any
  *     dimension whose rows are padded (FSW_ROWS_PADDED); anything else runs on a much slower
- *     edge-shape kernel with identical arithmetic.  fsw_repack_rows pads and unpads rows.
+ *     edge-shape kernel with identical arithmetic, but for the forward of up to 128 tokens (I >= 8), which
+ *     streams such weights as they are.  fsw_repack_rows pads and unpads rows.
  */
 #ifndef FUSEDSWIGLU_H_
 #define FUSEDSWIGLU_H_
@@ -66,8 +67,9 @@ enum { FSW_DTYPE_BF16 = 0, FSW_DTYPE_FP16 = 1 };
  * elements, every leading dimension is a multiple of 8 (below 2^21) and every pointer is 16-byte aligned (else
  * FSW_ERR_ALIGNMENT, with nothing enqueued).  These padding columns take part in the arithmetic: they must be zeros in
  * inputs, and in results the kernels write what zero columns give: zeros, or NaN in the rows that an infinity or a NaN of
- * the other operand reaches (pad such a result anew, fsw_repack_rows, before it becomes an input).  The exception is
- * grad_out of fsw_swiglu_backward, which stays dense, [T,I] with leading dimension I. */
+ * the other operand reaches (pad such a result anew, fsw_repack_rows, before it becomes an input).  The exceptions are
+ * in fsw_swiglu_backward: grad_out stays dense, [T,I] with leading dimension I, and what the padding of xw_gate and xw_up
+ * holds does not matter. */
 #define FSW_ROWS_PADDED 0x400
 
 enum {
