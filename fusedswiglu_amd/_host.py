@@ -38,7 +38,7 @@ def load():
             module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_fsw_host", PATH, loader=loader))
             loader.exec_module(module)
             module.setup(_abi.check, ops._general_backward, ops._general_down_backward, _launch._PAD_MIN_WORK,
-                         _launch._PAD_MIN_WORK // _launch._PAD_MIN_STEPS_SHARE, _launch._TILED_MAX_LD, _launch._STREAM_MAX_TOKENS)
+                         _launch._PAD_MIN_WORK // _launch._PAD_MIN_STEPS_SHARE, _launch._TILED_MAX_LD)
             _module = module
     return _module
 

@@ -35,7 +35,7 @@ PyObject* g_check = nullptr;
 PyObject* g_swiglu_backward = nullptr;
 PyObject* g_down_backward = nullptr;
 // the rule for padded copies (pads_rows in _launch.py)
-int64_t g_pad_min_work = 0, g_pad_min_steps = 0, g_max_ld = 0, g_stream_max_tokens = 0;
+int64_t g_pad_min_work = 0, g_pad_min_steps = 0, g_max_ld = 0;
 
 // A failed library call: the Python exception that the launchers raise.
 void check(int status) {
@@ -211,12 +211,10 @@ void run_forward(const Tensor& x, Weights w, bool save, Tensor& out, Tensor& g, 
   const c10::DeviceGuard guard(x.device());
   Rows rx = rows_of(x);
   const int64_t T = rx.rows, D = w.D, I = w.I;
-  // (_streams_unaligned of _launch.py: no copies; pre-activations lie in padded rows all the same)
-  const bool streams = T <= g_stream_max_tokens && I >= 8 && !w.whole();
-  const bool padded = ((D | I | rx.ld | w.ld) & 7 || (rx.p | w.pg | w.pu) & 15) && !(streams && !save) && pads_rows(T, D, I, false);
-  const Call c(x, w.out_in, padded && !streams);
+  const bool padded = ((D | I | rx.ld | w.ld) & 7 || (rx.p | w.pg | w.pu) & 15) && pads_rows(T, D, I, false);
+  const Call c(x, w.out_in, padded);
   Tensor keep_x, keep_w[2];
-  if (padded && !streams) {
+  if (padded) {
     Copies todo;
     pad_rows(c, rx, keep_x, todo);
     pad_weights(c, w, keep_w, todo);
@@ -531,15 +529,14 @@ PyObject* py_down_proj(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// setup(check, swiglu_backward, down_backward, least work and steps for padded copies, longest rows of the tiled kernels, most
-// tokens of a forward that streams unaligned weights)
+// setup(check, swiglu_backward, down_backward, least work and steps for padded copies, longest rows of the tiled kernels)
 PyObject* py_setup(PyObject*, PyObject* args) {
   PyObject *a, *b, *c;
-  long long work, steps, ld, tokens;
-  if (!PyArg_ParseTuple(args, "OOOLLLL", &a, &b, &c, &work, &steps, &ld, &tokens)) return nullptr;
+  long long work, steps, ld;
+  if (!PyArg_ParseTuple(args, "OOOLLL", &a, &b, &c, &work, &steps, &ld)) return nullptr;
   Py_INCREF(a), Py_INCREF(b), Py_INCREF(c);
   g_check = a, g_swiglu_backward = b, g_down_backward = c;
-  g_pad_min_work = work, g_pad_min_steps = steps, g_max_ld = ld, g_stream_max_tokens = tokens;
+  g_pad_min_work = work, g_pad_min_steps = steps, g_max_ld = ld;
   Py_RETURN_NONE;
 }
 

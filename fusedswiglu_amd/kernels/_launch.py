@@ -190,19 +190,6 @@ def _wants_padding(T: int, D: int, I: int, product: Tuple[int, int, int], *ts: t
     return bool(bits & 7) and pads_rows(T, D, I, product)
 
 
-# A forward of up to this many tokens reads each weight once, so padded copies of the weights would treble its traffic; the
-# library streams such rows as they are (1 / 8 / 32 / 64 / 128 tokens, padded copies against the stream, us: 1023 x 3071 [D, I] 158
-# (edge kernel) / 23.3 / 23.0 / 24.0 / 28.2 and 13.7 / 14.1 / 11.8 / 14.5 / 20.9; 4095 x 11003 [D, I] 102 / 104 / 106 / 111 / 122 and
-# 59 / 63 / 72 / 87 / 123, [I, D] 114 / 116 / 119 / 125 / 139 and 49 / 54 / 65 / 82 / 120; 8190 x 20001 [I, D] 405 / 406 / 407 / 413 /
-# 426 and 126 / 133 / 169 / 215 / 290).  Pre-activations that are kept lie in padded rows all the same, as the backward wants
-# them.  Where x alone is unaligned its copy is small and the aligned kernels read the rest as it is.
-_STREAM_MAX_TOKENS = 128
-
-
-def _streams_unaligned(T: int, I: int, wg: torch.Tensor, wu: torch.Tensor) -> bool:
-    return T <= _STREAM_MAX_TOKENS and I >= 8 and not (_whole_chunks(wg) and _whole_chunks(wu))
-
-
 def _weight_dims(w: torch.Tensor, weights_out_in: bool) -> Tuple[int, int]:
     """(D, I) of a gate/up weight in either layout."""
     return (w.shape[1], w.shape[0]) if weights_out_in else (w.shape[0], w.shape[1])
@@ -235,8 +222,7 @@ def fused_swiglu_fwd(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, 
     T = x2.shape[0]
     out_shape = tuple(x.shape[:-1]) + (I,)
     px, pg, pu, ldx, ldw = x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), _ld(x2), _ld(wg)
-    if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and pads_rows(T, D, I, (T, I, D)) and (
-            save_preactivations or not _streams_unaligned(T, I, wg, wu)):
+    if ((D | I | ldx | ldw) & 7 or (px | pg | pu) & 15) and pads_rows(T, D, I, (T, I, D)):
         return _padded_fwd(x2, wg, wu, dtype, out_shape, D, I, save_preactivations, weights_out_in, dense_preactivations)
     out = torch.empty(out_shape, device=dev, dtype=dtype)
     g = torch.empty_like(out) if save_preactivations else None
@@ -249,19 +235,17 @@ def fused_swiglu_fwd(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, 
 
 
 def _padded_fwd(x2, wg, wu, dtype, out_shape, D, I, save_preactivations, weights_out_in, dense_preactivations):
-    """fused_swiglu_fwd on padded copies, or for few tokens on the operands as they are.  The pre-activations stay padded, views of [T, I rounded up to 8], unless the
+    """fused_swiglu_fwd on padded copies.  The pre-activations stay padded, views of [T, I rounded up to 8], unless the
     caller wants them dense."""
     T, dev = x2.shape[0], x2.device
     with _on_device(dev):
-        streams = _streams_unaligned(T, I, wg, wu)
-        if not streams:
-            (x2,), (wg, wu) = _padded_copies(x2), _padded_copies(wg, wu)
+        (x2,), (wg, wu) = _padded_copies(x2), _padded_copies(wg, wu)
         out = _padded_result(T, I, x2)
         g, u = (torch.empty_like(out), torch.empty_like(out)) if save_preactivations else (None, None)
         _abi.check(_abi.lib().fsw_swiglu_forward(
             x2.data_ptr(), wg.data_ptr(), wu.data_ptr(), out.data_ptr(),
             g.data_ptr() if g is not None else None, u.data_ptr() if u is not None else None,
-            T, D, I, _ld(x2), _ld(wg), _pad8(I), _code(dtype, weights_out_in, not streams), _stream_ptr(dev)))
+            T, D, I, _ld(x2), _ld(wg), _pad8(I), _code(dtype, weights_out_in, True), _stream_ptr(dev)))
         out = _unpadded(out, I).view(out_shape)
         if dense_preactivations and g is not None and I & 7:
             dense = torch.empty((T, I), device=dev, dtype=dtype), torch.empty((T, I), device=dev, dtype=dtype)

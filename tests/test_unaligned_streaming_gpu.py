@@ -57,8 +57,8 @@ def test_against_float64(T, D, I, oi):
 
 @pytest.mark.parametrize("oi", [False, True], ids=["DI", "ID"])
 @pytest.mark.parametrize("T,D,I", [(8, 2047, 5001), (128, 1023, 2730), (129, 1023, 2730)])
-def test_launchers_agree_on_the_route(T, D, I, oi):
-    """Native and general host path, with and without pre-activations (those in padded rows): the same bits"""
+def test_padded_copies_stay_alike(T, D, I, oi):
+    """Calls that the launchers copy into padded rows first: the same bits with and without pre-activations, native and general"""
     torch.manual_seed(T)
     x = torch.randn(T, D, device=DEV).bfloat16()
     wg, wu = ((torch.randn(*((I, D) if oi else (D, I)), device=DEV) * D ** -0.5).bfloat16() for _ in range(2))
