@@ -118,7 +118,7 @@ struct Weights {
       if (r.rows != g.size(0) || (out_in ? g.size(0) : g.size(1)) % 2) return;
       D = out_in ? g.size(1) : g.size(0);
       I = (out_in ? g.size(0) : g.size(1)) / 2;
-      ld = out_in ? r.ld : g.stride(0);
+      ld = r.ld;
       pg = r.p;
       pu = pg + 2 * static_cast<uintptr_t>(out_in ? I * ld : I);
     } else {

@@ -92,6 +92,21 @@ def test_same_bits_in_every_form(general, kind, size):
     assert same(step(fn, batched), general(step, fn, batched))
 
 
+@pytest.mark.parametrize("oi", [False, True], ids=["DI", "ID"])
+def test_packed_weight_of_one_row_with_any_stride(general, oi):
+    """The stride of a dimension of size 1 says nothing: one row of [D, 2I] weights, or of [2I, D] ones with D = 1, as a
+    transposed view whose strides are both 1, and with a stride far longer than the row."""
+    torch.manual_seed(3)
+    I = 24
+    x, column = tensor(5, 1), tensor(2 * I, 1)
+    weights = [column, torch.as_strided(column, (2 * I, 1), (1, 7))] if oi else [column.t(), torch.as_strided(column, (1, 2 * I), (999, 1))]
+    for w in weights:
+        fn = lambda x, w: ops.swiglu_packed(x, w, weights_out_in=oi)  # noqa: E731
+        dense = w.clone(memory_format=torch.contiguous_format)
+        assert w.is_contiguous() and same([general(fn, x, w)], [fn(x, dense)])
+        assert same([fn(x, w)], [fn(x, dense)]) and same(step(fn, [x, w]), general(step, fn, [x, w]))
+
+
 def plain_call():
     torch.manual_seed(0)
     return [tensor(2, 16, 64), tensor(64, 128), tensor(64, 128)]
