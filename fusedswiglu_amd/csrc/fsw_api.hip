@@ -58,6 +58,13 @@ int launched(const char* fn, hipError_t e) {
   return FSW_OK;
 }
 
+// Whether the memory of two arrays of the same rows and columns and of 16-bit elements meets (rows of one may lie between those of the
+// other: counted as meeting).
+bool overlap(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t rows, int64_t cols) {
+  const uintptr_t a0 = (uintptr_t)a, b0 = (uintptr_t)b;
+  return a0 < b0 + 2 * (uintptr_t)((rows - 1) * ldb + cols) && b0 < a0 + 2 * (uintptr_t)((rows - 1) * lda + cols);
+}
+
 // The two gradients of the down projection as GEMMs: w = act^T grad_y ([D,I] weights: grad_y^T act), x = grad_y W_down^T
 // ([D,I] weights: grad_y W_down).
 void down_gradients(const void* act, const void* grad_y, const void* w_down, void* grad_act, void* grad_w_down, int64_t T,
@@ -363,12 +370,14 @@ int fsw_weight_grad(const void* x, const void* grad_xw_up, const void* grad_xw_g
 // Both gradients of the gating gradients, arguments checked: in one launch, or the weight gradient and then the input gradient
 // (measured at 8192 x 4096 x 12288, the input gradient runs 4 % faster behind it than behind the gating-gradient kernel - its
 // dG / dU operand is still in the memory-side cache - and the step 0.3 % faster).
+// A grad_x in the place of x always takes two launches: the weight gradient has then read all of x before it is overwritten.
 static int gradients_checked(const char* fn, const fsw::Problem& p, int elem, void* workspace, int64_t workspace_bytes, hipStream_t s) {
   const bool ws_ok = workspace && workspace_bytes > 0 && ((uintptr_t)workspace & 15) == 0;
   void* ws = ws_ok ? workspace : nullptr;
   const int64_t ws_bytes = ws_ok ? workspace_bytes : 0;
   const bool x_fast = fsw::fast_path_ok_input_grad(p), w_fast = fsw::fast_path_ok_weight_grad(p);
-  if (x_fast && w_fast) {
+  const bool over_x = overlap(p.x, p.ldx, p.dx, p.lddx, p.T, fsw::result_cols(p.D));
+  if (x_fast && w_fast && !over_x) {
     bool done = false;
     const hipError_t e = fsw::launch_grads_pair(elem, p, s, ws, ws_bytes, &done);
     if (done || e != hipSuccess) return launched(fn, e);

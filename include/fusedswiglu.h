@@ -227,6 +227,7 @@ FSW_API int fsw_weight_grad(const void* x, const void* grad_xw_up, const void* g
  * without work they share one launch, which needs `workspace` to hold the partial tiles of both
  * (fsw_workspace_bytes(7, ...)); the results have the same bits as from the two calls with scratch of the sizes they ask for.
  *   x, grad_x [T,D] (ldx, ld_dx)   w_gate, w_up (ldw)   grad_xw_gate, grad_xw_up [T,I] (ldo)   grad_w_gate, grad_w_up (ld_dw)
+ * grad_x may be x itself: it is then written behind the weight gradient, in a launch of its own.
  */
 FSW_API int fsw_swiglu_gradients(const void* x, const void* w_gate, const void* w_up, const void* grad_xw_gate,
                          const void* grad_xw_up, void* grad_x, void* grad_w_gate, void* grad_w_up, int64_t T, int64_t D,
@@ -241,7 +242,7 @@ FSW_API int fsw_swiglu_gradients(const void* x, const void* w_gate, const void* 
  *   grad_out, xw_gate, xw_up, grad_xw_gate, grad_xw_up [T,I] dense (leading dimension I)
  *   x [T,D] (ldx)   w_gate, w_up (ldw)   grad_x [T,D] (ld_dx)   grad_w_gate, grad_w_up (ld_dw)
  * grad_xw_gate and grad_xw_up are results too (the gating gradients), always written.  grad_x may be NULL, and
- * grad_w_gate / grad_w_up both NULL: that gradient is skipped (ctx.needs_input_grad).  The larger of
+ * grad_w_gate / grad_w_up both NULL: that gradient is skipped (ctx.needs_input_grad).  grad_x may be x itself.  The larger of
  * fsw_workspace_bytes(1, ...) and fsw_workspace_bytes(2, ...) serves both GEMMs one after the other, fsw_workspace_bytes(7, ...)
  * in one launch as well.
  */
@@ -279,6 +280,7 @@ FSW_API int fsw_down_proj_weight_grad(const void* act, const void* grad_y, void*
 /*
  * Both gradients in one call: fsw_down_proj_input_grad and fsw_down_proj_weight_grad, in one launch where that is faster
  * and `workspace` holds the partial tiles of both (step 8 of fsw_workspace_bytes); the same bits as from the two calls.
+ * No result may overlap an operand.
  */
 FSW_API int fsw_down_proj_backward(const void* act, const void* grad_y, const void* w_down, void* grad_act, void* grad_w_down,
                                    int64_t T, int64_t I, int64_t D, int64_t ld_act, int64_t ldy, int64_t ldw, int64_t ld_dact,

@@ -5,6 +5,7 @@ products; and against those here too, rel-L2 <= 1e-2 (bfloat16, fused_swiglu/tes
 import pytest
 import torch
 
+from fusedswiglu_amd import _abi
 from fusedswiglu_amd.kernels import _launch
 
 pytestmark = pytest.mark.gpu
@@ -83,3 +84,34 @@ def test_every_form_of_the_operands(shape, out_in):
             da, dWd = _launch.down_proj_backward(x, dU, (wg if out_in else wg).t().contiguous(), **kw)
             assert torch.equal(da, _launch.down_proj_input_grad(x, wg.t().contiguous(), **kw))
             assert torch.equal(dWd, _launch.down_proj_weight_grad(dU, x, **kw))
+
+
+@pytest.mark.parametrize("out_in", [False, True], ids=["DI", "ID"])
+@pytest.mark.parametrize("shape", [(1016, 800, 192), (706, 1120, 528), (4077, 32, 656), (2048, 512, 1536)], ids=lambda s: "x".join(map(str, s)))
+def test_input_gradient_over_x(shape, out_in):
+    """grad_x in the place of x, as where memory is short, or a row of it further on: the weight gradient reads all of x first."""
+    T, D, I = shape
+    dtype, kw = torch.bfloat16, dict(dtype=torch.bfloat16, weights_out_in=out_in)
+    torch.manual_seed(2)
+    x, dG, dU, dout, g, u = make(dtype, T, D), *(make(dtype, T, I) for _ in range(5))
+    wg, wu = (make(dtype, *((I, D) if out_in else (D, I)), std=D ** -0.5) for _ in range(2))
+    L, flag = _abi.lib(), _abi.WEIGHTS_OUT_IN if out_in else 0
+    stream = torch.cuda.current_stream().cuda_stream
+    ws = torch.empty(max(1, L.fsw_workspace_bytes(_abi.STEP_GRADIENTS | flag, T, D, I)), device=DEV, dtype=torch.uint8)
+    cols = wg.shape[1]
+    for further in (0, 1):
+        room = torch.empty(T + 1, D, device=DEV, dtype=dtype)
+        room[:T] = x
+        over = room[further:further + T]
+        dWg, dWu = torch.empty_like(wg), torch.empty_like(wu)
+        _abi.check(L.fsw_swiglu_gradients(room.data_ptr(), wg.data_ptr(), wu.data_ptr(), dG.data_ptr(), dU.data_ptr(), over.data_ptr(),
+                                          dWg.data_ptr(), dWu.data_ptr(), T, D, I, D, cols, I, D, cols, ws.data_ptr(), ws.numel(), flag, stream))
+        want = _launch.fused_gradients(x, wg, wu, dU, dG, **kw)
+        assert all(torch.equal(a, b) for a, b in zip((over, dWu, dWg), want))
+        room[:T] = x
+        dG2, dU2 = torch.empty_like(dG), torch.empty_like(dU)
+        _abi.check(L.fsw_swiglu_backward(dout.data_ptr(), g.data_ptr(), u.data_ptr(), room.data_ptr(), wg.data_ptr(), wu.data_ptr(),
+                                         dG2.data_ptr(), dU2.data_ptr(), over.data_ptr(), dWg.data_ptr(), dWu.data_ptr(), T, D, I, D, cols,
+                                         D, cols, ws.data_ptr(), ws.numel(), flag, stream))
+        want = _launch.swiglu_backward(dout, x, wg, wu, g, u, dtype, weights_out_in=out_in)
+        assert all(torch.equal(a, b) for a, b in zip((over, dWg, dWu), want))
