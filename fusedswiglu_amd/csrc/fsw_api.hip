@@ -382,8 +382,11 @@ static int gradients_checked(const char* fn, const fsw::Problem& p, int elem, vo
     const hipError_t e = fsw::launch_grads_pair(elem, p, s, ws, ws_bytes, &done);
     if (done || e != hipSuccess) return launched(fn, e);
   }
-  if (int e = launched(fn, w_fast ? fsw::launch_weight_grad_fast(elem, p, s, ws, ws_bytes) : fsw::launch_weight_grad_generic(elem, p, s))) return e;
-  return launched(fn, x_fast ? fsw::launch_input_grad_fast(elem, p, s, ws, ws_bytes) : fsw::launch_input_grad_generic(elem, p, s));
+  // (no more scratch than either would have by itself: the same parts of its sums)
+  const int64_t ws_w = std::min<int64_t>(ws_bytes, fsw::splitk_workspace_bytes(p.w_out_in ? 5 : 2, p.T, p.D, p.I));
+  const int64_t ws_x = std::min<int64_t>(ws_bytes, fsw::splitk_workspace_bytes(p.w_out_in ? 4 : 1, p.T, p.D, p.I));
+  if (int e = launched(fn, w_fast ? fsw::launch_weight_grad_fast(elem, p, s, ws, ws_w) : fsw::launch_weight_grad_generic(elem, p, s))) return e;
+  return launched(fn, x_fast ? fsw::launch_input_grad_fast(elem, p, s, ws, ws_x) : fsw::launch_input_grad_generic(elem, p, s));
 }
 
 int fsw_swiglu_gradients(const void* x, const void* w_gate, const void* w_up, const void* grad_xw_gate, const void* grad_xw_up,
@@ -534,9 +537,13 @@ int fsw_down_proj_backward(const void* act, const void* grad_y, const void* w_do
                                                ws_ok ? workspace_bytes : 0, &done);
     if (done || e != hipSuccess) return launched(fn, e);
   }
-  if (int e = fsw_down_proj_input_grad(grad_y, w_down, grad_act, T, I, D, ldy, ldw, ld_dact, workspace, workspace_bytes, dtype, stream))
+  // (no more scratch than either would have by itself: the same parts of its sums)
+  const int flag = dtype & FSW_WEIGHTS_OUT_IN;
+  if (int e = fsw_down_proj_input_grad(grad_y, w_down, grad_act, T, I, D, ldy, ldw, ld_dact, workspace,
+                                       std::min(workspace_bytes, fsw_workspace_bytes(5 | flag, T, D, I)), dtype, stream))
     return e;
-  return fsw_down_proj_weight_grad(act, grad_y, grad_w_down, T, I, D, ld_act, ldy, ld_dw, workspace, workspace_bytes, dtype, stream);
+  return fsw_down_proj_weight_grad(act, grad_y, grad_w_down, T, I, D, ld_act, ldy, ld_dw, workspace,
+                                   std::min(workspace_bytes, fsw_workspace_bytes(6 | flag, T, D, I)), dtype, stream);
 }
 
 }  // extern "C"

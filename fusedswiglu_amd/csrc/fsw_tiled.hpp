@@ -347,12 +347,22 @@ double plane_bytes(const Plan& p, const GemmParams& g) {
   return p.splits > 1 ? 4.0 * p.splits * Cfg<MODE>::kResults * g.M * g.N : 0.0;
 }
 
+// What a GEMM by itself would be offered of scratch that is there for two: workspace_of, which asks for the plan of dense rows.
+// Where rows are not whole lines apart, plan() would take more parts than it asked for if it had the scratch.
+template <int MODE>
+long long scratch_for_one(const GemmParams& g, long long ws_bytes) {
+  const Lines here = lines_of<MODE>(g), dense = dense_lines<MODE>(g.M, g.N, g.K);
+  if (here.a == dense.a && here.b == dense.b) return ws_bytes;
+  return std::min(ws_bytes, workspace_of<MODE>(g.M, g.N, g.K));
+}
+
 template <int MODE_W, int MODE_X>
 PairPlan plan_pair(const GemmParams& w, const GemmParams& x, long long ws_bytes) {
   PairPlan none{}, best{};
   const Lines lw = lines_of<MODE_W>(w), lx = lines_of<MODE_X>(x);
   // The splits are those of two launches, so that a sum is made of the same parts in either case.
-  const Plan pw = plan<MODE_W>(w.M, w.N, w.K, ws_bytes, lw), px = plan<MODE_X>(x.M, x.N, x.K, ws_bytes, lx);
+  const Plan pw = plan<MODE_W>(w.M, w.N, w.K, scratch_for_one<MODE_W>(w, ws_bytes), lw);
+  const Plan px = plan<MODE_X>(x.M, x.N, x.K, scratch_for_one<MODE_X>(x, ws_bytes), lx);
   if (pw.tail_count > 0 || px.tail_count > 0) return none;
   const double planes = plane_bytes<MODE_W>(pw, w) + plane_bytes<MODE_X>(px, x);
   if (planes > (double)ws_bytes) return none;

@@ -86,6 +86,34 @@ def test_every_form_of_the_operands(shape, out_in):
             assert torch.equal(dWd, _launch.down_proj_weight_grad(dU, x, **kw))
 
 
+def with_room(t, more):
+    wide = torch.empty(t.shape[0], t.shape[1] + more, device=DEV, dtype=t.dtype)
+    wide[:, :t.shape[1]] = t
+    return wide[:, :t.shape[1]]
+
+
+@pytest.mark.parametrize("out_in", [False, True], ids=["DI", "ID"])
+@pytest.mark.parametrize("shape", [
+    (913, 64, 1624), (2557, 16, 384), (5441, 80, 1856), (5852, 1952, 192), (1347, 2712, 256), (4141, 2880, 88), (2019, 1344, 320),
+    (3652, 88, 1600), (846, 16, 1024), (6282, 256, 1088), (1664, 384, 1200)], ids=lambda s: "x".join(map(str, s)))
+def test_scratch_for_both_leaves_the_sums_alone(shape, out_in):
+    """Rows that are not whole lines apart, of sizes at which more scratch than a gradient by itself asks for would let its
+    reduction be split into more parts."""
+    T, D, I = shape
+    dtype, kw = torch.bfloat16, dict(dtype=torch.bfloat16, weights_out_in=out_in)
+    torch.manual_seed(3)
+    x, dG, dU = with_room(make(dtype, T, D), 40), *(with_room(make(dtype, T, I), 56) for _ in range(2))
+    wg, wu = (with_room(make(dtype, *((I, D) if out_in else (D, I)), std=D ** -0.5), 24) for _ in range(2))
+    dx, dWu, dWg = _launch.fused_gradients(x, wg, wu, dU, dG, **kw)
+    assert torch.equal(dx, _launch.fused_input_grad(dG, dU, wg, wu, **kw))
+    assert all(torch.equal(a, b) for a, b in zip((dWu, dWg), _launch.fused_weight_grad(x, dU, dG, **kw)))
+    gy, act = with_room(make(dtype, T, D), 24), with_room(make(dtype, T, I), 24)
+    wd = with_room(make(dtype, *((D, I) if out_in else (I, D)), std=I ** -0.5), 24)
+    da, dWd = _launch.down_proj_backward(gy, act, wd, **kw)
+    assert torch.equal(da, _launch.down_proj_input_grad(gy, wd, **kw))
+    assert torch.equal(dWd, _launch.down_proj_weight_grad(act, gy, **kw))
+
+
 @pytest.mark.parametrize("out_in", [False, True], ids=["DI", "ID"])
 @pytest.mark.parametrize("shape", [(1016, 800, 192), (706, 1120, 528), (4077, 32, 656), (2048, 512, 1536)], ids=lambda s: "x".join(map(str, s)))
 def test_input_gradient_over_x(shape, out_in):
