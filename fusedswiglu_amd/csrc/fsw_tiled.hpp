@@ -430,4 +430,9 @@ hipError_t launch_pair(GemmParams w, GemmParams x, hipStream_t s, void* ws, long
   return hipGetLastError();
 }
 
+// The pairs in float16: each is instantiated in another file than the same pair in bfloat16, so that no file takes all of the
+// compiler's time.
+hipError_t launch_grads_pair_fp16(const Problem& p, hipStream_t s, void* ws, long long ws_bytes, bool* done);
+hipError_t launch_gemm_pair_fp16(const GemmParams& w, const GemmParams& x, int layout, hipStream_t s, void* ws, long long ws_bytes, bool* done);
+
 }  // namespace fsw

@@ -12,8 +12,6 @@ hipError_t launch_gemm_pair_fp16(const GemmParams& w, const GemmParams& x, int l
   return layout == 1 ? launch_pair<FP16, kTN, kNT>(w, x, s, ws, ws_bytes, done) : launch_pair<FP16, kTN, kNN>(w, x, s, ws, ws_bytes, done);
 }
 
-hipError_t launch_grads_pair_fp16(const Problem& p, hipStream_t s, void* ws, long long ws_bytes, bool* done);
-
 hipError_t launch_grads_pair(int dtype, const Problem& p, hipStream_t s, void* ws, long long ws_bytes, bool* done) {
   if (dtype != kDtypeBF16) return launch_grads_pair_fp16(p, s, ws, ws_bytes, done);
   const GemmParams w = weight_grad_params(p), x = input_grad_params(p);

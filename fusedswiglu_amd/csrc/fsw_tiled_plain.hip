@@ -28,8 +28,6 @@ long long gemm_pair_workspace_bytes(const GemmProblem& w, const GemmProblem& x) 
   return std::max(one, x.layout == 1 ? pair_workspace<kTN, kNT>(gw, gx) : pair_workspace<kTN, kNN>(gw, gx));
 }
 
-hipError_t launch_gemm_pair_fp16(const GemmParams& w, const GemmParams& x, int layout, hipStream_t s, void* ws, long long ws_bytes, bool* done);
-
 hipError_t launch_gemm_pair(int dtype, const GemmProblem& w, const GemmProblem& x, hipStream_t s, void* ws, long long ws_bytes, bool* done) {
   const GemmParams gw = gemm_params(w), gx = gemm_params(x);
   if (dtype != kDtypeBF16) return launch_gemm_pair_fp16(gw, gx, x.layout, s, ws, ws_bytes, done);
