@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 import os
 import subprocess
+import sys
 import threading
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
@@ -85,7 +86,7 @@ def build_library(verbose: bool = False, jobs: int = 4) -> str:
     """Compile the HIP sources for gfx950 with hipcc (works without a GPU) and return the
     path of the shared library.  Always recompiles."""
     global _lib, _bench_lib
-    cmd = ["make", "-C", _CSRC, f"-j{jobs}", "-B"]
+    cmd = ["make", "-C", _CSRC, f"-j{jobs}", "-B", f"PYTHON={sys.executable}"]
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if verbose or res.returncode != 0:
         print(res.stdout)

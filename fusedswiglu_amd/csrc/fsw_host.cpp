@@ -11,6 +11,7 @@
 #include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
+#include <torch/version.h>
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
@@ -550,4 +551,8 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_fsw_host", nullptr, -1, metho
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__fsw_host() { return PyModule_Create(&module_def); }
+PyMODINIT_FUNC PyInit__fsw_host() {
+  PyObject* m = PyModule_Create(&module_def);
+  if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}
