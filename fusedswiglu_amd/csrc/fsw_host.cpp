@@ -9,6 +9,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/forward_grad.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 #include <torch/version.h>
@@ -381,7 +382,9 @@ variable_list swiglu_node_backward(AutogradContext* ctx, Tensor grad) {
   return {need_x ? dx : Tensor(), need_g ? dwg : Tensor(), need_u ? dwu : Tensor()};
 }
 
-struct SwigluNode : torch::autograd::Function<SwigluNode> {
+enum { kBF16Function, kHalfFunction, kOperatorCall };  // FusedSwiGLU, FastAccumFusedSwiGLU, ops.swiglu: what grad_fn is called
+template <int KIND>
+struct SwigluNode : torch::autograd::Function<SwigluNode<KIND>> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& wg, const Tensor& wu, int64_t flags) {
     return swiglu_node_forward(ctx, x, wg, wu, flags);
   }
@@ -459,6 +462,69 @@ struct DownNode : torch::autograd::Function<DownNode> {
   }
 };
 
+// ---- the nodes as grad_fn --------------------------------------------------------------------------------------------------
+// What the Python nodes of the general path show of themselves: their name, saved_tensors and needs_input_grad.
+template <typename T>
+torch::autograd::CppNode<T>* node_of(PyObject* self) {
+  return static_cast<torch::autograd::CppNode<T>*>(reinterpret_cast<torch::autograd::THPCppFunction*>(self)->cdata.get());
+}
+// weights: 2; 1 packed; 0 for the down projection, which saves its two arguments
+template <typename T, int WEIGHTS>
+PyObject* node_saved_tensors(PyObject* self, void*) {
+  HANDLE_TH_ERRORS
+  variable_list v = node_of<T>(self)->ctx_.get_saved_variables();
+  if (WEIGHTS == 1) v.erase(v.begin() + 2);
+  if (WEIGHTS > 0) {  // pre-activations: none where they are recomputed, else in x's shape, without the padding of their rows
+    const bool out_in = node_of<T>(self)->ctx_.saved_data["flags"].toInt() & kOutIn;
+    const Tensor x = v[0], w = v[1];
+    const int64_t I = (out_in ? w.size(0) : w.size(1)) / (WEIGHTS == 1 ? 2 : 1);
+    for (size_t i = v.size() - 2; i < v.size(); i++)
+      v[i] = v[i].defined() ? v[i].reshape(with_last(x, v[i].size(-1))).narrow(-1, 0, I) : at::empty({0}, x.options().requires_grad(false));
+  }
+  py::tuple t(v.size());
+  for (size_t i = 0; i < v.size(); i++) t[i] = py::reinterpret_steal<py::object>(THPVariable_Wrap(v[i]));
+  return t.release().ptr();
+  END_HANDLE_TH_ERRORS
+}
+// (of the tensors; the flags behind them never do)
+template <typename T, int TENSORS>
+PyObject* node_needs_input_grad(PyObject* self, void*) {
+  HANDLE_TH_ERRORS
+  py::tuple t(TENSORS);
+  for (int i = 0; i < TENSORS; i++) t[i] = py::bool_(node_of<T>(self)->ctx_.needs_input_grad(i));
+  return t.release().ptr();
+  END_HANDLE_TH_ERRORS
+}
+PyObject* node_set_sequence_nr(PyObject* self, PyObject* n) {
+  HANDLE_TH_ERRORS
+  const unsigned long long value = PyLong_AsUnsignedLongLong(n);
+  if (PyErr_Occurred()) return nullptr;
+  reinterpret_cast<torch::autograd::THPCppFunction*>(self)->cdata->set_sequence_nr(value);
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+PyObject* node_name(PyObject* self, PyObject*) { return PyObject_GetAttrString(reinterpret_cast<PyObject*>(Py_TYPE(self)), "__name__"); }
+
+template <typename T, int WEIGHTS, int TENSORS>
+bool show_node(const char* name) {
+  using namespace torch::autograd;  // (THPCppFunction_*)
+  static PyGetSetDef properties[] = {{"saved_tensors", node_saved_tensors<T, WEIGHTS>, nullptr, nullptr, nullptr},
+                                     {"needs_input_grad", node_needs_input_grad<T, TENSORS>, nullptr, nullptr, nullptr},
+                                     THP_FUNCTION_DEFAULT_PROPERTIES,
+                                     {nullptr, nullptr, nullptr, nullptr, nullptr}};
+  static PyMethodDef node_methods[] = {{"name", node_name, METH_NOARGS, nullptr},
+                                       {"register_hook", THPCppFunction_register_hook, METH_O, nullptr},
+                                       {"register_prehook", THPCppFunction_register_prehook, METH_O, nullptr},
+                                       {"_register_hook_dict", THPCppFunction_register_hook_dict, METH_O, nullptr},
+                                       {"_sequence_nr", THPCppFunction_sequence_nr, METH_NOARGS, nullptr},
+                                       {"_set_sequence_nr", node_set_sequence_nr, METH_O, nullptr},
+                                       {nullptr, nullptr, 0, nullptr}};
+  static PyTypeObject type;
+  if (!torch::autograd::_initFunctionPyTypeObject(type, name, properties, node_methods)) return false;
+  torch::autograd::registerCppFunction(typeid(torch::autograd::CppNode<T>), &type);
+  return true;
+}
+
 // ---- Python ------------------------------------------------------------------------------------------------------------------
 bool exact(PyObject* o) { return THPVariable_CheckExact(o) || reinterpret_cast<PyObject*>(Py_TYPE(o)) == ParameterClass; }
 
@@ -494,7 +560,10 @@ PyObject* py_swiglu(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (inference({&x, &wg, &wu})) Py_RETURN_NONE;
     const int64_t flags = (packed ? kPacked : 0) | (out_in ? kOutIn : 0) | (recompute ? kRecompute : 0) | (op ? kOperator : 0);
     const py::gil_scoped_release unlocked;
-    out = packed ? PackedNode::apply(x, wg, flags) : SwigluNode::apply(x, wg, wu, flags);
+    out = packed ? PackedNode::apply(x, wg, flags)
+          : op   ? SwigluNode<kOperatorCall>::apply(x, wg, wu, flags)
+          : x.scalar_type() == at::kHalf ? SwigluNode<kHalfFunction>::apply(x, wg, wu, flags)
+                                         : SwigluNode<kBF16Function>::apply(x, wg, wu, flags);
   } else {
     const py::gil_scoped_release unlocked;
     const at::AutoDispatchBelowADInplaceOrView below;
@@ -552,6 +621,16 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_fsw_host", nullptr, -1, metho
 }  // namespace
 
 PyMODINIT_FUNC PyInit__fsw_host() {
+  static const bool shown = [] {  // (once per process)
+#define FSW_NODE(name) "torch.autograd.function." name "Backward"
+    return show_node<SwigluNode<kBF16Function>, 2, 3>(FSW_NODE("FusedSwiGLU")) &&
+           show_node<SwigluNode<kHalfFunction>, 2, 3>(FSW_NODE("FastAccumFusedSwiGLU")) &&
+           show_node<SwigluNode<kOperatorCall>, 2, 3>(FSW_NODE("GeneratedBackwardFor_fusedswiglu_amd_swiglu_forward_default")) &&
+           show_node<PackedNode, 1, 2>(FSW_NODE("_PackedSwiGLU")) &&
+           show_node<DownNode, 0, 2>(FSW_NODE("GeneratedBackwardFor_fusedswiglu_amd_down_proj_forward_default"));
+#undef FSW_NODE
+  }();
+  if (!shown) return nullptr;
   PyObject* m = PyModule_Create(&module_def);
   if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) Py_CLEAR(m);
   return m;

@@ -220,6 +220,44 @@ def test_graph_rules():
     assert out.requires_grad
 
 
+@pytest.mark.parametrize("size", [(3, 16, 24, 40), (4, 65, 520, 538)], ids=["dense", "padded"])
+@pytest.mark.parametrize("kind", ["function", "half", "swiglu", "swiglu-ID-recompute", "packed", "packed-ID", "packed-recompute", "down"])
+def test_what_grad_fn_shows(general, kind, size):
+    """The node behind an output has the general path's name, saved tensors and account of the gradients that are wanted."""
+    torch.manual_seed(4)
+    B, S, D, I = size
+    oi, rc, dtype = "-ID" in kind, "recompute" in kind, torch.float16 if kind == "half" else BF
+    if kind == "down":
+        tensors, fn = [tensor(B, S, I), tensor(I, D)], ops.down_proj
+    elif kind.startswith("packed"):
+        tensors = [tensor(B, S, D), tensor(*((2 * I, D) if oi else (D, 2 * I)))]
+        fn = lambda x, w: ops.swiglu_packed(x, w, recompute=rc, weights_out_in=oi)  # noqa: E731
+    else:
+        tensors = [tensor(B, S, D, dtype=dtype), *(tensor(*((I, D) if oi else (D, I)), dtype=dtype) for _ in range(2))]
+        fn = {"function": FusedSwiGLU.apply, "half": FastAccumFusedSwiGLU.apply}.get(
+            kind, lambda x, g, u: ops.swiglu(x, g, u, recompute=rc, weights_out_in=oi))
+    for frozen in range(len(tensors)):
+        leaves = [t.detach().requires_grad_(i != frozen) for i, t in enumerate(tensors)]
+        outs = fn(*leaves), general(fn, *leaves)
+        a, b = (out.grad_fn for out in outs)
+        assert type(a).__name__ == type(b).__name__ and a.name() == b.name()
+        assert a.needs_input_grad[:len(tensors)] == b.needs_input_grad[:len(tensors)] == tuple(t.requires_grad for t in leaves)
+        assert len(a.saved_tensors) == len(b.saved_tensors)
+        for s, t in zip(a.saved_tensors, b.saved_tensors):
+            assert s.shape == t.shape and s.dtype == t.dtype and s.device == t.device and torch.equal(s, t)
+        assert [t.requires_grad for t in a.saved_tensors[:len(leaves)]] == [t.requires_grad for t in leaves]
+        assert [n[0] is None for n in a.next_functions] == [n[0] is None for n in b.next_functions][:len(a.next_functions)]
+    out = fn(*leaves)
+    torch.autograd.grad(out, leaves[0], torch.ones_like(out))
+    with pytest.raises(RuntimeError):
+        out.grad_fn.saved_tensors                                                          # freed with the graph
+    seen = []
+    out = fn(*leaves)
+    out.grad_fn.register_hook(lambda gi, go: seen.append(len(go)))
+    torch.autograd.grad(out, leaves[0], torch.ones_like(out))
+    assert seen == [1]
+
+
 def test_checkpoint_streams_and_threads(general):
     tensors = plain_call()
     want = general(step, FusedSwiGLU.apply, tensors)
