@@ -50,7 +50,12 @@ inline SkPlan plan_wide(long long M, long long Nh, long long K, int cus, bool w_
 // 10 %): all weights once at 6 TB/s; per CU its weights at 49 (128-column blocks: 26) bytes/ns and its LDS fill, x
 // included, at 50 (62) bytes/ns; start and end of a launch and of every further round of workgroups; the second launch of a
 // split and its fp32 partials.  Rows of [D, I] weights shorter than a 128-byte line are fetched as whole lines by every
-// block.
+// block.  128-column blocks in parts, up to 16 rows, [I, D], cost more than that fit knows: 0.2 us for the start of each part, and
+// where rows of the weights start between lines 10 % more for the weights, whose row segments then share lines.  With both, and
+// with `rows` of choose_within for every narrow block of such a product, 3 x 382 down projections of 1 to 16 rows, 1024 to 9400
+// columns and reductions of 1024 to 28672 take 1.010 of what the best of the forms takes, 1.039 before: 1 x 8704 -> 3568 16.0 -> 12.6
+// us, 10 x 8584 -> 8048 41.2 -> 29.9, 6 x 4088 -> 7984 22.3 -> 15.5; 8 of them take 1.03 to 1.10 of their time before, all of 16 rows
+// or below 11 us (16 x 14336 -> 3456 22.3 -> 24.1).
 inline double estimate_us(const SkPlan& p, long long M, long long Nh, long long K, int cus, bool w_kc) {
   const bool wide = p.slot == 128;
   const long long wgs = (Nh + p.bn - 1) / p.bn * p.splits, rounds = (wgs + cus - 1) / cus;
@@ -63,6 +68,7 @@ inline double estimate_us(const SkPlan& p, long long M, long long Nh, long long 
   const double start = w_kc ? (wide ? 0.6 : 4.2) : (wide ? 1.2 : 4.3), round = wide ? 2.0 : (w_kc ? 1.3 : 0.0);
   double us = std::max({4.0 * K * Nh / 6.0e6, useful / cu_rate, fill / fill_rate}) + start + round * (rounds - 1);
   if (p.splits > 1) us += (w_kc ? 1.7 : 2.3) + p.splits * M * Nh * 8.0 / 1.3e6;
+  if (wide && p.splits > 1 && w_kc && M <= 16) us += 0.2 * p.splits + (K % 64 ? 0.1 * 4.0 * K * Nh / 6.0e6 : 0.0);
   return us;
 }
 
@@ -81,9 +87,8 @@ inline double estimate_us(const SkPlan& p, long long M, long long Nh, long long 
 // estimate errs both ways there, narrow blocks took 0.84 to 1.24 of the time (geometric mean 1.0), and no simple rule parts them.
 // 8-column blocks whose gate and up rows share the 16 rows of an MFMA operand ([I, D], up to 16 rows; NarrowCfg): twice the
 // workgroups of 16-column blocks and no half-empty slots, and a result of up to 4096 columns needs neither parts nor the launch
-// that adds them.  Against what was chosen before (1 to 16 rows, nn.Linear's layout, 70 random down projections): 0.951 of the time
-// on average, worst 1.05, best 0.74; 1 x 11008 -> 4096 20.7 -> 18.9 us, 4 x 8704 -> 4096 18.7 -> 14.8, 1 x 9408 -> 2688 15.5 -> 12.5,
-// the input gradient of 2 x 3328 x 1152 in the other layout 5.6 -> 4.8.
+// that adds them: 1 / 8 / 16 x 11008 -> 4096 21.1 / 21.5 / 22.3 us in 16 parts of 128 columns, 18.9 / 19.7 / 21.6 so; 1 x 8704 -> 4096
+// 17.4 and 13.9.  A second round of them is longer than wider blocks (1 x 8704 -> 4112 20.8 us, 32 columns in parts 17.0).
 inline SkPlan choose_within(long long M, long long Nh, long long K, int cus, bool w_kc, bool whole_lines, bool plain,
                             long long max_splits) {
   SkPlan best = plan_wide(M, Nh, K, cus, w_kc, plain ? max_splits : 0);
@@ -91,6 +96,9 @@ inline SkPlan choose_within(long long M, long long Nh, long long K, int cus, boo
   if (w_kc && !plain && !whole_lines && M <= 32 && Nh > 32LL * cus) return best;
   double best_us = estimate_us(best, M, Nh, K, cus, w_kc);
   best_us /= plain ? (M <= 16 ? 1.05 : 1.15) : (w_kc ? 1.10 : 1.0);
+  // x rows that are there cost more than those that zero-fill (12 x 5440 -> 1984 10.3 us, paired 10.9; 6 x 9472 -> 2560 13.8 and 14.6)
+  const bool few = w_kc && plain && M <= 16;
+  const double rows = M <= 4 ? 1.0 : M <= 8 ? 1.04 : 1.08;
   for (int slot = 16; slot <= (w_kc ? 64 : 32); slot *= 2) {
     int mq = slot == 64 ? 2 : 1;
     while (16 * mq < M) mq *= 2;
@@ -111,13 +119,7 @@ inline SkPlan choose_within(long long M, long long Nh, long long K, int cus, boo
         if (blocks * splits < (splits > 1 ? 48 : 40)) continue;
         const int sps = (stages + splits - 1) / splits;
         const SkPlan pl{slot, mq, bn, (stages + sps - 1) / sps, sps, paired};
-        // (x rows that are there cost more than those that zero-fill: 12 x 5440 -> 1984 10.3 us, paired 10.9; 6 x 9472 -> 2560 13.8
-        // and 14.6)
-        double us = estimate_us(pl, M, Nh, K, cus, w_kc) * (!paired || M <= 4 ? 1.0 : M <= 8 ? 1.04 : 1.08);
-        // One full round of 8-column blocks against split blocks of 128: 3 us more than the estimate knows, for the start of many
-        // short parts and, between lines, for their rows (1 / 8 / 16 x 11008 -> 4096 20.7 -> 18.8, 21.4 -> 19.9, 23.0 -> 21.8 us,
-        // 4 x 12976 -> 4032 30.4 -> 22.6)
-        if (paired && splits == 1 && blocks <= cus && 8 * blocks >= 7LL * cus && best.slot == 128 && best.splits > 1) us -= 3.0;
+        const double us = estimate_us(pl, M, Nh, K, cus, w_kc) * (paired || few ? rows : 1.0);
         if (us < best_us) { best_us = us; best = pl; }
       }
     }

@@ -124,3 +124,14 @@ def test_narrow_blocks_where_weight_rows_are_not_whole_lines(M, N, K, slot):
 def test_no_third_round_of_16_columns(M, N, K, narrow):
     """16-column blocks of a down projection: half of N in two rounds of the chip at most."""
     assert (ask(_abi.bench_lib().fsw_plan_few_tokens, 1, 1, M, N, K, CUS, 16, results=4)[0] == 16) == narrow
+
+
+@pytest.mark.parametrize("M", [1, 8])
+@pytest.mark.parametrize("N", [2688, 3200, 3456, 3568, 3584, 3600, 4080, 4096])
+def test_one_round_of_8_columns_is_whole(M, N):
+    """Down projections of a few rows whose 8-column blocks fit one round of the chip take them, whatever share of it they fill; a
+    second round does not pay (x 8704 -> 3568 12.6 / 13.2 us on them, 16.0 / 16.4 in parts of 128 columns; -> 4112 20.8 / 22.3 and 17.3 /
+    18.1)."""
+    few = lambda n: ask(_abi.bench_lib().fsw_plan_few_tokens, 1, 1, M, n, 8704, CUS, 16, results=4)  # noqa: E731
+    assert few(N) == (16, 1, 8, 1)
+    assert few(4112)[2] > 8
