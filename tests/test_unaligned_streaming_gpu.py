@@ -11,6 +11,12 @@ from fusedswiglu_amd.kernels import _launch
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
+TOKENS = [1, 7, 16, 17, 32, 33, 64, 65, 128]
+SIZES = [(1, 8), (15, 23), (64, 33), (65, 32), (127, 9), (128, 31), (129, 40), (513, 65), (777, 1023), (1001, 2731)]  # D, I
+
+
+def dtype_of(T, D):
+    return torch.float16 if (T + D) % 3 == 0 else torch.bfloat16
 
 
 def rows_in_nan(rows, cols, pitch, offset, dtype, std):
@@ -34,11 +40,11 @@ def close(a, r, dtype):
 
 
 @pytest.mark.parametrize("oi", [False, True], ids=["DI", "ID"])
-@pytest.mark.parametrize("D,I", [(1, 8), (15, 23), (64, 33), (65, 32), (127, 9), (128, 31), (129, 40), (513, 65), (777, 1023), (1001, 2731)])
-@pytest.mark.parametrize("T", [1, 7, 16, 17, 32, 33, 64, 65, 128])
+@pytest.mark.parametrize("D,I", SIZES)
+@pytest.mark.parametrize("T", TOKENS)
 def test_against_float64(T, D, I, oi):
     torch.manual_seed(T * D + I)
-    dtype = torch.float16 if (T + D) % 3 == 0 else torch.bfloat16
+    dtype = dtype_of(T, D)
     save = (T + I) % 2 == 0
     rows, cols = (I, D) if oi else (D, I)
     x = rows_in_nan(T, D, D + T % 3, 1 + T % 2, dtype, 1.0)

@@ -3,9 +3,12 @@ compiled, in both element types.  A change of a rule or of its constants that mo
 import ctypes
 
 import pytest
+import torch
 
 import test_narrow_blocks_gpu
+import test_paired_blocks_gpu
 import test_tile_rows_gpu
+import test_unaligned_streaming_gpu
 import test_variants_gpu
 from fusedswiglu_amd import _abi
 
@@ -40,13 +43,21 @@ def tiled_variants(T, D, I, oi):
         yield mode, blocks, how
 
 
+def few_variant(kc, down, M, N, K):
+    """(reduction contiguous in the weights, column slot, 16-row blocks, down projection, split); 8 columns of either half in one
+    slot of 16 count as a slot of 8, with 0 blocks where x has 8 rows at most"""
+    slot, blocks, columns, splits = ask(_abi.bench_lib().fsw_plan_few_tokens, int(kc), int(down), M, N, K, CUS, 16, results=4)
+    if kc and columns == 8 and blocks == 1:
+        slot, blocks = 8, int(M > 8)
+    return bool(kc), slot, blocks, bool(down), splits > 1
+
+
 def few_variants(T, D, I, oi):
-    """(reduction contiguous in the weights, column slot, 16-row blocks, down projection, split)"""
+    """of every launcher's launches, as the Python launchers make them"""
     for down, kc, N, K in ((0, oi, (I + 7) & ~7, D), (1, oi, D, I), (1, not oi, I, D)):
         if down and (N & 7 or N // 2 % (8 if kc else 64)):
             continue                                                                     # runs on the tiled kernels
-        slot, blocks, _, splits = ask(_abi.bench_lib().fsw_plan_few_tokens, int(kc), down, T, N, K, CUS, 16, results=4)
-        yield bool(kc), slot, blocks, bool(down), splits > 1
+        yield few_variant(kc, down, T, N, K)
 
 
 def reached():
@@ -61,6 +72,8 @@ def reached():
         tiled |= {(*v, dtype) for v in tiled_variants(*case) for dtype in (0, 1)}
     for case in test_variants_gpu.FEW:
         few |= {(*v, dtype) for v in few_variants(*case) for dtype in (0, 1)}
+    for case in test_paired_blocks_gpu.CASES:
+        few |= {(*few_variant(1, 1, *case), dtype) for dtype in (0, 1)}
     return tiled, few
 
 
@@ -81,12 +94,21 @@ def test_tiled_kernels(variants):
 
 def test_weight_streaming_kernels(variants):
     """Slots of 16 columns hold up to 64 rows, slots of 64 columns need contiguous reductions and more than 16 rows; blocks of
-    128 columns have room for 32, 64 or 128 rows.  The forward is never split."""
+    128 columns have room for 32, 64 or 128 rows.  Slots of 8 need contiguous reductions and up to 16 rows.  The forward is never
+    split, nor are slots of 8."""
     blocks = {16: (1, 2, 4), 32: (1, 2, 4, 8), 64: (2, 4, 8), 128: (2, 4, 8)}
     want = {(kc, slot, b, down, split, dtype) for kc in (False, True) for slot in blocks if kc or slot != 64 for b in blocks[slot]
             for down in (False, True) for split in (False, True) if down or not split for dtype in (0, 1)}
+    want |= {(True, 8, b, down, False, dtype) for b in (0, 1) for down in (False, True) for dtype in (0, 1)}
     never = {(False, 16, 1, True, False, dtype) for dtype in (0, 1)}                      # a split comes out cheaper there
     assert variants[1] == want - never
+
+
+def test_unaligned_stream():
+    """32 columns in either layout, 16, 32, 64 or 128 rows of x."""
+    few = test_unaligned_streaming_gpu
+    got = {(oi, next(b for b in (1, 2, 4, 8) if T <= 16 * b), few.dtype_of(T, D)) for T in few.TOKENS for D, _ in few.SIZES for oi in (0, 1)}
+    assert got == {(oi, b, dtype) for oi in (0, 1) for b in (1, 2, 4, 8) for dtype in (torch.bfloat16, torch.float16)}
 
 
 @pytest.mark.parametrize("mode,M,N,K,whole_lines,ragged", [

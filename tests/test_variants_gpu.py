@@ -25,7 +25,7 @@ FEW = [
     (64, 1032, 5632, 1), (64, 1008, 6144, 1), (17, 840, 8272, 0), (32, 7296, 976, 0), (32, 6912, 1040, 0), (63, 8304, 904, 1),
     (2, 968, 8320, 1), (65, 2768, 3112, 1), (31, 1736, 8208, 1), (17, 976, 16432, 0), (63, 976, 16480, 0),
     (127, 976, 16512, 0), (17, 2768, 14504, 1), (32, 4160, 8704, 1), (32, 4168, 8704, 1), (1, 5448, 11704, 1),
-    (1, 648, 8208, 0),
+    (1, 648, 8208, 0), (8, 1096, 1544, 1), (9, 2056, 1288, 1),
 ]
 
 
