@@ -209,15 +209,34 @@ def test_graph_rules():
     torch.autograd.grad(out, [x], torch.ones_like(out))
     with pytest.raises(RuntimeError, match="second time"):
         torch.autograd.grad(out, [x], torch.ones_like(out))
-    # the module's operator refuses to be differentiated twice
-    out = ops.swiglu(x, g, u)
-    (dx,) = torch.autograd.grad(out, [x], torch.ones_like(out), create_graph=True)
-    if dx.requires_grad:
-        with pytest.raises(RuntimeError):
-            dx.sum().backward()
     out = FusedSwiGLU.apply(x, g, u)
     out.add_(1)                                                                            # an output may be changed in place
     assert out.requires_grad
+
+
+@pytest.mark.parametrize("oi", [False, True], ids=["DI", "ID"])
+@pytest.mark.parametrize("kind", ["swiglu", "swiglu-recompute", "packed", "packed-recompute", "down"])
+def test_a_recorded_backward_keeps_its_graph(general, kind, oi):
+    """Gradients of the module's entry points under create_graph=True go through their operators, which refuse to be differentiated:
+    a gradient without a graph would lose the second order without a word."""
+    torch.manual_seed(5)
+    D, I, rc = 24, 40, "recompute" in kind
+    if kind == "down":
+        tensors, fn = [tensor(3, 16, I), tensor(*((D, I) if oi else (I, D)))], lambda a, w: ops.down_proj(a, w, weights_out_in=oi)
+    elif kind.startswith("packed"):
+        tensors = [tensor(3, 16, D), tensor(*((2 * I, D) if oi else (D, 2 * I)))]
+        fn = lambda x, w: ops.swiglu_packed(x, w, recompute=rc, weights_out_in=oi)  # noqa: E731
+    else:
+        tensors = [tensor(3, 16, D), *(tensor(*((I, D) if oi else (D, I))) for _ in range(2))]
+        fn = lambda x, g, u: ops.swiglu(x, g, u, recompute=rc, weights_out_in=oi)  # noqa: E731
+    for run in (lambda *leaves: fn(*leaves), lambda *leaves: general(fn, *leaves)):
+        leaves = [t.clone().requires_grad_() for t in tensors]
+        out = run(*leaves)
+        grads = torch.autograd.grad(out, leaves, torch.ones_like(out), create_graph=True)
+        assert all(g.requires_grad for g in grads)
+        for g in grads:
+            with pytest.raises(RuntimeError):
+                torch.autograd.grad(g, leaves, torch.ones_like(g), retain_graph=True)
 
 
 @pytest.mark.parametrize("size", [(3, 16, 24, 40), (4, 65, 520, 538)], ids=["dense", "padded"])
