@@ -108,8 +108,9 @@ FSW_DEV u32x4 load_any(const char* p, int left) {
 // columns that are not stored.  The last stage is checked chunk by chunk, and those that end inside go element by element.
 // Bound: HBM for few rows of x (8190 x 20001 [I, D], 1 / 16 tokens: 5.2 / 4.7 TB/s), with more rows the copies of x in every
 // workgroup, and for [D, I] weights their 64-byte row segments, which straddle lines (3.7 / 3.4 TB/s).  Padded copies of the
-// weights and the aligned kernels move the weights three times: 405 / 407 and 368 / 369 us there, 126 / 141 and 178 / 193 here;
-// one token, which the edge-shape kernel took, 2047 x 5461: 309 and 353 us, 15 and 17 here.
+// weights and the aligned kernels move the weights three times: 405 / 407 and 368 / 369 us there, 126 / 141 and 178 / 193 here
+// (from the C entry: the Python launchers still copy what exceeds 2^24 multiply-adds); one token, which the edge-shape kernel took,
+// 2047 x 5461: 309 and 353 us, 15 and 17 here.
 template <typename E, int MQ, int BN, bool W_KC, bool UNALIGNED = false>
 __global__ __launch_bounds__(kSkThreads) void fsw_narrow_kernel(GemmParams p, SkArgs a) {
   using C = NarrowCfg<MQ, BN>;

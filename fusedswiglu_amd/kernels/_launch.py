@@ -112,6 +112,9 @@ def _code(dtype: torch.dtype, weights_out_in: bool, padded: bool = False) -> int
 # and each result padded until it is copied back (that step 116 -> 125 MB).  Padding pays from this
 # many multiply-adds per matrix product on (forward / backward, edge kernel against padded: 33 / 56 against 46 / 75 us at
 # 2^21.5, 39 / 100 against 46 / 77 at 2^24.5, 69 / 224 against 46 / 77 at 2^25.2) ...
+# Both limits weigh the copies against the edge-shape kernel.  A forward of up to 128 tokens (I >= 8) below them runs on the library's
+# stream of unaligned rows instead, which also beats the copies above them (1023 x 3071 [D, I], 5 tokens 14 us on the stream, 6 tokens 23
+# on copies): for such forwards the limits are too low, and wait for a rule of their own.
 _PAD_MIN_WORK = 1 << 24
 # ... if the edge-shape kernel is not done sooner than the copies and their launches.  Its time is a chain of 32-element
 # steps of the reduction, 2.4 us each while its 64 x 64 tiles are no more than 320: padding pays from 4300 steps x tiles per

@@ -44,9 +44,10 @@ extern "C" {
 #endif
 
 /* major*10000 + minor*100 + patch.
- * 0.4.0: fsw_swiglu_backward (the three backward steps in one call), fsw_swiglu_gradients, fsw_down_proj_backward
- *        and steps 7 and 8 of fsw_workspace_bytes; FSW_ROWS_PADDED, fsw_repack_rows / _group and
- *        fsw_elementwise_backward_rows / _group.
+ * 0.4.0: fsw_swiglu_backward (the three backward steps in one call); FSW_ROWS_PADDED, fsw_repack_rows and
+ *        fsw_elementwise_backward_rows.  Added later under the same number, so that a program that may meet an earlier
+ *        build looks the symbols up: fsw_swiglu_gradients, fsw_down_proj_backward, fsw_repack_group,
+ *        fsw_elementwise_backward_group; steps 7 and 8 of fsw_workspace_bytes (0 in that build).
  * 0.3.0: FSW_WEIGHTS_OUT_IN, the fsw_down_proj_* entry points, fsw_input_grad_noalloc and status 7,
  *        fsw_uses_tiled_kernel answers 2 for the weight-streaming kernels and knows steps 4 / 5 / 6,
  *        fsw_workspace_bytes may ask for up to 64 MiB for large gradient GEMMs (tail split).
@@ -93,7 +94,8 @@ FSW_API const char* fsw_last_error(void);
 /* Which kernel the arguments of the named step would run on: 1 the tiled MFMA kernels, 2 the
  * weight-streaming kernel (at most 128 tokens: the forward, and the down projection and its input gradient
  * when half their result columns are a multiple of 8 elements for a k-contiguous W_down - [D,I] in the
- * forward, [I,D] in the input gradient - and of 64 otherwise), 0 the edge-shape kernel.
+ * forward, [I,D] in the input gradient - and of 64 otherwise), 0 neither: the edge-shape kernel, or, for a
+ * forward of up to 128 tokens with I >= 8, the weight-streaming kernel's form for rows of any alignment.
  * step: 0 forward, 1 input_grad, 2 weight_grad, 3 gating_grad_recompute, 4 / 5 / 6 down projection forward /
  * input gradient / weight gradient, each optionally | FSW_WEIGHTS_OUT_IN.  ldx: the [T,D] arrays, ldw: the
  * weights, ldo: the [T,I] arrays, ld_grad: grad_x or the weight gradient.  Pure host logic. */

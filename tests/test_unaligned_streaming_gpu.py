@@ -62,9 +62,11 @@ def test_against_float64(T, D, I, oi):
 
 
 @pytest.mark.parametrize("oi", [False, True], ids=["DI", "ID"])
-@pytest.mark.parametrize("T,D,I", [(8, 2047, 5001), (128, 1023, 2730), (129, 1023, 2730)])
+@pytest.mark.parametrize("T,D,I", [(5, 1023, 3071), (6, 1023, 3071), (8, 2047, 5001), (128, 1023, 2730), (129, 1023, 2730)])
 def test_padded_copies_stay_alike(T, D, I, oi):
-    """Calls that the launchers copy into padded rows first: the same bits with and without pre-activations, native and general"""
+    """Calls that the launchers copy into padded rows first, and on the other side of that rule's limit one that streams its rows
+    as they are: the same bits with and without pre-activations, native and general"""
+    assert (T * D * I >= _launch._PAD_MIN_WORK) == (T > 5)
     torch.manual_seed(T)
     x = torch.randn(T, D, device=DEV).bfloat16()
     wg, wu = ((torch.randn(*((I, D) if oi else (D, I)), device=DEV) * D ** -0.5).bfloat16() for _ in range(2))
