@@ -610,10 +610,19 @@ PyObject* py_setup(PyObject*, PyObject* args) {
   Py_RETURN_NONE;
 }
 
+// pads_rows(T, D, I, backward) -> bool, for the test that holds it against the rule in Python
+PyObject* py_pads_rows(PyObject*, PyObject* args) {
+  long long T, D, I;
+  int backward;
+  if (!PyArg_ParseTuple(args, "LLLp", &T, &D, &I, &backward)) return nullptr;
+  return PyBool_FromLong(pads_rows(T, D, I, backward));
+}
+
 PyMethodDef methods[] = {
     {"swiglu", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_swiglu)), METH_FASTCALL, nullptr},
     {"down_proj", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_down_proj)), METH_FASTCALL, nullptr},
     {"setup", py_setup, METH_VARARGS, nullptr},
+    {"pads_rows", py_pads_rows, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_fsw_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

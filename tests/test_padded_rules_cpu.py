@@ -175,3 +175,22 @@ def test_short_reductions_stay_on_the_edge_kernel(recorded, T, D, I, padded, oi)
             recorded.calls.clear()
             ops._swiglu_backward(dy, x, w, w, saved, saved, True, True, True, True, oi)
             assert {p for _, _, p in recorded.calls} == {True}
+
+
+def test_native_rule_is_the_same():
+    """The native host path keeps its own copy of pads_rows: the same answer on both sides of every limit."""
+    import random
+
+    from fusedswiglu_amd import _host
+
+    rng = random.Random(0)
+    native, work = _host.load().pads_rows, _launch._PAD_MIN_WORK
+    for _ in range(20000):
+        D, I = (max(1, round(2 ** rng.uniform(0, 13))) for _ in range(2))
+        T = max(1, work // (D * I) + rng.choice([-1, 0, 1])) if rng.random() < 0.3 else max(1, round(2 ** rng.uniform(0, 15)))
+        if rng.random() < 0.1:
+            D, I = rng.sample([D, MAX_LD - 8 + rng.choice([-1, 0, 1])], 2)
+        assert native(T, D, I, False) == _launch.pads_rows(T, D, I, (T, I, D)), (T, D, I)
+        assert native(T, D, I, True) == _launch.pads_rows(T, D, I, *_launch.backward_products(T, D, I)), (T, D, I)
+    seen = {native(T, D, I, b) for T, D, I in ((5, 1023, 3071), (6, 1023, 3071), (256, 257, 693), (256, 641, 1731)) for b in (False, True)}
+    assert seen == {False, True}
